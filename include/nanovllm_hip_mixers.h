@@ -495,6 +495,38 @@ NV_API int nv_fixed_decay_memory(const void* q, const void* k, const void* v, in
                                  void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * The gated delta rule, the generalized delta rule and the gated-write memory with what is known of the step, so that each kind
+ * of portion gets its own launch: T rows in all, leading_singles sequences with one row each in front of the batch, `portions`
+ * as above for the sequences behind them.  Single tokens stream their states; longer portions run in chunks on the matrix cores
+ * (D 32, 64, 96 or 128, Dv a multiple of 16, D * Dv <= 16384) through a workspace of nv_recurrence_workspace_bytes (form: 0 gated
+ * delta, 1 generalized delta, 2 gated write).  Other sizes, or no workspace (NULL): as the entry points above, token by token.
+ */
+NV_API int64_t nv_recurrence_workspace_bytes(int form, int64_t T, int H, int D, int Dv, int num_seqs, int leading_singles,
+                                             int dtype);
+NV_API int nv_gated_delta_rule_portions(const void* q, const void* k, const void* v, int64_t q_stride, int64_t k_stride,
+                                        int64_t v_stride, const void* a_raw, int64_t a_stride, const void* b_raw,
+                                        int64_t b_stride, const void* gate_raw, int64_t gate_stride, const float* A_log,
+                                        const float* dt_bias, const float* norm_w, float* state, void* out,
+                                        int64_t out_stride, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                                        const int32_t* state_slots, int num_seqs, int64_t T, int H, int G, int D, int Dv,
+                                        float eps, int leading_singles, int portions, int dtype, void* workspace,
+                                        int64_t workspace_bytes, void* stream);
+NV_API int nv_general_delta_rule_portions(const void* r, const void* k, const void* v, int64_t r_stride, int64_t k_stride,
+                                          int64_t v_stride, const void* w_raw, int64_t w_stride, const void* a_raw,
+                                          int64_t a_stride, const void* gate_raw, int64_t gate_stride, const float* w_bias,
+                                          const float* a_bias, const float* norm_w, float* state, void* out,
+                                          int64_t out_stride, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                                          const int32_t* state_slots, int num_seqs, int64_t T, int H, int D, float eps,
+                                          float decay_rate, float key_eps, int leading_singles, int portions, int dtype,
+                                          void* workspace, int64_t workspace_bytes, void* stream);
+NV_API int nv_gated_write_memory_portions(const void* q, const void* f_raw, const void* v, int64_t q_stride, int64_t f_stride,
+                                          int64_t v_stride, const float* f_bias, const float* lower, const float* norm_w,
+                                          float* state, void* out, int64_t out_stride, const int32_t* cu_seqlens_q,
+                                          const int32_t* cu_seqlens_k, const int32_t* state_slots, int num_seqs, int64_t T,
+                                          int H, int Dk, int Dv, float eps, int leading_singles, int portions, int dtype,
+                                          void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * In front of nv_attn_scoremod_paged: q [T, H * D] and k [T, G * D] are RMS-normed over the whole row (one weight per column),
  * rotated on the first rot_dims dimensions of every head (pair (i, i + rot_dims/2) by position * freq[i], cos and sin times
  * magnitude); q_out [T, H, D] contiguous, k and v [T, G * Dv] scattered into the paged caches (slot < 0: skipped).

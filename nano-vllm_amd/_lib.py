@@ -12,7 +12,7 @@ import threading
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libnanovllm_hip.so")
 MIXERS_LIB_PATH = os.path.join(_HERE, "lib", "libnanovllm_hip_mixers.so")
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 _vp, _i32, _i64, _f32 = C.c_void_p, C.c_int, C.c_int64, C.c_float
 
@@ -142,6 +142,15 @@ MIXERS_PROTOTYPES = {
     "nv_selective_scan_workspace_bytes": (_i64, [_i32, _i64, _i32, _i32, _i32, _i32]),
     "nv_selective_scan": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _vp,
                                  _vp, _i32, _i64, _i32, _i32, _i32, _i32, _i32, _vp, _i64, _vp]),
+    "nv_recurrence_workspace_bytes": (_i64, [_i32, _i64, _i32, _i32, _i32, _i32, _i32, _i32]),
+    "nv_gated_delta_rule_portions": (_i32, [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp,
+                                            _vp, _vp, _i64, _vp, _vp, _vp, _i32, _i64, _i32, _i32, _i32, _i32, _f32, _i32, _i32,
+                                            _i32, _vp, _i64, _vp]),
+    "nv_general_delta_rule_portions": (_i32, [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp,
+                                              _vp, _vp, _i64, _vp, _vp, _vp, _i32, _i64, _i32, _i32, _f32, _f32, _f32, _i32,
+                                              _i32, _i32, _vp, _i64, _vp]),
+    "nv_gated_write_memory_portions": (_i32, [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp,
+                                              _i32, _i64, _i32, _i32, _i32, _f32, _i32, _i32, _i32, _vp, _i64, _vp]),
     "nv_fixed_decay_workspace_bytes": (_i64, [_i32, _i64, _i32, _i32, _i32, _i32, _i32, _i32]),
     "nv_fixed_decay_memory": (_i32, [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _i32, _i64, _i32, _i32,
                                      _i32, _i32, _i32, _i32, _i32, _vp, _i64, _vp]),

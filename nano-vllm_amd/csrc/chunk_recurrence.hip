@@ -1,0 +1,920 @@
+// Recurrences whose memory S [D, Dv] (key channel x value channel, fp32) decays with one factor per key channel and is
+// rewritten along its own read-out.  Three forms; x0 .. x3 are the raw projections, everything after them is fp32:
+//
+//   gated    (x0 = q, x1 = k, x2 = a_raw)   k, q unit vectors (q times D^-1/2);  w = exp(-exp(c0_h) softplus(x2 + c1))
+//            S <- diag(w) S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q
+//   general  (x0 = r, x1 = k, x2 = w_raw, x3 = a_raw)   u = k / |k|;  w = exp(-p0 sigmoid(x2 + c0));  a = sigmoid(x3 + c1)
+//            S <- diag(w) S - (a u)(u^T S) + k v^T  (both terms read the old state);  o = S^T r
+//   write    (x0 = q, x1 = f_raw)   w = c1 + (1 - c1) sigmoid(x1 + c0);  k = 1 - w;  S <- diag(w) S + k v^T;  o = S^T silu(q)
+//
+// A token-by-token loop is bound by its serial chain (one pass over the state a token and the LDS reads of the token's vectors
+// by every lane), so portions run in CHUNKS of 8 tokens.  With G_t the product of the decays from the chunk's start through
+// token t, and S the state in front of the chunk, each form is
+//
+//   C = [K; Q] S        16 rows: what the tokens' k (u) and q (r) find in S, K_t = k_t G_t (general: u_t G_(t-1)), Q_t = q_t G_t
+//   [U; O] = M C + M2 V 16 x 16 and 16 x 8 matrices of the chunk alone: the tokens' influence on each other, solved
+//   S <- diag(G_8) S + K^^T V (general, write) + X^^T U (gated, general),   K^_t = k_t G_8 / G_t
+//
+// (write has no U and no M: O = C + M2 V).  M and M2 come from the pair products P_ts = sum_d l_t,d r_s,d G_t / G_s, s <= t, and
+// the inverse of a unit lower triangular 8 x 8 matrix by forward substitution.  All large products are
+// v_mfma_f32_16x16x4_f32: operands and sums stay fp32.
+//
+// G_t / G_s does not factor through one reference without overflow when a channel decays fast, so both sides are taken relative
+// to the middle of the chunk: four factors on either side.  There the factors are held above 2^-25: the largest product is
+// 2^100, and a ratio that holding changes is one of numbers below 2^-25 in front of sums whose rounding is 2^-24.
+//
+// Two launches: the first makes every chunk's operands (a wave per chunk and head, all chunks at once), the second walks the
+// chunks of a (sequence, head, 16 value columns) with the state in MFMA accumulators (128 channels: 32 registers) and reads the
+// operands from memory in the order of its lanes.  fp32 MFMAs run on the vector units, so waves that prepared operands beside
+// them (one launch, everything through LDS) took the same issue slots: 653 us instead of 284 on gated, 4 prompts of 1501 .. 2048 tokens,
+// 16 heads 128 x 128.
+// Accumulators of one product are the operand of the next in place: a lane holds rows 4 g + e (g: its group of 16 lanes), so
+// MFMA e of a tile contracts the four rows {4 g + e}, and the other operand is read in that order (16 bytes a lane).  U comes out
+// in the lower half of the lanes; two v_permlane32_swap spread its 8 rows over all four groups, so that an update of a 16-channel
+// tile takes two MFMAs.  The chunk takes 54 (gated) / 70 (general) / 50 (write) MFMAs of 32 cycles per 16 columns of 128 channels.
+//
+// Measured against the token-by-token launches (16 heads 128 x 128, bf16 rows), whole call: gated, 4 prompts of 1501 .. 2048 tokens
+// 3123 -> 284 us; general, 3 prompts of 700 .. 2000: 3645 -> 290; write, 8 chunks of 509 over carried states: 431 -> 117; gated, 256
+// single tokens: 393 -> 112 (4.8 TB/s of states, what a large copy reaches).  Of the 284 us the second launch is 219, 257 chunks
+// in a row at 0.85 us: 0.43 us of MFMAs, the rest the chain of exchange, M and update between them.
+//
+// The read-outs go to a scratch of fp32 rows, because a row's norm spans the workgroups of its value columns; a last launch
+// norms, weights and gates them.  Single tokens run in a launch of their own that streams every state once.
+#include <type_traits>
+
+#include "chunk_recurrence.h"
+#include "row_pieces.h"
+#include "../../include/nanovllm_hip_mixers.h"
+
+namespace nv {
+
+constexpr int kCrChunk = 8;
+constexpr float kCrHold = 2.98023224e-8f;             // 2^-25
+constexpr float kCrLog2e = 1.4426950408889634f, kCrLn2 = 0.6931471805599453f;
+
+__device__ __forceinline__ float cr_exp(float x) { return __builtin_amdgcn_exp2f(x * kCrLog2e); }
+__device__ __forceinline__ float cr_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
+// log(1 + exp(x)) = max(x, 0) + log1p(u), u = exp(-|x|); log1p(u) = u log(w) / (w - 1) with w = 1 + u rounded (the rounding
+// of w cancels: D. Goldberg, "What Every Computer Scientist Should Know About Floating-Point Arithmetic", theorem 4).
+__device__ __forceinline__ float cr_softplus(float x) {
+    const float u = cr_exp(-fabsf(x)), w = 1.0f + u, d = w - 1.0f;
+    const float l = d == 0.f ? u : __builtin_amdgcn_logf(w) * kCrLn2 * (u * __builtin_amdgcn_rcpf(d));
+    return fmaxf(x, 0.f) + l;
+}
+
+// Decay and vectors of one token and channel from its raw projections (x: in the order of x0 .. x3).
+struct CrElem {
+    float w, k, q, a;                                 // decay; k (raw scale); q / r; removal rate times k (general)
+};
+template <int FORM>
+__device__ __forceinline__ CrElem cr_elem(const float* x, float c0, float c1, float p0) {
+    CrElem e;
+    if constexpr (FORM == kCrGated) {
+        e.w = cr_exp(-c0 * cr_softplus(x[2] + c1));   // c0: exp(A_log)
+        e.k = x[1];
+        e.q = x[0];
+        e.a = 0.f;
+    } else if constexpr (FORM == kCrGeneral) {
+        e.w = cr_exp(-p0 * cr_sigmoid(x[2] + c0));
+        e.k = x[1];
+        e.q = x[0];
+        e.a = cr_sigmoid(x[3] + c1) * x[1];
+    } else {
+        e.w = c1 + (1.0f - c1) * cr_sigmoid(x[1] + c0);
+        e.k = 1.0f - e.w;
+        e.q = x[0] * cr_sigmoid(x[0]);
+        e.a = 0.f;
+    }
+    return e;
+}
+
+// An element on its way from memory in a register of its own: packed halves would make every load wait for the one before.
+template <typename T> struct CrRaw;
+template <> struct CrRaw<__bf16> {
+    typedef uint32_t type;
+    static __device__ __forceinline__ uint32_t load(const __bf16* p) { return *(const uint16_t*)p; }
+    static __device__ __forceinline__ float value(uint32_t r) { return __builtin_bit_cast(float, r << 16); }
+};
+// Two neighbouring elements by one load (VEC) or two.
+template <typename T, bool VEC> struct CrPair;
+template <> struct CrPair<__bf16, true> {
+    uint32_t r;
+    __device__ __forceinline__ void load(const __bf16* p) { r = *(const uint32_t*)p; }
+    __device__ __forceinline__ float value(int i) const { return i ? bf16_hi(r) : bf16_lo(r); }
+    __device__ __forceinline__ void store(__bf16* p, bool in) const { *(uint32_t*)p = in ? r : 0u; }
+};
+template <> struct CrPair<float, true> {
+    float2 r;
+    __device__ __forceinline__ void load(const float* p) { r = *(const float2*)p; }
+    __device__ __forceinline__ float value(int i) const { return i ? r.y : r.x; }
+    __device__ __forceinline__ void store(float* p, bool in) const { *(float2*)p = in ? r : make_float2(0.f, 0.f); }
+};
+template <typename T> struct CrPair<T, false> {
+    typename CrRaw<T>::type r[2];
+    __device__ __forceinline__ void load(const T* p) {
+        r[0] = CrRaw<T>::load(p);
+        r[1] = CrRaw<T>::load(p + 1);
+    }
+    __device__ __forceinline__ float value(int i) const { return CrRaw<T>::value(r[i]); }
+    __device__ __forceinline__ void store(T* p, bool in) const {
+        p[0] = in ? (T)value(0) : (T)0.f;
+        p[1] = in ? (T)value(1) : (T)0.f;
+    }
+};
+template <> struct CrRaw<float> {
+    typedef float type;
+    static __device__ __forceinline__ float load(const float* p) { return *p; }
+    static __device__ __forceinline__ float value(float r) { return r; }
+};
+
+__device__ __forceinline__ f32x4 cr_mfma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ float cr_lane(float x, int lane) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
+}
+// The lower half's `lo` in the lower half of the lanes, the lower half's `hi` in the upper one.
+__device__ __forceinline__ float cr_spread(float lo, float hi) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, lo), __builtin_bit_cast(int, hi), false, false)[0]);
+}
+// LDS writes of this wave / of the workgroup's waves are done; loads from memory stay in flight.
+__device__ __forceinline__ void cr_wave_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ void cr_group_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// PER neighbouring elements of a row of V by one load.
+template <typename T, int PER> struct CrColumns : CrPair<T, true> {};
+template <typename T> struct CrColumns<T, 1> {
+    typename CrRaw<T>::type r;
+    __device__ __forceinline__ void load(const T* p) { r = CrRaw<T>::load(p); }
+    __device__ __forceinline__ float value(int) const { return CrRaw<T>::value(r); }
+};
+
+// Where a chunk's operands lie in the workspace: one record per (head, chunk), in the order in which the lanes of the second
+// launch read them, a head's chunks one after the other, beside them the chunks' rows of V ([head][record][8][Dv], zeros past the
+// sequence's end); read-outs are [head][row][Dv] too.  The second launch has few loads in flight, so streams that stay within a page
+// for several chunks matter to it (heads side by side, every chunk on pages of its own: 302 us instead of 264).  Records of a sequence start at (first row + 7 x its number) / 8: enough for the chunks in front, whatever
+// the lengths, without a scan over them.
+template <int FORM, int D>
+struct CrRecord {
+    static constexpr int kRows = FORM == kCrWrite ? 8 : 16;       // of [K; Q]: write has no K
+    static constexpr int kUpd = FORM == kCrGeneral ? 2 : 1;       // update operands: K^ and / or X^
+    static constexpr int kq = 0;                                  // [tile][g][row][4 channels]
+    static constexpr int upd = kq + kRows * D;                    // [operand][tile][g][channel][2 tokens]
+    static constexpr int decay = upd + kUpd * 8 * D;              // [channel]
+    static constexpr int m = decay + D;                           // [16][16]
+    static constexpr int m2 = m + (FORM == kCrWrite ? 0 : 256);   // [16][8] (write: [8][8])
+    static constexpr int words = m2 + 8 * kRows;
+};
+// (rows and numbers counted from the first sequence of the launch)
+__device__ __host__ __forceinline__ int64_t cr_first_record(int64_t first_row, int seq) { return (first_row + 7LL * seq) / 8; }
+
+// ------------------------------------------------------------------------------------------------ first launch
+// A wave per (chunk, head); a lane owns two neighbouring channels and all 8 tokens, so running products need no exchange.  LDS
+// (the wave's own) only turns the pair products' operands and [K; Q] into the order of the matrix cores.
+template <typename T, int FORM, int D>
+struct CrPrepLds {
+    static constexpr int kRow = D + 4;                            // rows of D channels start on different banks
+    static constexpr int kRight = FORM == kCrGeneral ? 16 : 8;
+    float left[16 * kRow], right[kRight * kRow];                  // pair products' operands; then left holds [K; Q]
+};
+
+template <typename T, int FORM, int D, bool VEC>
+__global__ __launch_bounds__(256) void recurrence_chunks_kernel(const ChunkRecurrenceArgs a, const int first_seq) {
+    constexpr int NM = D / 16, NX = FORM == kCrGated ? 3 : FORM == kCrGeneral ? 4 : 2;
+    typedef CrPrepLds<T, FORM, D> Lds;
+    typedef CrRecord<FORM, D> Rec;
+    typedef CrRaw<T> In;
+    constexpr int ROW = Lds::kRow;
+    __shared__ __attribute__((aligned(16))) Lds all[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, g = lane >> 4, h = blockIdx.y * 4 + wave;
+    const int64_t rec = blockIdx.x;
+    const int row0 = a.cu_q[first_seq];
+    int lo = first_seq, hi = a.num_seqs;              // the last sequence whose records start at or in front of this one
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (cr_first_record(a.cu_q[mid] - row0, mid - first_seq) <= rec) lo = mid; else hi = mid;
+    }
+    const int b = lo, q0 = a.cu_q[b], len = a.cu_q[b + 1] - q0;
+    const int64_t c64 = rec - cr_first_record(q0 - row0, b - first_seq);
+    if (len < 2 || c64 * kCrChunk >= len || h >= a.H) return;
+    const int t0 = q0 + (int)c64 * kCrChunk, n = min(kCrChunk, q0 + len - t0);
+    float* out = a.chunks + (h * a.records + rec) * Rec::words;
+    Lds& lds = all[wave];
+
+    const bool in_row = 2 * lane < D;
+    const int d = in_row ? 2 * lane : 0;
+    CrPair<T, VEC> raw[NX][8];
+    {
+        const void* xs[4] = {a.x0, a.x1, a.x2, a.x3};
+        const int64_t ss[4] = {a.s0, a.s1, a.s2, a.s3};
+#pragma unroll
+        for (int j = 0; j < NX; ++j) {
+            const int hj = (FORM == kCrGated && j < 2) ? h / a.group : h;
+            const T* p = (const T*)xs[j] + (int64_t)t0 * ss[j] + (int64_t)hj * D;
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {             // (past the end: the chunk's first row, dropped below)
+                const T* row = p + (t < n ? t : 0) * ss[j];
+                raw[j][t].load(row + d);
+            }
+        }
+    }
+    {
+        const T* v = (const T*)a.v + (int64_t)t0 * a.sv + (int64_t)h * a.Dv;
+        T* to = (T*)a.columns + (h * a.records + rec) * 8 * a.Dv;
+        for (int c = 2 * lane; c < a.Dv; c += 128) {
+            CrPair<T, VEC> r[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) r[t].load(v + (t < n ? t : 0) * a.sv + c);
+#pragma unroll
+            for (int t = 0; t < 8; ++t) r[t].store(to + t * a.Dv + c, t < n);
+        }
+    }
+    float beta = 0.f;                                 // raw, of token lane % 8
+    if constexpr (FORM == kCrGated) beta = CrRaw<T>::value(In::load((const T*)a.b_raw + (int64_t)(t0 + min(lane & 7, n - 1)) * a.b_stride + h));
+    float c0[2], c1[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        c0[i] = FORM == kCrGated ? expf(a.c0[h]) : a.c0[h * D + d + i];
+        c1[i] = a.c1[h * D + d + i];
+    }
+    CrElem el[8][2];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            float in[4];
+#pragma unroll
+            for (int j = 0; j < NX; ++j) in[j] = raw[j][t].value(i);
+            el[t][i] = cr_elem<FORM>(in, c0[i], c1[i], a.p0);
+            if (t >= n || !in_row) el[t][i] = CrElem{1.f, 0.f, 0.f, 0.f};
+        }
+    }
+    float kk = 0.f, qq = 0.f;                         // sums of squares of token lane % 8
+    if constexpr (FORM != kCrWrite) {
+        auto squares = [&](auto of) {                 // 8 tokens' sums over 64 lanes: halved three times over the lanes, then summed
+            float s[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) s[t] = of(t);
+            const bool o1 = lane & 1, o2 = lane & 2, o4 = lane & 4;
+            float u[4], w[2];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) u[t] = (o1 ? s[2 * t + 1] : s[2 * t]) + dpp_f32<0xB1>(o1 ? s[2 * t] : s[2 * t + 1]);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) w[t] = (o2 ? u[2 * t + 1] : u[2 * t]) + dpp_f32<0x4E>(o2 ? u[2 * t] : u[2 * t + 1]);
+            float r = (o4 ? w[1] : w[0]) + __shfl_xor(o4 ? w[0] : w[1], 4);
+            r += __shfl_xor(r, 8);
+            r += __shfl_xor(r, 16);
+            return r + __shfl_xor(r, 32);
+        };
+        kk = squares([&](int t) { return el[t][0].k * el[t][0].k + el[t][1].k * el[t][1].k; });
+        if constexpr (FORM == kCrGated) qq = squares([&](int t) { return el[t][0].q * el[t][0].q + el[t][1].q * el[t][1].q; });
+    }
+    // ---- relative to the middle: left sides G_t / G_4, right sides G_4 / G_t, factors held above 2^-25
+    float held[2][8];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        held[i][3] = 1.f;                             // of tokens 0 .. 3: products behind the token; 4 .. 7: through the token
+#pragma unroll
+        for (int t = 2; t >= 0; --t) held[i][t] = held[i][t + 1] * fmaxf(el[t + 1][i].w, kCrHold);
+        held[i][4] = fmaxf(el[4][i].w, kCrHold);
+#pragma unroll
+        for (int t = 5; t < 8; ++t) held[i][t] = held[i][t - 1] * fmaxf(el[t][i].w, kCrHold);
+    }
+    if (in_row) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            float lv[2], rv[2], hb[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const float inv = __builtin_amdgcn_rcpf(held[i][t]);
+                lv[i] = t < 4 ? inv : held[i][t];
+                rv[i] = t < 4 ? held[i][t] : inv;
+                if constexpr (FORM == kCrGeneral)     // the old state: through the token before
+                    hb[i] = t == 0 ? __builtin_amdgcn_rcpf(held[i][0] * fmaxf(el[0][i].w, kCrHold))
+                                   : t < 4 ? __builtin_amdgcn_rcpf(held[i][t - 1]) : t == 4 ? 1.f : held[i][t - 1];
+                else hb[i] = lv[i];
+            }
+            if constexpr (FORM != kCrWrite) *(float2*)(lds.left + t * ROW + d) = make_float2(el[t][0].k * hb[0], el[t][1].k * hb[1]);
+            *(float2*)(lds.left + (8 + t) * ROW + d) = make_float2(el[t][0].q * lv[0], el[t][1].q * lv[1]);
+            *(float2*)(lds.right + t * ROW + d) = make_float2(el[t][0].k * rv[0], el[t][1].k * rv[1]);
+            if constexpr (FORM == kCrGeneral)
+                *(float2*)(lds.right + (8 + t) * ROW + d) = make_float2(el[t][0].a * rv[0], el[t][1].a * rv[1]);
+        }
+    }
+    cr_wave_sync();
+    f32x4 p = {0.f, 0.f, 0.f, 0.f}, p1 = p;           // entry (row 4 g + e, column l16): rows k | q, columns k | a k
+    {
+        const int lrow = FORM == kCrWrite ? (8 + (l16 & 7)) : l16;
+        const float* lf = lds.left + lrow * ROW + 4 * g;
+        const float* rt = lds.right + (Lds::kRight == 16 ? l16 : (l16 & 7)) * ROW + 4 * g;
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            const f32x4 x = *(const f32x4*)(lf + 16 * m), y = *(const f32x4*)(rt + 16 * m);
+            p = cr_mfma(x[0], y[0], p);
+            p1 = cr_mfma(x[1], y[1], p1);
+            p = cr_mfma(x[2], y[2], p);
+            p1 = cr_mfma(x[3], y[3], p1);
+        }
+    }
+    p += p1;
+    // ---- [K; Q], K^, X^ and the chunk's decay
+    float G[2][8], F[2][8];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        G[i][0] = el[0][i].w;
+        F[i][7] = 1.f;
+#pragma unroll
+        for (int t = 1; t < 8; ++t) {
+            G[i][t] = G[i][t - 1] * el[t][i].w;
+            F[i][7 - t] = F[i][8 - t] * el[8 - t][i].w;
+        }
+    }
+    cr_wave_sync();
+    if (in_row) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            if constexpr (FORM == kCrGated)
+                *(float2*)(lds.left + t * ROW + d) = make_float2(el[t][0].k * G[0][t], el[t][1].k * G[1][t]);
+            if constexpr (FORM == kCrGeneral)
+                *(float2*)(lds.left + t * ROW + d) = make_float2(t ? el[t][0].k * G[0][t ? t - 1 : 0] : el[t][0].k,
+                                                                 t ? el[t][1].k * G[1][t ? t - 1 : 0] : el[t][1].k);
+            *(float2*)(lds.left + (8 + t) * ROW + d) = make_float2(el[t][0].q * G[0][t], el[t][1].q * G[1][t]);
+        }
+        *(float2*)(out + Rec::decay + d) = make_float2(G[0][7], G[1][7]);
+        // token pairs in the order of the lane groups that supply them: of V 0 1 | 2 3 | 4 5 | 6 7, of U 0 1 | 4 5 | 2 3 | 6 7
+        auto store = [&](int which, auto of, bool u) {
+#pragma unroll
+            for (int pos = 0; pos < 4; ++pos) {
+                const int t = u ? (pos == 1 ? 4 : pos == 2 ? 2 : 2 * pos) : 2 * pos;
+                float* to = out + Rec::upd + which * 8 * D + (((d >> 4) * 4 + pos) * 16 + (d & 15)) * 2;
+                *(f32x4*)to = f32x4{of(t, 0) * F[0][t], of(t + 1, 0) * F[0][t + 1], of(t, 1) * F[1][t], of(t + 1, 1) * F[1][t + 1]};
+            }
+        };
+        if constexpr (FORM == kCrGated) store(0, [&](int t, int i) { return el[t][i].k; }, true);
+        else store(0, [&](int t, int i) { return el[t][i].k; }, false);
+        if constexpr (FORM == kCrGeneral) store(1, [&](int t, int i) { return el[t][i].a; }, true);
+    }
+    cr_wave_sync();
+    if constexpr (FORM == kCrWrite) {
+        // lanes: (tile, g, row) of 8 rows, 16 bytes each
+#pragma unroll
+        for (int i = 0; i < NM / 2; ++i) {
+            const int at = i * 64 + lane;             // tile at / 32, g (at / 8) % 4, row at % 8
+            *(f32x4*)(out + Rec::kq + at * 4) = *(const f32x4*)(lds.left + (8 + (at & 7)) * ROW + 16 * (at >> 5) + 4 * ((at >> 3) & 3));
+        }
+    } else {
+#pragma unroll
+        for (int m = 0; m < NM; ++m) *(f32x4*)(out + Rec::kq + (m * 64 + lane) * 4) = *(const f32x4*)(lds.left + l16 * ROW + 16 * m + 4 * g);
+    }
+    // ---- M and M2
+    float* m = out + Rec::m;
+    float* m2 = out + Rec::m2;
+    if constexpr (FORM == kCrWrite) {
+        if (g < 2 && l16 < 8) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) m2[(4 * g + e) * 8 + l16] = l16 <= 4 * g + e ? p[e] : 0.f;
+        }
+        return;
+    }
+    const int j = lane & 7;
+    const bool in = j < n;
+    const float kn = in ? 1.0f / sqrtf(kk + a.p1) : 0.f;                               // of token lane % 8
+    const float qn = FORM == kCrGated ? 1.0f / sqrtf((qq + a.p1) * (float)D) : 1.0f;
+    // Lanes 0 - 7: columns of M for the rows K; lanes 8 - 15: columns of M2; lanes 16 - 23: columns of M for the rows Q.
+    const int kind = lane >> 3;
+    float y[8], o[8];
+    if constexpr (FORM == kCrGated) {
+        // u = T beta (v - kn K^T S), T = (I + A)^-1, A_ts = beta_t kn_t kn_s P_ts (s < t);  y_t = kn_t u_t is what X^ = k G_8 / G_t
+        // takes, o_t = qn_t (Q^T S + sum_(s <= t) P'_ts y_s)
+        beta = in ? cr_sigmoid(beta) : 0.f;
+        const float rhs = kind == 0 ? -beta * kn * kn : kind == 1 ? beta * kn : 0.f;
+        const float scale = beta * kn * kn;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            float s = 0.f;
+#pragma unroll
+            for (int i = 0; i < t; ++i) s += cr_lane(p[t & 3], (t >> 2) * 16 + i) * y[i];
+            y[t] = (t == j ? rhs : 0.f) - cr_lane(scale, t) * s;
+        }
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            float s = (kind == 2 && t == j) ? 1.f : 0.f;
+#pragma unroll
+            for (int i = 0; i <= t; ++i) s += cr_lane(p[t & 3], (2 + (t >> 2)) * 16 + i) * y[i];
+            o[t] = s * cr_lane(qn, t);
+        }
+    } else {
+        // x_t = u_t^T S_(t-1) = kn_t (K^T S + sum_(s < t) P_ts(k, k) v_s - P_ts(k, a k) kn_s x_s);  y_t = kn_t x_t, taken with
+        // a minus sign by X^ = a k G_8 / G_t;  o_t = Q^T S + sum_(s <= t) P_ts(r, k) v_s - P_ts(r, a k) y_s
+        const float kn2 = kn * kn;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const float nt = __shfl(p[t & 3], (t >> 2) * 16 + j);
+            float s = kind == 0 ? (t == j ? 1.f : 0.f) : kind == 1 ? (t > j ? nt : 0.f) : 0.f;
+#pragma unroll
+            for (int i = 0; i < t; ++i) s -= cr_lane(p[t & 3], (t >> 2) * 16 + 8 + i) * y[i];
+            y[t] = cr_lane(kn2, t) * s;
+        }
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const float bt = __shfl(p[t & 3], (2 + (t >> 2)) * 16 + j);
+            float s = kind == 2 ? (t == j ? 1.f : 0.f) : kind == 1 ? (t >= j ? bt : 0.f) : 0.f;
+#pragma unroll
+            for (int i = 0; i <= t; ++i) s -= cr_lane(p[t & 3], (2 + (t >> 2)) * 16 + 8 + i) * y[i];
+            o[t] = s;
+        }
+    }
+    if (kind < 3) {
+        float* to = kind == 1 ? m2 + j : m + (kind == 2 ? 8 : 0) + j;
+        const int ld = kind == 1 ? 8 : 16;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            to[t * ld] = FORM == kCrGeneral ? -y[t] : y[t];
+            to[(8 + t) * ld] = o[t];
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------------ second launch
+// RS waves per (sequence, head, 16 value columns), each with D / RS key channels of the state in MFMA accumulators; RS = 2: the
+// waves' parts of [K; Q] S are exchanged through LDS.  A workgroup has four of these waves, one on each SIMD of a CU, and four that
+// do nothing but move: records and columns of V four chunks ahead into registers and two ahead into LDS (three slots), read-outs from LDS to
+// memory.  One barrier a chunk.  The products alone are bound by their chain (product, exchange, M, update); with the loads and
+// stores in the same waves every chunk also paid for their issue (gated, 4 x 1501 .. 2048 tokens, 16 heads: 264 us instead of 219).
+template <typename T, int FORM, int D, int RS>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void recurrence_states_kernel(
+    const ChunkRecurrenceArgs a, const int first_seq) {
+    constexpr int NM = D / 16 / RS;                   // tiles of a wave
+    typedef CrRecord<FORM, D> Rec;
+    constexpr int ROUNDS = (Rec::words + 1023) / 1024;
+    constexpr int COLS = 64 / RS, PER = 2 / RS;       // value columns of the workgroup; elements of a row of V a thread moves
+    __shared__ __attribute__((aligned(16))) float slots[3][Rec::words];
+    __shared__ __attribute__((aligned(8))) float vs[3][kCrChunk][COLS], os[2][kCrChunk][COLS];
+    __shared__ f32x4 part[RS == 1 ? 1 : 2][4][64];
+    // Workgroups go to the eight XCDs in turn: an XCD takes neighbouring heads.
+    const int pair = gridDim.x % 8 == 0 ? (int)(blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8) : (int)blockIdx.x;
+    const int b = first_seq + pair / a.H, h = pair % a.H;
+    const int q0 = a.cu_q[b], len = a.cu_q[b + 1] - q0;
+    if (len < 2) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int chunks = (len + kCrChunk - 1) / kCrChunk, Dv = a.Dv;
+
+    if (wave >= 4) {
+        // ---------------------------------------------------------------- the movers
+        const int tid = threadIdx.x - 256;
+        const int64_t first = (int64_t)h * a.records + cr_first_record(q0 - a.cu_q[first_seq], b - first_seq);
+        const float* rec = a.chunks + first * Rec::words;
+        const int tok = tid >> 5, col = (tid & 31) * PER, col_all = blockIdx.y * COLS + col;
+        // (columns past the end: the last ones, used by waves that write nothing)
+        const T* v = (const T*)a.columns + first * 8 * Dv + tok * Dv + min(col_all, Dv - PER);
+        float* o = a.raw + ((int64_t)h * a.T + q0 + tok) * Dv + col_all;
+        struct Staged {
+            f32x4 r[ROUNDS];
+            CrColumns<T, PER> v;
+        };
+        auto fetch = [&](int c, Staged& st) {
+            c = min(c, chunks - 1);
+            const float* rc = rec + (int64_t)c * Rec::words;
+            st.v.load(v + (int64_t)c * 8 * Dv);
+#pragma unroll
+            for (int i = 0; i < ROUNDS; ++i)
+                if ((i + 1) * 1024 <= Rec::words || i * 1024 + tid * 4 < Rec::words) st.r[i] = *(const f32x4*)(rc + (uint32_t)(i * 1024 + tid * 4));
+        };
+        auto stage = [&](int at, const Staged& st) {
+#pragma unroll
+            for (int e = 0; e < PER; ++e) vs[at][tok][col + e] = st.v.value(e);
+#pragma unroll
+            for (int i = 0; i < ROUNDS; ++i)
+                if ((i + 1) * 1024 <= Rec::words || i * 1024 + tid * 4 < Rec::words) *(f32x4*)(slots[at] + i * 1024 + tid * 4) = st.r[i];
+        };
+        auto store = [&](int c) {
+            if (c * kCrChunk + tok < len && col_all < Dv) {
+#pragma unroll
+                for (int e = 0; e < PER; ++e) o[(int64_t)c * kCrChunk * Dv + e] = os[c & 1][tok][col + e];
+            }
+        };
+        Staged s0, s1;
+        fetch(0, s0);
+        fetch(1, s1);
+        stage(0, s0);
+        stage(1, s1);
+        fetch(2, s0);
+        fetch(3, s1);
+        cr_group_barrier();
+        int at = 2, c = 0;
+        auto move = [&](int c, Staged& st) {          // behind the barrier of chunk c: st holds chunk c + 2 and takes c + 4
+            cr_group_barrier();
+            stage(at, st);
+            at = at == 2 ? 0 : at + 1;
+            fetch(c + 4, st);
+            if (c > 0) store(c - 1);
+        };
+        for (; c + 1 < chunks; c += 2) {              // (no way out of the middle: the waits at the loop's head stay exact)
+            move(c, s0);
+            move(c + 1, s1);
+        }
+        if (c < chunks) move(c, s0);
+        cr_group_barrier();
+        store(chunks - 1);
+        return;
+    }
+
+    // -------------------------------------------------------------------- the state
+    const int rp = wave % RS, l16 = lane & 15, g = lane >> 4, d0 = rp * (D / RS);
+    int tile = blockIdx.y * (4 / RS) + wave / RS;
+    const bool live = tile * 16 < Dv, fresh = a.cu_k[b + 1] - a.cu_k[b] == len;
+    if (!live) tile = 0;                              // (waves without columns repeat the first ones' and write nothing)
+    const int in_group = (wave / RS) * 16 + l16;
+    float* slot = a.state + ((int64_t)a.slots[b] * a.H + h) * (int64_t)D * Dv + (int64_t)(d0 + 4 * g) * Dv + tile * 16 + l16;
+    f32x4 S[NM];                                      // rows 4 g + e of the wave's tiles
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[m][e] = fresh ? 0.f : slot[(int64_t)(16 * m + e) * Dv];
+    }
+    const int at_kq = Rec::kq + (FORM == kCrWrite ? (g * 8 + (l16 & 7)) * 4 + d0 * 8 : lane * 4 + d0 * 16);
+    constexpr int kq_tile = 16 * Rec::kRows;
+    const int at_upd = Rec::upd + lane * 2 + d0 * 8, at_dec = Rec::decay + d0 + ((l16 + 4 * g) & 15), at_m = Rec::m + l16 * 16 + 4 * g;
+    const int at_m2 = Rec::m2 + (FORM == kCrWrite ? l16 & 7 : l16) * 8 + 2 * g;
+    f32x4 x[NM];
+    auto read_x = [&](int at) {
+#pragma unroll
+        for (int m = 0; m < NM; ++m) x[m] = *(const f32x4*)(slots[at] + kq_tile * m + at_kq);
+    };
+    cr_group_barrier();
+    read_x(0);
+    int at = 0;
+    for (int c = 0; c < chunks; ++c) {                // chunk c from slot `at`
+        const float* rc = slots[at];
+        f32x4 y;
+        float dec[NM];                                // lane e of group g: the decay of row 4 g + e of the tile
+        float2 uk[NM], ux[NM];
+        float vv[2];
+        const float2 y2 = *(const float2*)(rc + at_m2);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) vv[e] = vs[at][2 * g + e][in_group];
+        if constexpr (FORM != kCrWrite) y = *(const f32x4*)(rc + at_m);
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            dec[m] = rc[16 * m + at_dec];
+            if constexpr (FORM != kCrGated) uk[m] = *(const float2*)(rc + 128 * m + at_upd);
+            if constexpr (FORM != kCrWrite) ux[m] = *(const float2*)(rc + (Rec::kUpd - 1) * 8 * D + 128 * m + at_upd);
+        }
+        f32x4 c0 = {0.f, 0.f, 0.f, 0.f}, d = c0;
+        __builtin_amdgcn_sched_barrier(0);            // the reads are on their way before the products
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) c0 = cr_mfma(x[m][e], S[m][e], c0);
+        }
+        d = cr_mfma(y2.x, vv[0], d);
+        d = cr_mfma(y2.y, vv[1], d);
+        if constexpr (RS > 1) part[c & 1][wave][lane] = c0;
+        cr_group_barrier();                           // chunk c + 1 is in its slot; chunk c - 1's slot is free
+        f32x4 other;
+        if constexpr (RS > 1) other = part[c & 1][wave ^ 1][lane];
+        at = at == 2 ? 0 : at + 1;
+        read_x(at);
+        // the state moves on: rows 4 g + e of tile m decay, then take the chunk's writes
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            S[m][0] *= dpp_f32<0x150>(dec[m]);        // row_newbcast e: lane e of the group
+            S[m][1] *= dpp_f32<0x151>(dec[m]);
+            S[m][2] *= dpp_f32<0x152>(dec[m]);
+            S[m][3] *= dpp_f32<0x153>(dec[m]);
+        }
+        if constexpr (FORM != kCrGated) {
+#pragma unroll
+            for (int m = 0; m < NM; ++m) S[m] = cr_mfma(uk[m].x, vv[0], S[m]);
+#pragma unroll
+            for (int m = 0; m < NM; ++m) S[m] = cr_mfma(uk[m].y, vv[1], S[m]);
+        }
+        if constexpr (RS > 1) c0 += other;
+        if constexpr (FORM == kCrWrite) {
+            d += c0;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) d = cr_mfma(y[e], c0[e], d);
+            // tokens 0, 1 | 4, 5 of U sit in groups 0 | 1, tokens 2, 3 | 6, 7 move to groups 2 | 3
+            const float u0 = cr_spread(d[0], d[2]), u1 = cr_spread(d[1], d[3]);
+#pragma unroll
+            for (int m = 0; m < NM; ++m) S[m] = cr_mfma(ux[m].x, u0, S[m]);
+#pragma unroll
+            for (int m = 0; m < NM; ++m) S[m] = cr_mfma(ux[m].y, u1, S[m]);
+        }
+        // write: rows 0 - 7 of the products are the read-outs (8 - 15 repeat them), else rows 8 - 15
+        if (rp == 0 && (FORM == kCrWrite ? g < 2 : g >= 2)) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) os[c & 1][4 * (g & 1) + e][in_group] = d[e];
+        }
+    }
+    cr_group_barrier();
+    if (!live) return;
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) slot[(int64_t)(16 * m + e) * Dv] = S[m][e];
+    }
+}
+
+// ------------------------------------------------------------------------------------------------ read-outs
+// out = o / sqrt(mean(o^2) + eps) * norm_w * sigmoid(gate) per token and head; 16 lanes a row, pieces of four columns.  A workgroup
+// takes a token; SEARCH: tokens that are their sequence's only row are another launch's.
+template <typename T, bool VEC, bool SEARCH>
+__global__ __launch_bounds__(256) void recurrence_finish_kernel(const ChunkRecurrenceArgs a, const int first_seq) {
+    const int t = a.cu_q[first_seq] + blockIdx.x, l16 = threadIdx.x & 15;
+    if (t >= a.cu_q[a.num_seqs]) return;
+    if constexpr (SEARCH) {
+        int lo = 0, hi = a.num_seqs;
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (a.cu_q[mid] <= t) lo = mid; else hi = mid;
+        }
+        if (a.cu_q[lo + 1] - a.cu_q[lo] < 2) return;
+    }
+    const int Dv = a.Dv;
+    constexpr int V = VEC ? 4 : 1;
+    constexpr int P = 16 / V;                         // pieces of a lane: up to 256 columns
+    for (int h = threadIdx.x >> 4; h < a.H; h += 16) {
+        const float* o = a.raw + ((int64_t)h * a.T + t) * Dv;
+        const float* w = a.norm_w + (int64_t)h * a.norm_head_stride;
+        const T* gate = (const T*)a.gate_raw + (int64_t)t * a.gate_stride + (int64_t)h * Dv;
+        Cols<V> x[P], gt[P];
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+            const int c = V * (l16 + 16 * j);
+            if (c < Dv) {
+                x[j] = row_load<V>(o + c);
+                if (a.gate_raw != nullptr) gt[j] = row_load<V>(gate + c);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+            if (V * (l16 + 16 * j) < Dv) {
+#pragma unroll
+                for (int e = 0; e < V; ++e) ss += x[j].v[e] * x[j].v[e];
+            }
+        }
+        const float rstd = 1.0f / sqrtf(row16_sum(ss) / (float)Dv + a.eps);
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+            const int c = V * (l16 + 16 * j);
+            if (c < Dv) {
+                const Cols<V> wt = row_load<V>(w + c);
+#pragma unroll
+                for (int e = 0; e < V; ++e) {
+                    x[j].v[e] *= rstd * wt.v[e];
+                    if (a.gate_raw != nullptr) x[j].v[e] *= cr_sigmoid(gt[j].v[e]);
+                }
+                row_store<V>((T*)a.out + (int64_t)t * a.out_stride + (int64_t)h * Dv + c, x[j]);
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------------ single tokens
+// One token of a sequence: bound by its state, which is read and written once.  A workgroup per (sequence, head) holds the state in
+// registers, four neighbouring columns of ROWS rows a thread (all loads in flight at once); what the token finds in the old state
+// and what it reads out come from one pass: with p = S^T k (decayed as the form wants it) the read-out of the new state
+// is that of the decayed old one plus the write's part, which is a number per token (k . q and the like) times the columns written.
+template <typename T, int FORM, int ROWS>
+__global__ __launch_bounds__(256) void single_recurrence_kernel(const ChunkRecurrenceArgs a, const int pieces) {
+    constexpr int NX = FORM == kCrGated ? 3 : FORM == kCrGeneral ? 4 : 2;
+    __shared__ float ws[256], ks[256], qs[256], as[256], red[4][4];
+    __shared__ __attribute__((aligned(16))) float part[2][256 * 4];
+    const int b = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+    const int t = a.cu_q[b], D = a.D, Dv = a.Dv;
+    if (a.cu_q[b + 1] - t != 1) return;
+    const bool fresh = a.cu_k[b + 1] - a.cu_k[b] == 1;
+    const int c = (tid % pieces) * 4, group = tid / pieces, groups = 256 / pieces;      // (pieces is a power of two)
+    const bool live = c < Dv;
+    // the token's rows first: they are waited for first
+    float x[4] = {};
+    const int dd = tid < D ? tid : 0;
+    {
+        const void* xs[4] = {a.x0, a.x1, a.x2, a.x3};
+        const int64_t ss[4] = {a.s0, a.s1, a.s2, a.s3};
+#pragma unroll
+        for (int j = 0; j < NX; ++j) {
+            const int hj = (FORM == kCrGated && j < 2) ? h / a.group : h;
+            x[j] = (float)((const T*)xs[j])[(int64_t)t * ss[j] + (int64_t)hj * D + dd];
+        }
+    }
+    const float c0 = FORM == kCrGated ? expf(a.c0[h]) : a.c0[(int64_t)h * D + dd], c1 = a.c1[(int64_t)h * D + dd];
+    float v[4], gate[4], nw[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        v[e] = live ? (float)((const T*)a.v)[(int64_t)t * a.sv + (int64_t)h * Dv + c + e] : 0.f;
+        gate[e] = (live && a.gate_raw != nullptr) ? (float)((const T*)a.gate_raw)[(int64_t)t * a.gate_stride + (int64_t)h * Dv + c + e] : 0.f;
+        nw[e] = live ? a.norm_w[(int64_t)h * a.norm_head_stride + c + e] : 0.f;
+    }
+    float beta = 0.f;
+    if constexpr (FORM == kCrGated) beta = (float)((const T*)a.b_raw)[(int64_t)t * a.b_stride + h];
+    float* st = a.state + ((int64_t)a.slots[b] * a.H + h) * (int64_t)D * Dv + c;
+    f32x4 S[ROWS];
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+        const int d = group + i * groups;
+        S[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (live && d < D && !fresh) S[i] = *(const f32x4*)(st + (int64_t)d * Dv);
+    }
+    {
+        CrElem el = cr_elem<FORM>(x, c0, c1, a.p0);
+        if (tid >= D) el = CrElem{1.f, 0.f, 0.f, 0.f};
+        const float s0 = wave_sum(el.k * el.k);
+        const float s1 = wave_sum(FORM == kCrGated ? el.q * el.q : el.a * el.q), s2 = wave_sum(el.k * el.q);
+        if ((tid & 63) == 0) {
+            red[0][tid >> 6] = s0;
+            red[1][tid >> 6] = s1;
+            red[2][tid >> 6] = s2;
+        }
+        ws[tid] = el.w;
+        ks[tid] = el.k;
+        qs[tid] = el.q;
+        as[tid] = el.a;
+    }
+    __syncthreads();
+    const float kk = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]), s1 = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
+    const float kq = (red[2][0] + red[2][1]) + (red[2][2] + red[2][3]);
+    const float kn = FORM == kCrWrite ? 1.f : 1.0f / sqrtf(kk + a.p1);
+    const float qn = FORM == kCrGated ? 1.0f / sqrtf((s1 + a.p1) * (float)D) : 1.f;
+    f32x4 pk = {0.f, 0.f, 0.f, 0.f}, pq = pk;         // S^T k (general: of the old state), (w S)^T q over this thread's rows
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+        const int d = group + i * groups;
+        if (d < D) {
+            if constexpr (FORM == kCrGeneral) pk += S[i] * ks[d];
+            S[i] *= ws[d];
+            if constexpr (FORM == kCrGated) pk += S[i] * ks[d];
+            pq += S[i] * qs[d];
+        }
+    }
+    if constexpr (FORM != kCrWrite) *(f32x4*)(part[0] + tid * 4) = pk;
+    *(f32x4*)(part[1] + tid * 4) = pq;
+    __syncthreads();
+    f32x4 sk = {0.f, 0.f, 0.f, 0.f}, sq = sk;
+    for (int j = 0; j < groups; ++j) {
+        if constexpr (FORM != kCrWrite) sk += *(const f32x4*)(part[0] + (j * pieces + tid % pieces) * 4);
+        sq += *(const f32x4*)(part[1] + (j * pieces + tid % pieces) * 4);
+    }
+    const f32x4 vv = {v[0], v[1], v[2], v[3]};
+    f32x4 o, add, sub = {0.f, 0.f, 0.f, 0.f};         // new state: decayed old + k add - a sub
+    if constexpr (FORM == kCrGated) {
+        add = (vv - sk * kn) * (cr_sigmoid(beta) * kn);
+        o = (sq + add * kq) * qn;
+    } else if constexpr (FORM == kCrGeneral) {
+        add = vv;
+        sub = sk * (kn * kn);
+        o = sq + vv * kq - sub * s1;
+    } else {
+        add = vv;
+        o = sq + vv * kq;
+    }
+    if (live) {
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) {
+            const int d = group + i * groups;
+            if (d < D) {
+                S[i] += add * ks[d];
+                if constexpr (FORM == kCrGeneral) S[i] -= sub * as[d];
+                *(f32x4*)(st + (int64_t)d * Dv) = S[i];
+            }
+        }
+    }
+    float ss = live ? (o[0] * o[0] + o[1] * o[1]) + (o[2] * o[2] + o[3] * o[3]) : 0.f;
+    for (int m = 1; m < pieces; m *= 2) ss += __shfl_xor(ss, m);        // (pieces <= 64: a row's columns lie in one wave)
+    if (live && group == 0) {
+        const float rstd = 1.0f / sqrtf(ss / (float)Dv + a.eps);
+        T* out = (T*)a.out + (int64_t)t * a.out_stride + (int64_t)h * Dv + c;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float r = o[e] * rstd * nw[e];
+            if (a.gate_raw != nullptr) r *= cr_sigmoid(gate[e]);
+            out[e] = (T)r;
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------------ launches
+// Sizes both launches take: the single tokens' one holds a state in at most 32 pieces of four columns a thread.
+static bool recurrence_built(int D, int Dv) {
+    return (D == 32 || D == 64 || D == 96 || D == 128) && Dv % 16 == 0 && Dv <= 256 && D * Dv <= 128 * 128;
+}
+
+// The workspace of T rows in seqs sequences: records, their rows of V, read-outs; every part starts on 16 bytes.
+struct CrWorkspace {
+    int64_t records, chunks, columns, raw;            // how many (per head); bytes of the parts
+    CrWorkspace(int form, int64_t T, int H, int D, int Dv, int seqs, int dtype) {
+        const int rows = form == kCrWrite ? 8 : 16;
+        const int words = rows * D + (form == kCrGeneral ? 2 : 1) * 8 * D + D + (form == kCrWrite ? 0 : 256) + 8 * rows;
+        records = cr_first_record(T, seqs) + 1;
+        chunks = records * H * words * 4;
+        columns = records * H * 8 * Dv * (dtype == NV_DTYPE_BF16 ? 2 : 4);
+        raw = T * H * Dv * 4;
+    }
+    int64_t bytes() const { return chunks + columns + raw; }
+};
+
+template <typename T, int FORM, int D>
+static void chunks_of_size(const ChunkRecurrenceArgs& a, int first_seq, hipStream_t s) {
+    const int seqs = a.num_seqs - first_seq;
+    const dim3 prep((unsigned)a.records, (unsigned)((a.H + 3) / 4)), pairs((unsigned)(seqs * a.H));
+    const uintptr_t piece = 2 * sizeof(T) - 1;        // two channels by one load
+    const bool vec = a.sv % 2 == 0 && a.s0 % 2 == 0 && a.s1 % 2 == 0 && a.s2 % 2 == 0 && a.s3 % 2 == 0 &&
+                     (((uintptr_t)a.v | (uintptr_t)a.x0 | (uintptr_t)a.x1 | (uintptr_t)a.x2 | (uintptr_t)a.x3) & piece) == 0;
+    if (vec) hipLaunchKernelGGL((recurrence_chunks_kernel<T, FORM, D, true>), prep, dim3(256), 0, s, a, first_seq);
+    else hipLaunchKernelGGL((recurrence_chunks_kernel<T, FORM, D, false>), prep, dim3(256), 0, s, a, first_seq);
+    // two waves for a state's 16 columns while one each leaves a good part of the 1024 SIMDs idle
+    const int tiles = a.Dv / 16;
+    if ((int64_t)pairs.x * tiles <= 768)
+        hipLaunchKernelGGL((recurrence_states_kernel<T, FORM, D, 2>), dim3(pairs.x, (unsigned)((tiles + 1) / 2)), dim3(512), 0, s, a, first_seq);
+    else
+        hipLaunchKernelGGL((recurrence_states_kernel<T, FORM, D, 1>), dim3(pairs.x, (unsigned)((tiles + 3) / 4)), dim3(512), 0, s, a, first_seq);
+}
+
+template <typename T, int FORM>
+static int chunks_of(const ChunkRecurrenceArgs& a, int first_seq, bool singles_behind, hipStream_t s) {
+    switch (a.D) {
+        case 32: chunks_of_size<T, FORM, 32>(a, first_seq, s); break;
+        case 64: chunks_of_size<T, FORM, 64>(a, first_seq, s); break;
+        case 96: chunks_of_size<T, FORM, 96>(a, first_seq, s); break;
+        default: chunks_of_size<T, FORM, 128>(a, first_seq, s); break;
+    }
+    const dim3 rows((unsigned)a.T);
+    const bool vec = a.gate_stride % 4 == 0 && a.out_stride % 4 == 0 &&
+                     ((uintptr_t)a.gate_raw | (uintptr_t)a.out | (uintptr_t)a.norm_w | (uintptr_t)a.raw) % 16 == 0;
+    if (vec && singles_behind) hipLaunchKernelGGL((recurrence_finish_kernel<T, true, true>), rows, dim3(256), 0, s, a, first_seq);
+    else if (vec) hipLaunchKernelGGL((recurrence_finish_kernel<T, true, false>), rows, dim3(256), 0, s, a, first_seq);
+    else hipLaunchKernelGGL((recurrence_finish_kernel<T, false, true>), rows, dim3(256), 0, s, a, first_seq);
+    return check_launch("chunked recurrence");
+}
+
+template <typename T, int FORM>
+static int singles_of(const ChunkRecurrenceArgs& a, hipStream_t s) {
+    int pieces = 1;
+    while (pieces * 4 < a.Dv) pieces *= 2;            // at most 64
+    const int rows = (a.D + 256 / pieces - 1) / (256 / pieces);
+    const dim3 grid((unsigned)a.num_seqs, (unsigned)a.H), block(256);
+    if (rows <= 4) hipLaunchKernelGGL((single_recurrence_kernel<T, FORM, 4>), grid, block, 0, s, a, pieces);
+    else if (rows <= 8) hipLaunchKernelGGL((single_recurrence_kernel<T, FORM, 8>), grid, block, 0, s, a, pieces);
+    else if (rows <= 16) hipLaunchKernelGGL((single_recurrence_kernel<T, FORM, 16>), grid, block, 0, s, a, pieces);
+    else hipLaunchKernelGGL((single_recurrence_kernel<T, FORM, 32>), grid, block, 0, s, a, pieces);
+    return check_launch("single-token recurrence");
+}
+
+#define NV_CR_DISPATCH(FN, ...)                                                                                       \
+    if (dtype == NV_DTYPE_BF16)                                                                                       \
+        return form == kCrGated ? FN<__bf16, kCrGated>(__VA_ARGS__)                                                   \
+                                : form == kCrGeneral ? FN<__bf16, kCrGeneral>(__VA_ARGS__) : FN<__bf16, kCrWrite>(__VA_ARGS__); \
+    return form == kCrGated ? FN<float, kCrGated>(__VA_ARGS__)                                                        \
+                            : form == kCrGeneral ? FN<float, kCrGeneral>(__VA_ARGS__) : FN<float, kCrWrite>(__VA_ARGS__)
+
+int launch_chunk_recurrence(int form, const ChunkRecurrenceArgs& a, int first_seq, bool singles_behind, int dtype, hipStream_t s) {
+    NV_CR_DISPATCH(chunks_of, a, first_seq, singles_behind, s);
+}
+int launch_single_recurrence(int form, const ChunkRecurrenceArgs& a, int dtype, hipStream_t s) {
+    NV_CR_DISPATCH(singles_of, a, s);
+}
+#undef NV_CR_DISPATCH
+
+bool run_recurrence_portions(int form, ChunkRecurrenceArgs a, int lead, int portions, int dtype, void* workspace,
+                             int64_t workspace_bytes, hipStream_t s, int* rc) {
+    *rc = NV_OK;
+    const bool rest = lead < a.num_seqs && a.T > lead && (portions & (NV_PORTION_FEW | NV_PORTION_LONG));
+    const bool singles_behind = lead < a.num_seqs && (portions & NV_PORTION_SINGLE);
+    const int64_t far = 1LL << 28;                    // rows of a chunk are addressed by 32-bit offsets
+    if (!recurrence_built(a.D, a.Dv) || (uintptr_t)a.state % 16 != 0 || a.s0 >= far || a.s1 >= far || a.s2 >= far || a.s3 >= far ||
+        a.sv >= far || (int64_t)a.H * a.Dv >= far || a.T >= (1LL << 31) || (rest && workspace == nullptr))
+        return false;
+    const CrWorkspace ws(form, a.T, a.H, a.D, a.Dv, a.num_seqs - lead, dtype);
+    const int64_t need = ws.bytes();
+    if (rest && workspace_bytes < need) {
+        set_error("recurrence: workspace of %lld bytes, need %lld", (long long)workspace_bytes, (long long)need);
+        *rc = NV_ERR_WORKSPACE;
+        return true;
+    }
+    if (lead > 0 || singles_behind) {
+        ChunkRecurrenceArgs one = a;
+        if (!singles_behind) one.num_seqs = lead;
+        *rc = launch_single_recurrence(form, one, dtype, s);
+        if (*rc != NV_OK) return true;
+    }
+    a.chunks = (float*)workspace;
+    a.columns = (char*)workspace + ws.chunks;
+    a.raw = (float*)((char*)a.columns + ws.columns);
+    a.records = ws.records;
+    if (rest) *rc = launch_chunk_recurrence(form, a, lead, singles_behind, dtype, s);
+    return true;
+}
+
+}  // namespace nv
+
+extern "C" int64_t nv_recurrence_workspace_bytes(int form, int64_t T, int H, int D, int Dv, int num_seqs, int leading_singles,
+                                                 int dtype) {
+    if (form < 0 || form > 2 || T <= 0 || H <= 0 || D <= 0 || Dv <= 0 || leading_singles < 0 || num_seqs <= leading_singles ||
+        !nv::recurrence_built(D, Dv))
+        return 0;
+    return nv::CrWorkspace(form, T, H, D, Dv, num_seqs - leading_singles, dtype).bytes();
+}

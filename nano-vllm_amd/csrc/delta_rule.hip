@@ -24,7 +24,7 @@
 // tokens for its 16 columns, and the normalised read-out of the tile is written by all waves together.
 #include <algorithm>
 
-#include "nv_common.h"
+#include "chunk_recurrence.h"
 #include "../../include/nanovllm_hip_mixers.h"
 
 namespace nv {
@@ -456,6 +456,19 @@ extern "C" int nv_gated_delta_rule(const void* q, const void* k, const void* v, 
                                    int64_t out_stride, const int* cu_seqlens_q, const int* cu_seqlens_k,
                                    const int* state_slots, int num_seqs, int H, int G, int D, int Dv, float eps,
                                    int dtype, void* stream) {
+    return nv_gated_delta_rule_portions(q, k, v, q_stride, k_stride, v_stride, a_raw, a_stride, b_raw, b_stride, gate_raw,
+                                        gate_stride, A_log, dt_bias, norm_w, state, out, out_stride, cu_seqlens_q, cu_seqlens_k,
+                                        state_slots, num_seqs, 0, H, G, D, Dv, eps, 0, 7, dtype, nullptr, 0, stream);
+}
+
+extern "C" int nv_gated_delta_rule_portions(const void* q, const void* k, const void* v, int64_t q_stride, int64_t k_stride,
+                                   int64_t v_stride, const void* a_raw, int64_t a_stride, const void* b_raw,
+                                   int64_t b_stride, const void* gate_raw, int64_t gate_stride, const float* A_log,
+                                   const float* dt_bias, const float* norm_w, float* state, void* out,
+                                   int64_t out_stride, const int* cu_seqlens_q, const int* cu_seqlens_k,
+                                   const int* state_slots, int num_seqs, int64_t T, int H, int G, int D, int Dv,
+                                   float eps, int leading_singles, int portions, int dtype, void* workspace,
+                                   int64_t workspace_bytes, void* stream) {
     using namespace nv;
     NV_REQUIRE(num_seqs >= 0 && H > 0 && G > 0 && D > 0 && Dv > 0, NV_ERR_INVALID_ARG, "nv_gated_delta_rule: bad sizes");
     if (num_seqs == 0) return NV_OK;
@@ -466,7 +479,25 @@ extern "C" int nv_gated_delta_rule(const void* q, const void* k, const void* v, 
     NV_REQUIRE(D <= 256 && Dv <= 256, NV_ERR_UNSUPPORTED, "nv_gated_delta_rule: D=%d, Dv=%d exceed 256", D, Dv);
     NV_REQUIRE(dtype == NV_DTYPE_BF16 || dtype == NV_DTYPE_F32, NV_ERR_INVALID_ARG, "nv_gated_delta_rule: bad dtype");
     NV_REQUIRE(H < 65536, NV_ERR_UNSUPPORTED, "nv_gated_delta_rule: launch too large");
+    NV_REQUIRE(leading_singles >= 0 && leading_singles <= num_seqs, NV_ERR_INVALID_ARG, "nv_gated_delta_rule: bad portions");
     hipStream_t s = (hipStream_t)stream;
+    {
+        ChunkRecurrenceArgs c{};
+        c.x0 = q; c.x1 = k; c.x2 = a_raw; c.v = v;
+        c.s0 = q_stride; c.s1 = k_stride; c.s2 = a_stride; c.sv = v_stride;
+        c.b_raw = b_raw; c.b_stride = b_stride;
+        c.c0 = A_log; c.c1 = dt_bias;
+        c.gate_raw = gate_raw; c.gate_stride = gate_stride;
+        c.norm_w = norm_w;
+        c.state = state;
+        c.out = out; c.out_stride = out_stride;
+        c.cu_q = cu_seqlens_q; c.cu_k = cu_seqlens_k; c.slots = state_slots;
+        c.num_seqs = num_seqs; c.H = H; c.group = H / G; c.D = D; c.Dv = Dv;
+        c.T = T;
+        c.eps = eps; c.p1 = 1e-6f;
+        int rc;
+        if (run_recurrence_portions(kCrGated, c, leading_singles, portions, dtype, workspace, workspace_bytes, s, &rc)) return rc;
+    }
     if (dtype == NV_DTYPE_BF16)
         return launch_delta<__bf16>(q, k, v, q_stride, k_stride, v_stride, a_raw, a_stride, b_raw, b_stride, gate_raw,
                                     gate_stride, A_log, dt_bias, norm_w, state, out, out_stride, cu_seqlens_q,

@@ -27,6 +27,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "chunk_recurrence.h"
 #include "fixed_decay.h"
 #include "../../include/nanovllm_hip_mixers.h"
 
@@ -349,6 +350,17 @@ extern "C" int nv_gated_write_memory(const void* q, const void* f_raw, const voi
                                      float* state, void* out, int64_t out_stride, const int32_t* cu_seqlens_q,
                                      const int32_t* cu_seqlens_k, const int32_t* state_slots, int num_seqs, int H, int Dk,
                                      int Dv, float eps, int dtype, void* stream) {
+    return nv_gated_write_memory_portions(q, f_raw, v, q_stride, f_stride, v_stride, f_bias, lower, norm_w, state, out, out_stride,
+                                          cu_seqlens_q, cu_seqlens_k, state_slots, num_seqs, 0, H, Dk, Dv, eps, 0, 7, dtype, nullptr,
+                                          0, stream);
+}
+
+extern "C" int nv_gated_write_memory_portions(const void* q, const void* f_raw, const void* v, int64_t q_stride, int64_t f_stride,
+                                     int64_t v_stride, const float* f_bias, const float* lower, const float* norm_w,
+                                     float* state, void* out, int64_t out_stride, const int32_t* cu_seqlens_q,
+                                     const int32_t* cu_seqlens_k, const int32_t* state_slots, int num_seqs, int64_t T,
+                                     int H, int Dk, int Dv, float eps, int leading_singles, int portions, int dtype,
+                                     void* workspace, int64_t workspace_bytes, void* stream) {
     using namespace nv;
     NV_REQUIRE(num_seqs >= 0 && H > 0 && Dk > 0 && Dv > 0, NV_ERR_INVALID_ARG, "nv_gated_write_memory: bad sizes");
     if (num_seqs == 0) return NV_OK;
@@ -357,7 +369,23 @@ extern "C" int nv_gated_write_memory(const void* q, const void* f_raw, const voi
     NV_REQUIRE(Dk <= 256 && Dv <= 256, NV_ERR_UNSUPPORTED, "nv_gated_write_memory: Dk=%d, Dv=%d exceed 256", Dk, Dv);
     NV_REQUIRE(dtype == NV_DTYPE_BF16 || dtype == NV_DTYPE_F32, NV_ERR_INVALID_ARG, "nv_gated_write_memory: bad dtype");
     NV_REQUIRE(H < 65536, NV_ERR_UNSUPPORTED, "nv_gated_write_memory: launch too large");
+    NV_REQUIRE(leading_singles >= 0 && leading_singles <= num_seqs, NV_ERR_INVALID_ARG, "nv_gated_write_memory: bad portions");
     hipStream_t s = (hipStream_t)stream;
+    {
+        ChunkRecurrenceArgs c{};
+        c.x0 = q; c.x1 = f_raw; c.v = v;
+        c.s0 = q_stride; c.s1 = f_stride; c.sv = v_stride;
+        c.c0 = f_bias; c.c1 = lower;
+        c.norm_w = norm_w;
+        c.state = state;
+        c.out = out; c.out_stride = out_stride;
+        c.cu_q = cu_seqlens_q; c.cu_k = cu_seqlens_k; c.slots = state_slots;
+        c.num_seqs = num_seqs; c.H = H; c.group = 1; c.D = Dk; c.Dv = Dv;
+        c.T = T;
+        c.eps = eps;
+        int rc;
+        if (run_recurrence_portions(kCrWrite, c, leading_singles, portions, dtype, workspace, workspace_bytes, s, &rc)) return rc;
+    }
     if (dtype == NV_DTYPE_BF16) {
         GmArgs<__bf16> a{(const __bf16*)q, nullptr, (const __bf16*)v, q_stride, 0, v_stride, (const __bf16*)f_raw, f_stride,
                          nullptr, nullptr, 0, nullptr, 0, nullptr, f_bias, lower, norm_w, 0, state, nullptr, nullptr,

@@ -18,7 +18,7 @@
 // normalised, gated read-out of the tile is written by all waves together.
 #include <algorithm>
 
-#include "nv_common.h"
+#include "chunk_recurrence.h"
 #include "../../include/nanovllm_hip_mixers.h"
 
 namespace nv {
@@ -199,6 +199,19 @@ extern "C" int nv_general_delta_rule(const void* r, const void* k, const void* v
                                      int64_t out_stride, const int* cu_seqlens_q, const int* cu_seqlens_k,
                                      const int* state_slots, int num_seqs, int H, int D, float eps, float decay_rate,
                                      float key_eps, int dtype, void* stream) {
+    return nv_general_delta_rule_portions(r, k, v, r_stride, k_stride, v_stride, w_raw, w_stride, a_raw, a_stride, gate_raw,
+                                          gate_stride, w_bias, a_bias, norm_w, state, out, out_stride, cu_seqlens_q, cu_seqlens_k,
+                                          state_slots, num_seqs, 0, H, D, eps, decay_rate, key_eps, 0, 7, dtype, nullptr, 0, stream);
+}
+
+extern "C" int nv_general_delta_rule_portions(const void* r, const void* k, const void* v, int64_t r_stride, int64_t k_stride,
+                                     int64_t v_stride, const void* w_raw, int64_t w_stride, const void* a_raw,
+                                     int64_t a_stride, const void* gate_raw, int64_t gate_stride, const float* w_bias,
+                                     const float* a_bias, const float* norm_w, float* state, void* out,
+                                     int64_t out_stride, const int* cu_seqlens_q, const int* cu_seqlens_k,
+                                     const int* state_slots, int num_seqs, int64_t T, int H, int D, float eps,
+                                     float decay_rate, float key_eps, int leading_singles, int portions, int dtype,
+                                     void* workspace, int64_t workspace_bytes, void* stream) {
     using namespace nv;
     NV_REQUIRE(num_seqs >= 0 && H > 0 && D > 0, NV_ERR_INVALID_ARG, "nv_general_delta_rule: bad sizes");
     if (num_seqs == 0) return NV_OK;
@@ -208,7 +221,24 @@ extern "C" int nv_general_delta_rule(const void* r, const void* k, const void* v
     NV_REQUIRE(D <= 256, NV_ERR_UNSUPPORTED, "nv_general_delta_rule: D=%d exceeds 256", D);
     NV_REQUIRE(dtype == NV_DTYPE_BF16 || dtype == NV_DTYPE_F32, NV_ERR_INVALID_ARG, "nv_general_delta_rule: bad dtype");
     NV_REQUIRE(H < 65536, NV_ERR_UNSUPPORTED, "nv_general_delta_rule: launch too large");
+    NV_REQUIRE(leading_singles >= 0 && leading_singles <= num_seqs, NV_ERR_INVALID_ARG, "nv_general_delta_rule: bad portions");
     hipStream_t s = (hipStream_t)stream;
+    {
+        ChunkRecurrenceArgs c{};
+        c.x0 = r; c.x1 = k; c.x2 = w_raw; c.x3 = a_raw; c.v = v;
+        c.s0 = r_stride; c.s1 = k_stride; c.s2 = w_stride; c.s3 = a_stride; c.sv = v_stride;
+        c.c0 = w_bias; c.c1 = a_bias;
+        c.gate_raw = gate_raw; c.gate_stride = gate_stride;
+        c.norm_w = norm_w; c.norm_head_stride = D;
+        c.state = state;
+        c.out = out; c.out_stride = out_stride;
+        c.cu_q = cu_seqlens_q; c.cu_k = cu_seqlens_k; c.slots = state_slots;
+        c.num_seqs = num_seqs; c.H = H; c.group = 1; c.D = D; c.Dv = D;
+        c.T = T;
+        c.eps = eps; c.p0 = decay_rate; c.p1 = key_eps;
+        int rc;
+        if (run_recurrence_portions(kCrGeneral, c, leading_singles, portions, dtype, workspace, workspace_bytes, s, &rc)) return rc;
+    }
     if (dtype == NV_DTYPE_BF16)
         return launch_general_delta<__bf16>(r, k, v, r_stride, k_stride, v_stride, w_raw, w_stride, a_raw, a_stride,
                                             gate_raw, gate_stride, w_bias, a_bias, norm_w, state, out, out_stride,

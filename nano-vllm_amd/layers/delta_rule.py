@@ -46,4 +46,5 @@ class GatedDeltaRule(nn.Module):
         gate_raw [T, H*Dv] as projected; state [slots, H, D, Dv] float32.  Returns [T, H*Dv]."""
         ctx = get_context()
         return ops.gated_delta_rule(q, k, v, a_raw, b_raw, gate_raw, self.A_log, self.dt_bias, self.norm_weight, state,
-                                    ctx.cu_seqlens_q, ctx.cu_seqlens_k, ctx.state_slots, self.eps)
+                                    ctx.cu_seqlens_q, ctx.cu_seqlens_k, ctx.state_slots, self.eps,
+                                    ctx.max_seqlen_q, ctx.num_leading_decode, ctx.portion_kinds)

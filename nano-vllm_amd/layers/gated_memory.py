@@ -61,7 +61,8 @@ class GatedWriteMemory(nn.Module):
         """q, f_raw: [T, H, Dk] as projected; v: [T, H, Dv]; returns [T, H * Dv]."""
         ctx = get_context()
         return ops.gated_write_memory(q, f_raw, v, self.f_bias, self.lower, self.norm_weight, cache["state"],
-                                      ctx.cu_seqlens_q, ctx.cu_seqlens_k, ctx.state_slots, self.eps)
+                                      ctx.cu_seqlens_q, ctx.cu_seqlens_k, ctx.state_slots, self.eps,
+                                      ctx.max_seqlen_q, ctx.num_leading_decode, ctx.portion_kinds)
 
 
 class FixedDecayMemory(nn.Module):

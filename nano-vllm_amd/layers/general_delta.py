@@ -34,4 +34,4 @@ class GeneralDeltaRule(nn.Module):
         ctx = get_context()
         return ops.general_delta_rule(r, k, v, w_raw, a_raw, gate_raw, self.w_bias, self.a_bias, self.norm_weight, state,
                                       ctx.cu_seqlens_q, ctx.cu_seqlens_k, ctx.state_slots, self.eps, self.decay_rate,
-                                      self.key_eps)
+                                      self.key_eps, ctx.max_seqlen_q, ctx.num_leading_decode, ctx.portion_kinds)

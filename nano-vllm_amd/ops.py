@@ -533,13 +533,27 @@ def causal_conv_silu(x: torch.Tensor, weight: torch.Tensor, conv_state: torch.Te
     return y
 
 
+def _portions(dll, form: int, rows: torch.Tensor, T: int, H: int, D: int, Dv: int, B: int, max_seqlen_q: int, leading_singles: Optional[int],
+              portions: int) -> tuple:
+    """(leading single tokens, kinds of portions behind them, workspace or None) of a recurrent layer's step.  max_seqlen_q: the
+    most rows of a sequence (0: not known); leading_singles: sequences in front of the batch with exactly one row each;
+    portions: the kinds of portions behind them (`portion_kinds`; 7: not known)."""
+    lead = B if max_seqlen_q == 1 else int(leading_singles or 0)
+    _need(0 <= lead <= B, "leading_singles exceeds the batch")
+    if lead == B:                          # single tokens need none
+        return lead, int(portions), None
+    need = dll.nv_recurrence_workspace_bytes(form, T, H, D, Dv, B, lead, _dt(rows, "rows"))
+    return lead, int(portions), torch.empty(need, dtype=torch.uint8, device=rows.device) if need > 0 else None
+
+
 def gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a_raw: torch.Tensor, b_raw: torch.Tensor,
                      gate_raw: torch.Tensor, A_log: torch.Tensor, dt_bias: torch.Tensor, norm_weight: torch.Tensor,
                      state: torch.Tensor, cu_seqlens_q: torch.Tensor, cu_seqlens_k: torch.Tensor,
-                     state_slots: torch.Tensor, eps: float) -> torch.Tensor:
+                     state_slots: torch.Tensor, eps: float, max_seqlen_q: int = 0, leading_singles: Optional[int] = 0,
+                     portions: int = 7) -> torch.Tensor:
     """Gated delta rule with per-channel decay over a step's rows, state [slots, H, D, Dv] float32 updated in
     place; q, k: [T, G, D]; v: [T, H, Dv]; a_raw: [T, H * D]; b_raw: [T, H]; gate_raw: [T, H * Dv];
-    returns the normalised, gated read-out [T, H * Dv]."""
+    returns the normalised, gated read-out [T, H * Dv].  max_seqlen_q, leading_singles, portions: see `_portions`."""
     dt = _dt(q, "q")
     _rows_ok(q, "q")
     _rows_ok(k, "k")
@@ -560,12 +574,14 @@ def gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a_raw: t
     _need(cu_seqlens_q.numel() == B + 1 and cu_seqlens_k.numel() == B + 1, "one state slot per sequence")
     out = torch.empty((T, H * Dv), dtype=q.dtype, device=q.device)
     dll = _lib.mixers()
-    rc = dll.nv_gated_delta_rule(q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), k.stride(0), v.stride(0),
+    lead, portions, ws = _portions(dll, 0, q, T, H, D, Dv, B, max_seqlen_q, leading_singles, portions)
+    rc = dll.nv_gated_delta_rule_portions(q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), k.stride(0), v.stride(0),
                                  a_raw.data_ptr(), a_raw.stride(0), b_raw.data_ptr(), b_raw.stride(0),
                                  gate_raw.data_ptr(), gate_raw.stride(0), _f32c(A_log, "A_log"),
                                  _f32c(dt_bias, "dt_bias"), _f32c(norm_weight, "norm_weight"), state.data_ptr(),
                                  out.data_ptr(), out.stride(0), cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(),
-                                 state_slots.data_ptr(), B, H, G, D, Dv, float(eps), dt, _stream(q))
+                                 state_slots.data_ptr(), B, T, H, G, D, Dv, float(eps), lead, portions, dt, _ptr(ws),
+                                 ws.numel() if ws is not None else 0, _stream(q))
     _lib.check(rc, "nv_gated_delta_rule", dll)
     return out
 
@@ -678,9 +694,11 @@ def token_gate(z: torch.Tensor, table: torch.Tensor, ids: torch.Tensor, offset: 
 def general_delta_rule(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, w_raw: torch.Tensor, a_raw: torch.Tensor,
                        gate_raw: torch.Tensor, w_bias: torch.Tensor, a_bias: torch.Tensor, norm_weight: torch.Tensor,
                        state: torch.Tensor, cu_seqlens_q: torch.Tensor, cu_seqlens_k: torch.Tensor,
-                       state_slots: torch.Tensor, eps: float, decay_rate: float, key_eps: float) -> torch.Tensor:
+                       state_slots: torch.Tensor, eps: float, decay_rate: float, key_eps: float, max_seqlen_q: int = 0,
+                       leading_singles: Optional[int] = 0, portions: int = 7) -> torch.Tensor:
     """Generalized delta rule over a step's rows, state [slots, H, D, D] float32 updated in place; r, k, v: [T, H, D];
-    w_raw, a_raw, gate_raw: [T, H * D]; returns the normalised, gated read-out [T, H * D]."""
+    w_raw, a_raw, gate_raw: [T, H * D]; returns the normalised, gated read-out [T, H * D].  max_seqlen_q,
+    leading_singles, portions: see `_portions`."""
     dt = _dt(r, "r")
     T, H, D = r.shape
     for t, n in ((r, "r"), (k, "k"), (v, "v")):
@@ -698,13 +716,14 @@ def general_delta_rule(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, w_raw:
     _need(cu_seqlens_q.numel() == B + 1 and cu_seqlens_k.numel() == B + 1, "one state slot per sequence")
     out = torch.empty((T, H * D), dtype=r.dtype, device=r.device)
     dll = _lib.mixers()
-    rc = dll.nv_general_delta_rule(r.data_ptr(), k.data_ptr(), v.data_ptr(), r.stride(0), k.stride(0), v.stride(0),
+    lead, portions, ws = _portions(dll, 1, r, T, H, D, D, B, max_seqlen_q, leading_singles, portions)
+    rc = dll.nv_general_delta_rule_portions(r.data_ptr(), k.data_ptr(), v.data_ptr(), r.stride(0), k.stride(0), v.stride(0),
                                    w_raw.data_ptr(), w_raw.stride(0), a_raw.data_ptr(), a_raw.stride(0),
                                    gate_raw.data_ptr(), gate_raw.stride(0), _f32c(w_bias, "w_bias"),
                                    _f32c(a_bias, "a_bias"), _f32c(norm_weight, "norm_weight"), state.data_ptr(),
                                    out.data_ptr(), out.stride(0), cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(),
-                                   state_slots.data_ptr(), B, H, D, float(eps), float(decay_rate), float(key_eps), dt,
-                                   _stream(r))
+                                   state_slots.data_ptr(), B, T, H, D, float(eps), float(decay_rate), float(key_eps), lead,
+                                   portions, dt, _ptr(ws), ws.numel() if ws is not None else 0, _stream(r))
     _lib.check(rc, "nv_general_delta_rule", dll)
     return out
 
@@ -1297,10 +1316,11 @@ def mlstm_memory(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gates_pre: t
 
 def gated_write_memory(q: torch.Tensor, f_raw: torch.Tensor, v: torch.Tensor, f_bias: torch.Tensor, lower: torch.Tensor,
                        norm_weight: torch.Tensor, state: torch.Tensor, cu_seqlens_q: torch.Tensor,
-                       cu_seqlens_k: torch.Tensor, state_slots: torch.Tensor, eps: float) -> torch.Tensor:
+                       cu_seqlens_k: torch.Tensor, state_slots: torch.Tensor, eps: float, max_seqlen_q: int = 0,
+                       leading_singles: Optional[int] = 0, portions: int = 7) -> torch.Tensor:
     """Gated linear recurrence whose forget gate decides what is written; q, f_raw: [T, H, Dk] as projected; v: [T, H, Dv];
     f_bias, lower [H * Dk], norm_weight [Dv] float32; state [slots, H, Dk, Dv] float32 updated in place; returns
-    [T, H * Dv]."""
+    [T, H * Dv].  max_seqlen_q, leading_singles, portions: see `_portions`."""
     dt = _dt(q, "q")
     T, H, Dk = q.shape
     Dv = v.shape[2]
@@ -1314,10 +1334,12 @@ def gated_write_memory(q: torch.Tensor, f_raw: torch.Tensor, v: torch.Tensor, f_
     B = _seq_meta(cu_seqlens_q, cu_seqlens_k, state_slots)
     out = torch.empty((T, H * Dv), dtype=q.dtype, device=q.device)
     dll = _lib.mixers()
-    rc = dll.nv_gated_write_memory(q.data_ptr(), f_raw.data_ptr(), v.data_ptr(), q.stride(0), f_raw.stride(0), v.stride(0),
+    lead, portions, ws = _portions(dll, 2, q, T, H, Dk, Dv, B, max_seqlen_q, leading_singles, portions)
+    rc = dll.nv_gated_write_memory_portions(q.data_ptr(), f_raw.data_ptr(), v.data_ptr(), q.stride(0), f_raw.stride(0), v.stride(0),
                                    _f32c(f_bias, "f_bias"), _f32c(lower, "lower"), _f32c(norm_weight, "norm_weight"),
                                    state.data_ptr(), out.data_ptr(), out.stride(0), cu_seqlens_q.data_ptr(),
-                                   cu_seqlens_k.data_ptr(), state_slots.data_ptr(), B, H, Dk, Dv, float(eps), dt, _stream(q))
+                                   cu_seqlens_k.data_ptr(), state_slots.data_ptr(), B, T, H, Dk, Dv, float(eps), lead, portions,
+                                   dt, _ptr(ws), ws.numel() if ws is not None else 0, _stream(q))
     _lib.check(rc, "nv_gated_write_memory", dll)
     return out
 

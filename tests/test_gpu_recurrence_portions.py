@@ -1,0 +1,92 @@
+"""GPU: the recurrences with a decay per head and key channel against the eager stand-ins of the same layers, at the sizes where
+their launches change: around the chunk of 8 tokens, single tokens in front of, between and beside longer portions, fresh and
+carried states, every built number of key channels, value columns that do not fill a workgroup, decays from none to total."""
+import pytest
+import torch
+
+import nanovllm_amd as nv
+from nanovllm_amd import ops
+from nanovllm_amd.layers import delta_rule, gated_memory, general_delta
+from oracle import ref_benarax_modules, ref_mixer_modules, ref_tutedra_modules
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+STEPS = {   # rows of the sequences; keys in front of them
+    "chunk_edges": ([2, 7, 8, 9, 16, 17], [0, 3, 0, 5, 1, 0]),
+    "mixed": ([1, 1, 30, 1, 0, 65], [4, 0, 7, 2, 3, 0]),
+    "singles": ([1, 1, 1], [0, 9, 1]),
+    "long": ([300], [0]),
+}
+
+
+def _context(rows, before, hints):
+    cu = lambda xs: torch.tensor([0] + torch.tensor(xs).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+    lead = 0
+    while lead < len(rows) and rows[lead] == 1:
+        lead += 1
+    known = dict(max_seqlen_q=max(rows), num_leading_decode=lead, portion_kinds=ops.portion_kinds(rows[lead:])) if hints else {}
+    slots = [(3 * i + 1) % (len(rows) + 2) if (len(rows) + 2) % 3 else i for i in range(len(rows))]
+    return nv.CacheContext(cu_seqlens_q=cu(rows), cu_seqlens_k=cu([r + n for r, n in zip(rows, before)]),
+                           state_slots=torch.tensor(slots, dtype=torch.int32, device=DEV), **known)
+
+
+def _layers(form, H, D, Dv, mk):
+    if form == "gated":
+        a, r = (m.GatedDeltaRule(H, H // 2, D, Dv, 1e-5, device=DEV) for m in (delta_rule, ref_mixer_modules))
+    elif form == "general":
+        a, r = (m.GeneralDeltaRule(H, D, 1e-5, device=DEV) for m in (general_delta, ref_benarax_modules))
+    else:
+        a, r = (m.GatedWriteMemory(H, D, Dv, 1e-5, device=DEV) for m in (gated_memory, ref_tutedra_modules))
+    spread = torch.linspace(-6, 8, H * D, device=DEV)[torch.randperm(H * D, generator=torch.Generator().manual_seed(1)).to(DEV)]
+    with torch.no_grad():
+        a.norm_weight.copy_(1 + 0.3 * mk(a.norm_weight.numel()))
+        if form == "gated":            # decays from exp(-0.02) to exp(-22) per token
+            a.A_log.copy_(torch.linspace(-1, 1, H, device=DEV))
+            a.dt_bias.copy_(spread)
+        elif form == "general":
+            a.w_bias.copy_(spread)
+            a.a_bias.copy_(0.5 * mk(H * D))
+        else:                          # forget gates from 0.997 to 4e-6
+            a.f_bias.copy_(-2 * spread + 4)
+            a.lower.copy_(torch.where(spread > 3, 0.0, 0.3) * torch.rand(H * D, device=DEV))
+    r.load_state_dict(a.state_dict())
+    return a, r
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("step", list(STEPS))
+@pytest.mark.parametrize("form,D,Dv", [("gated", 128, 128), ("gated", 64, 80), ("gated", 96, 16), ("general", 128, 128),
+                                       ("general", 64, 64), ("general", 32, 32), ("write", 128, 128), ("write", 32, 144),
+                                       ("write", 40, 24)])
+def test_portions(form, D, Dv, step, dtype):
+    rows, before = STEPS[step]
+    H, T = 4, sum(rows)
+    g = torch.Generator(device=DEV).manual_seed(7 * D + Dv)
+    mk = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    a, r = _layers(form, H, D, Dv, mk)
+    G = H // 2 if form == "gated" else H
+    q, k, v = mk(T, G, D).to(dtype), mk(T, H if form == "write" else G, D).to(dtype), mk(T, H, Dv + 8)[:, :, :Dv].contiguous().to(dtype)
+    wide = mk(T, H * Dv + 1).to(dtype)
+    gate = wide[:, 1:] if Dv == 80 else wide[:, :-1].contiguous()      # rows that do not start on 16 bytes
+    w, rate, b = mk(T, H * D).to(dtype), mk(T, H * D).to(dtype), mk(T, H).to(dtype)
+    if D == 64:                            # rows that start on any element
+        w = mk(T, H * D + 1).to(dtype)[:, 1:]
+    state = mk(len(rows) + 2, H, D, Dv)
+    call = {"gated": lambda m, s: m(q, k, v, w, b, gate, s), "general": lambda m, s: m(q, k, v, w, rate, gate, s),
+            "write": lambda m, s: m(q, k, v, {"state": s})}[form]
+    nv.set_context(_context(rows, before, False))
+    want_state = state.clone()
+    want = call(r, want_state)
+    # float32: sums of up to 128 products of order one taken in another order, read-outs divided by their root mean square;
+    # bfloat16: one rounding of the output (2^-9 of values up to 8)
+    tol = dict(rtol=5e-5, atol=5e-5) if dtype == torch.float32 else dict(rtol=1e-2, atol=2e-2)
+    scale = want_state.abs().max().item()
+    for hints in (True, False):
+        nv.set_context(_context(rows, before, hints))
+        got_state = state.clone()
+        got = call(a, got_state)
+        torch.cuda.synchronize()
+        torch.testing.assert_close(got.float(), want.float(), **tol)
+        torch.testing.assert_close(got_state, want_state, rtol=2e-5, atol=2e-6 * scale)
+    nv.set_context(None)
