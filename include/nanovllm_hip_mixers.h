@@ -86,6 +86,10 @@ NV_API int nv_attn_scoremod_paged_vld(const void* q, const void* k_cache, const 
                                       int64_t out_stride, void* workspace, int64_t workspace_bytes, void* stream);
 /* Scratch bytes the launches above need for these sizes (key slices of single rows; 0 when it needs none). */
 NV_API int64_t nv_attn_scoremod_workspace_bytes(int num_seqs, int64_t T, int H, int G, int Dv, int max_seqlen_k);
+/* The same with key ranges for prompt portions counted in (few long portions of few sequences are cut along their keys when the
+ * workspace holds it). */
+NV_API int64_t nv_attn_scoremod_step_workspace_bytes(int num_seqs, int64_t T, int H, int G, int D, int Dv, int block_size,
+                                                     int max_seqlen_q, int max_seqlen_k, int dtype);
 
 /*
  * Short causal convolution over time per channel, then SiLU, with the last taps-1 inputs of every sequence carried

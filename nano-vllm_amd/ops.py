@@ -497,7 +497,7 @@ def attn_scoremod_paged(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.T
         n_dist = dist_bias.shape[1]
     out = torch.empty((T, H * Dv), dtype=q.dtype, device=q.device)
     dll = _lib.mixers()
-    need = dll.nv_attn_scoremod_workspace_bytes(B, T, H, G, Dv, int(max_seqlen_k))
+    need = dll.nv_attn_scoremod_step_workspace_bytes(B, T, H, G, D, Dv, bs, int(max_seqlen_q), int(max_seqlen_k), dt)
     ws = _workspace(q.device, need) if need else None
     rc = dll.nv_attn_scoremod_paged_vld(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), v_ld, out.data_ptr(),
                                     cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(), block_tables.data_ptr(), B,

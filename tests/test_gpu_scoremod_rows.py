@@ -1,0 +1,52 @@
+"""GPU: score-modified attention on pages of whole key tiles against the eager stand-in: portions around the 32-row blocks and the 64-key
+tiles, every group size's way of sharing a workgroup, key and value sizes 64 / 128, each form of the scores, long portions of one
+sequence (cut into key ranges) and single rows beside portions."""
+import pytest
+import torch
+
+import nanovllm_amd as nv
+from nanovllm_amd.layers import attention
+from oracle import ref_mixer_modules as ref
+from test_gpu_mixers import DEV, _context
+
+pytestmark = pytest.mark.gpu
+
+STEPS = {"edges": ([1, 31, 32, 33, 64, 65, 2], [64, 31, 96, 161, 64, 129, 66]), "portions": ([200, 1, 130], [200, 77, 600]),
+         "ranges": ([40], [2500]), "singles": ([1] * 5, [1500, 63, 64, 65, 1])}
+FORMS = {"plain": dict(), "cap_sink": dict(softcap=25.0, use_sink=True, rot_dims=32), "high_cap": dict(softcap=60.0, temp_coef=0.5, temp_every=64),
+         "cap_bias_sink": dict(softcap=25.0, use_sink=True, bias=True), "bias": dict(bias=True)}
+
+
+@pytest.mark.parametrize("step", list(STEPS))
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("shape", [(4, 2, 128, 128, 64), (4, 4, 64, 64, 128), (8, 1, 64, 128, 64), (6, 2, 128, 64, 256)])
+def test_portions(shape, form, step):
+    H, G, D, Dv, bs = shape
+    kw = dict(FORMS[form])
+    bias = kw.pop("bias", False)
+    n_qs, n_ks = STEPS[step]
+    nb = sum(-(-n // bs) for n in n_ks) + 2
+    a, r = (m.ScoreModAttention(H, G, D, Dv, D ** -0.5, device=DEV, **kw) for m in (attention, ref))
+    g = torch.Generator(device=DEV).manual_seed(H * D + Dv)
+    if bias:
+        table = torch.randn(H, 90, generator=g, device=DEV)
+        a.set_distance_bias(table)
+        r.set_distance_bias(table)
+    if a.sink is not None:
+        with torch.no_grad():
+            a.sink.copy_(3 * torch.randn(H, generator=g, device=DEV))
+            r.sink.copy_(a.sink)
+    ctx, pos = _context(n_qs, n_ks, bs, nb, seed=4)
+    ctx.num_decode_seqs = sum(n == 1 for n in n_qs)
+    T = sum(n_qs)
+    mk = lambda *s: (2 * torch.randn(*s, generator=g, device=DEV)).to(torch.bfloat16)
+    q, k, v = mk(T, H, D), mk(T, G, D), mk(T, G, Dv)
+    kc, vc = mk(nb, bs, G, D), mk(nb, bs, G, Dv)
+    kc_r, vc_r = kc.clone(), vc.clone()
+    nv.set_context(ctx)
+    o, o_r = a(q, k, v, pos, kc, vc), r(q, k, v, pos, kc_r, vc_r)
+    nv.set_context(None)
+    torch.testing.assert_close(kc.float(), kc_r.float(), rtol=2e-2, atol=2e-2)
+    assert torch.equal(vc, vc_r)
+    # probabilities and outputs are rounded to bf16 (2^-9 each) and values are of order two
+    torch.testing.assert_close(o.float(), o_r.float(), rtol=2e-2, atol=2e-2)
