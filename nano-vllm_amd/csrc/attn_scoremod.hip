@@ -410,6 +410,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void attn_scoremod_tile_kernel(
 // small launch that also puts the sink into the denominator.
 constexpr int kDecRep = 8;             // query heads per kv head handled at once (larger groups take further passes)
 constexpr int kDecThreads = 256;
+constexpr float kDecLog2e = 1.4426950408889634f, kDecLn2 = 0.6931471805599453f, kDecInit = -1.0e30f;
 
 template <typename T> struct Vec16;
 template <> struct Vec16<__bf16> { static constexpr int n = 8; };
@@ -428,6 +429,54 @@ __device__ __forceinline__ void load16<float>(const float* p, float* o) {
     const float4 u = *(const float4*)p;
     o[0] = u.x; o[1] = u.y; o[2] = u.z; o[3] = u.w;
 }
+// The four waves' running (max, sum, accumulator) of REP heads meet in LDS (red: [4 waves][repm][2 + Dv]), wave w finishes heads
+// w, w + 4, ...: an output row, or a slice's state in the workspace.
+template <typename T, int REP>
+__device__ __forceinline__ void decode_finish(float* red, int repm, int rep, int head0, int wave, int lane, int split, int splits, int t,
+                                              int64_t T_rows, int H, int Dv, const float* sink, T* out, int64_t out_stride, float* ws) {
+    const int rs = 2 + Dv;
+    __syncthreads();
+    for (int r = wave; r < rep; r += 4) {
+        float mm = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) mm = fmaxf(mm, red[(w * repm + r) * rs]);
+        float ll = 0.f, f[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const float mw = red[(w * repm + r) * rs];
+            f[w] = mw == -INFINITY ? 0.f : expf(mw - mm);      // a wave (or the whole slice) may have had no keys
+            ll += f[w] * red[(w * repm + r) * rs + 1];
+        }
+        const int head = head0 + r;
+        if (splits == 1) {
+            float den = ll, osc = 1.f;
+            if (sink) {
+                const float sk = sink[head], m2 = fmaxf(mm, sk);
+                osc = expf(mm - m2);
+                den = ll * osc + expf(sk - m2);
+            }
+            for (int c = lane; c < Dv; c += 64) {
+                float o = 0.f;
+#pragma unroll
+                for (int w = 0; w < 4; ++w) o += f[w] * red[(w * repm + r) * rs + 2 + c];
+                out[(int64_t)t * out_stride + (int64_t)head * Dv + c] = (T)(o * osc / den);
+            }
+        } else {
+            float* wrow = ws + (((int64_t)split * T_rows + t) * H + head) * rs;
+            if (lane == 0) {
+                wrow[0] = mm;
+                wrow[1] = ll;
+            }
+            for (int c = lane; c < Dv; c += 64) {
+                float o = 0.f;
+#pragma unroll
+                for (int w = 0; w < 4; ++w) o += f[w] * red[(w * repm + r) * rs + 2 + c];
+                wrow[2 + c] = o;
+            }
+        }
+    }
+}
+
 // REP: query heads of a group taken per pass (1, 2, 4 or 8): the per-head registers are sized by it, so small groups
 // run at high occupancy.
 template <typename T, int REP>
@@ -560,46 +609,164 @@ __global__ __launch_bounds__(kDecThreads) void attn_scoremod_decode_kernel(
                 }
             }
         }
-        __syncthreads();
-        for (int r = wave; r < rep; r += 4) {                 // wave w finishes heads w, w + 4, ...
-            float mm = -INFINITY;
+        decode_finish<T, REP>(red, repm, rep, head0, wave, lane, split, splits, t, T_rows, H, Dv, sink, out, out_stride, ws);
+    }
+}
+
+// The same for bf16 rows of 64 or 128 columns on pages of whole tiles: lanes share a row from the start.  A load instruction of the
+// wave covers whole rows (16 bytes a lane), for the keys as for the values, a tile's loads are all on their way while the one
+// before is computed, and a key's score is joined over its row's lanes by DPP adds.  (A lane that walks a key row of its own touches 64 rows
+// with every load and has eight of them in flight.)  CAP: a soft cap of at most 40 and no bias; the cap is the reference of the
+// exponentials, without a maximum.  256 rows over 513 .. 768 keys, 16 / 8 heads of 128, whole call with its
+// preparation: 219 -> 110 us, 6.1 TB/s; 64 rows over 1500 keys, eight heads a kv head: 99 -> 42 us (with a bias 102 -> 98).
+template <int CK, int CV, int REP, bool CAP>      // 16-byte pieces of a key row, of a value row
+__global__ __launch_bounds__(kDecThreads, 2) void attn_scoremod_decode_pieces_kernel(
+    const __bf16* __restrict__ q, const __bf16* __restrict__ k_cache, const __bf16* __restrict__ v_cache, __bf16* __restrict__ out,
+    float* __restrict__ ws, const int* __restrict__ cu_q, const int* __restrict__ cu_k, const int* __restrict__ block_tables,
+    int max_blocks, int H, int G, int block_size, float scale, float softcap, const float* __restrict__ sink,
+    const float* __restrict__ dist_bias, int n_dist, int64_t q_stride, int64_t out_stride, int64_t v_ld, int splits, int slice_keys,
+    int64_t T_rows, int max_block) {
+    // keys of a tile: eight loads a lane (four with eight heads), twice, beside the heads' registers
+    constexpr int KT = (CK + CV == 16 ? 32 : 16) / (REP <= 4 ? 1 : 2);
+    constexpr int LK = KT * CK / 64, LV = KT * CV / 64, RK = 64 / CK, RV = 64 / CV;     // loads a tile, rows a load
+    constexpr int D = 8 * CK, Dv = 8 * CV, RS = 2 + Dv;
+    __shared__ float red[4 * REP * RS], pw[4][REP][KT];
+    const int b = blockIdx.x, g = blockIdx.y, split = blockIdx.z;
+    const int t = cu_q[b];
+    if (cu_q[b + 1] - t != 1) return;                 // rows of longer portions belong to the other kernels
+    const int n_keys = cu_k[b + 1] - cu_k[b], pos = n_keys - 1, rep_all = H / G;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int* table = block_tables + (int64_t)b * max_blocks;
+    const int k_lo = split * slice_keys, k_hi = min(n_keys, k_lo + slice_keys);
+    const int pk = lane & (CK - 1), sk_ = lane / CK, pv = lane & (CV - 1), sv = lane / CV;
+    const float cap_in = softcap > 0.f ? 2.f * kDecLog2e * scale / softcap : 0.f, cap2 = softcap * kDecLog2e;
+    struct Tile { uint4 k[LK], v[LV]; };
+    auto fetch = [&](int base, Tile& x) {             // (keys past the slice's end: its last one, finite and of weight 0)
+        const int off = base % block_size, last = k_hi - 1 - base;
+        const int phys = min(max(__builtin_amdgcn_readfirstlane(table[base / block_size]), 0), max_block);
+        const int64_t row0 = ((int64_t)phys * block_size + off) * G + g;
+        const __bf16* kb = k_cache + row0 * D + pk * 8;
+        const __bf16* vb = v_cache + row0 * v_ld + pv * 8;
 #pragma unroll
-            for (int w = 0; w < 4; ++w) mm = fmaxf(mm, red[(w * repm + r) * rs]);
-            float ll = 0.f, f[4];
+        for (int i = 0; i < LK; ++i) x.k[i] = load_stream16((const uint4*)(kb + (int64_t)min(i * RK + sk_, last) * G * D));
 #pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                const float mw = red[(w * repm + r) * rs];
-                f[w] = mw == -INFINITY ? 0.f : expf(mw - mm);  // a wave (or the whole slice) may have had no keys
-                ll += f[w] * red[(w * repm + r) * rs + 1];
+        for (int i = 0; i < LV; ++i) x.v[i] = load_stream16((const uint4*)(vb + (int64_t)min(i * RV + sv, last) * G * v_ld));
+    };
+    for (int h0 = 0; h0 < rep_all; h0 += REP) {
+        const int rep = min(REP, rep_all - h0), head0 = g * rep_all + h0;
+        const int first = k_lo + wave * KT;
+        Tile x0, x1;
+        if (first < k_hi) fetch(first, x0);
+        float qf[REP][8], m[REP], l[REP], acc[REP][8];
+#pragma unroll
+        for (int r = 0; r < REP; ++r) {
+            load16<__bf16>(q + (int64_t)t * q_stride + (int64_t)(head0 + min(r, rep - 1)) * D + pk * 8, qf[r]);
+            m[r] = CAP ? cap2 : kDecInit;             // log2 units
+            l[r] = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[r][e] = 0.f;
+        }
+        auto step = [&](int base, const Tile& x) {
+            float p[REP][LK];
+#pragma unroll
+            for (int i = 0; i < LK; ++i) {
+                float kv[8];
+                const uint4 u = x.k[i];
+                kv[0] = bf16_lo(u.x); kv[1] = bf16_hi(u.x); kv[2] = bf16_lo(u.y); kv[3] = bf16_hi(u.y);
+                kv[4] = bf16_lo(u.z); kv[5] = bf16_hi(u.z); kv[6] = bf16_lo(u.w); kv[7] = bf16_hi(u.w);
+                const int j = base + i * RK + sk_;
+#pragma unroll
+                for (int r = 0; r < REP; ++r) {
+                    float s = qf[r][0] * kv[0];
+#pragma unroll
+                    for (int e = 1; e < 8; ++e) s += qf[r][e] * kv[e];
+                    s += dpp_f32<0xB1>(s);
+                    s += dpp_f32<0x4E>(s);
+                    s += dpp_f32<0x141>(s);
+                    if constexpr (CK == 16) s += dpp_f32<0x140>(s);
+                    if constexpr (CAP) {
+                        s = __builtin_amdgcn_exp2f(-2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(s * cap_in) + 1.0f));
+                        p[r][i] = j < k_hi ? s : 0.f;
+                    } else {
+                        if (softcap > 0.f) s = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(s * cap_in) + 1.0f);
+                        else s *= scale * kDecLog2e;
+                        if (dist_bias) s += kDecLog2e * dist_bias[(int64_t)(head0 + min(r, rep - 1)) * n_dist + min(max(pos - j, 0), n_dist - 1)];
+                        p[r][i] = j < k_hi ? s : -INFINITY;
+                    }
+                }
             }
-            const int head = head0 + r;
-            if (splits == 1) {
-                float den = ll, osc = 1.f;
-                if (sink) {
-                    const float sk = sink[head], m2 = fmaxf(mm, sk);
-                    osc = expf(mm - m2);
-                    den = ll * osc + expf(sk - m2);
-                }
-                for (int c = lane; c < Dv; c += 64) {
-                    float o = 0.f;
+            if constexpr (!CAP) {
 #pragma unroll
-                    for (int w = 0; w < 4; ++w) o += f[w] * red[(w * repm + r) * rs + 2 + c];
-                    out[(int64_t)t * out_stride + (int64_t)head * Dv + c] = (T)(o * osc / den);
-                }
-            } else {
-                float* wrow = ws + (((int64_t)split * T_rows + t) * H + head) * rs;
-                if (lane == 0) {
-                    wrow[0] = mm;
-                    wrow[1] = ll;
-                }
-                for (int c = lane; c < Dv; c += 64) {
-                    float o = 0.f;
+                for (int r = 0; r < REP; ++r) {
+                    float tm = p[r][0];
 #pragma unroll
-                    for (int w = 0; w < 4; ++w) o += f[w] * red[(w * repm + r) * rs + 2 + c];
-                    wrow[2 + c] = o;
+                    for (int i = 1; i < LK; ++i) tm = fmaxf(tm, p[r][i]);
+                    for (int o = CK; o < 64; o *= 2) tm = fmaxf(tm, __shfl_xor(tm, o));
+                    const float m_new = fmaxf(m[r], tm), corr = __builtin_amdgcn_exp2f(m[r] - m_new);
+                    m[r] = m_new;
+                    l[r] *= corr;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) acc[r][e] *= corr;
+#pragma unroll
+                    for (int i = 0; i < LK; ++i) p[r][i] = __builtin_amdgcn_exp2f(p[r][i] - m_new);
                 }
+            }
+#pragma unroll
+            for (int r = 0; r < REP; ++r) {
+#pragma unroll
+                for (int i = 0; i < LK; ++i) l[r] += p[r][i];
+            }
+            if constexpr (CK != CV) {                 // the value rows lie in other lanes: the weights go through LDS (the wave's own)
+                if (pk == 0) {
+#pragma unroll
+                    for (int r = 0; r < REP; ++r)
+#pragma unroll
+                        for (int i = 0; i < LK; ++i) pw[wave][r][i * RK + sk_] = p[r][i];
+                }
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            }
+#pragma unroll
+            for (int i = 0; i < LV; ++i) {
+                float vv[8];
+                const uint4 u = x.v[i];
+                vv[0] = bf16_lo(u.x); vv[1] = bf16_hi(u.x); vv[2] = bf16_lo(u.y); vv[3] = bf16_hi(u.y);
+                vv[4] = bf16_lo(u.z); vv[5] = bf16_hi(u.z); vv[6] = bf16_lo(u.w); vv[7] = bf16_hi(u.w);
+#pragma unroll
+                for (int r = 0; r < REP; ++r) {
+                    const float w = CK == CV ? p[r][CK == CV ? i : 0] : pw[wave][r][i * RV + sv];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) acc[r][e] += w * vv[e];
+                }
+            }
+            if constexpr (CK != CV) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        };
+        int base = first;
+        for (; base + 4 * KT < k_hi; base += 8 * KT) {        // the slice's tiles are dealt to the four waves in turn
+            fetch(base + 4 * KT, x1);
+            step(base, x0);
+            if (base + 8 * KT < k_hi) fetch(base + 8 * KT, x0);
+            step(base + 4 * KT, x1);
+        }
+        if (base < k_hi) step(base, x0);
+        __syncthreads();                              // (a second pass over the heads: the first one's states have been read)
+#pragma unroll
+        for (int r = 0; r < REP; ++r) {
+            for (int o = CK; o < 64; o *= 2) l[r] += __shfl_xor(l[r], o);
+            for (int o = CV; o < 64; o *= 2) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) acc[r][e] += __shfl_xor(acc[r][e], o);
+            }
+            float* dst = red + (wave * REP + r) * RS;
+            if (lane == 0) {
+                dst[0] = l[r] > 0.f ? m[r] * kDecLn2 : -INFINITY;             // natural units, as the merge has them
+                dst[1] = l[r];
+            }
+            if (sv == 0) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) dst[2 + pv * 8 + e] = acc[r][e];
             }
         }
+        decode_finish<__bf16, REP>(red, REP, rep, head0, wave, lane, split, splits, t, T_rows, H, Dv, sink, out, out_stride, ws);
     }
 }
 
@@ -815,7 +982,7 @@ extern "C" int nv_attn_scoremod_paged_vld(const void* q, const void* k_cache, co
     while ((vn << cpr_log2) < Dv) ++cpr_log2;
     const bool dec_ok = singles && D % vn == 0 && Dv % vn == 0 && Dv <= 256 && v_ld % vn == 0 && cpr_log2 <= 6 && dec_lds <= 64 * 1024 &&
                         ((uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0;
-    // Rows of whole 32-column subtiles on pages of whole tiles: the 32 x 32 launch (498 -> 117 us with its preparation on 4 prompts of
+    // Rows of whole 32-column subtiles on pages of whole tiles: the 32 x 32 launch (498 -> 130 us with its preparation on 4 prompts of
     // 1777 .. 2048 tokens, 16 / 8 heads of 128, soft cap and sink); other sizes: the 16 x 16 one.
     const bool rows_ok = bf && max_seqlen_q > 1 && scoremod_rows_built(D, Dv, block_size) && v_ld % 8 == 0 && q_stride % 8 == 0 &&
                          out_stride % 8 == 0 && (int64_t)G * std::max<int64_t>(v_ld, D) < (1LL << 24) &&
@@ -876,7 +1043,33 @@ extern "C" int nv_attn_scoremod_paged_vld(const void* q, const void* k_cache, co
     else if (repm == 2) NV_DEC_LAUNCH(TT, 2); \
     else if (repm <= 4) NV_DEC_LAUNCH(TT, 4); \
     else NV_DEC_LAUNCH(TT, 8);
-        if (bf) { NV_DEC_BY_REP(__bf16) } else { NV_DEC_BY_REP(float) }
+        if (bf && (D == 64 || D == 128) && (Dv == 64 || Dv == 128) && block_size % 32 == 0 && q_stride % 8 == 0 &&
+            (uintptr_t)q % 16 == 0) {
+            const bool cap = softcap > 0.f && softcap <= 40.f && !dist_bias;
+            const int max_block = (int)std::max<int64_t>(0, std::min<int64_t>(num_blocks - 1, 0x7fffffff));
+#define NV_DEC_PIECES(CK, CV, R, CAP)                                                                                            \
+    hipLaunchKernelGGL((attn_scoremod_decode_pieces_kernel<CK, CV, R, CAP>), dgrid, dim3(kDecThreads), 0, s, (const __bf16*)q,   \
+                       (const __bf16*)k_cache, (const __bf16*)v_cache, (__bf16*)out, (float*)workspace, cu_seqlens_q,            \
+                       cu_seqlens_k, block_tables, max_blocks_per_seq, H, G, block_size, scale, softcap, sink, dist_bias,        \
+                       n_dist, q_stride, out_stride, v_ld, plan.splits, plan.slice_keys, T, max_block)
+#define NV_DEC_PIECES_CAP(CK, CV, R)                \
+    do {                                            \
+        if (cap) NV_DEC_PIECES(CK, CV, R, true);    \
+        else NV_DEC_PIECES(CK, CV, R, false);       \
+    } while (0)
+#define NV_DEC_PIECES_REP(CK, CV)                        \
+    if (repm == 1) NV_DEC_PIECES_CAP(CK, CV, 1);         \
+    else if (repm == 2) NV_DEC_PIECES_CAP(CK, CV, 2);    \
+    else if (repm <= 4) NV_DEC_PIECES_CAP(CK, CV, 4);    \
+    else NV_DEC_PIECES_CAP(CK, CV, 8);
+            if (D == 64 && Dv == 64) { NV_DEC_PIECES_REP(8, 8) }
+            else if (D == 64) { NV_DEC_PIECES_REP(8, 16) }
+            else if (Dv == 64) { NV_DEC_PIECES_REP(16, 8) }
+            else { NV_DEC_PIECES_REP(16, 16) }
+#undef NV_DEC_PIECES_REP
+#undef NV_DEC_PIECES_CAP
+#undef NV_DEC_PIECES
+        } else if (bf) { NV_DEC_BY_REP(__bf16) } else { NV_DEC_BY_REP(float) }
 #undef NV_DEC_BY_REP
 #undef NV_DEC_LAUNCH
 #undef NV_DEC_ARGS

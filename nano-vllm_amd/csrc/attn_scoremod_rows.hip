@@ -6,14 +6,15 @@
 // double-buffered, swizzled in 8-row x 32-column subtiles), and
 //     S^T (keys x rows) = K Q^T        v_mfma_f32_32x32x16_bf16: A = K rows from LDS, B = Q^T in registers
 //     O^T (columns x rows) += V^T P^T  A = V rows read transposed (ds_read_b64_tr_b16), B = P^T, the registers of S^T as bf16
-// A row's scores live in two lanes, so a running maximum is one exchange a tile.  With a soft cap and no bias the cap itself bounds
-// the scores: exponentials are taken relative to the cap, without a maximum (cap <= 40: the smallest, exp(-80), is a normal number
-// in both formats).
+// A row's scores live in two lanes, so a maximum is one exchange a tile.  It is the row's true running maximum (a tile that does not
+// raise it in any row skips the rescale): its largest weight is an exact 1, and an error against 64 bits of 0.0026 stays what it was
+// on 16 x 16 tiles.  Exponentials relative to the soft cap, without any maximum, measured 0.0028 (119 us for the call below), the same
+// with probabilities as the sum of two bf16 numbers 0.0022 (148 us).
 //
 // What bounds it: the vector units.  64 soft-capped scores cost a SIMD two exponentials and a reciprocal at quarter rate, about 70
 // cycles with what is around them, beside 32 cycles of matrix products.  Measured (4 prompts of 1777 .. 2048 tokens, 16 / 8 heads of 128,
-// soft cap and sink): 104 us, 578 TFLOP/s; the launch on 16 x 16 tiles with values transposed through registers, which other sizes
-// still take, 455 us.
+// soft cap and sink, the call with its preparation of 21 us): 130 us; with the launch on 16 x 16 tiles, values transposed through
+// registers, which other sizes still take, 498 us (44 of them preparation).
 #include <algorithm>
 #include <type_traits>
 
@@ -23,14 +24,12 @@ namespace nv {
 
 constexpr int kSrTile = 64;
 constexpr float kSrLog2e = 1.4426950408889634f;
-constexpr float kSrRaise = 8.0f;                      // log2 units a tile may exceed the running maximum without a rescale
 constexpr float kSrInit = -1.0e30f;
-constexpr int kSrWave = 256 / 64;
 
 typedef __attribute__((ext_vector_type(8))) short sr_s16x8;
 typedef __attribute__((address_space(3))) s16x4 sr_lds_s16x4;
 
-enum { kSrPlain = 0, kSrCap = 1, kSrGeneral = 2 };    // scale only | soft cap alone, the cap as reference | cap and / or bias
+enum { kSrPlain = 0, kSrCap = 1, kSrGeneral = 2 };    // scale only | soft cap alone | bias, with a cap or without
 
 // byte offset of 16-byte chunk `ch` of row `row` in the image of a tile whose rows are 32 * C32 columns wide
 template <int C32>
@@ -40,10 +39,6 @@ __device__ __forceinline__ int sr_off(int row, int ch) {
 __device__ __forceinline__ float sr_max_xor32(float x) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float sr_sum_xor32(float x) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
 template <int D32, int V32, int MOD>
@@ -84,8 +79,15 @@ __global__ __launch_bounds__(256, 2) void scoremod_rows_kernel(const ScoremodRow
 #pragma unroll
         for (int i = 0; i < 16; ++i) oacc[d][i] = 0.f;
     const float cap2 = p.softcap * kSrLog2e;
-    float m_run = MOD == kSrCap ? cap2 : kSrInit, l_run = 0.f;
-    const float* bias = MOD == kSrGeneral && p.dist_bias ? p.dist_bias + (int64_t)hq * p.n_dist : nullptr;
+    float m_run = kSrInit;                            // the row's maximum so far, log2 units
+    // The denominator is a product with ones, which the matrix cores have time for (every register of it is the same sum).
+    f32x16 lacc;
+    bf16x8 ones;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) lacc[i] = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.0f;
+    const float* bias = MOD == kSrGeneral ? p.dist_bias + (int64_t)hq * p.n_dist : nullptr;
 
     // staging: one DMA instruction fills 1 KiB of LDS linearly (lane l: bytes 16 l ..), two subtiles; a lane picks the (row, chunk)
     // that the image has there.  Wave w takes pieces w, w + 4, .. of K and of V.
@@ -155,82 +157,54 @@ __global__ __launch_bounds__(256, 2) void scoremod_rows_kernel(const ScoremodRow
         }
         // register i of block kb is key kt + 32 kb + (i & 3) + 8 (i >> 2) + 4 hh; row rw0 + r
         const bool edge = kt + kSrTile - 1 > rw0 + shift;     // some row of the wave does not see all of the tile
-        if constexpr (MOD == kSrCap) {
-            // relative to the cap: log2 weight = -2 cap2 / (exp(2 s / cap) + 1)
-            float psum = 0.f;
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
+        for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const float E = __builtin_amdgcn_exp2f(s[kb][i] * p.cap_in);
-                    s[kb][i] = __builtin_amdgcn_exp2f(-2.f * cap2 * __builtin_amdgcn_rcpf(E + 1.0f));
+            for (int i = 0; i < 16; ++i) {
+                float x = s[kb][i];
+                if (MOD == kSrCap || (MOD == kSrGeneral && p.softcap > 0.f))       // cap tanh(s / cap) = cap - 2 cap / (exp(2 s / cap) + 1)
+                    x = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x * p.cap_in) + 1.0f);
+                else
+                    x *= p.scale_log2;
+                if constexpr (MOD == kSrGeneral) {
+                    const int j = kt + kb * 32 + (i & 3) + 8 * (i >> 2) + 4 * hh;
+                    x += kSrLog2e * bias[min(max(qpos - j, 0), p.n_dist - 1)];
                 }
-            if (edge) {
-#pragma unroll
-                for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i)
-                        s[kb][i] = kt + kb * 32 + (i & 3) + 8 * (i >> 2) + 4 * hh <= qpos ? s[kb][i] : 0.f;
+                s[kb][i] = x;
             }
+        if (edge) {
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) psum += s[kb][i];
-            l_run += psum;
-        } else {
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    float x = s[kb][i];
-                    if constexpr (MOD == kSrGeneral) {
-                        if (p.softcap > 0.f) x = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x * p.cap_in) + 1.0f);
-                        else x *= p.scale_log2;
-                        const int j = kt + kb * 32 + (i & 3) + 8 * (i >> 2) + 4 * hh;
-                        if (bias != nullptr) x += kSrLog2e * bias[min(max(qpos - j, 0), p.n_dist - 1)];
-                    } else {
-                        x *= p.scale_log2;
-                    }
-                    s[kb][i] = x;
-                }
-            if (edge) {
-#pragma unroll
-                for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i)
-                        s[kb][i] = kt + kb * 32 + (i & 3) + 8 * (i >> 2) + 4 * hh <= qpos ? s[kb][i] : -INFINITY;
-            }
-            float tmax = s[0][0];
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, s[kb][i]);
-            tmax = sr_max_xor32(tmax);
-            if (!__all(tmax <= m_run + kSrRaise)) {   // rare after the first tiles
-                const float m_new = fmaxf(m_run, tmax), alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-                m_run = m_new;
-                l_run *= alpha;
-#pragma unroll
-                for (int d = 0; d < V32; ++d)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) oacc[d][i] *= alpha;
-            }
-            float psum = 0.f;
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    s[kb][i] = __builtin_amdgcn_exp2f(s[kb][i] - m_run);
-                    psum += s[kb][i];
-                }
-            l_run += psum;
+                for (int i = 0; i < 16; ++i)
+                    s[kb][i] = kt + kb * 32 + (i & 3) + 8 * (i >> 2) + 4 * hh <= qpos ? s[kb][i] : -INFINITY;
         }
+        float tmax = s[0][0];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, s[kb][i]);
+        tmax = sr_max_xor32(tmax);
+        if (!__all(tmax <= m_run)) {   // rare after the first tiles
+            const float m_new = fmaxf(m_run, tmax), alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+            m_run = m_new;
+            lacc[0] *= alpha;
+#pragma unroll
+            for (int d = 0; d < V32; ++d)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) oacc[d][i] *= alpha;
+        }
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[kb][i] = __builtin_amdgcn_exp2f(s[kb][i] - m_run);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {                 // 16 keys each
             const int kb = c >> 1, s2 = c & 1;
             bf16x8 pb;
 #pragma unroll
             for (int j = 0; j < 8; ++j) pb[j] = (__bf16)s[kb][8 * s2 + j];
+            lacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, pb, lacc, 0, 0, 0);
             const int row1 = kb * 32 + 16 * s2 + 4 * hh + (i16 >> 2), row2 = row1 + 8;
 #pragma unroll
             for (int d = 0; d < V32; ++d) {
@@ -249,7 +223,7 @@ __global__ __launch_bounds__(256, 2) void scoremod_rows_kernel(const ScoremodRow
         if (t + 1 < nt) tile_step(std::integral_constant<int, 1>{}, t + 1);
     }
 
-    float l = sr_sum_xor32(l_run);
+    float l = lacc[0];
     __syncthreads();                                  // every wave is done with the tiles
     if (!wave_live) return;
     unsigned char* stg = lds + wave * (32 * STG);
@@ -352,7 +326,7 @@ ScoremodRowsPlan scoremod_rows_plan(int num_seqs, int64_t T, int H, int G, int D
 template <int D32, int V32>
 static void rows_by_mod(const ScoremodRowsParams& p, hipStream_t s) {
     const dim3 grid((unsigned)(p.grid_base * p.nsplit));
-    if (p.dist_bias != nullptr || p.softcap > 40.f) hipLaunchKernelGGL((scoremod_rows_kernel<D32, V32, kSrGeneral>), grid, dim3(256), 0, s, p);
+    if (p.dist_bias != nullptr) hipLaunchKernelGGL((scoremod_rows_kernel<D32, V32, kSrGeneral>), grid, dim3(256), 0, s, p);
     else if (p.softcap > 0.f) hipLaunchKernelGGL((scoremod_rows_kernel<D32, V32, kSrCap>), grid, dim3(256), 0, s, p);
     else hipLaunchKernelGGL((scoremod_rows_kernel<D32, V32, kSrPlain>), grid, dim3(256), 0, s, p);
 }
