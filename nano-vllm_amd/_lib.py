@@ -91,6 +91,7 @@ MIXERS_PROTOTYPES = {
     "nv_latent_prep_store": (_i32, [_vp, _i64, _i32, _vp, _i64, _i64, _vp, _i64, _vp, _vp, _f32, _i32, _vp, _vp, _vp, _vp,
                                     _vp, _i32, _i64, _i32, _i32, _i32, _f32, _vp]),
     "nv_moe_route": (_i32, [_vp, _vp, _vp, _i64, _i32, _i32, _vp]),
+    "nv_moe_tile_rows_for": (_i32, [_i64, _i32, _i32, _i32, _vp, _i64, _vp, _vp, _i32]),
     "nv_moe_tile_rows": (_i32, [_i64, _i32]),
     "nv_moe_max_tiles": (_i64, [_i64, _i32, _i32]),
     "nv_moe_align": (_i32, [_vp, _vp, _vp, _i64, _i32, _i32, _vp]),

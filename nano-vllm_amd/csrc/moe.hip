@@ -20,6 +20,7 @@
 // [E, rows_out, rows_in] with the contraction index contiguous, as stored.  The launch is sized for the most tiles any
 // routing can produce; workgroups beyond the table's count return at once.
 #include <algorithm>
+#include <type_traits>
 
 #include "mfma_tile.h"
 #include "../../include/nanovllm_hip_mixers.h"
@@ -198,39 +199,253 @@ __global__ __launch_bounds__(64) void moe_route_softmax_kernel(const float* __re
 }
 
 // One workgroup.  meta: [0] = number of tiles, then (expert, first position, rows) per tile.  A pair whose id is not in
-// 0 .. E - 1 (a choice that needs no product) gets no position.
+// 0 .. E - 1 (a choice that needs no product) gets no position.  Every wave counts and places its own range of the pairs through
+// counters of its own (COPIES of them; one for few pairs and when they would not fit LDS): 64 lanes on one table beside 15 other waves spent the time
+// on each other's additions (32768 pairs, 32 experts: 43 -> 21 us).
+template <int COPIES>
 __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__ ids, int* __restrict__ sorted_pairs,
                                                          int* __restrict__ meta, int64_t P, int E, int tile_rows) {
-    extern __shared__ int sm[];                    // [E] counts, [E] cursors
-    int* count = sm;
-    int* cursor = sm + E;
-    const int tid = threadIdx.x;
-    for (int e = tid; e < E; e += 1024) count[e] = 0;
+    extern __shared__ int sm[];                    // [COPIES][E] counts, then cursors; [E + 1] first position, [E + 1] first tile
+    int* first = sm + COPIES * E;
+    int* first_tile = first + E + 1;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    int* mine = sm + (COPIES > 1 ? wave : 0) * E;
+    for (int i = tid; i < COPIES * E; i += 1024) sm[i] = 0;
     __syncthreads();
-    for (int64_t p = tid; p < P; p += 1024) {
-        const int e = ids[p];
-        if (e >= 0 && e < E) atomicAdd(&count[e], 1);
+    const int64_t per = ((P + 15) / 16 + 63) / 64 * 64, p0 = wave * per, p1 = p0 + per < P ? p0 + per : P;
+    for (int64_t p = p0 + lane; p < p1; p += 256) {          // four loads on their way
+        int e[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) e[u] = p + 64 * u < p1 ? ids[p + 64 * u] : -1;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (e[u] >= 0 && e[u] < E) atomicAdd(&mine[e[u]], 1);
+    }
+    __syncthreads();
+    for (int e = tid; e < E; e += 1024) {          // counts to the copies' offsets within the expert, the total to first[e + 1]
+        int off = 0;
+        for (int c = 0; c < COPIES; ++c) {
+            const int n = sm[c * E + e];
+            sm[c * E + e] = off;
+            off += n;
+        }
+        first[e + 1] = off;
+        first_tile[e + 1] = (off + tile_rows - 1) / tile_rows;
     }
     __syncthreads();
     if (tid == 0) {
-        int off = 0, n = 0;
+        first[0] = first_tile[0] = 0;
         for (int e = 0; e < E; ++e) {
-            const int c = count[e];
-            cursor[e] = off;
-            for (int m = 0; m < c; m += tile_rows) {
-                meta[1 + 3 * n] = e;
-                meta[2 + 3 * n] = off + m;
-                meta[3 + 3 * n] = min(tile_rows, c - m);
-                ++n;
-            }
-            off += c;
+            first[e + 1] += first[e];
+            first_tile[e + 1] += first_tile[e];
         }
-        meta[0] = n;
+        meta[0] = first_tile[E];
     }
     __syncthreads();
-    for (int64_t p = tid; p < P; p += 1024) {
-        const int e = ids[p];
-        if (e >= 0 && e < E) sorted_pairs[atomicAdd(&cursor[e], 1)] = (int)p;
+    for (int e = tid; e < E; e += 1024) {
+        for (int c = 0; c < COPIES; ++c) sm[c * E + e] += first[e];
+        for (int n = first_tile[e], m = first[e]; n < first_tile[e + 1]; ++n, m += tile_rows) {
+            meta[1 + 3 * n] = e;
+            meta[2 + 3 * n] = m;
+            meta[3 + 3 * n] = min(tile_rows, first[e + 1] - m);
+        }
+    }
+    __syncthreads();
+    for (int64_t p = p0 + lane; p < p1; p += 256) {
+        int e[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) e[u] = p + 64 * u < p1 ? ids[p + 64 * u] : -1;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (e[u] >= 0 && e[u] < E) sorted_pairs[atomicAdd(&mine[e[u]], 1)] = (int)(p + 64 * u);
+    }
+}
+
+// Many rows per expert, bf16: a workgroup of four waves takes 128 rows of one expert and 256 weight rows (gate and up: 128 columns of
+// both), a wave 64 x 128 of it on v_mfma_f32_32x32x16_bf16 (weights as the first operand, so that a lane holds four neighbouring
+// columns of a row).  Slices 32 deep go straight into LDS (LDS-DMA, chunks swizzled by row so that the 16-byte operand reads are free
+// of bank conflicts); two workgroups share a CU, so that one's products cover the other's barrier, first loads and epilogue.
+// 64 x 128 a wave, because LDS reads come next: 6 KiB for 8 MFMAs of 32 cycles, three quarters of what a CU's LDS delivers; 64 x 64
+// would take all of it.  Rows past the tile repeat its first one, weight rows past N the last one; neither is written.
+// What bounds it: the latency of the slices.  Three buffers, two slices in flight, and one LDS object per buffer: with one array the
+// compiler waits for the loads just issued before it reads another buffer (656 us for the whole call below with two halves of one
+// array, 619 with two objects, 590 .. 605 with three).  Slices 64 deep, one workgroup a CU: 642 us.
+// 8192 tokens, top 4 of 32 experts, width 2048, ff 1024: gate and up 433 -> 338 us, down 354 -> 240 us (the tiles of 64 x 128 below,
+// which other sizes still take, against these); the call 780 -> 600 us.
+constexpr int kMoeBigRows = 128;
+__device__ __forceinline__ int big_off(int row, int ch) { return row * 64 + ((ch ^ ((row >> 2) & 3)) * 16); }
+
+template <int MODE>
+__global__ __launch_bounds__(256, 2) void moe_big_kernel(
+    const __bf16* __restrict__ a, int64_t a_stride, const __bf16* __restrict__ w, const int* __restrict__ sorted_pairs,
+    const int* __restrict__ meta, const float* __restrict__ pair_w, __bf16* __restrict__ y, float* __restrict__ out, int top, int N,
+    int K, float limit, float alpha, float up_shift) {
+    constexpr bool GATE_UP = MODE == 1, GATHER = MODE != 0;
+    constexpr int COLS = GATE_UP ? 128 : 256, XB = kMoeBigRows * 64, BUF = XB + 256 * 64;       // bytes: rows' slice, both slices
+    __shared__ __attribute__((aligned(16))) unsigned char buf0[BUF], buf1[BUF], buf2[BUF];
+    __shared__ int src_row[kMoeBigRows];
+    // Workgroups go to the eight XCDs in turn; an XCD takes a run of the tiles that there are, all column blocks of a tile next to each
+    // other: its L2 then holds a tile's rows for all of them and an expert's weights for its tiles (tiles next to each other instead:
+    // no difference at the call above).
+    const int n_cols = (N + COLS - 1) / COLS, items = meta[0] * n_cols, per_xcd = (items + 7) / 8, at = blockIdx.x / 8;
+    const int item = (blockIdx.x & 7) * per_xcd + at;
+    if (at >= per_xcd || item >= items) return;
+    const int tile = item / n_cols, n0 = (item % n_cols) * COLS;
+    const int e = meta[1 + 3 * tile], row0 = meta[2 + 3 * tile], rows = meta[3 + 3 * tile];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, hh = lane >> 5, wr = wave >> 1, wc = wave & 1;
+    for (int i = tid; i < kMoeBigRows; i += 256) src_row[i] = sorted_pairs[row0 + min(i, rows - 1)];
+    __syncthreads();
+    const __bf16* we = w + (int64_t)e * ((GATE_UP ? 2 : 1) * (int64_t)N) * K;
+    // a piece of 1 KiB: 16 rows of 64 bytes, lane l fills bytes 16 l .. of it
+    const int p_row = lane >> 2, p_ch = (lane & 3) ^ ((p_row >> 2) & 3);
+    const char *xp[2], *wp[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int r = (wave * 2 + i) * 16 + p_row;
+        const int64_t at = GATHER ? (int64_t)(src_row[r] / top) : row0 + min(r, rows - 1);
+        xp[i] = (const char*)(a + at * a_stride + p_ch * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int lr = (wave * 4 + i) * 16 + p_row;   // weight row of the workgroup: gate rows, then up rows
+        const int64_t n = GATE_UP ? (lr >> 7) * (int64_t)N + min(n0 + (lr & 127), N - 1) : min(n0 + lr, N - 1);
+        wp[i] = (const char*)(we + n * K + p_ch * 8);
+    }
+    auto stage = [&](unsigned char* dst) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)xp[i],
+                                             (__attribute__((address_space(3))) void*)(dst + (wave * 2 + i) * 1024), 16, 0, 0);
+            xp[i] += 64;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)wp[i],
+                                             (__attribute__((address_space(3))) void*)(dst + XB + (wave * 4 + i) * 1024), 16, 0, 0);
+            wp[i] += 64;
+        }
+    };
+    f32x16 acc[4][2];                                 // [weight block: gate 0, 1, up 0, 1 | 0 .. 3][row block]
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[j][x][i] = 0.f;
+    auto multiply = [&](const unsigned char* xs) {
+        const unsigned char* ws = xs + XB;
+        bf16x8 xf[2][2], wf[2][4];                    // all operands of the slice are on their way before the first product
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+#pragma unroll
+            for (int x = 0; x < 2; ++x) xf[s][x] = *(const bf16x8*)(xs + big_off(wr * 64 + x * 32 + l32, 2 * s + hh));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int lr = GATE_UP ? (j >> 1) * 128 + wc * 64 + (j & 1) * 32 : wc * 128 + j * 32;
+                wf[s][j] = *(const bf16x8*)(ws + big_off(lr + l32, 2 * s + hh));
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int x = 0; x < 2; ++x) acc[j][x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[s][j], xf[s][x], acc[j][x], 0, 0, 0);
+    };
+    // One slice: this wave's part of it has landed (all but the newest `flying` loads have) and the wave is done reading the one
+    // before; past the barrier so it is for all waves, and the slice after the next one goes where the one before was.
+    // (The builtin, which the compiler's own count of loads in flight follows; __syncthreads would wait for all of them.)
+    auto step = [&](bool more, bool stages, const unsigned char* now, unsigned char* after_next) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);            // (nor may the products sink below the wait)
+        if (more) __builtin_amdgcn_s_waitcnt(0x76);   // vmcnt(6) lgkmcnt(0): the six of the next slice stay in flight
+        else __builtin_amdgcn_s_waitcnt(0x70);        // vmcnt(0) lgkmcnt(0)
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (stages) stage(after_next);
+        __builtin_amdgcn_sched_barrier(0);            // (the compiler would start the loads behind the products)
+        multiply(now);
+    };
+    const int slices = K / 32;                        // at least 2 (K is a multiple of 64)
+    stage(buf0);
+    stage(buf1);
+    int t = 0;
+    for (; t + 4 < slices; t += 3) {
+        step(true, true, buf0, buf2);
+        step(true, true, buf1, buf0);
+        step(true, true, buf2, buf1);
+    }
+    const int left = slices - t;                      // 2 .. 4
+    step(true, left > 2, buf0, buf2);
+    step(left > 2, left > 3, buf1, buf0);
+    if (left > 2) step(left > 3, false, buf2, buf1);
+    if (left > 3) step(false, false, buf0, buf2);
+    __syncthreads();                                  // the slices are done with: each wave turns its blocks through LDS of its own
+    // lane (l32, hh) holds of row 64 wr + 32 x + l32 the weight rows 8 (i >> 2) + 4 hh + (i & 3) of each block
+    if constexpr (MODE != 0) {
+        constexpr int CW = GATE_UP ? 64 : 128, LD = CW * 2 + 16;       // columns of the wave; bytes of a staged row
+        unsigned char* st = (wave < 2 ? buf0 : buf1) + (wave & 1) * 32 * LD;
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+#pragma unroll
+            for (int j = 0; j < (GATE_UP ? 2 : 4); ++j)
+#pragma unroll
+                for (int i = 0; i < 16; i += 4) {
+                    float v[4];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        if constexpr (GATE_UP) {
+                            const float g = fminf(acc[j][x][i + t], limit);
+                            const float u = fminf(fmaxf(acc[j + 2][x][i + t], -limit), limit);
+                            v[t] = g / (1.0f + expf(-alpha * g)) * (u + up_shift);
+                        } else {
+                            const float u = fmaxf(acc[j][x][i + t], 0.f);
+                            v[t] = u * u;
+                        }
+                    }
+                    *(uint2*)(st + l32 * LD + (j * 32 + 2 * i + 4 * hh) * 2) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+                }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            constexpr int LPR = CW / 8;               // lanes a row, 16 bytes each
+#pragma unroll
+            for (int it = 0; it < 32 * LPR / 64; ++it) {
+                const int rr = it * (64 / LPR) + lane / LPR, c = (lane % LPR) * 8, r = wr * 64 + x * 32 + rr, n = n0 + wc * CW + c;
+                const uint4 v = *(const uint4*)(st + rr * LD + c * 2);
+                if (r < rows && n < N) *(uint4*)(y + (int64_t)(row0 + r) * N + n) = v;
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
+    } else {
+        constexpr int LD = 64 * 4 + 16;
+        unsigned char* st = (wave < 2 ? buf0 : buf1) + (wave & 1) * 32 * LD;
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {    // 64 columns at a time
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int i = 0; i < 16; i += 4) {
+                        const f32x16& c = acc[2 * half + j][x];
+                        *(float4*)(st + l32 * LD + (j * 32 + 2 * i + 4 * hh) * 4) = make_float4(c[i], c[i + 1], c[i + 2], c[i + 3]);
+                    }
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+                for (int it = 0; it < 8; ++it) {
+                    const int rr = it * 4 + (lane >> 4), c = (lane & 15) * 4, r = wr * 64 + x * 32 + rr, n = n0 + wc * 128 + half * 64 + c;
+                    float4 v = *(const float4*)(st + rr * LD + c * 4);
+                    if (r < rows && n < N) {
+                        const int pair = src_row[r];
+                        const float f = pair_w[pair];
+                        v.x *= f; v.y *= f; v.z *= f; v.w *= f;
+                        *(float4*)(out + (int64_t)pair * N + n) = v;
+                    }
+                }
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            }
+        }
     }
 }
 
@@ -348,9 +563,17 @@ template <typename T, int MODE>
 static void launch_grouped(const void* a, int64_t a_stride, const void* w, const int* sorted_pairs, const int* meta,
                            const float* pair_w, void* y, float* out, int top, int N, int K, float limit, float alpha,
                            float up_shift, int max_tiles, int tile_rows, hipStream_t s) {
+    if constexpr (sizeof(T) == 2) {
+        if (tile_rows == kMoeBigRows) {               // (the caller has checked sizes and alignment)
+            constexpr int cols = MODE == 1 ? 128 : 256;
+            hipLaunchKernelGGL(moe_big_kernel<MODE>, dim3((unsigned)(((int64_t)max_tiles * ((N + cols - 1) / cols) + 7) / 8 * 8)), dim3(256), 0, s,
+                               (const T*)a, a_stride, (const T*)w, sorted_pairs, meta, pair_w, (T*)y, out, top, N, K, limit, alpha, up_shift);
+            return;
+        }
+    }
     const int vec = TileMma<T>::kVec;
     const int vec_ok = K % vec == 0 && a_stride % vec == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0;
-    // many rows per expert: 64 x 128 tiles (a wave owns 32 columns; 128-row tiles measured slower: one workgroup per CU);
+    // many rows per expert: 64 x 128 tiles (a wave owns 32 columns; 128 rows of this kernel measured slower: one workgroup per CU);
     // few: 16 x 64 tiles, more workgroups per weight byte
 #define NV_MOE_LAUNCH(MT, NT)                                                                                          \
     hipLaunchKernelGGL((moe_grouped_kernel<T, MT, NT, MODE>), dim3((unsigned)(max_tiles * ((N + 64 * NT - 1) / (64 * NT)))), \
@@ -378,6 +601,18 @@ extern "C" int nv_moe_route(const float* logits, int32_t* ids, float* weights, i
 
 extern "C" int nv_moe_tile_rows(int64_t pairs, int E) { return pairs >= 32 * (int64_t)E ? 64 : 16; }
 
+// Rows of 128 take pairs of whole 32-deep slices and 16-byte pieces of both products' rows.
+static bool moe_big_ok(int dtype, const void* a, int64_t a_stride, const void* w, int N, int K) {
+    return dtype == NV_DTYPE_BF16 && K % 64 == 0 && N % 8 == 0 && a_stride % 8 == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0;
+}
+
+// 128 rows from 96 per expert on: fewer leave most of a tile empty.
+extern "C" int nv_moe_tile_rows_for(int64_t pairs, int E, int width, int ff, const void* h, int64_t h_stride, const void* up,
+                                    const void* down, int dtype) {
+    const bool big = pairs >= 96 * (int64_t)E && moe_big_ok(dtype, h, h_stride, up, ff, width) && moe_big_ok(dtype, down, ff, down, width, ff);
+    return big ? nv::kMoeBigRows : nv_moe_tile_rows(pairs, E);
+}
+
 extern "C" int64_t nv_moe_max_tiles(int64_t pairs, int E, int tile_rows) {
     return pairs / tile_rows + std::min<int64_t>(pairs, E);
 }
@@ -385,12 +620,18 @@ extern "C" int64_t nv_moe_max_tiles(int64_t pairs, int E, int tile_rows) {
 extern "C" int nv_moe_align(const int32_t* ids, int32_t* sorted_pairs, int32_t* meta, int64_t pairs, int E,
                             int tile_rows, void* stream) {
     using namespace nv;
-    NV_REQUIRE(pairs >= 0 && E > 0 && E <= 4096 && (tile_rows == 16 || tile_rows == 64), NV_ERR_INVALID_ARG,
+    NV_REQUIRE(pairs >= 0 && E > 0 && E <= 4096 && (tile_rows == 16 || tile_rows == 64 || tile_rows == 128), NV_ERR_INVALID_ARG,
                "nv_moe_align: bad sizes");
     NV_REQUIRE(ids && sorted_pairs && meta, NV_ERR_INVALID_ARG, "nv_moe_align: null pointer");
     NV_REQUIRE(pairs < (1LL << 31), NV_ERR_UNSUPPORTED, "nv_moe_align: too many pairs");
-    hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(1024), sizeof(int) * 2 * (size_t)E, (hipStream_t)stream, ids,
-                       sorted_pairs, meta, pairs, E, tile_rows);
+    const size_t tables = sizeof(int) * 2 * ((size_t)E + 1);
+    // few pairs: one table, since joining the copies then costs more than the additions (128 pairs: 0.6 us of the whole call)
+    if (E <= 512 && pairs >= 4096)
+        hipLaunchKernelGGL(moe_align_kernel<16>, dim3(1), dim3(1024), sizeof(int) * 16 * (size_t)E + tables, (hipStream_t)stream, ids,
+                           sorted_pairs, meta, pairs, E, tile_rows);
+    else
+        hipLaunchKernelGGL(moe_align_kernel<1>, dim3(1), dim3(1024), sizeof(int) * (size_t)E + tables, (hipStream_t)stream, ids,
+                           sorted_pairs, meta, pairs, E, tile_rows);
     return check_launch("nv_moe_align");
 }
 
@@ -405,11 +646,13 @@ extern "C" int nv_moe_gate_up_act(const void* h, int64_t h_stride, const void* g
                                   const int32_t* meta, void* y, int dtype, int64_t pairs, int E, int top, int width,
                                   int ff, float limit, float alpha, float up_shift, int tile_rows, void* stream) {
     using namespace nv;
-    NV_REQUIRE(pairs >= 0 && E > 0 && top > 0 && width > 0 && ff > 0 && (tile_rows == 16 || tile_rows == 64),
+    NV_REQUIRE(pairs >= 0 && E > 0 && top > 0 && width > 0 && ff > 0 && (tile_rows == 16 || tile_rows == 64 || tile_rows == 128),
                NV_ERR_INVALID_ARG, "nv_moe_gate_up: bad sizes");
     if (pairs == 0) return NV_OK;
     NV_REQUIRE(h && gate_up && sorted_pairs && meta && y, NV_ERR_INVALID_ARG, "nv_moe_gate_up: null pointer");
     NV_REQUIRE(dtype == NV_DTYPE_BF16 || dtype == NV_DTYPE_F32, NV_ERR_INVALID_ARG, "nv_moe_gate_up: bad dtype");
+    NV_REQUIRE(tile_rows != 128 || ((uintptr_t)y % 16 == 0 && moe_big_ok(dtype, h, h_stride, gate_up, ff, width)), NV_ERR_UNSUPPORTED,
+               "nv_moe_gate_up: tiles of 128 rows take bf16 rows in whole pieces");
     const int64_t tiles = nv_moe_max_tiles(pairs, E, tile_rows);
     NV_REQUIRE(tiles * ((ff + kMoeBN - 1) / kMoeBN) < (1LL << 31), NV_ERR_UNSUPPORTED, "nv_moe_gate_up: launch too large");
     hipStream_t s = (hipStream_t)stream;
@@ -426,11 +669,13 @@ extern "C" int nv_moe_down(const void* y, const void* down, const int32_t* sorte
                            const float* pair_weights, float* out, int dtype, int64_t pairs, int E, int width, int ff,
                            int tile_rows, void* stream) {
     using namespace nv;
-    NV_REQUIRE(pairs >= 0 && E > 0 && width > 0 && ff > 0 && (tile_rows == 16 || tile_rows == 64), NV_ERR_INVALID_ARG,
+    NV_REQUIRE(pairs >= 0 && E > 0 && width > 0 && ff > 0 && (tile_rows == 16 || tile_rows == 64 || tile_rows == 128), NV_ERR_INVALID_ARG,
                "nv_moe_down: bad sizes");
     if (pairs == 0) return NV_OK;
     NV_REQUIRE(y && down && sorted_pairs && meta && pair_weights && out, NV_ERR_INVALID_ARG, "nv_moe_down: null pointer");
     NV_REQUIRE(dtype == NV_DTYPE_BF16 || dtype == NV_DTYPE_F32, NV_ERR_INVALID_ARG, "nv_moe_down: bad dtype");
+    NV_REQUIRE(tile_rows != 128 || ((uintptr_t)out % 16 == 0 && moe_big_ok(dtype, y, ff, down, width, ff)), NV_ERR_UNSUPPORTED,
+               "nv_moe_down: tiles of 128 rows take bf16 rows in whole pieces");
     const int64_t tiles = nv_moe_max_tiles(pairs, E, tile_rows);
     NV_REQUIRE(tiles * ((width + kMoeBN - 1) / kMoeBN) < (1LL << 31), NV_ERR_UNSUPPORTED, "nv_moe_down: launch too large");
     hipStream_t s = (hipStream_t)stream;
@@ -464,11 +709,13 @@ extern "C" int nv_moe_up_relu2(const void* h, int64_t h_stride, const void* up, 
                                const int32_t* meta, void* y, int dtype, int64_t pairs, int E, int top, int width, int ff,
                                int tile_rows, void* stream) {
     using namespace nv;
-    NV_REQUIRE(pairs >= 0 && E > 0 && top > 0 && width > 0 && ff > 0 && (tile_rows == 16 || tile_rows == 64),
+    NV_REQUIRE(pairs >= 0 && E > 0 && top > 0 && width > 0 && ff > 0 && (tile_rows == 16 || tile_rows == 64 || tile_rows == 128),
                NV_ERR_INVALID_ARG, "nv_moe_up_relu2: bad sizes");
     if (pairs == 0) return NV_OK;
     NV_REQUIRE(h && up && sorted_pairs && meta && y, NV_ERR_INVALID_ARG, "nv_moe_up_relu2: null pointer");
     NV_REQUIRE(dtype == NV_DTYPE_BF16 || dtype == NV_DTYPE_F32, NV_ERR_INVALID_ARG, "nv_moe_up_relu2: bad dtype");
+    NV_REQUIRE(tile_rows != 128 || ((uintptr_t)y % 16 == 0 && moe_big_ok(dtype, h, h_stride, up, ff, width)), NV_ERR_UNSUPPORTED,
+               "nv_moe_up_relu2: tiles of 128 rows take bf16 rows in whole pieces");
     const int64_t tiles = nv_moe_max_tiles(pairs, E, tile_rows);
     NV_REQUIRE(tiles * ((ff + kMoeBN - 1) / kMoeBN) < (1LL << 31), NV_ERR_UNSUPPORTED, "nv_moe_up_relu2: launch too large");
     hipStream_t s = (hipStream_t)stream;

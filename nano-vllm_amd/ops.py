@@ -793,7 +793,7 @@ def moe_experts(h: torch.Tensor, logits: torch.Tensor, gate_up: torch.Tensor, do
     if T == 0:
         return out
     _lib.check(dll.nv_moe_route(logits.data_ptr(), ids.data_ptr(), wgt.data_ptr(), T, E, int(top), s), "nv_moe_route", dll)
-    rows = dll.nv_moe_tile_rows(P, E)
+    rows = dll.nv_moe_tile_rows_for(P, E, W, ff, h.data_ptr(), h.stride(0), gate_up.data_ptr(), down.data_ptr(), dt)
     tiles = dll.nv_moe_max_tiles(P, E, rows)
     sorted_pairs = torch.empty(P, dtype=torch.int32, device=dev)
     meta = torch.empty(1 + 3 * tiles, dtype=torch.int32, device=dev)
@@ -1140,7 +1140,7 @@ def moe_silu_experts(h: torch.Tensor, ids: torch.Tensor, weights: Optional[torch
     if weights is None:
         weights = torch.ones((T, top), dtype=torch.float32, device=dev)
     _need(weights.shape == (T, top), "weights must be [T, top]")
-    rows = dll.nv_moe_tile_rows(P, E)
+    rows = dll.nv_moe_tile_rows_for(P, E, W, ff, h.data_ptr(), h.stride(0), gate_up.data_ptr(), down.data_ptr(), dt)
     tiles = dll.nv_moe_max_tiles(P, E, rows)
     sorted_pairs = torch.empty(P, dtype=torch.int32, device=dev)
     meta = torch.empty(1 + 3 * tiles, dtype=torch.int32, device=dev)
@@ -1381,7 +1381,7 @@ def moe_relu2_experts(h: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
     out = torch.empty((T, top, W), dtype=torch.float32, device=dev)
     if T == 0:
         return out
-    rows = dll.nv_moe_tile_rows(P, E)
+    rows = dll.nv_moe_tile_rows_for(P, E, W, ff, h.data_ptr(), h.stride(0), up.data_ptr(), down.data_ptr(), dt)
     tiles = dll.nv_moe_max_tiles(P, E, rows)
     sorted_pairs = torch.empty(P, dtype=torch.int32, device=dev)
     meta = torch.empty(1 + 3 * tiles, dtype=torch.int32, device=dev)
