@@ -12,6 +12,8 @@
 //
 //   rows kernel    sequences with several tokens in the step: a workgroup of four waves takes 128 rows; key tiles of 64
 //                  (32 for wide rows) are staged once for the four waves, double-buffered.
+//                  The loads of the next tile run beside the products of this one only with an LDS object per buffer (16 heads,
+//                  256 columns, 1024 rows of each of 2 sequences of 3000 .. 6001 keys: 303 -> 234 us against two halves of one array).
 //   single kernel  sequences with one token: a workgroup takes up to 32 heads; its four waves take the key tiles of 32 in
 //                  turn, each staging its own (no barrier in the loop), and join their states through LDS.
 //
@@ -197,7 +199,10 @@ template <int D32, int DV32, int KB, int OCC>
 __global__ __launch_bounds__(256, OCC) void attn_latent_rows_kernel(const LatentParams p) {
     constexpr int D = 32 * D32, KT = 32 * KB, kTile = KT * D * 2, kPieces = D32 * KB / 2;
     static_assert(D32 * KB % 2 == 0, "a wave stages whole pieces");
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];      // two tiles; the output staging area at the end
+    // A tile each; two waves' output staging areas at the end.  Two objects, not one array: the compiler tells a tile's reads from
+    // the other tile's LDS-DMA by the object, and with one array it waits for the DMA just issued before the first read.
+    constexpr int BUF = kTile > 2 * kLatRows * kLatStageRow ? kTile : 2 * kLatRows * kLatStageRow;
+    __shared__ __attribute__((aligned(16))) unsigned char buf0[BUF], buf1[BUF];
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int split = blockIdx.y, dv0 = blockIdx.z * DV32, Dv = p.Dv;
@@ -226,34 +231,36 @@ __global__ __launch_bounds__(256, OCC) void attn_latent_rows_kernel(const Latent
         lat_piece<D32>(wave * kPieces + i, lane, dma_row[i], ch);
         dma_off[i] = (uint32_t)(dma_row[i] * (D * 2) + ch * 16);
     }
-    auto stage = [&](int buf, int entry, int t) {
+    auto stage = [&](unsigned char* buf, int entry, int t) {
         const unsigned char* base = lat_tile_base(p, __builtin_amdgcn_readfirstlane(entry), (t % p.tiles_per_block) * KT, D * 2);
         const int last = n_k - 1 - t * KT;                   // rows behind the sequence's end re-read its last row
-        unsigned char* dst = lds + buf * kTile + wave * kPieces * 1024;
+        unsigned char* dst = buf + wave * kPieces * 1024;
 #pragma unroll
         for (int i = 0; i < kPieces; ++i)
             lat_dma(base + (dma_off[i] - (uint32_t)(max(dma_row[i] - last, 0) * (D * 2))), dst + i * 1024);
     };
     int entry_next = 0;
-    if (t_begin < t_end) stage(0, table[t_begin / p.tiles_per_block], t_begin);
+    if (t_begin < t_end) stage(buf0, table[t_begin / p.tiles_per_block], t_begin);
     if (t_begin + 1 < t_end) entry_next = table[(t_begin + 1) / p.tiles_per_block];
-    int buf = 0;
-    for (int t = t_begin; t < t_end; ++t) {
+    auto tile_step = [&](const unsigned char* now, unsigned char* next, int t) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();                                     // tile t has landed for all, the other buffer is free
-        if (t + 1 < t_end) stage(buf ^ 1, entry_next, t + 1);
+        if (t + 1 < t_end) stage(next, entry_next, t + 1);
         if (t + 2 < t_end) entry_next = table[(t + 2) / p.tiles_per_block];
         const int kt = t * KT;
         if (wave_live && kt <= wave_last_pos)                // (uniform per wave)
-            w.step(lds + buf * kTile, lane, kt, qpos, kt + KT - 1 > wave_first_pos, p.scale_log2, dv0);
-        buf ^= 1;
+            w.step(now, lane, kt, qpos, kt + KT - 1 > wave_first_pos, p.scale_log2, dv0);
+    };
+    for (int t = t_begin; t < t_end; t += 2) {
+        tile_step(buf0, buf1, t);
+        if (t + 1 < t_end) tile_step(buf1, buf0, t + 1);
     }
     const float l_tot = lat_sum_xor32(w.l_run);
     __syncthreads();                                         // every wave is done reading tiles
     if (!wave_live) return;
     // Lane (r, h) holds columns 32 d + 8 (i >> 2) + 4 h + (i & 3) of row r: through the wave's staging area to 128-byte row
     // segments.
-    unsigned char* stg = lds + wave * (kLatRows * kLatStageRow);
+    unsigned char* stg = (wave < 2 ? buf0 : buf1) + (wave & 1) * (kLatRows * kLatStageRow);
     const int rows_here = rows - rw0;
     const int64_t grow = (int64_t)q_begin * p.H + rw0;
     if (p.nsplit > 1) {
@@ -472,14 +479,6 @@ static LatentPlan latent_single_plan(int B, int H, int max_k) {
 template <int D32, int DV32>
 static int launch_latent_rows(LatentParams p, int max_q, int max_k, hipStream_t s) {
     constexpr int KB = D32 <= 8 ? 2 : 1, OCC = D32 <= 5 || (D32 == 6 && DV32 == 4) ? 2 : 1, D = 32 * D32;
-    constexpr size_t rows_lds = (size_t)std::max(2 * 32 * KB * D * 2, 4 * kLatRows * kLatStageRow);
-    static_assert(rows_lds <= 160 * 1024, "LDS of a compute unit");
-    const void* fn = (const void*)attn_latent_rows_kernel<D32, DV32, KB, OCC>;
-    static bool raised = rows_lds <= 64 * 1024;              // beyond the default limit of dynamic LDS: raise it once
-    if (!raised) {
-        if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)rows_lds) != hipSuccess) return NV_ERR_LAUNCH;
-        raised = true;
-    }
     const LatentPlan plan = latent_rows_plan(p.B, p.H, max_q, max_k, D);
     p.nsplit = plan.nsplit;
     p.tiles_per_split = plan.tiles_per_split;
@@ -487,7 +486,7 @@ static int launch_latent_rows(LatentParams p, int max_q, int max_k, hipStream_t 
     p.tiles_per_block = p.block_size / (32 * KB);
     p.dv_groups = p.Dv / (32 * DV32);
     hipLaunchKernelGGL((attn_latent_rows_kernel<D32, DV32, KB, OCC>),
-                       dim3((unsigned)(p.B * p.row_tiles), (unsigned)p.nsplit, (unsigned)p.dv_groups), dim3(256), rows_lds, s, p);
+                       dim3((unsigned)(p.B * p.row_tiles), (unsigned)p.nsplit, (unsigned)p.dv_groups), dim3(256), 0, s, p);
     return check_launch("nv_attn_latent_paged (rows kernel)");
 }
 template <int D32, int DV32>
