@@ -15,6 +15,9 @@
 //                          channel, and the read-out normalised: o / rms(o) * norm_w * sigmoid(gate_raw).
 //                          Everything after the raw projections is fp32.
 //
+// With a workspace and head sizes in steps of 32 up to 128 the recurrence runs in chunks of 8 tokens on the matrix cores
+// (chunk_recurrence.hip).  What follows is the launch for the other sizes and for calls without a workspace.
+//
 // Layout of the recurrence: one workgroup per (sequence, head).  A lane owns one value column and a quarter of the
 // key rows (a contiguous run: its quad index r owns rows r * RPL .. r * RPL + RPL - 1, read from LDS four at a time; the
 // four runs sit RPL + 4 words apart so that the quad's 16-byte reads fall on different banks), so the state lives in

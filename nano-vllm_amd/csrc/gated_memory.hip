@@ -17,6 +17,8 @@
 //   fixed form             (one constant decay per head; fixed_decay.hip takes long portions and owns the entry point)
 //       w = decay[h];   k = silu(k_raw);   v = silu(v_raw);   r = silu(q_raw);   out = o in fp32
 //
+// With a workspace and built sizes the gated write runs in chunks (chunk_recurrence.hip); the launch here serves the rest.
+//
 // Layout as in the decayed-memory kernel next door: one workgroup per (sequence, head); a lane owns one value column
 // and a quarter of the key rows (its quad index q owns rows q * RPL .. q * RPL + RPL - 1, read from LDS four at a time,
 // the four runs RPL + 4 words apart so that a quad's 16-byte reads fall on different banks), so the state lives in

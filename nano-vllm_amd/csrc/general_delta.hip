@@ -8,7 +8,8 @@
 //     S <- diag(w) S - (a * u)(u^T S) + k v^T                           both terms read the old state
 //     o = S^T r;   out = o / sqrt(mean(o^2) + eps) * norm_w * sigmoid(gate_raw)
 //
-// Everything after the raw projections is fp32.  Layout as in the gated delta rule next door: one workgroup per
+// Everything after the raw projections is fp32.  With a workspace and built sizes the tokens run in chunks
+// (chunk_recurrence.hip); the launch here serves the rest.  Layout as in the gated delta rule next door: one workgroup per
 // (sequence, head); a lane owns one value column and a quarter of the key rows (its quad index r owns rows
 // r * RPL .. r * RPL + RPL - 1, read from LDS four at a time, the four runs RPL + 4 words apart so that a quad's 16-byte
 // reads fall on different banks), so the state lives in registers and the token loop has no workgroup barrier: the
