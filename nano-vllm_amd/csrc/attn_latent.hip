@@ -13,7 +13,7 @@
 //   rows kernel    sequences with several tokens in the step: a workgroup of four waves takes 128 rows; key tiles of 64
 //                  (32 for wide rows) are staged once for the four waves, double-buffered.
 //                  The loads of the next tile run beside the products of this one only with an LDS object per buffer (16 heads,
-//                  256 columns, 1024 rows of each of 2 sequences of 3000 .. 6001 keys: 303 -> 234 us against two halves of one array).
+//                  256 columns, 1024 rows of each of 2 sequences of 3000 and 6001 keys: 302 -> 233 us against two halves of one array).
 //   single kernel  sequences with one token: a workgroup takes up to 32 heads; its four waves take the key tiles of 32 in
 //                  turn, each staging its own (no barrier in the loop), and join their states through LDS.
 //
@@ -99,18 +99,40 @@ struct LatentWave {
 
     // A tile of 32 KB keys at `lds`, the first of them key kt; the lane's row sees keys <= qpos (masked: some row of the wave
     // does not see all of the tile).  The wave accumulates the value columns from 32 dv0 on.
+    // FAR: operands of the first product two steps ahead, the key blocks in turn (rows kernel: 233 -> 221 us at the call above; the
+    // single kernel, whose waves cover each other, lost 1 % with it).
+    template <bool FAR>
     __device__ __forceinline__ void step(const unsigned char* lds, int lane, int kt, int qpos, bool masked, float scale_log2,
                                          int dv0) {
         const int r = lane & 31, h = lane >> 5, i16 = lane & 15, g16 = (lane >> 4) & 1;
         f32x16 sacc[KB];
 #pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
+        for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
             for (int i = 0; i < 16; ++i) sacc[kb][i] = 0.f;
+        if constexpr (!FAR) {
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                for (int s = 0; s < 2 * D32; ++s) {
+                    const bf16x8 a = *(const bf16x8*)(lds + lat_off<D32>(kb * 32 + r, 2 * s + h));
+                    sacc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[s], sacc[kb], 0, 0, 0);
+                }
+        } else {
+            constexpr int AHEAD = 2;                                 // operand steps on their way before a product needs them
+            bf16x8 a[2 * D32][KB];
+            auto fetch = [&](int s) {
+#pragma unroll
+                for (int kb = 0; kb < KB; ++kb) a[s][kb] = *(const bf16x8*)(lds + lat_off<D32>(kb * 32 + r, 2 * s + h));
+            };
+#pragma unroll
+            for (int s = 0; s < AHEAD; ++s) fetch(s);
 #pragma unroll
             for (int s = 0; s < 2 * D32; ++s) {
-                const bf16x8 a = *(const bf16x8*)(lds + lat_off<D32>(kb * 32 + r, 2 * s + h));
-                sacc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[s], sacc[kb], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);                   // (left alone, a product waits for the read just before it)
+                if (s + AHEAD < 2 * D32) fetch(s + AHEAD);
+#pragma unroll
+                for (int kb = 0; kb < KB; ++kb) sacc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s][kb], qf[s], sacc[kb], 0, 0, 0);
             }
         }
         // register i of block kb is key kt + 32 kb + (i & 3) + 8 (i >> 2) + 4 h
@@ -249,7 +271,7 @@ __global__ __launch_bounds__(256, OCC) void attn_latent_rows_kernel(const Latent
         if (t + 2 < t_end) entry_next = table[(t + 2) / p.tiles_per_block];
         const int kt = t * KT;
         if (wave_live && kt <= wave_last_pos)                // (uniform per wave)
-            w.step(now, lane, kt, qpos, kt + KT - 1 > wave_first_pos, p.scale_log2, dv0);
+            w.template step<true>(now, lane, kt, qpos, kt + KT - 1 > wave_first_pos, p.scale_log2, dv0);
     };
     for (int t = t_begin; t < t_end; t += 2) {
         tile_step(buf0, buf1, t);
@@ -348,7 +370,7 @@ __global__ __launch_bounds__(256, OCC) void attn_latent_single_kernel(const Late
     for (; t < t_end; t += 4) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // this wave's own tile has landed
         if (NBUF == 2 && t + 4 < t_end) stage(buf ^ 1, t + 4);
-        w.step(mine + buf * kTile, lane, t * KT, n_k - 1, t * KT + KT > n_k, p.scale_log2, dv0);
+        w.template step<false>(mine + buf * kTile, lane, t * KT, n_k - 1, t * KT + KT > n_k, p.scale_log2, dv0);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // its reads are done before the buffer is filled again
         if (NBUF == 1 && t + 4 < t_end) stage(0, t + 4);
         if (NBUF == 2) buf ^= 1;
