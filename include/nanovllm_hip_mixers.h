@@ -507,7 +507,8 @@ NV_API int nv_fixed_decay_memory(const void* q, const void* k, const void* v, in
  * of portion gets its own launch: T rows in all, leading_singles sequences with one row each in front of the batch, `portions`
  * as above for the sequences behind them.  Single tokens stream their states; longer portions run in chunks on the matrix cores
  * (D 32, 64, 96 or 128, Dv a multiple of 16, D * Dv <= 16384) through a workspace of nv_recurrence_workspace_bytes (form: 0 gated
- * delta, 1 generalized delta, 2 gated write).  Other sizes, or no workspace (NULL): as the entry points above, token by token.
+ * delta, 1 generalized delta, 2 gated write).  Other sizes, no workspace (NULL) or T not known (0) while longer portions are
+ * possible: as the entry points above, token by token.
  */
 NV_API int64_t nv_recurrence_workspace_bytes(int form, int64_t T, int H, int D, int Dv, int num_seqs, int leading_singles,
                                              int dtype);

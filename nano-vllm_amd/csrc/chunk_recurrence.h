@@ -36,8 +36,8 @@ struct ChunkRecurrenceArgs {
 int launch_chunk_recurrence(int form, const ChunkRecurrenceArgs& a, int first_seq, bool singles_behind, int dtype, hipStream_t s);
 int launch_single_recurrence(int form, const ChunkRecurrenceArgs& a, int dtype, hipStream_t s);
 
-// The launches of a step by what is known of its portions; *rc is NV_OK when the sizes, the rows or a missing workspace leave
-// the step to the token-by-token launch (false).
+// The launches of a step by what is known of its portions; false, with *rc NV_OK and nothing launched, when the sizes, the rows, a
+// missing workspace or an unknown number of rows (T = 0) leave a step that may hold longer portions to the token-by-token launch.
 bool run_recurrence_portions(int form, ChunkRecurrenceArgs a, int leading_singles, int portions, int dtype, void* workspace,
                              int64_t workspace_bytes, hipStream_t s, int* rc);
 

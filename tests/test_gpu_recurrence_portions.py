@@ -90,3 +90,64 @@ def test_portions(form, D, Dv, step, dtype):
         torch.testing.assert_close(got.float(), want.float(), **tol)
         torch.testing.assert_close(got_state, want_state, rtol=2e-5, atol=2e-6 * scale)
     nv.set_context(None)
+
+
+def _operands(form, rows, before, H, D, Dv, dtype, seed, extra=0):
+    """A layer, its eager stand-in, the raw projections by name and the states."""
+    T = sum(rows)
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    mk = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    a, r = _layers(form, H, D, Dv, mk)
+    G = H // 2 if form == "gated" else H
+    x = dict(q=mk(T, G, D), k=mk(T, G, D), v=mk(T, H, Dv), w=mk(T, H * D), a=mk(T, H * D), b=mk(T, H), gate=mk(T, H * Dv))
+    return a, r, {n: t.to(dtype) for n, t in x.items()}, mk(len(rows) + 2, H, D, Dv)
+
+
+def _forward(form, m, x, state):
+    if form == "gated":
+        return m(x["q"], x["k"], x["v"], x["w"], x["b"], x["gate"], state)
+    if form == "general":
+        return m(x["q"], x["k"], x["v"], x["w"], x["a"], x["gate"], state)
+    return m(x["q"], x["k"], x["v"], {"state": state})
+
+
+@pytest.mark.parametrize("entry", ["plain", "no_workspace", "no_rows"])
+@pytest.mark.parametrize("form", ["gated", "general", "write"])
+def test_entries_without_workspace(form, entry):
+    """The C entries without portions, and those with portions but no workspace or an unknown number of rows, go token by token at
+    sizes that have a launch in chunks too."""
+    from nanovllm_amd import _lib
+    rows, before = [1, 9, 30, 1], [4, 0, 7, 0]
+    H, D, T = 4, 128, sum(rows)
+    a, r, x, state = _operands(form, rows, before, H, D, D, torch.float32, 5)
+    ctx = _context(rows, before, True)
+    nv.set_context(ctx)
+    want_state, got_state = state.clone(), state.clone()
+    want = _forward(form, r, x, want_state)
+    nv.set_context(None)
+    out = torch.full((T, H * D), float("nan"), device=DEV)
+    dll, p = _lib.mixers(), lambda t: t.data_ptr()
+    q, k, v = (x[n] for n in "qkv")
+    seqs = [p(ctx.cu_seqlens_q), p(ctx.cu_seqlens_k), p(ctx.state_slots), len(rows)]
+    sizes = {"gated": [H, H // 2, D, D, 1e-5], "general": [H, D, 1e-5, getattr(a, "decay_rate", 0.0), getattr(a, "key_eps", 0.0)],
+             "write": [H, D, D, 1e-5]}[form]
+    head = [p(q), p(k), p(v), q.stride(0), k.stride(0), v.stride(0)]
+    if form == "gated":
+        head += [p(x["w"]), H * D, p(x["b"]), H, p(x["gate"]), H * D, p(a.A_log), p(a.dt_bias), p(a.norm_weight)]
+    elif form == "general":
+        head += [p(x["w"]), H * D, p(x["a"]), H * D, p(x["gate"]), H * D, p(a.w_bias), p(a.a_bias), p(a.norm_weight)]
+    else:
+        head += [p(a.f_bias), p(a.lower), p(a.norm_weight)]
+    head += [p(got_state), p(out), H * D] + seqs
+    name = {"gated": "nv_gated_delta_rule", "general": "nv_general_delta_rule", "write": "nv_gated_write_memory"}[form]
+    dt, stream = ops._dt(q, "q"), ops._stream(q)
+    if entry == "plain":
+        rc = getattr(dll, name)(*head, *sizes, dt, stream)
+    else:                                  # a workspace without the number of rows is not used
+        ws = torch.empty(1 << 24, dtype=torch.uint8, device=DEV) if entry == "no_rows" else None
+        rc = getattr(dll, name + "_portions")(*head, 0 if entry == "no_rows" else T, *sizes, 1, ops.portion_kinds(rows[1:]), dt,
+                                              p(ws) if ws is not None else None, ws.numel() if ws is not None else 0, stream)
+    _lib.check(rc, name, dll)
+    torch.cuda.synchronize()
+    torch.testing.assert_close(out, want, rtol=5e-5, atol=5e-5)          # (the bounds of test_portions)
+    torch.testing.assert_close(got_state, want_state, rtol=2e-5, atol=2e-6 * want_state.abs().max().item())
