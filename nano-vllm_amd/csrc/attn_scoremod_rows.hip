@@ -277,12 +277,12 @@ __global__ __launch_bounds__(256) void scoremod_rows_merge_kernel(const Scoremod
     const float* base = p.part + ((int64_t)(q_begin + row) * p.H + hq) * p.nsplit * ps;
     float mm = p.sink != nullptr ? p.sink[hq] * kSrLog2e : kSrInit;
     for (int s = 0; s < p.nsplit; ++s)
-        if (base[s * ps + Dv + 1] > 0.f) mm = fmaxf(mm, base[s * ps + Dv]);
+        if (base[s * ps + Dv + 1] != 0.f) mm = fmaxf(mm, base[s * ps + Dv]);
     float den = p.sink != nullptr ? __builtin_amdgcn_exp2f(p.sink[hq] * kSrLog2e - mm) : 0.f;
     float o[2] = {0.f, 0.f};                          // columns lane, lane + 64
     for (int s = 0; s < p.nsplit; ++s) {
         const float l = base[s * ps + Dv + 1];
-        if (!(l > 0.f)) continue;
+        if (l == 0.f) continue;                       // an empty range (not one whose sum is not a number: it counts)
         const float f = __builtin_amdgcn_exp2f(base[s * ps + Dv] - mm);
         den += f * l;
 #pragma unroll

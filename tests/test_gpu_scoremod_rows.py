@@ -50,3 +50,35 @@ def test_portions(shape, form, step):
     assert torch.equal(vc, vc_r)
     # probabilities and outputs are rounded to bf16 (2^-9 each) and values are of order two
     torch.testing.assert_close(o.float(), o_r.float(), rtol=2e-2, atol=2e-2)
+
+
+def _step(H, G, D, Dv, bs, n_qs, n_ks, seed=4, scale=None, spread=1.0, **kw):
+    """A layer, its stand-in, the step's rows and caches (bfloat16)."""
+    a, r = (m.ScoreModAttention(H, G, D, Dv, scale or D ** -0.5, device=DEV, **kw) for m in (attention, ref))
+    g = torch.Generator(device=DEV).manual_seed(H * D + Dv)
+    nb = sum(-(-n // bs) for n in n_ks) + 2
+    ctx, pos = _context(n_qs, n_ks, bs, nb, seed=seed)
+    ctx.num_decode_seqs = sum(n == 1 for n in n_qs)
+    mk = lambda *s: (spread * torch.randn(*s, generator=g, device=DEV)).to(torch.bfloat16)
+    T = sum(n_qs)
+    return a, r, ctx, pos, mk(T, H, D), mk(T, G, D), mk(T, G, Dv), mk(nb, bs, G, D), mk(nb, bs, G, Dv)
+
+
+@pytest.mark.parametrize("where", ["own", "first"])
+@pytest.mark.parametrize("n_qs,n_ks", [([40], [2500]), ([70, 33], [200, 161])])
+@pytest.mark.parametrize("softcap", [0.0, 25.0, 60.0])
+def test_a_key_that_is_not_a_number(softcap, n_qs, n_ks, where):
+    """Every row that sees such a key is not a number, whatever key ranges there are; the other heads do not notice."""
+    H, G, D, bs = 4, 2, 128, 64
+    a, r, ctx, pos, q, k, v, kc, vc = _step(H, G, D, D, bs, n_qs, n_ks, softcap=softcap)
+    nv.set_context(ctx)
+    clean = a(q, k, v, pos, kc.clone(), vc.clone()).view(-1, H, D)
+    if where == "own":
+        k[0, 1] = float("nan")             # the first new token's: all rows of the sequence see it
+    else:
+        kc[ctx.block_tables[0, 0], 0, 1] = float("nan")
+    got = a(q, k, v, pos, kc, vc).view(-1, H, D)
+    nv.set_context(None)
+    n = n_qs[0]
+    assert got[:n, 2:].isnan().all()
+    assert torch.equal(got[:, :2], clean[:, :2]) and torch.equal(got[n:], clean[n:])
