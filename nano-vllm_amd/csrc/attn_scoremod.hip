@@ -758,7 +758,8 @@ __global__ __launch_bounds__(kDecThreads, 2) void attn_scoremod_decode_pieces_ke
             }
             float* dst = red + (wave * REP + r) * RS;
             if (lane == 0) {
-                dst[0] = l[r] > 0.f ? m[r] * kDecLn2 : -INFINITY;             // natural units, as the merge has them
+                // natural units, as the merge has them; no keys: -inf (a sum that is not a number is no empty one)
+                dst[0] = l[r] == 0.f ? -INFINITY : m[r] * kDecLn2;
                 dst[1] = l[r];
             }
             if (sv == 0) {

@@ -65,7 +65,7 @@ def _step(H, G, D, Dv, bs, n_qs, n_ks, seed=4, scale=None, spread=1.0, **kw):
 
 
 @pytest.mark.parametrize("where", ["own", "first"])
-@pytest.mark.parametrize("n_qs,n_ks", [([40], [2500]), ([70, 33], [200, 161])])
+@pytest.mark.parametrize("n_qs,n_ks", [([40], [2500]), ([70, 33], [200, 161]), ([1], [1281]), ([1], [1400]), ([1] * 3, [1500, 63, 64])])
 @pytest.mark.parametrize("softcap", [0.0, 25.0, 60.0])
 def test_a_key_that_is_not_a_number(softcap, n_qs, n_ks, where):
     """Every row that sees such a key is not a number, whatever key ranges there are; the other heads do not notice."""
