@@ -65,7 +65,8 @@ __global__ __launch_bounds__(256, 2) void scoremod_rows_kernel(const ScoremodRow
     const int shift = n_k - n_q, rw0 = q0 + (wave / p.hpw) * 32;            // row i sees keys <= i + shift
     const bool wave_live = rw0 < n_q;
     const int max_key = min(min(q0 + rows_per_wg, n_q) - 1 + shift, n_k - 1);
-    const int t_begin = split * p.tiles_per_split, nt = min(max_key / kSrTile + 1, t_begin + p.tiles_per_split);
+    // (no key at all, e.g. a sequence that has none: no tile, or its rows' clamp to the last key would leave the cache)
+    const int t_begin = split * p.tiles_per_split, nt = min(max_key < 0 ? 0 : max_key / kSrTile + 1, t_begin + p.tiles_per_split);
 
     bf16x8 qf[2 * D32];                               // lane (r, hh): Q[row r][16 s + 8 hh ..]
     {

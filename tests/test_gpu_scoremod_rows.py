@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import nanovllm_amd as nv
+from nanovllm_amd import ops
 from nanovllm_amd.layers import attention
 from oracle import ref_mixer_modules as ref
 from test_gpu_mixers import DEV, _context
@@ -82,3 +83,21 @@ def test_a_key_that_is_not_a_number(softcap, n_qs, n_ks, where):
     n = n_qs[0]
     assert got[:n, 2:].isnan().all()
     assert torch.equal(got[:, :2], clean[:, :2]) and torch.equal(got[n:], clean[n:])
+
+
+@pytest.mark.parametrize("sink", [False, True])
+@pytest.mark.parametrize("n_qs,n_ks", [([40, 70], [0, 200]), ([3, 33], [1, 50]), ([130], [0])])
+def test_rows_without_keys(n_qs, n_ks, sink):
+    """Rows that no key precedes are zero (nothing is read for them), whatever stands beside them."""
+    H, G, D, bs = 4, 2, 128, 64
+    a, r, ctx, pos, q, k, v, kc, vc = _step(H, G, D, D, bs, n_qs, [max(n, m) for n, m in zip(n_qs, n_ks)], use_sink=True)
+    cu_k = torch.tensor([0] + torch.tensor(n_ks).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+    call = lambda q, cu_q, cu_k, bt, most: ops.attn_scoremod_paged(q, kc, vc, cu_q, cu_k, bt, D ** -0.5, 0.0, a.sink if sink else None, None,
+                                                                  max(n_qs), most, 0)
+    got = call(q, ctx.cu_seqlens_q, cu_k, ctx.block_tables, max(n_ks))
+    assert got[:n_qs[0] - n_ks[0]].eq(0).all()
+    if len(n_qs) > 1:
+        n = n_qs[0]
+        alone = call(q[n:], torch.tensor([0, n_qs[1]], dtype=torch.int32, device=DEV),
+                     torch.tensor([0, n_ks[1]], dtype=torch.int32, device=DEV), ctx.block_tables[1:], n_ks[1])
+        torch.testing.assert_close(got[n:], alone, rtol=1e-2, atol=1e-2)     # (key ranges may differ)
