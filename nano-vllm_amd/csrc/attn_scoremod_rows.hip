@@ -7,14 +7,16 @@
 //     S^T (keys x rows) = K Q^T        v_mfma_f32_32x32x16_bf16: A = K rows from LDS, B = Q^T in registers
 //     O^T (columns x rows) += V^T P^T  A = V rows read transposed (ds_read_b64_tr_b16), B = P^T, the registers of S^T as bf16
 // A row's scores live in two lanes, so a maximum is one exchange a tile.  It is the row's true running maximum (a tile that does not
-// raise it in any row skips the rescale): its largest weight is an exact 1, and an error against 64 bits of 0.0026 stays what it was
-// on 16 x 16 tiles.  Exponentials relative to the soft cap, without any maximum, measured 0.0028 (119 us for the call below), the same
-// with probabilities as the sum of two bf16 numbers 0.0022 (148 us).
+// raise it in any row skips the rescale), so that its largest weight is an exact 1, and the denominator sums the weights in front of
+// their rounding to bf16, both as on the 16 x 16 tiles: outputs of the call below differ from theirs by 9e-5 and are 0.00258 from
+// the same in 64 bits (2-norms relative to the output rows, bf16), on either.  Exponentials relative to the soft cap, without any
+// maximum: 0.0028 and 119 us; the same with probabilities as the sum of two bf16 numbers: 0.0022 and 148 us.
 //
 // What bounds it: the vector units.  64 soft-capped scores cost a SIMD two exponentials and a reciprocal at quarter rate, about 70
 // cycles with what is around them, beside 32 cycles of matrix products.  Measured (4 prompts of 1777 .. 2048 tokens, 16 / 8 heads of 128,
-// soft cap and sink, the call with its preparation of 21 us): 130 us; with the launch on 16 x 16 tiles, values transposed through
-// registers, which other sizes still take, 498 us (44 of them preparation).
+// soft cap and sink, the call with its preparation of 21 us): 127 us (129 with the denominator as a product of rounded weights with
+// ones); with the launch on 16 x 16 tiles, values transposed through registers, which other sizes still take, 496 us (44 of them
+// preparation).
 #include <algorithm>
 #include <type_traits>
 
@@ -39,6 +41,10 @@ __device__ __forceinline__ int sr_off(int row, int ch) {
 __device__ __forceinline__ float sr_max_xor32(float x) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float sr_sum_xor32(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
 template <int D32, int V32, int MOD>
@@ -81,13 +87,8 @@ __global__ __launch_bounds__(256, 2) void scoremod_rows_kernel(const ScoremodRow
         for (int i = 0; i < 16; ++i) oacc[d][i] = 0.f;
     const float cap2 = p.softcap * kSrLog2e;
     float m_run = kSrInit;                            // the row's maximum so far, log2 units
-    // The denominator is a product with ones, which the matrix cores have time for (every register of it is the same sum).
-    f32x16 lacc;
-    bf16x8 ones;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) lacc[i] = 0.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.0f;
+    // The denominator, this lane's keys: a sum of the weights as computed (of the rounded ones it would be off by up to 2^-9).
+    float l_run = 0.f;
     const float* bias = MOD == kSrGeneral ? p.dist_bias + (int64_t)hq * p.n_dist : nullptr;
 
     // staging: one DMA instruction fills 1 KiB of LDS linearly (lane l: bytes 16 l ..), two subtiles; a lane picks the (row, chunk)
@@ -189,23 +190,27 @@ __global__ __launch_bounds__(256, 2) void scoremod_rows_kernel(const ScoremodRow
         if (!__all(tmax <= m_run)) {   // rare after the first tiles
             const float m_new = fmaxf(m_run, tmax), alpha = __builtin_amdgcn_exp2f(m_run - m_new);
             m_run = m_new;
-            lacc[0] *= alpha;
+            l_run *= alpha;
 #pragma unroll
             for (int d = 0; d < V32; ++d)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) oacc[d][i] *= alpha;
         }
+        float l_part[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) s[kb][i] = __builtin_amdgcn_exp2f(s[kb][i] - m_run);
+            for (int i = 0; i < 16; ++i) {
+                s[kb][i] = __builtin_amdgcn_exp2f(s[kb][i] - m_run);
+                l_part[i & 3] += s[kb][i];
+            }
+        l_run += (l_part[0] + l_part[1]) + (l_part[2] + l_part[3]);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {                 // 16 keys each
             const int kb = c >> 1, s2 = c & 1;
             bf16x8 pb;
 #pragma unroll
             for (int j = 0; j < 8; ++j) pb[j] = (__bf16)s[kb][8 * s2 + j];
-            lacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, pb, lacc, 0, 0, 0);
             const int row1 = kb * 32 + 16 * s2 + 4 * hh + (i16 >> 2), row2 = row1 + 8;
 #pragma unroll
             for (int d = 0; d < V32; ++d) {
@@ -224,7 +229,7 @@ __global__ __launch_bounds__(256, 2) void scoremod_rows_kernel(const ScoremodRow
         if (t + 1 < nt) tile_step(std::integral_constant<int, 1>{}, t + 1);
     }
 
-    float l = lacc[0];
+    float l = sr_sum_xor32(l_run);
     __syncthreads();                                  // every wave is done with the tiles
     if (!wave_live) return;
     unsigned char* stg = lds + wave * (32 * STG);

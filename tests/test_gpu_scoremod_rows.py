@@ -101,3 +101,29 @@ def test_rows_without_keys(n_qs, n_ks, sink):
         alone = call(q[n:], torch.tensor([0, n_qs[1]], dtype=torch.int32, device=DEV),
                      torch.tensor([0, n_ks[1]], dtype=torch.int32, device=DEV), ctx.block_tables[1:], n_ks[1])
         torch.testing.assert_close(got[n:], alone, rtol=1e-2, atol=1e-2)     # (key ranges may differ)
+
+
+@pytest.mark.parametrize("n_qs,n_ks", [([64, 40], [190, 170]), ([40], [2500])])
+def test_denominators_of_portions(n_qs, n_ks):
+    """The denominator is a sum of float32 weights: all but one weight are just below one, where bfloat16 rounds them up."""
+    H, G, D, bs = 4, 2, 128, 64
+    a, r, ctx, pos, q, k, v, kc, vc = _step(H, G, D, D, bs, n_qs, n_ks, scale=1.0)
+    q.zero_()[..., 0] = 1.0
+    for t in (k, kc):
+        t.zero_()[..., 0] = -0.0017013549  # exp of it is 0.9983: 1 in bfloat16
+    v.zero_()
+    vc.zero_()
+    first = ctx.block_tables[:, 0].long()
+    kc[first, 0] = 0.0                     # the largest weight, and the only one with values
+    vc[first, 0] = (1 + torch.rand(G, D, generator=torch.Generator(device=DEV).manual_seed(1), device=DEV)).to(torch.bfloat16)
+    nv.set_context(ctx)
+    o = a(q, k, v, pos, kc, vc)
+    nv.set_context(None)
+    w = torch.tensor(-0.0017013549, dtype=torch.bfloat16).double().exp().item()
+    at = 0
+    for b, (n, m) in enumerate(zip(n_qs, n_ks)):
+        seen = torch.arange(m - n, m, dtype=torch.float64, device=DEV)   # keys in front of each row, with its own
+        want = vc[first[b], 0].double().repeat_interleave(H // G, 0).flatten()[None] / (1 + seen * w)[:, None]
+        # one rounding of the outputs, unbiased over rows * H * D of them; rounded weights would give 1.7e-3
+        assert abs((o[at:at + n].double() / want - 1).mean().item()) < 4e-4
+        at += n
