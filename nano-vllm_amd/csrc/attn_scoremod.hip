@@ -613,12 +613,29 @@ __global__ __launch_bounds__(kDecThreads) void attn_scoremod_decode_kernel(
     }
 }
 
+// cap tanh(s / cap) in log2 units, from a raw score s: cap_in = scale / cap, to2 = scale log2(e), cap2 = cap log2(e).  Right to a few
+// units in the last place for every score, so that the error is one of the score, not of the cap (cap - 2 cap / (e^2y + 1) alone
+// loses a small score against a large cap).  Below |y| = 0.6 a polynomial: (tanh(y) / y - 1) / y^2 through five Chebyshev points in
+// y^2, at most 1.3 * 2^-24 off.  ALL_SMALL: no score of the wave is larger, as with scores well inside the cap; then it costs no more
+// than the exponential and the reciprocal would.
+template <bool ALL_SMALL>
+__device__ __forceinline__ float dec_capped(float s, float cap_in, float to2, float cap2) {
+    const float y = s * cap_in, z = y * y, x = s * to2;
+    const float q = (((-0.0062691197f * z + 0.021110959f) * z - 0.053873949f) * z + 0.13332915f) * z - 0.33333331f;
+    const float small = x + x * (z * q);
+    if constexpr (ALL_SMALL) return small;
+    const float cap = copysignf(cap2, y), e = __builtin_amdgcn_exp2f(fabsf(y) * (2.f * kDecLog2e));
+    return fabsf(y) < 0.6f ? small : cap - 2.f * cap * __builtin_amdgcn_rcpf(e + 1.0f);
+}
+
 // The same for bf16 rows of 64 or 128 columns on pages of whole tiles: lanes share a row from the start.  A load instruction of the
 // wave covers whole rows (16 bytes a lane), for the keys as for the values, a tile's loads are all on their way while the one
 // before is computed, and a key's score is joined over its row's lanes by DPP adds.  (A lane that walks a key row of its own touches 64 rows
-// with every load and has eight of them in flight.)  CAP: a soft cap of at most 40 and no bias; the cap is the reference of the
-// exponentials, without a maximum.  256 rows over 513 .. 768 keys, 16 / 8 heads of 128, whole call with its
-// preparation: 219 -> 110 us, 6.1 TB/s; 64 rows over 1500 keys, eight heads a kv head: 99 -> 42 us (with a bias 102 -> 98).
+// with every load and has eight of them in flight.)  CAP: a soft cap of at most 40 and no bias; e^40 times any number of
+// keys is far from overflow, so the exponentials need no maximum.  256 rows over 513 .. 768 keys, 16 / 8 heads of 128, whole call with its
+// preparation: 219 -> 110 us, 6.1 TB/s.  64 rows over 1500 keys, 64 / 8 heads of 128, which the vector units bound: cap 30
+// 231 -> 121 us, neither cap nor bias 227 -> 145, a bias 243 -> 196 (eight heads without CAP spill 8 to 22 registers; four at a
+// time, which do not, read the keys twice: 266 with a bias, 162 without).
 template <int CK, int CV, int REP, bool CAP>      // 16-byte pieces of a key row, of a value row
 __global__ __launch_bounds__(kDecThreads, 2) void attn_scoremod_decode_pieces_kernel(
     const __bf16* __restrict__ q, const __bf16* __restrict__ k_cache, const __bf16* __restrict__ v_cache, __bf16* __restrict__ out,
@@ -639,7 +656,7 @@ __global__ __launch_bounds__(kDecThreads, 2) void attn_scoremod_decode_pieces_ke
     const int* table = block_tables + (int64_t)b * max_blocks;
     const int k_lo = split * slice_keys, k_hi = min(n_keys, k_lo + slice_keys);
     const int pk = lane & (CK - 1), sk_ = lane / CK, pv = lane & (CV - 1), sv = lane / CV;
-    const float cap_in = softcap > 0.f ? 2.f * kDecLog2e * scale / softcap : 0.f, cap2 = softcap * kDecLog2e;
+    const float cap_in = softcap > 0.f ? scale / softcap : 0.f, to2 = scale * kDecLog2e, cap2 = softcap * kDecLog2e;
     struct Tile { uint4 k[LK], v[LV]; };
     auto fetch = [&](int base, Tile& x) {             // (keys past the slice's end: its last one, finite and of weight 0)
         const int off = base % block_size, last = k_hi - 1 - base;
@@ -661,20 +678,19 @@ __global__ __launch_bounds__(kDecThreads, 2) void attn_scoremod_decode_pieces_ke
 #pragma unroll
         for (int r = 0; r < REP; ++r) {
             load16<__bf16>(q + (int64_t)t * q_stride + (int64_t)(head0 + min(r, rep - 1)) * D + pk * 8, qf[r]);
-            m[r] = CAP ? cap2 : kDecInit;             // log2 units
+            m[r] = CAP ? 0.f : kDecInit;              // log2 units
             l[r] = 0.f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) acc[r][e] = 0.f;
         }
         auto step = [&](int base, const Tile& x) {
-            float p[REP][LK];
+            float p[REP][LK], most = 0.f;             // raw scores, then weights; the largest raw score
 #pragma unroll
             for (int i = 0; i < LK; ++i) {
                 float kv[8];
                 const uint4 u = x.k[i];
                 kv[0] = bf16_lo(u.x); kv[1] = bf16_hi(u.x); kv[2] = bf16_lo(u.y); kv[3] = bf16_hi(u.y);
                 kv[4] = bf16_lo(u.z); kv[5] = bf16_hi(u.z); kv[6] = bf16_lo(u.w); kv[7] = bf16_hi(u.w);
-                const int j = base + i * RK + sk_;
 #pragma unroll
                 for (int r = 0; r < REP; ++r) {
                     float s = qf[r][0] * kv[0];
@@ -684,16 +700,30 @@ __global__ __launch_bounds__(kDecThreads, 2) void attn_scoremod_decode_pieces_ke
                     s += dpp_f32<0x4E>(s);
                     s += dpp_f32<0x141>(s);
                     if constexpr (CK == 16) s += dpp_f32<0x140>(s);
-                    if constexpr (CAP) {
-                        s = __builtin_amdgcn_exp2f(-2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(s * cap_in) + 1.0f));
-                        p[r][i] = j < k_hi ? s : 0.f;
-                    } else {
-                        if (softcap > 0.f) s = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(s * cap_in) + 1.0f);
-                        else s *= scale * kDecLog2e;
-                        if (dist_bias) s += kDecLog2e * dist_bias[(int64_t)(head0 + min(r, rep - 1)) * n_dist + min(max(pos - j, 0), n_dist - 1)];
-                        p[r][i] = j < k_hi ? s : -INFINITY;
-                    }
+                    p[r][i] = s;
+                    most = fmaxf(most, fabsf(s));
                 }
+            }
+            auto each = [&](auto of) {
+#pragma unroll
+                for (int i = 0; i < LK; ++i)
+#pragma unroll
+                    for (int r = 0; r < REP; ++r) p[r][i] = of(p[r][i], r, base + i * RK + sk_);
+            };
+            if (CAP || softcap > 0.f) {
+                if (__all(most * cap_in < 0.6f)) each([&](float s, int, int) { return dec_capped<true>(s, cap_in, to2, cap2); });
+                else each([&](float s, int, int) { return dec_capped<false>(s, cap_in, to2, cap2); });
+            } else {
+                each([&](float s, int, int) { return s * to2; });
+            }
+            if constexpr (CAP) {
+                each([&](float s, int, int j) { return j < k_hi ? __builtin_amdgcn_exp2f(s) : 0.f; });
+            } else {
+                if (dist_bias)
+                    each([&](float s, int r, int j) {
+                        return s + kDecLog2e * dist_bias[(int64_t)(head0 + min(r, rep - 1)) * n_dist + min(max(pos - j, 0), n_dist - 1)];
+                    });
+                each([&](float s, int, int j) { return j < k_hi ? s : -INFINITY; });
             }
             if constexpr (!CAP) {
 #pragma unroll
@@ -983,7 +1013,7 @@ extern "C" int nv_attn_scoremod_paged_vld(const void* q, const void* k_cache, co
     while ((vn << cpr_log2) < Dv) ++cpr_log2;
     const bool dec_ok = singles && D % vn == 0 && Dv % vn == 0 && Dv <= 256 && v_ld % vn == 0 && cpr_log2 <= 6 && dec_lds <= 64 * 1024 &&
                         ((uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0;
-    // Rows of whole 32-column subtiles on pages of whole tiles: the 32 x 32 launch (498 -> 130 us with its preparation on 4 prompts of
+    // Rows of whole 32-column subtiles on pages of whole tiles: the 32 x 32 launch (496 -> 127 us with its preparation on 4 prompts of
     // 1777 .. 2048 tokens, 16 / 8 heads of 128, soft cap and sink); other sizes: the 16 x 16 one.
     const bool rows_ok = bf && max_seqlen_q > 1 && scoremod_rows_built(D, Dv, block_size) && v_ld % 8 == 0 && q_stride % 8 == 0 &&
                          out_stride % 8 == 0 && (int64_t)G * std::max<int64_t>(v_ld, D) < (1LL << 24) &&

@@ -127,3 +127,21 @@ def test_denominators_of_portions(n_qs, n_ks):
         # one rounding of the outputs, unbiased over rows * H * D of them; rounded weights would give 1.7e-3
         assert abs((o[at:at + n].double() / want - 1).mean().item()) < 4e-4
         at += n
+
+
+@pytest.mark.parametrize("softcap", [25.0, 60.0, 1000.0, 1e6])
+@pytest.mark.parametrize("bias", [False, True])
+def test_single_rows_any_soft_cap(softcap, bias):
+    """Scores small against the soft cap: the error is one of the score, not of the cap."""
+    H, G, D, bs = 8, 4, 64, 64
+    n_ks = [700, 64, 130]
+    a, r, ctx, pos, q, k, v, kc, vc = _step(H, G, D, 128, bs, [1] * 3, n_ks, softcap=softcap)
+    if bias:
+        table = torch.randn(H, 90, generator=torch.Generator(device=DEV).manual_seed(2), device=DEV)
+        a.set_distance_bias(table)
+        r.set_distance_bias(table)
+    nv.set_context(ctx)
+    o, o_r = a(q, k, v, pos, kc, vc), r(q, k, v, pos, kc, vc)
+    nv.set_context(None)
+    # fp32 throughout and one rounding of the output (2^-9) on both sides
+    torch.testing.assert_close(o.float(), o_r.float(), rtol=2 ** -7, atol=1e-3)
