@@ -711,7 +711,7 @@ __global__ __launch_bounds__(kDecThreads, 2) void attn_scoremod_decode_pieces_ke
                     for (int r = 0; r < REP; ++r) p[r][i] = of(p[r][i], r, base + i * RK + sk_);
             };
             if (CAP || softcap > 0.f) {
-                if (__all(most * cap_in < 0.6f)) each([&](float s, int, int) { return dec_capped<true>(s, cap_in, to2, cap2); });
+                if (__all(most * fabsf(cap_in) < 0.6f)) each([&](float s, int, int) { return dec_capped<true>(s, cap_in, to2, cap2); });
                 else each([&](float s, int, int) { return dec_capped<false>(s, cap_in, to2, cap2); });
             } else {
                 each([&](float s, int, int) { return s * to2; });

@@ -129,13 +129,14 @@ def test_denominators_of_portions(n_qs, n_ks):
         at += n
 
 
-@pytest.mark.parametrize("softcap", [25.0, 60.0, 1000.0, 1e6])
+@pytest.mark.parametrize("softcap", [1.0, 25.0, 60.0, 1000.0, 1e6])
 @pytest.mark.parametrize("bias", [False, True])
-def test_single_rows_any_soft_cap(softcap, bias):
+@pytest.mark.parametrize("sign", [1, -1])
+def test_single_rows_any_soft_cap(sign, softcap, bias):
     """Scores small against the soft cap: the error is one of the score, not of the cap."""
     H, G, D, bs = 8, 4, 64, 64
     n_ks = [700, 64, 130]
-    a, r, ctx, pos, q, k, v, kc, vc = _step(H, G, D, 128, bs, [1] * 3, n_ks, softcap=softcap)
+    a, r, ctx, pos, q, k, v, kc, vc = _step(H, G, D, 128, bs, [1] * 3, n_ks, scale=sign * D ** -0.5, softcap=softcap)
     if bias:
         table = torch.randn(H, 90, generator=torch.Generator(device=DEV).manual_seed(2), device=DEV)
         a.set_distance_bias(table)
