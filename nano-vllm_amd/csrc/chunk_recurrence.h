@@ -24,6 +24,7 @@ struct ChunkRecurrenceArgs {
     float* chunks;                             // the chunks' operands: [H, records, ..]
     void* columns;                             // their rows of V: [H, records, 8, Dv]
     float* raw;                                // [H, T, Dv]: read-outs in front of their norm
+    uint32_t* odd;                             // [H, records]: some value of the chunk is not finite
     int64_t records;
     const int *cu_q, *cu_k, *slots;
     int num_seqs, H, group, D, Dv;             // group: heads that share a row of x0 and x1

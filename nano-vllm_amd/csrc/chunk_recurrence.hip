@@ -19,6 +19,9 @@
 // the inverse of a unit lower triangular 8 x 8 matrix by forward substitution.  All large products are
 // v_mfma_f32_16x16x4_f32: operands and sums stay fp32.
 //
+// A zero of M or M2 keeps a token's row out of a product only while the row is finite.  Where a chunk holds a value that is not, its
+// sequence and head take these products token by token, so that no earlier token and, from q, no state sees it.
+//
 // G_t / G_s does not factor through one reference without overflow when a channel decays fast, so both sides are taken relative
 // to the middle of the chunk: four factors on either side.  There the factors are held above 2^-25: the largest product is
 // 2^100, and a ratio that holding changes is one of numbers below 2^-25 in front of sums whose rounding is 2^-24.
@@ -219,6 +222,7 @@ __global__ __launch_bounds__(256) void recurrence_chunks_kernel(const ChunkRecur
             }
         }
     }
+    float odd[8] = {};                                // NaN with a value that is not finite
     {
         const T* v = (const T*)a.v + (int64_t)t0 * a.sv + (int64_t)h * a.Dv;
         T* to = (T*)a.columns + (h * a.records + rec) * 8 * a.Dv;
@@ -227,7 +231,11 @@ __global__ __launch_bounds__(256) void recurrence_chunks_kernel(const ChunkRecur
 #pragma unroll
             for (int t = 0; t < 8; ++t) r[t].load(v + (t < n ? t : 0) * a.sv + c);
 #pragma unroll
-            for (int t = 0; t < 8; ++t) r[t].store(to + t * a.Dv + c, t < n);
+            for (int t = 0; t < 8; ++t) {
+                r[t].store(to + t * a.Dv + c, t < n);
+                odd[t] += r[t].value(0) * 0.f;
+                odd[t] += r[t].value(1) * 0.f;
+            }
         }
     }
     float beta = 0.f;                                 // raw, of token lane % 8
@@ -245,11 +253,17 @@ __global__ __launch_bounds__(256) void recurrence_chunks_kernel(const ChunkRecur
         for (int i = 0; i < 2; ++i) {
             float in[4];
 #pragma unroll
-            for (int j = 0; j < NX; ++j) in[j] = raw[j][t].value(i);
+            for (int j = 0; j < NX; ++j) {
+                in[j] = raw[j][t].value(i);
+                odd[t] += in[j] * 0.f;
+            }
             el[t][i] = cr_elem<FORM>(in, c0[i], c1[i], a.p0);
             if (t >= n || !in_row) el[t][i] = CrElem{1.f, 0.f, 0.f, 0.f};
         }
     }
+    const float sum_odd = ((odd[0] + odd[1]) + (odd[2] + odd[3])) + ((odd[4] + odd[5]) + (odd[6] + odd[7])) + beta * 0.f;
+    const bool any_odd = __any(sum_odd != 0.f);
+    if (lane == 0) a.odd[h * a.records + rec] = any_odd;
     float kk = 0.f, qq = 0.f;                         // sums of squares of token lane % 8
     if constexpr (FORM != kCrWrite) {
         auto squares = [&](auto of) {                 // 8 tokens' sums over 64 lanes: halved three times over the lanes, then summed
@@ -533,6 +547,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int e = 0; e < 4; ++e) S[m][e] = fresh ? 0.f : slot[(int64_t)(16 * m + e) * Dv];
     }
+    uint32_t odd = 0;                                 // some chunk of the sequence and head holds a value that is not finite
+    {
+        const uint32_t* flags = a.odd + (int64_t)h * a.records + cr_first_record(q0 - a.cu_q[first_seq], b - first_seq);
+        for (int c = lane; c < chunks; c += 64) odd |= flags[c];
+        odd = __any(odd != 0);
+    }
     const int at_kq = Rec::kq + (FORM == kCrWrite ? (g * 8 + (l16 & 7)) * 4 + d0 * 8 : lane * 4 + d0 * 16);
     constexpr int kq_tile = 16 * Rec::kRows;
     const int at_upd = Rec::upd + lane * 2 + d0 * 8, at_dec = Rec::decay + d0 + ((l16 + 4 * g) & 15), at_m = Rec::m + l16 * 16 + 4 * g;
@@ -545,7 +565,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     cr_group_barrier();
     read_x(0);
     int at = 0;
-    for (int c = 0; c < chunks; ++c) {                // chunk c from slot `at`
+    auto chunk = [&](auto odd_tag, int c) {           // chunk c from slot `at`
+        constexpr bool ODD = decltype(odd_tag)::value;
         const float* rc = slots[at];
         f32x4 y;
         float dec[NM];                                // lane e of group g: the decay of row 4 g + e of the tile
@@ -591,11 +612,38 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             for (int m = 0; m < NM; ++m) S[m] = cr_mfma(uk[m].y, vv[1], S[m]);
         }
         if constexpr (RS > 1) c0 += other;
+        if constexpr (!ODD) {
+            if constexpr (FORM != kCrWrite) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) d = cr_mfma(y[e], c0[e], d);
+            }
+        } else {
+            // A zero above the diagonal keeps a later token out only while that token's value is finite: token by token, each
+            // from operands that end with it; a row of Q counts for its own read-out alone.
+            f32x4 rows = d;
+#pragma unroll 1
+            for (int t = 0; t < kCrChunk; ++t) {
+                f32x4 u = {0.f, 0.f, 0.f, 0.f};
+                u = cr_mfma(y2.x, 2 * g <= t ? vv[0] : 0.f, u);
+                u = cr_mfma(y2.y, 2 * g + 1 <= t ? vv[1] : 0.f, u);
+                f32x4 o = u;
+                if constexpr (FORM != kCrWrite) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int at = (4 * g + e) & 7;
+                        u = cr_mfma(y[e], g < 2 && at <= t ? c0[e] : 0.f, u);
+                        o = cr_mfma(y[e], (g < 2 ? at <= t : at == t) ? c0[e] : 0.f, o);
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (((4 * g + e) & 7) == t) rows[e] = g < 2 ? u[e] : o[e];
+            }
+            d = rows;
+        }
         if constexpr (FORM == kCrWrite) {
             d += c0;
         } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) d = cr_mfma(y[e], c0[e], d);
             // tokens 0, 1 | 4, 5 of U sit in groups 0 | 1, tokens 2, 3 | 6, 7 move to groups 2 | 3
             const float u0 = cr_spread(d[0], d[2]), u1 = cr_spread(d[1], d[3]);
 #pragma unroll
@@ -608,6 +656,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
             for (int e = 0; e < 4; ++e) os[c & 1][4 * (g & 1) + e][in_group] = d[e];
         }
+    };
+    if (odd == 0) {
+        for (int c = 0; c < chunks; ++c) chunk(std::false_type{}, c);
+    } else {
+        for (int c = 0; c < chunks; ++c) chunk(std::true_type{}, c);
     }
     cr_group_barrier();
     if (!live) return;
@@ -803,9 +856,10 @@ static bool recurrence_built(int D, int Dv) {
     return (D == 32 || D == 64 || D == 96 || D == 128) && Dv % 16 == 0 && Dv <= 256 && D * Dv <= 128 * 128;
 }
 
-// The workspace of T rows in seqs sequences: records, their rows of V, read-outs; every part starts on 16 bytes.
+// The workspace of T rows in seqs sequences: records, their rows of V, read-outs, flags; the parts in front of the flags are whole
+// 16-byte pieces.
 struct CrWorkspace {
-    int64_t records, chunks, columns, raw;            // how many (per head); bytes of the parts
+    int64_t records, chunks, columns, raw, odd;       // how many (per head); bytes of the parts
     CrWorkspace(int form, int64_t T, int H, int D, int Dv, int seqs, int dtype) {
         const int rows = form == kCrWrite ? 8 : 16;
         const int words = rows * D + (form == kCrGeneral ? 2 : 1) * 8 * D + D + (form == kCrWrite ? 0 : 256) + 8 * rows;
@@ -813,8 +867,9 @@ struct CrWorkspace {
         chunks = records * H * words * 4;
         columns = records * H * 8 * Dv * (dtype == NV_DTYPE_BF16 ? 2 : 4);
         raw = T * H * Dv * 4;
+        odd = records * H * 4;
     }
-    int64_t bytes() const { return chunks + columns + raw; }
+    int64_t bytes() const { return chunks + columns + raw + odd; }
 };
 
 template <typename T, int FORM, int D>
@@ -905,6 +960,7 @@ bool run_recurrence_portions(int form, ChunkRecurrenceArgs a, int lead, int port
     a.chunks = (float*)workspace;
     a.columns = (char*)workspace + ws.chunks;
     a.raw = (float*)((char*)a.columns + ws.columns);
+    a.odd = (uint32_t*)((char*)a.raw + ws.raw);
     a.records = ws.records;
     if (rest) *rc = launch_chunk_recurrence(form, a, lead, singles_behind, dtype, s);
     return true;

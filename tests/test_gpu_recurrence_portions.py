@@ -151,3 +151,54 @@ def test_entries_without_workspace(form, entry):
     torch.cuda.synchronize()
     torch.testing.assert_close(out, want, rtol=5e-5, atol=5e-5)          # (the bounds of test_portions)
     torch.testing.assert_close(got_state, want_state, rtol=2e-5, atol=2e-6 * want_state.abs().max().item())
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("form,name", [("gated", "q"), ("gated", "k"), ("gated", "v"), ("gated", "w"), ("gated", "b"), ("gated", "gate"),
+                                       ("general", "q"), ("general", "k"), ("general", "v"), ("general", "w"), ("general", "a"),
+                                       ("write", "q"), ("write", "k"), ("write", "v")])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("Dv", [16, 128])                               # two waves for a state's columns and one
+def test_values_that_are_not_finite(form, name, value, dtype, Dv):
+    """What is not finite in one token's row reaches that row and what comes after it, as token by token: no row in front of it,
+    no other head, no other sequence; and what it makes finite (a gate fully open or closed) is finite."""
+    H, D, at = 4, 128, 11                  # token 3 of the second chunk of the first sequence
+    Dv = D if form == "general" else Dv
+    rows, before = [21, 9, 13], [0, 5, 0]
+    if Dv == 128:
+        rows, before = rows * 16, before * 16
+    n, ctx = rows[0], _context(rows, before, True)
+    a, r, x, state = _operands(form, rows, before, H, D, Dv, dtype, 9)
+    nv.set_context(ctx)
+    clean_state = state.clone()
+    clean = _forward(form, a, x, clean_state)
+    x[name] = x[name].clone()
+    if x[name].dim() == 3:
+        x[name][at, 0, 3] = value
+    else:
+        x[name][at, 3 if name != "b" else 0] = value                     # (b: one value per head)
+    got_state = state.clone()
+    got = _forward(form, a, x, got_state)
+    slot = int(ctx.state_slots[0])
+    others = [s for s in range(state.shape[0]) if s != slot]
+    one = state[slot:slot + 1].clone()     # the first sequence alone through the stand-in
+    ctx = _context(rows[:1], before[:1], True)
+    ctx.state_slots = torch.zeros(1, dtype=torch.int32, device=DEV)
+    nv.set_context(ctx)
+    want = _forward(form, r, {k: t[:n] for k, t in x.items()}, one).detach()
+    nv.set_context(None)
+    heads = lambda t: t[:n].float().view(n, H, Dv)
+    hit = 2 if form == "gated" and name in "qk" else 1                   # heads that share the row
+    assert torch.equal(got[:at], clean[:at]) and torch.equal(got[n:], clean[n:])
+    assert torch.equal(heads(got)[:, hit:], heads(clean)[:, hit:])
+    assert torch.equal(got_state[others], clean_state[others])
+    if name == "v" and abs(value) == float("inf"):
+        # Its column of the state holds infinities of both signs: a read-out as a sum over them is NaN and its norm takes the row
+        # along, one from the write's own product is infinite and leaves zeros beside it.  Only its own column counts.
+        assert not heads(got)[at:, 0, 3].isfinite().any() and not heads(want)[at:, 0, 3].isfinite().any()
+        got[at:n, :Dv] = want[at:, :Dv] = 0
+    for g, w, tol in ((heads(got), heads(want), dict(rtol=5e-5, atol=5e-5) if dtype == torch.float32 else dict(rtol=1e-2, atol=2e-2)),
+                      (got_state[slot], one[0], dict(rtol=2e-5, atol=2e-6 * clean_state.abs().max().item()))):
+        ok = w.isfinite()
+        assert torch.equal(g.isfinite(), ok)
+        torch.testing.assert_close(g[ok], w[ok], **tol)                  # (the bounds of test_portions)
