@@ -22,10 +22,12 @@
 // A zero of M or M2 keeps a token's row out of a product only while the row is finite.  Where a chunk holds a value that is not, its
 // sequence and head take these products token by token, so that no earlier token and, from q, no state sees it.
 //
-// G_t / G_s does not factor through one reference without overflow when a channel decays fast, so both sides are taken relative
-// to the middle of the chunk: four factors on either side.  There the factors are held above 2^-25: the largest product is
-// 2^100, and a ratio that holding changes is one of numbers below 2^-25 in front of sums whose rounding is 2^-24.
-//
+// G_t / G_s does not factor through one reference without overflow when a channel decays fast.  Both sides are taken relative to
+// the middle of the chunk, four factors on either side, where no channel of the chunk has four that multiply to less than 2^-80 (a
+// right side then keeps its 24 bits down to 2^-46 of the raw key).  Other chunks take the pairs in four sets by where s and t part:
+// in halves, quarters or neighbours of the chunk, each relative to the boundary between the two, where every factor is a decay and
+// nothing is divided, and s = t.  A wave decides by its chunk alone.
+
 // Two launches: the first makes every chunk's operands (a wave per chunk and head, all chunks at once), the second walks the
 // chunks of a (sequence, head, 16 value columns) with the state in MFMA accumulators (128 channels: 32 registers) and reads the
 // operands from memory in the order of its lanes.  fp32 MFMAs run on the vector units, so waves that prepared operands beside
@@ -52,7 +54,7 @@
 namespace nv {
 
 constexpr int kCrChunk = 8;
-constexpr float kCrHold = 2.98023224e-8f;             // 2^-25
+constexpr float kCrNear = 8.27180613e-25f;            // 2^-80
 
 __device__ __forceinline__ float cr_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
 // log(1 + exp(x)) = max(x, 0) + log(1 + u), u = exp(-|x|) <= 1; log(1 + u) = 2 atanh(s), s = u / (2 + u) <= 1/3, by its series
@@ -293,54 +295,94 @@ __global__ __launch_bounds__(256) void recurrence_chunks_kernel(const ChunkRecur
         kk = squares([&](int t) { return el[t][0].k * el[t][0].k + el[t][1].k * el[t][1].k; });
         if constexpr (FORM == kCrGated) qq = squares([&](int t) { return el[t][0].q * el[t][0].q + el[t][1].q * el[t][1].q; });
     }
-    // ---- relative to the middle: left sides G_t / G_4, right sides G_4 / G_t, factors held above 2^-25
-    float held[2][8];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        held[i][3] = 1.f;                             // of tokens 0 .. 3: products behind the token; 4 .. 7: through the token
-#pragma unroll
-        for (int t = 2; t >= 0; --t) held[i][t] = held[i][t + 1] * fmaxf(el[t + 1][i].w, kCrHold);
-        held[i][4] = fmaxf(el[4][i].w, kCrHold);
-#pragma unroll
-        for (int t = 5; t < 8; ++t) held[i][t] = held[i][t - 1] * fmaxf(el[t][i].w, kCrHold);
-    }
-    if (in_row) {
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            float lv[2], rv[2], hb[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const float inv = __builtin_amdgcn_rcpf(held[i][t]);
-                lv[i] = t < 4 ? inv : held[i][t];
-                rv[i] = t < 4 ? held[i][t] : inv;
-                if constexpr (FORM == kCrGeneral)     // the old state: through the token before
-                    hb[i] = t == 0 ? __builtin_amdgcn_rcpf(held[i][0] * fmaxf(el[0][i].w, kCrHold))
-                                   : t < 4 ? __builtin_amdgcn_rcpf(held[i][t - 1]) : t == 4 ? 1.f : held[i][t - 1];
-                else hb[i] = lv[i];
-            }
-            if constexpr (FORM != kCrWrite) *(float2*)(lds.left + t * ROW + d) = make_float2(el[t][0].k * hb[0], el[t][1].k * hb[1]);
-            *(float2*)(lds.left + (8 + t) * ROW + d) = make_float2(el[t][0].q * lv[0], el[t][1].q * lv[1]);
-            *(float2*)(lds.right + t * ROW + d) = make_float2(el[t][0].k * rv[0], el[t][1].k * rv[1]);
-            if constexpr (FORM == kCrGeneral)
-                *(float2*)(lds.right + (8 + t) * ROW + d) = make_float2(el[t][0].a * rv[0], el[t][1].a * rv[1]);
-        }
-    }
-    cr_wave_sync();
-    f32x4 p = {0.f, 0.f, 0.f, 0.f}, p1 = p;           // entry (row 4 g + e, column l16): rows k | q, columns k | a k
-    {
+    // ---- pair products: entry (row 4 g + e, column l16): rows k | q, columns k | a k
+    f32x4 p = {0.f, 0.f, 0.f, 0.f};
+    auto products = [&] {                             // of the operands in LDS
+        cr_wave_sync();
+        f32x4 p0 = {0.f, 0.f, 0.f, 0.f}, p1 = p0;
         const int lrow = FORM == kCrWrite ? (8 + (l16 & 7)) : l16;
         const float* lf = lds.left + lrow * ROW + 4 * g;
         const float* rt = lds.right + (Lds::kRight == 16 ? l16 : (l16 & 7)) * ROW + 4 * g;
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
             const f32x4 x = *(const f32x4*)(lf + 16 * m), y = *(const f32x4*)(rt + 16 * m);
-            p = cr_mfma(x[0], y[0], p);
+            p0 = cr_mfma(x[0], y[0], p0);
             p1 = cr_mfma(x[1], y[1], p1);
-            p = cr_mfma(x[2], y[2], p);
+            p0 = cr_mfma(x[2], y[2], p0);
             p1 = cr_mfma(x[3], y[3], p1);
         }
+        return p0 + p1;
+    };
+    // relative to the middle: left sides G_t / G_4, right sides G_4 / G_t
+    float side[2][8];
+    bool near = true;                                 // (false with a decay that is not a number)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        side[i][3] = 1.f;                             // of tokens 0 .. 3: products behind the token; 4 .. 7: through the token
+#pragma unroll
+        for (int t = 2; t >= 0; --t) side[i][t] = side[i][t + 1] * el[t + 1][i].w;
+        side[i][4] = el[4][i].w;
+#pragma unroll
+        for (int t = 5; t < 8; ++t) side[i][t] = side[i][t - 1] * el[t][i].w;
+        near = near && side[i][0] * el[0][i].w >= kCrNear && side[i][7] >= kCrNear;
     }
-    p += p1;
+    if (__all(near)) {
+        if (in_row) {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                float lv[2], rv[2], hb[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const float inv = __builtin_amdgcn_rcpf(side[i][t]);
+                    lv[i] = t < 4 ? inv : side[i][t];
+                    rv[i] = t < 4 ? side[i][t] : inv;
+                    if constexpr (FORM == kCrGeneral) // the old state: through the token before
+                        hb[i] = t == 0 ? __builtin_amdgcn_rcpf(side[i][0] * el[0][i].w)
+                                       : t < 4 ? __builtin_amdgcn_rcpf(side[i][t - 1]) : t == 4 ? 1.f : side[i][t - 1];
+                    else hb[i] = lv[i];
+                }
+                if constexpr (FORM != kCrWrite) *(float2*)(lds.left + t * ROW + d) = make_float2(el[t][0].k * hb[0], el[t][1].k * hb[1]);
+                *(float2*)(lds.left + (8 + t) * ROW + d) = make_float2(el[t][0].q * lv[0], el[t][1].q * lv[1]);
+                *(float2*)(lds.right + t * ROW + d) = make_float2(el[t][0].k * rv[0], el[t][1].k * rv[1]);
+                if constexpr (FORM == kCrGeneral)
+                    *(float2*)(lds.right + (8 + t) * ROW + d) = make_float2(el[t][0].a * rv[0], el[t][1].a * rv[1]);
+            }
+        }
+        p = products();
+    } else {
+#pragma unroll 1
+        for (int part = 4; part >= 0; part = part == 1 ? 0 : part == 0 ? -1 : part / 2) {       // 4, 2, 1; 0: s = t
+            if (in_row) {
+                float lv[2] = {1.f, 1.f}, rv[2] = {1.f, 1.f};
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {         // from the start of its part through the token
+                    if ((t & (part - 1)) == 0) lv[0] = lv[1] = 1.f;
+                    const float before[2] = {lv[0], lv[1]};
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) lv[i] *= part ? el[t][i].w : 1.f;
+                    const float* kv = FORM == kCrGeneral ? before : lv;
+                    if constexpr (FORM != kCrWrite) *(float2*)(lds.left + t * ROW + d) = make_float2(el[t][0].k * kv[0], el[t][1].k * kv[1]);
+                    *(float2*)(lds.left + (8 + t) * ROW + d) = make_float2(el[t][0].q * lv[0], el[t][1].q * lv[1]);
+                }
+#pragma unroll
+                for (int t = 7; t >= 0; --t) {        // behind the token to the end of its part
+                    if (((t + 1) & (part - 1)) == 0) rv[0] = rv[1] = 1.f;
+                    *(float2*)(lds.right + t * ROW + d) = make_float2(el[t][0].k * rv[0], el[t][1].k * rv[1]);
+                    if constexpr (FORM == kCrGeneral)
+                        *(float2*)(lds.right + (8 + t) * ROW + d) = make_float2(el[t][0].a * rv[0], el[t][1].a * rv[1]);
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) rv[i] *= part ? el[t][i].w : 1.f;
+                }
+            }
+            const f32x4 of = products();
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int apart = ((4 * g + e) & 7) ^ (l16 & 7);
+                if (part ? apart >= part && apart < 2 * part : apart == 0) p[e] = of[e];
+            }
+            cr_wave_sync();
+        }
+    }
     // ---- [K; Q], K^, X^ and the chunk's decay
     float G[2][8], F[2][8];
 #pragma unroll

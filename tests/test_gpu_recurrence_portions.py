@@ -245,3 +245,34 @@ def test_decays_keep_their_precision(rows):
         big = want > 1e-30
         off.append((((got[..., 0].double() - want) / want)[big] ** 2).mean().sqrt().item())
     assert off[0] <= 1.1 * off[1], off
+
+
+@pytest.mark.parametrize("at", range(8, 16))
+@pytest.mark.parametrize("form", ["gated", "general", "write"])
+def test_total_decay_behind_large_values(form, at):
+    """A token whose decays forget everything sees nothing of what was written before it, also within its chunk and however large
+    that was: its factors are below any that the pair products could divide by."""
+    H, D, rows, before = 4, 128, [24, 13], [0, 3]
+    a, r, x, state = _operands(form, rows, before, H, D, D, torch.float32, 13)
+    for m in (a, r):
+        if form == "gated":
+            m.A_log.data.zero_()
+            m.dt_bias.data.fill_(-8.0)
+        elif form == "general":
+            m.decay_rate = 60.0
+            m.w_bias.data.zero_()
+        else:
+            m.lower.data.zero_()
+            m.f_bias.data.zero_()
+    keep, forget = {"gated": (0.0, 60.0), "general": (-12.0, 12.0), "write": (1.0, -60.0)}[form]
+    decay = x["k"] if form == "write" else x["w"]
+    decay.mul_(0.1).add_(keep)
+    decay[at] = forget
+    x["a"][at] = -60.0                             # (general: nothing of the old state is moved either)
+    x["v"][:at] *= 1e6
+    got_state, want_state = state.clone(), state.clone()
+    nv.set_context(_context(rows, before, True))
+    want, got = _forward(form, r, x, want_state), _forward(form, a, x, got_state)
+    nv.set_context(None)
+    torch.testing.assert_close(got, want, rtol=5e-5, atol=5e-5)          # (the bounds of test_portions)
+    torch.testing.assert_close(got_state, want_state, rtol=2e-5, atol=2e-6 * state.abs().max().item())
