@@ -61,7 +61,8 @@ class LLMEngine:
         if stateful and max_num_seqs is None:
             max_num_seqs = 64                 # rows of the state tensors: the most requests live at once
         self.runner = ModelRunner(model, cfg, block_size, num_kvcache_blocks, gpu_memory_utilization, device,
-                                  dtype=dtype, use_graphs=use_graphs, num_state_slots=max_num_seqs if stateful else None)
+                                  dtype=dtype, use_graphs=use_graphs, num_state_slots=max_num_seqs if stateful else None,
+                                  max_num_batched_tokens=max_num_batched_tokens)
         self.scheduler = Scheduler(self.runner.num_kvcache_blocks, block_size, max_num_batched_tokens,
                                    long_prefill_token_threshold, eos if eos is not None else cfg.eos_token_id,
                                    max_num_seqs, num_state_slots=max_num_seqs if stateful else None,

@@ -196,14 +196,17 @@ class _DecodeGraph:
 class ModelRunner:
     def __init__(self, model: torch.nn.Module, cfg, block_size: int = 256, num_kvcache_blocks: int | None = None,
                  gpu_memory_utilization: float = 0.9, device: str | torch.device = "cuda",
-                 dtype: torch.dtype = torch.bfloat16, use_graphs: bool = False, num_state_slots: int | None = None):
+                 dtype: torch.dtype = torch.bfloat16, use_graphs: bool = False, num_state_slots: int | None = None,
+                 max_num_batched_tokens: int = 0):
         """num_state_slots: rows of the per-sequence state tensors of models with recurrent layers (the most
-        requests that can be live at once)."""
+        requests that can be live at once).  max_num_batched_tokens: the most rows of a step, for the scratch memory that
+        recurrent layers allocate per step (0: none is set aside)."""
         self.model, self.cfg, self.block_size = model, cfg, block_size
         self.device, self.dtype = torch.device(device), dtype
         self.kv_cache: torch.Tensor | None = None
         self.cache_specs = model.cache_specs() if hasattr(model, "cache_specs") else None
         self.num_state_slots = num_state_slots
+        self.max_num_batched_tokens = max_num_batched_tokens
         self.has_state = self.cache_specs is not None and any(isinstance(c, SlotStateSpec) for c in self.cache_specs)
         if self.has_state and not num_state_slots:
             raise ValueError("this model keeps a state per sequence: num_state_slots (max live requests) must be given")
@@ -246,18 +249,28 @@ class ModelRunner:
         shard = getattr(self.model, "shard", None)
         return shard.local_kv_heads if shard is not None else self.cfg.num_key_value_heads
 
-    def _init_spec_caches(self, num_blocks: int | None, utilization: float) -> int:
-        """Models that describe their caches (`cache_specs()`): one paged K/V pair per attention run, all sharing
-        the block numbering, and the per-sequence state tensors of the recurrent runs with `num_state_slots` rows."""
+    def _step_scratch_bytes(self) -> int:
+        """What the layers of a step allocate for themselves, one after the other."""
+        if not self.max_num_batched_tokens:
+            return 0
+        return max((m.step_scratch_bytes(self.max_num_batched_tokens, self.num_state_slots or 0, self.dtype)
+                    for m in self.model.modules() if hasattr(m, "step_scratch_bytes")), default=0)
+
+    def _spec_blocks_that_fit(self, utilization: float) -> int:
         state_bytes = sum(spec.slot_bytes(self.dtype) for spec in self.cache_specs if isinstance(spec, SlotStateSpec))
         state_bytes *= self.num_state_slots or 0
         per_block = self.block_bytes()
+        free, total = torch.cuda.mem_get_info(self.device)
+        budget = int(total * utilization) - (total - free) - state_bytes - self._step_scratch_bytes()
+        return budget // per_block if per_block else 1
+
+    def _init_spec_caches(self, num_blocks: int | None, utilization: float) -> int:
+        """Models that describe their caches (`cache_specs()`): one paged K/V pair per attention run, all sharing
+        the block numbering, and the per-sequence state tensors of the recurrent runs with `num_state_slots` rows."""
         if num_blocks is None:
             if self.device.type != "cuda":
                 raise ValueError("num_kvcache_blocks must be given when not running on a GPU")
-            free, total = torch.cuda.mem_get_info(self.device)
-            budget = int(total * utilization) - (total - free) - state_bytes
-            num_blocks = budget // per_block if per_block else 1
+            num_blocks = self._spec_blocks_that_fit(utilization)
         assert num_blocks > 0, "no memory left for the KV cache"
         caches = []
         for spec in self.cache_specs:

@@ -41,6 +41,10 @@ class GatedDeltaRule(nn.Module):
         self.dt_bias = nn.Parameter(torch.zeros(num_heads * head_dim, **f32))
         self.norm_weight = nn.Parameter(torch.ones(v_head_dim, **f32))
 
+    def step_scratch_bytes(self, rows: int, sequences: int, dtype: torch.dtype) -> int:
+        """Device bytes a step of up to these rows and sequences allocates for itself."""
+        return ops.recurrence_scratch_bytes(0, rows, self.num_heads, self.head_dim, self.v_head_dim, sequences, dtype)
+
     def forward(self, q, k, v, a_raw, b_raw, gate_raw, state: torch.Tensor) -> torch.Tensor:
         """q, k: [T, G, D]; v: [T, H, Dv] (after the short convolution); a_raw [T, H*D], b_raw [T, H],
         gate_raw [T, H*Dv] as projected; state [slots, H, D, Dv] float32.  Returns [T, H*Dv]."""

@@ -57,6 +57,10 @@ class GatedWriteMemory(nn.Module):
     def state_shapes(self) -> dict:
         return {"state": ((self.num_heads, self.key_dim, self.value_dim), torch.float32)}
 
+    def step_scratch_bytes(self, rows: int, sequences: int, dtype: torch.dtype) -> int:
+        """Device bytes a step of up to these rows and sequences allocates for itself."""
+        return ops.recurrence_scratch_bytes(2, rows, self.num_heads, self.key_dim, self.value_dim, sequences, dtype)
+
     def forward(self, q, f_raw, v, cache: dict) -> torch.Tensor:
         """q, f_raw: [T, H, Dk] as projected; v: [T, H, Dv]; returns [T, H * Dv]."""
         ctx = get_context()

@@ -28,6 +28,10 @@ class GeneralDeltaRule(nn.Module):
         self.w_bias = nn.Parameter(torch.zeros(num_heads * head_dim, **f32))
         self.norm_weight = nn.Parameter(torch.ones(num_heads * head_dim, **f32))
 
+    def step_scratch_bytes(self, rows: int, sequences: int, dtype: torch.dtype) -> int:
+        """Device bytes a step of up to these rows and sequences allocates for itself."""
+        return ops.recurrence_scratch_bytes(1, rows, self.num_heads, self.head_dim, self.head_dim, sequences, dtype)
+
     def forward(self, r, k, v, w_raw, a_raw, gate_raw, state: torch.Tensor) -> torch.Tensor:
         """r, k, v: [T, H, D]; w_raw, a_raw, gate_raw: [T, H * D] as projected; state [slots, H, D, D] float32.
         Returns [T, H * D]."""

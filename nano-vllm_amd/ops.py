@@ -540,10 +540,17 @@ def _portions(dll, form: int, rows: torch.Tensor, T: int, H: int, D: int, Dv: in
     portions: the kinds of portions behind them (`portion_kinds`; 7: not known)."""
     lead = B if max_seqlen_q == 1 else int(leading_singles or 0)
     _need(0 <= lead <= B, "leading_singles exceeds the batch")
-    if lead == B:                          # single tokens need none
+    if lead == B or not int(portions) & ~1:                # single tokens need none
         return lead, int(portions), None
     need = dll.nv_recurrence_workspace_bytes(form, T, H, D, Dv, B, lead, _dt(rows, "rows"))
     return lead, int(portions), torch.empty(need, dtype=torch.uint8, device=rows.device) if need > 0 else None
+
+
+def recurrence_scratch_bytes(form: int, rows: int, H: int, D: int, Dv: int, seqs: int, dtype: torch.dtype) -> int:
+    """The most bytes a recurrent layer allocates for a step of up to `rows` rows in up to `seqs` sequences (form: 0 gated delta
+    rule, 1 generalized delta rule, 2 gated write)."""
+    return int(_lib.mixers().nv_recurrence_workspace_bytes(form, rows, H, D, Dv, seqs, 0,
+                                                           _lib.DTYPE_BF16 if dtype == _BF16 else _lib.DTYPE_F32))
 
 
 def gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a_raw: torch.Tensor, b_raw: torch.Tensor,

@@ -1,0 +1,47 @@
+"""Scratch memory of the recurrent layers: asked for only by steps that use it, and set aside when the caches are sized."""
+import pytest
+import torch
+import torch.nn as nn
+
+from nanovllm_amd import _lib, ops
+from nanovllm_amd.engine.cache_spec import PagedKVSpec, SlotStateSpec
+from nanovllm_amd.engine.model_runner import ModelRunner
+from nanovllm_amd.layers.delta_rule import GatedDeltaRule
+from nanovllm_amd.layers.gated_memory import GatedWriteMemory
+from nanovllm_amd.layers.general_delta import GeneralDeltaRule
+
+H, D = 4, 128
+
+
+class _Model(nn.Module):
+    def __init__(self):
+        super().__init__()
+        self.rules = nn.ModuleList([GatedDeltaRule(H, H, D, D, 1e-5), GeneralDeltaRule(H, D, 1e-5), GatedWriteMemory(H, D, D, 1e-5),
+                                    GatedDeltaRule(H, H, 40, D, 1e-5)])
+
+    def cache_specs(self):
+        return [PagedKVSpec(2, 64, 64)] + [SlotStateSpec({"state": ((H, D, D), torch.float32)})] * 3
+
+    def bind_caches(self, caches):
+        pass
+
+
+@pytest.mark.parametrize("rows", [0, 1, 5000])
+def test_caches_leave_room_for_the_scratch_of_the_largest_step(monkeypatch, rows):
+    runner = ModelRunner(_Model(), None, 16, 3, device="cpu", num_state_slots=6, max_num_batched_tokens=rows)
+    free, total = 3 << 30, 4 << 30
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device: (free, total))
+    need = [_lib.mixers().nv_recurrence_workspace_bytes(form, rows, H, D, D, 6, 0, _lib.DTYPE_BF16) for form in range(3)]
+    assert (min(need) > 0) == (rows > 0)
+    left = int(total * 0.9) - (total - free) - 3 * 6 * H * D * D * 4 - max(need)
+    assert runner._spec_blocks_that_fit(0.9) == left // (16 * 2 * 128 * 2)
+
+
+def test_sizes_without_a_launch_in_chunks_need_none():
+    assert _Model().rules[3].step_scratch_bytes(5000, 6, torch.bfloat16) == 0
+
+
+@pytest.mark.parametrize("max_rows,lead,portions", [(1, 0, 7), (0, 3, 7), (0, 1, 1), (0, 0, 0)])
+def test_single_tokens_allocate_nothing(max_rows, lead, portions):
+    """All sequences of one row each, known as such by any of the step's three hints."""
+    assert ops._portions(None, 0, None, 3, H, D, D, 3, max_rows, lead, portions)[2] is None
