@@ -146,3 +146,17 @@ def test_single_rows_any_soft_cap(sign, softcap, bias):
     nv.set_context(None)
     # fp32 throughout and one rounding of the output (2^-9) on both sides
     torch.testing.assert_close(o.float(), o_r.float(), rtol=2 ** -7, atol=1e-3)
+
+
+@pytest.mark.parametrize("step", list(STEPS))
+@pytest.mark.parametrize("softcap", [0.0, 25.0])
+@pytest.mark.parametrize("D,Dv,at", [(128, 64, 0), (128, 64, 64), (128, 64, 8), (128, 128, 0), (64, 64, 0)])
+def test_values_as_columns_of_the_keys(D, Dv, at, softcap, step):
+    """Value rows with a stride of their own, as a column range of the key rows: what a dense copy of them gives, bit for bit."""
+    H, G, bs = 4, 2, 64
+    n_qs, n_ks = STEPS[step]
+    a, r, ctx, pos, q, k, v, kc, vc = _step(H, G, D, Dv, bs, n_qs, n_ks)
+    values = kc[..., at:at + Dv]
+    got, want = (ops.attn_scoremod_paged(q, kc, x, ctx.cu_seqlens_q, ctx.cu_seqlens_k, ctx.block_tables, D ** -0.5, softcap, None, None,
+                                         max(n_qs), max(n_ks)) for x in (values, values.contiguous()))
+    assert got.isfinite().all() and torch.equal(got, want)
