@@ -993,9 +993,9 @@ bool run_recurrence_portions(int form, ChunkRecurrenceArgs a, int lead, int port
     // (T = 0: not known, as from the entry points without portions; there may be longer portions then)
     const bool rest = lead < a.num_seqs && (a.T <= 0 || a.T > lead) && (portions & (NV_PORTION_FEW | NV_PORTION_LONG));
     const bool singles_behind = lead < a.num_seqs && (portions & NV_PORTION_SINGLE);
-    const int64_t far = 1LL << 28;                    // rows of a chunk are addressed by 32-bit offsets
-    if (!recurrence_built(a.D, a.Dv) || (uintptr_t)a.state % 16 != 0 || a.s0 >= far || a.s1 >= far || a.s2 >= far || a.s3 >= far ||
-        a.sv >= far || (int64_t)a.H * a.Dv >= far || a.T >= (1LL << 31) || (rest && (workspace == nullptr || a.T <= 0)))
+    // (rows, and sequences times heads, number workgroups in 32 bits; strides are 64 bits throughout)
+    if (!recurrence_built(a.D, a.Dv) || (uintptr_t)a.state % 16 != 0 || a.T >= (1LL << 31) || (int64_t)a.num_seqs * a.H >= (1LL << 31) ||
+        (rest && (workspace == nullptr || a.T <= 0)))
         return false;
     const CrWorkspace ws(form, a.T, a.H, a.D, a.Dv, a.num_seqs - lead, dtype);
     const int64_t need = ws.bytes();
