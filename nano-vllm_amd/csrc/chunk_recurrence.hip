@@ -27,11 +27,11 @@
 // right side then keeps its 24 bits down to 2^-46 of the raw key).  Other chunks take the pairs in four sets by where s and t part:
 // in halves, quarters or neighbours of the chunk, each relative to the boundary between the two, where every factor is a decay and
 // nothing is divided, and s = t.  A wave decides by its chunk alone.
-
+//
 // Two launches: the first makes every chunk's operands (a wave per chunk and head, all chunks at once), the second walks the
 // chunks of a (sequence, head, 16 value columns) with the state in MFMA accumulators (128 channels: 32 registers) and reads the
 // operands from memory in the order of its lanes.  fp32 MFMAs run on the vector units, so waves that prepared operands beside
-// them (one launch, everything through LDS) took the same issue slots: 653 us instead of 284 on gated, 4 prompts of 1501 .. 2048 tokens,
+// them (one launch, everything through LDS) took the same issue slots: 653 us instead of 292 on gated, 4 prompts of 1501 .. 2048 tokens,
 // 16 heads 128 x 128.
 // Accumulators of one product are the operand of the next in place: a lane holds rows 4 g + e (g: its group of 16 lanes), so
 // MFMA e of a tile contracts the four rows {4 g + e}, and the other operand is read in that order (16 bytes a lane).  U comes out
@@ -39,9 +39,13 @@
 // tile takes two MFMAs.  The chunk takes 54 (gated) / 70 (general) / 50 (write) MFMAs of 32 cycles per 16 columns of 128 channels.
 //
 // Measured against the token-by-token launches (16 heads 128 x 128, bf16 rows), whole call: gated, 4 prompts of 1501 .. 2048 tokens
-// 3123 -> 284 us; general, 3 prompts of 700 .. 2000: 3645 -> 290; write, 8 chunks of 509 over carried states: 431 -> 117; gated, 256
-// single tokens: 393 -> 112 (4.8 TB/s of states, what a large copy reaches).  Of the 284 us the second launch is 219, 257 chunks
-// in a row at 0.85 us: 0.43 us of MFMAs, the rest the chain of exchange, M and update between them.
+// 3123 -> 292 us; general, 3 prompts of 700 .. 2000: 3645 -> 293; write, 8 chunks of 509 over carried states: 431 -> 119; gated, 256
+// single tokens: 393 -> 113 (4.8 TB/s of states, what a large copy reaches).  Of the 292 us the first launch is 73 and the second 218,
+// 257 chunks in a row at 0.85 us: 0.43 us of MFMAs, the rest the chain of exchange, M and update between them.
+//
+// Against 64 bits (float32 rows, 1 to 300 tokens a sequence): states 0.9 to 1.5 times the token-by-token launch's error, all below
+// 3.3e-7; read-outs 1.5e-7 to 2.6e-7 where that has 1.1e-7 to 2.4e-7, because a chunk's sums are taken in another order.  Of bf16
+// read-outs, which are 1.7e-3 off by their own rounding, neither shows.
 //
 // The read-outs go to a scratch of fp32 rows, because a row's norm spans the workgroups of its value columns; a last launch
 // norms, weights and gates them.  Single tokens run in a launch of their own that streams every state once.
