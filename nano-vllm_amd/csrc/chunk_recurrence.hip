@@ -31,7 +31,7 @@
 // Two launches: the first makes every chunk's operands (a wave per chunk and head, all chunks at once), the second walks the
 // chunks of a (sequence, head, 16 value columns) with the state in MFMA accumulators (128 channels: 32 registers) and reads the
 // operands from memory in the order of its lanes.  fp32 MFMAs run on the vector units, so waves that prepared operands beside
-// them (one launch, everything through LDS) took the same issue slots: 653 us instead of 292 on gated, 4 prompts of 1501 .. 2048 tokens,
+// them (one launch, everything through LDS) took the same issue slots: 653 us instead of 286 on gated, 4 prompts of 1501 .. 2048 tokens,
 // 16 heads 128 x 128.
 // Accumulators of one product are the operand of the next in place: a lane holds rows 4 g + e (g: its group of 16 lanes), so
 // MFMA e of a tile contracts the four rows {4 g + e}, and the other operand is read in that order (16 bytes a lane).  U comes out
@@ -39,12 +39,13 @@
 // tile takes two MFMAs.  The chunk takes 54 (gated) / 70 (general) / 50 (write) MFMAs of 32 cycles per 16 columns of 128 channels.
 //
 // Measured against the token-by-token launches (16 heads 128 x 128, bf16 rows), whole call: gated, 4 prompts of 1501 .. 2048 tokens
-// 3123 -> 292 us; general, 3 prompts of 700 .. 2000: 3645 -> 293; write, 8 chunks of 509 over carried states: 431 -> 119; gated, 256
+// 3123 -> 286 us; general, 3 prompts of 700 .. 2000: 3645 -> 285; write, 8 chunks of 509 over carried states: 431 -> 116; gated, 256
 // single tokens: 393 -> 113 (4.8 TB/s of states, what a large copy reaches).  Of the 292 us the first launch is 73 and the second 218,
 // 257 chunks in a row at 0.85 us: 0.43 us of MFMAs, the rest the chain of exchange, M and update between them.
 //
 // Against 64 bits (float32 rows, 1 to 300 tokens a sequence): states 0.9 to 1.5 times the token-by-token launch's error, all below
-// 3.3e-7; read-outs 1.5e-7 to 2.6e-7 where that has 1.1e-7 to 2.4e-7, because a chunk's sums are taken in another order.  Of bf16
+// 3.3e-7; read-outs 1.0 to 1.24 times (1.2e-7 to 2.4e-7), because a chunk's sums are taken in another order: C and the pair products
+// are four sums each, since one sum over all key channels has its roundings one after the other (1.6 times the error).  Of bf16
 // read-outs, which are 1.7e-3 off by their own rounding, neither shows.
 //
 // The read-outs go to a scratch of fp32 rows, because a row's norm spans the workgroups of its value columns; a last launch
@@ -303,7 +304,7 @@ __global__ __launch_bounds__(256) void recurrence_chunks_kernel(const ChunkRecur
     f32x4 p = {0.f, 0.f, 0.f, 0.f};
     auto products = [&] {                             // of the operands in LDS
         cr_wave_sync();
-        f32x4 p0 = {0.f, 0.f, 0.f, 0.f}, p1 = p0;
+        f32x4 p0 = {0.f, 0.f, 0.f, 0.f}, p1 = p0, p2 = p0, p3 = p0;
         const int lrow = FORM == kCrWrite ? (8 + (l16 & 7)) : l16;
         const float* lf = lds.left + lrow * ROW + 4 * g;
         const float* rt = lds.right + (Lds::kRight == 16 ? l16 : (l16 & 7)) * ROW + 4 * g;
@@ -312,10 +313,10 @@ __global__ __launch_bounds__(256) void recurrence_chunks_kernel(const ChunkRecur
             const f32x4 x = *(const f32x4*)(lf + 16 * m), y = *(const f32x4*)(rt + 16 * m);
             p0 = cr_mfma(x[0], y[0], p0);
             p1 = cr_mfma(x[1], y[1], p1);
-            p0 = cr_mfma(x[2], y[2], p0);
-            p1 = cr_mfma(x[3], y[3], p1);
+            p2 = cr_mfma(x[2], y[2], p2);
+            p3 = cr_mfma(x[3], y[3], p3);
         }
-        return p0 + p1;
+        return (p0 + p1) + (p2 + p3);
     };
     // relative to the middle: left sides G_t / G_4, right sides G_4 / G_t
     float side[2][8];
@@ -637,15 +638,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             if constexpr (FORM != kCrGated) uk[m] = *(const float2*)(rc + 128 * m + at_upd);
             if constexpr (FORM != kCrWrite) ux[m] = *(const float2*)(rc + (Rec::kUpd - 1) * 8 * D + 128 * m + at_upd);
         }
-        f32x4 c0 = {0.f, 0.f, 0.f, 0.f}, d = c0;
+        f32x4 c0 = {0.f, 0.f, 0.f, 0.f}, d = c0, c1 = c0, c2 = c0, c3 = c0;   // (four sums: a quarter of the roundings one after the other)
         __builtin_amdgcn_sched_barrier(0);            // the reads are on their way before the products
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) c0 = cr_mfma(x[m][e], S[m][e], c0);
+            c0 = cr_mfma(x[m][0], S[m][0], c0);
+            c1 = cr_mfma(x[m][1], S[m][1], c1);
+            c2 = cr_mfma(x[m][2], S[m][2], c2);
+            c3 = cr_mfma(x[m][3], S[m][3], c3);
         }
         d = cr_mfma(y2.x, vv[0], d);
         d = cr_mfma(y2.y, vv[1], d);
+        __builtin_amdgcn_sched_barrier(0);            // (d's products run while the last of C comes out: 298 -> 286 us, gated)
+        c0 = (c0 + c1) + (c2 + c3);
         if constexpr (RS > 1) part[c & 1][wave][lane] = c0;
         cr_group_barrier();                           // chunk c + 1 is in its slot; chunk c - 1's slot is free
         f32x4 other;

@@ -276,3 +276,45 @@ def test_total_decay_behind_large_values(form, at):
     nv.set_context(None)
     torch.testing.assert_close(got, want, rtol=5e-5, atol=5e-5)          # (the bounds of test_portions)
     torch.testing.assert_close(got_state, want_state, rtol=2e-5, atol=2e-6 * state.abs().max().item())
+
+
+def test_read_outs_keep_their_precision():
+    """Read-outs of float32 rows against 64 bits, in a portion of one chunk: both launches sum 128 products with about 32 roundings
+    one after the other, so the chunk's error is that of the token-by-token entry and of the few sums over its tokens (measured:
+    1.11 times; with one sum over all key channels 1.62 times)."""
+    from nanovllm_amd import _lib
+    B, rows, H, D, Dv = 16, 8, 16, 128, 128
+    T = B * rows
+    g = torch.Generator(device=DEV).manual_seed(11)
+    mk = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    m = delta_rule.GatedDeltaRule(H, H, D, Dv, 1e-5, device=DEV)
+    m.A_log.data.copy_(torch.linspace(1, 16, H, device=DEV).log())
+    m.dt_bias.data.copy_(torch.linspace(-7, -2, H * D, device=DEV))
+    q, k, v, raw, b, gate = mk(T, H, D), mk(T, H, D), mk(T, H, Dv), 0.5 * mk(T, H * D), mk(T, H), mk(T, H * Dv)
+    state = 0.3 * mk(B, H, D, Dv)
+    # the same in 64 bits
+    unit = lambda t: t / torch.sqrt((t * t).sum(-1, keepdim=True) + 1e-6)
+    seqs = lambda t, *s: t.double().view(B, rows, H, *s)
+    w = torch.exp(-m.A_log.double().exp()[:, None] * torch.log1p(torch.exp(seqs(raw, D) + m.dt_bias.double().view(H, D))))
+    k64, q64, v64, beta = unit(seqs(k, D)), unit(seqs(q, D)) * D ** -0.5, seqs(v, Dv), torch.sigmoid(seqs(b))
+    S, o = state.double(), []
+    for t in range(rows):
+        S = S * w[:, t, :, :, None]
+        u = (v64[:, t] - (S * k64[:, t, :, :, None]).sum(2)) * beta[:, t, :, None]
+        S = S + k64[:, t, :, :, None] * u[:, :, None]
+        o.append((S * q64[:, t, :, :, None]).sum(2))
+    o = torch.stack(o, 1)
+    want = (o / torch.sqrt((o * o).mean(-1, keepdim=True) + 1e-5) * torch.sigmoid(seqs(gate, Dv))).view(T, H * Dv)
+    ctx = _context([rows] * B, [1] * B, True)
+    ctx.state_slots = torch.arange(B, dtype=torch.int32, device=DEV)
+    nv.set_context(ctx)
+    got = m(q, k, v, raw, b, gate, state.clone()).detach()
+    nv.set_context(None)
+    p, dll, tokens, st = lambda t: t.data_ptr(), _lib.mixers(), torch.empty(T, H * Dv, device=DEV), state.clone()
+    rc = dll.nv_gated_delta_rule(p(q), p(k), p(v), H * D, H * D, H * Dv, p(raw), H * D, p(b), H, p(gate), H * Dv, p(m.A_log), p(m.dt_bias),
+                                 p(m.norm_weight), p(st), p(tokens), H * Dv, p(ctx.cu_seqlens_q), p(ctx.cu_seqlens_k), p(ctx.state_slots),
+                                 B, H, H, D, Dv, 1e-5, ops._dt(v, "v"), ops._stream(v))
+    _lib.check(rc, "nv_gated_delta_rule", dll)
+    torch.cuda.synchronize()
+    off = [((x.double() - want).norm() / want.norm()).item() for x in (got, tokens)]
+    assert off[0] <= 1.35 * off[1], off
