@@ -39,9 +39,9 @@
 // tile takes two MFMAs.  The chunk takes 54 (gated) / 70 (general) / 50 (write) MFMAs of 32 cycles per 16 columns of 128 channels.
 //
 // Measured against the token-by-token launches (16 heads 128 x 128, bf16 rows), whole call: gated, 4 prompts of 1501 .. 2048 tokens
-// 3123 -> 286 us; general, 3 prompts of 700 .. 2000: 3645 -> 285; write, 8 chunks of 509 over carried states: 431 -> 116; gated, 256
-// single tokens: 393 -> 113 (4.8 TB/s of states, what a large copy reaches).  Of the 292 us the first launch is 73 and the second 218,
-// 257 chunks in a row at 0.85 us: 0.43 us of MFMAs, the rest the chain of exchange, M and update between them.
+// 3123 -> 286 us; general, 3 prompts of 700 .. 2000: 3645 -> 285; write, 8 chunks of 509 over carried states: 431 -> 115; gated, 256
+// single tokens: 393 -> 113 (4.8 TB/s of states, what a large copy reaches).  Of the 286 us the first launch is 74 and the second 208,
+// 257 chunks in a row at 0.81 us: 0.43 us of MFMAs, the rest the chain of exchange, M and update between them.
 //
 // Against 64 bits (float32 rows, 1 to 300 tokens a sequence): states 0.9 to 1.5 times the token-by-token launch's error, all below
 // 3.3e-7; read-outs 1.0 to 1.24 times (1.2e-7 to 2.4e-7), because a chunk's sums are taken in another order: C and the pair products
