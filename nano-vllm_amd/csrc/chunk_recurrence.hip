@@ -8,44 +8,52 @@
 //   write    (x0 = q, x1 = f_raw)   w = c1 + (1 - c1) sigmoid(x1 + c0);  k = 1 - w;  S <- diag(w) S + k v^T;  o = S^T silu(q)
 //
 // A token-by-token loop is bound by its serial chain (one pass over the state a token and the LDS reads of the token's vectors
-// by every lane), so portions run in CHUNKS of 8 tokens.  With G_t the product of the decays from the chunk's start through
+// by every lane), so portions run in CHUNKS of 16 tokens.  With G_t the product of the decays from the chunk's start through
 // token t, and S the state in front of the chunk, each form is
 //
-//   C = [K; Q] S        16 rows: what the tokens' k (u) and q (r) find in S, K_t = k_t G_t (general: u_t G_(t-1)), Q_t = q_t G_t
-//   [U; O] = M C + M2 V 16 x 16 and 16 x 8 matrices of the chunk alone: the tokens' influence on each other, solved
-//   S <- diag(G_8) S + K^^T V (general, write) + X^^T U (gated, general),   K^_t = k_t G_8 / G_t
+//   C = K S, Q S         what the tokens' k and q (r) find in S: K_t = k_t G_t (general: k_t G_(t-1)), Q_t = q_t G_t, 16 rows each
+//   U = T (V - K S)      gated; general: U = T (K S + PK V); write has none: the tokens' influence on each other, solved
+//   O = Q S + PQ U       (general: + PV V; write: PV V alone)
+//   S <- diag(G_16) S + K^^T V (general, write) + X^^T U (gated, general),   K^_t = k_t G_16 / G_t
 //
-// (write has no U and no M: O = C + M2 V).  M and M2 come from the pair products P_ts = sum_d l_t,d r_s,d G_t / G_s, s <= t, and
-// the inverse of a unit lower triangular 8 x 8 matrix by forward substitution.  All large products are
+// T is the inverse of a unit lower triangular 16 x 16 matrix by forward substitution, with the tokens' factors on either side; PQ, PV
+// and PK are lower triangles; all come from the pair products P_ts = sum_d l_t,d r_s,d G_t / G_s, s <= t.  Gated keys and queries are
+// scaled to unit length on their way into K, Q and X^, so that V - K S needs no factors.  All large products are
 // v_mfma_f32_16x16x4_f32: operands and sums stay fp32.
 //
-// A zero of M or M2 keeps a token's row out of a product only while the row is finite.  Where a chunk holds a value that is not, its
+// A zero of a triangle keeps a token's row out of a product only while the row is finite.  Where a chunk holds a value that is not, its
 // sequence and head take these products token by token, so that no earlier token and, from q, no state sees it.
 //
 // G_t / G_s does not factor through one reference without overflow when a channel decays fast.  Both sides are taken relative to
-// the middle of the chunk, four factors on either side, where no channel of the chunk has four that multiply to less than 2^-80 (a
-// right side then keeps its 24 bits down to 2^-46 of the raw key).  Other chunks take the pairs in four sets by where s and t part:
-// in halves, quarters or neighbours of the chunk, each relative to the boundary between the two, where every factor is a decay and
-// nothing is divided, and s = t.  A wave decides by its chunk alone.
+// the middle of the chunk, eight factors on either side, where no channel of the chunk has eight that multiply to less than 2^-80 (a
+// right side then keeps its 24 bits down to 2^-46 of the raw key).  Other chunks take the pairs in five sets by where s and t part:
+// in halves, quarters, eighths or neighbours of the chunk, each relative to the boundary between the two, where every factor is a decay
+// and nothing is divided, and s = t.  A chunk and head decide by themselves.
 //
-// Two launches: the first makes every chunk's operands (a wave per chunk and head, all chunks at once), the second walks the
+// Two launches: the first makes every chunk's operands (two waves per chunk and head, all chunks at once), the second walks the
 // chunks of a (sequence, head, 16 value columns) with the state in MFMA accumulators (128 channels: 32 registers) and reads the
-// operands from memory in the order of its lanes.  fp32 MFMAs run on the vector units, so waves that prepared operands beside
-// them (one launch, everything through LDS) took the same issue slots: 653 us instead of 286 on gated, 4 prompts of 1501 .. 2048 tokens,
-// 16 heads 128 x 128.
+// operands from memory in the order of its lanes.  Operands prepared beside the products (one launch, everything through LDS) took the
+// same issue slots: 653 us instead of 286 on gated, 4 prompts of 1501 .. 2048 tokens, 16 heads 128 x 128, in chunks of 8.
 // Accumulators of one product are the operand of the next in place: a lane holds rows 4 g + e (g: its group of 16 lanes), so
-// MFMA e of a tile contracts the four rows {4 g + e}, and the other operand is read in that order (16 bytes a lane).  U comes out
-// in the lower half of the lanes; two v_permlane32_swap spread its 8 rows over all four groups, so that an update of a 16-channel
-// tile takes two MFMAs.  The chunk takes 54 (gated) / 70 (general) / 50 (write) MFMAs of 32 cycles per 16 columns of 128 channels.
+// MFMA e of a tile contracts the four rows {4 g + e}, and the other operand is read in that order (16 bytes a lane); U, 16 rows, fills
+// all four groups.  The chunk takes 104 (gated) / 144 (general) / 68 (write) MFMAs of 32 cycles per 16 columns of 128 channels.
 //
-// Measured against the token-by-token launches (16 heads 128 x 128, bf16 rows), whole call: gated, 4 prompts of 1501 .. 2048 tokens
-// 3123 -> 286 us; general, 3 prompts of 700 .. 2000: 3645 -> 285; write, 8 chunks of 509 over carried states: 431 -> 115; gated, 256
-// single tokens: 393 -> 113 (4.8 TB/s of states, what a large copy reaches).  Of the 286 us the first launch is 74 and the second 208,
-// 257 chunks in a row at 0.81 us: 0.43 us of MFMAs, the rest the chain of exchange, M and update between them.
+// Why 16 tokens: the products per token are those of chunks of 8, but a chunk's chain of exchange, triangle and update is paid half as
+// often, and Q S, which no other product waits for, is multiplied while the parts of K S are exchanged.  Whole calls, chunks of 8 against
+// 16, 16 heads 128 x 128, bf16 rows: gated, 4 prompts of 1501 .. 2048 tokens 285 -> 254 us (second launch 204 -> 166); general, 3 prompts
+// of 700 .. 2000: 285 -> 261; write, 8 portions of 509 over carried states: 115 -> 94, one prompt of 2048: 197 -> 118.  Where every SIMD
+// has a whole state's columns (general, 16 prompts of 300 .. 500) it is the products that count: 283 and 290; the shortest portions pay
+// for rows that are not there (general, 8 of 17: 28 and 33).  Token by token: gated 3123, general 3645, write 431; gated, 256 single
+// tokens: 393 -> 113 (4.8 TB/s of states, what a large copy reaches).
+// Of the 254 us the first launch is 83 (instructions: some 1700 a wave, half of them decays), the second 166, 129 chunks in a row at
+// 1.28 us: 0.83 us of MFMAs (15.3 ns each, back to back), the rest LDS latency and the chain.  Tried and slower: all large products
+// as six bf16 products of three parts each, split by the movers (198 us for the second launch: the LDS traffic of the parts; 144 without
+// them), the same for the updates alone (176), four waves a state on eight product waves (180).
 //
 // Against 64 bits (float32 rows, 1 to 300 tokens a sequence): states 0.9 to 1.5 times the token-by-token launch's error, all below
 // 3.3e-7; read-outs 1.0 to 1.24 times (1.2e-7 to 2.4e-7), because a chunk's sums are taken in another order: C and the pair products
-// are four sums each, since one sum over all key channels has its roundings one after the other (1.6 times the error).  Of bf16
+// are four sums each, since one sum over all key channels has its roundings one after the other (1.6 times the error).  Chunks of 16
+// against chunks of 8, 30 to 900 tokens: read-outs 0.99 to 1.02 times the error, states 0.99 to 1.00 (general 1.04 to 1.10).  Of bf16
 // read-outs, which are 1.7e-3 off by their own rounding, neither shows.
 //
 // The read-outs go to a scratch of fp32 rows, because a row's norm spans the workgroups of its value columns; a last launch
@@ -58,7 +66,7 @@
 
 namespace nv {
 
-constexpr int kCrChunk = 8;
+constexpr int kCrChunk = 16;
 constexpr float kCrNear = 8.27180613e-25f;            // 2^-80
 
 __device__ __forceinline__ float cr_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
@@ -120,13 +128,15 @@ template <> struct CrPair<__bf16, true> {
     uint32_t r;
     __device__ __forceinline__ void load(const __bf16* p) { r = *(const uint32_t*)p; }
     __device__ __forceinline__ float value(int i) const { return i ? bf16_hi(r) : bf16_lo(r); }
-    __device__ __forceinline__ void store(__bf16* p, bool in) const { *(uint32_t*)p = in ? r : 0u; }
+    __device__ __forceinline__ void keep(bool in) { r = in ? r : 0u; }
+    __device__ __forceinline__ void store(__bf16* p) const { *(uint32_t*)p = r; }
 };
 template <> struct CrPair<float, true> {
     float2 r;
     __device__ __forceinline__ void load(const float* p) { r = *(const float2*)p; }
     __device__ __forceinline__ float value(int i) const { return i ? r.y : r.x; }
-    __device__ __forceinline__ void store(float* p, bool in) const { *(float2*)p = in ? r : make_float2(0.f, 0.f); }
+    __device__ __forceinline__ void keep(bool in) { r = in ? r : make_float2(0.f, 0.f); }
+    __device__ __forceinline__ void store(float* p) const { *(float2*)p = r; }
 };
 template <typename T> struct CrPair<T, false> {
     typename CrRaw<T>::type r[2];
@@ -135,9 +145,13 @@ template <typename T> struct CrPair<T, false> {
         r[1] = CrRaw<T>::load(p + 1);
     }
     __device__ __forceinline__ float value(int i) const { return CrRaw<T>::value(r[i]); }
-    __device__ __forceinline__ void store(T* p, bool in) const {
-        p[0] = in ? (T)value(0) : (T)0.f;
-        p[1] = in ? (T)value(1) : (T)0.f;
+    __device__ __forceinline__ void keep(bool in) {
+        r[0] = in ? r[0] : 0;
+        r[1] = in ? r[1] : 0;
+    }
+    __device__ __forceinline__ void store(T* p) const {
+        p[0] = (T)value(0);
+        p[1] = (T)value(1);
     }
 };
 template <> struct CrRaw<float> {
@@ -150,63 +164,71 @@ __device__ __forceinline__ f32x4 cr_mfma(float a, float b, f32x4 c) { return __b
 __device__ __forceinline__ float cr_lane(float x, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
 }
-// The lower half's `lo` in the lower half of the lanes, the lower half's `hi` in the upper one.
-__device__ __forceinline__ float cr_spread(float lo, float hi) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, lo), __builtin_bit_cast(int, hi), false, false)[0]);
-}
 // LDS writes of this wave / of the workgroup's waves are done; loads from memory stay in flight.
 __device__ __forceinline__ void cr_wave_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 __device__ __forceinline__ void cr_group_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+template <int N> using CrRow = __attribute__((ext_vector_type(N))) float;
 // PER neighbouring elements of a row of V by one load.
 template <typename T, int PER> struct CrColumns : CrPair<T, true> {};
-template <typename T> struct CrColumns<T, 1> {
-    typename CrRaw<T>::type r;
-    __device__ __forceinline__ void load(const T* p) { r = CrRaw<T>::load(p); }
-    __device__ __forceinline__ float value(int) const { return CrRaw<T>::value(r); }
+template <> struct CrColumns<__bf16, 4> {
+    uint2 r;
+    __device__ __forceinline__ void load(const __bf16* p) { r = *(const uint2*)p; }
+    __device__ __forceinline__ float value(int i) const { return i & 1 ? bf16_hi(i < 2 ? r.x : r.y) : bf16_lo(i < 2 ? r.x : r.y); }
+};
+template <> struct CrColumns<float, 4> {
+    f32x4 r;
+    __device__ __forceinline__ void load(const float* p) { r = *(const f32x4*)p; }
+    __device__ __forceinline__ float value(int i) const { return r[i]; }
 };
 
 // Where a chunk's operands lie in the workspace: one record per (head, chunk), in the order in which the lanes of the second
-// launch read them, a head's chunks one after the other, beside them the chunks' rows of V ([head][record][8][Dv], zeros past the
+// launch read them, a head's chunks one after the other, beside them the chunks' rows of V ([head][record][16][Dv], zeros past the
 // sequence's end); read-outs are [head][row][Dv] too.  The second launch has few loads in flight, so streams that stay within a page
-// for several chunks matter to it (heads side by side, every chunk on pages of its own: 302 us instead of 264).  Records of a sequence start at (first row + 7 x its number) / 8: enough for the chunks in front, whatever
-// the lengths, without a scan over them.
+// for several chunks matter to it (heads side by side, every chunk on pages of its own: 302 us instead of 264, chunks of 8).  Records of a
+// sequence start at (first row + 15 x its number) / 16: enough for the chunks in front, whatever the lengths, without a scan over them.
 template <int FORM, int D>
 struct CrRecord {
-    static constexpr int kRows = FORM == kCrWrite ? 8 : 16;       // of [K; Q]: write has no K
+    static constexpr int kRows = FORM == kCrWrite ? 16 : 32;      // of [K; Q]: write has no K
     static constexpr int kUpd = FORM == kCrGeneral ? 2 : 1;       // update operands: K^ and / or X^
-    static constexpr int kq = 0;                                  // [tile][g][row][4 channels]
-    static constexpr int upd = kq + kRows * D;                    // [operand][tile][g][channel][2 tokens]
-    static constexpr int decay = upd + kUpd * 8 * D;              // [channel]
-    static constexpr int m = decay + D;                           // [16][16]
-    static constexpr int m2 = m + (FORM == kCrWrite ? 0 : 256);   // [16][8] (write: [8][8])
-    static constexpr int words = m2 + 8 * kRows;
+    static constexpr int kMat = FORM == kCrWrite ? 1 : FORM == kCrGated ? 2 : 4;      // gated: T, PQ; general: T, PQ, PV, PK; write: PV
+    static constexpr int kq = 0;                                  // [K, Q][tile][g][row][4 channels]
+    static constexpr int upd = kq + kRows * D;                    // [operand][tile][g][channel][4 tokens]
+    static constexpr int decay = upd + kUpd * 16 * D;             // [channel]
+    static constexpr int m = decay + D;                           // [matrix][16][16]
+    static constexpr int words = m + kMat * 256;
 };
 // (rows and numbers counted from the first sequence of the launch)
-__device__ __host__ __forceinline__ int64_t cr_first_record(int64_t first_row, int seq) { return (first_row + 7LL * seq) / 8; }
+__device__ __host__ __forceinline__ int64_t cr_first_record(int64_t first_row, int seq) {
+    return (first_row + (int64_t)(kCrChunk - 1) * seq) / kCrChunk;
+}
 
 // ------------------------------------------------------------------------------------------------ first launch
-// A wave per (chunk, head); a lane owns two neighbouring channels and all 8 tokens, so running products need no exchange.  LDS
-// (the wave's own) only turns the pair products' operands and [K; Q] into the order of the matrix cores.
-template <typename T, int FORM, int D>
+// Two waves per (chunk, head), eight tokens each; a lane owns two neighbouring channels of its eight tokens, so running products need
+// no exchange but of the halves' totals.  LDS turns the pair products' operands, K and Q into the order of the matrix cores; one wave
+// multiplies the rows K and solves for T, the other one multiplies the rows Q.  One wave with all 16 tokens spills registers (general:
+// 95 us where this takes 70, 3 prompts of 700 .. 2000 tokens; gated 88 and 83).
+template <int D>
 struct CrPrepLds {
     static constexpr int kRow = D + 4;                            // rows of D channels start on different banks
-    static constexpr int kRight = FORM == kCrGeneral ? 16 : 8;
-    float left[16 * kRow], right[kRight * kRow];                  // pair products' operands; then left holds [K; Q]
+    float k[16 * kRow], q[16 * kRow], right[16 * kRow];           // left sides, then [K; Q]; right sides
+    float total[2][D], kn[16], qn[16], beta[16];
+    uint32_t odd[2], far[2];
 };
 
 template <typename T, int FORM, int D, bool VEC>
-__global__ __launch_bounds__(256) void recurrence_chunks_kernel(const ChunkRecurrenceArgs a, const int first_seq) {
-    constexpr int NM = D / 16, NX = FORM == kCrGated ? 3 : FORM == kCrGeneral ? 4 : 2;
-    typedef CrPrepLds<T, FORM, D> Lds;
+__global__ __launch_bounds__(128, FORM == kCrGeneral ? 2 : 3) void recurrence_chunks_kernel(const ChunkRecurrenceArgs a, const int first_seq) {
+    constexpr int NM = D / 16, NX = FORM == kCrGated ? 3 : FORM == kCrGeneral ? 4 : 2, L = kCrChunk, N = L / 2;
+    constexpr bool HAS_K = FORM != kCrWrite;
+    typedef CrPrepLds<D> Lds;
     typedef CrRecord<FORM, D> Rec;
     typedef CrRaw<T> In;
     constexpr int ROW = Lds::kRow;
-    __shared__ __attribute__((aligned(16))) Lds all[4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l16 = lane & 15, g = lane >> 4, h = blockIdx.y * 4 + wave;
+    __shared__ __attribute__((aligned(16))) Lds lds;
+    const int lane = threadIdx.x & 63, half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, g = lane >> 4, h = blockIdx.y;
     const int64_t rec = blockIdx.x;
     const int row0 = a.cu_q[first_seq];
     int lo = first_seq, hi = a.num_seqs;              // the last sequence whose records start at or in front of this one
@@ -216,14 +238,13 @@ __global__ __launch_bounds__(256) void recurrence_chunks_kernel(const ChunkRecur
     }
     const int b = lo, q0 = a.cu_q[b], len = a.cu_q[b + 1] - q0;
     const int64_t c64 = rec - cr_first_record(q0 - row0, b - first_seq);
-    if (len < 2 || c64 * kCrChunk >= len || h >= a.H) return;
-    const int t0 = q0 + (int)c64 * kCrChunk, n = min(kCrChunk, q0 + len - t0);
+    if (len < 2 || c64 * L >= len) return;            // (for the whole workgroup)
+    const int t0 = q0 + (int)c64 * L, n16 = min(L, q0 + len - t0), n = min(N, max(n16 - half * N, 0)), th = half * N;
     float* out = a.chunks + (h * a.records + rec) * Rec::words;
-    Lds& lds = all[wave];
 
-    const bool in_row = 2 * lane < D;
+    const bool in_row = D == 128 || 2 * lane < D;
     const int d = in_row ? 2 * lane : 0;
-    CrPair<T, VEC> raw[NX][8];
+    CrPair<T, VEC> raw[NX][N];
     {
         const void* xs[4] = {a.x0, a.x1, a.x2, a.x3};
         const int64_t ss[4] = {a.s0, a.s1, a.s2, a.s3};
@@ -232,295 +253,297 @@ __global__ __launch_bounds__(256) void recurrence_chunks_kernel(const ChunkRecur
             const int hj = (FORM == kCrGated && j < 2) ? h / a.group : h;
             const T* p = (const T*)xs[j] + (int64_t)t0 * ss[j] + (int64_t)hj * D;
 #pragma unroll
-            for (int t = 0; t < 8; ++t) {             // (past the end: the chunk's first row, dropped below)
-                const T* row = p + (t < n ? t : 0) * ss[j];
+            for (int t = 0; t < N; ++t) {             // (past the end: the chunk's first row, dropped below)
+                const T* row = p + (t < n ? th + t : 0) * ss[j];
                 raw[j][t].load(row + d);
             }
         }
     }
-    float odd[8] = {};                                // NaN with a value that is not finite
+    float odd[4] = {};                                // NaN with a value that is not finite
     {
         const T* v = (const T*)a.v + (int64_t)t0 * a.sv + (int64_t)h * a.Dv;
-        T* to = (T*)a.columns + (h * a.records + rec) * 8 * a.Dv;
+        T* to = (T*)a.columns + ((h * a.records + rec) * L + th) * a.Dv;
         for (int c = 2 * lane; c < a.Dv; c += 128) {
-            CrPair<T, VEC> r[8];
+            CrPair<T, VEC> r[N];
 #pragma unroll
-            for (int t = 0; t < 8; ++t) r[t].load(v + (t < n ? t : 0) * a.sv + c);
+            for (int t = 0; t < N; ++t) r[t].load(v + (t < n ? th + t : 0) * a.sv + c);
 #pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                r[t].store(to + t * a.Dv + c, t < n);
-                odd[t] += r[t].value(0) * 0.f;
-                odd[t] += r[t].value(1) * 0.f;
+            for (int t = 0; t < N; ++t) {
+                r[t].keep(t < n);
+                r[t].store(to + t * a.Dv + c);
+                odd[t & 3] = fmaf(r[t].value(0), 0.f, odd[t & 3]);
+                odd[t & 3] = fmaf(r[t].value(1), 0.f, odd[t & 3]);
             }
         }
     }
     float beta = 0.f;                                 // raw, of token lane % 8
-    if constexpr (FORM == kCrGated) beta = CrRaw<T>::value(In::load((const T*)a.b_raw + (int64_t)(t0 + min(lane & 7, n - 1)) * a.b_stride + h));
+    if constexpr (FORM == kCrGated)
+        beta = CrRaw<T>::value(In::load((const T*)a.b_raw + (int64_t)(t0 + min(th + (lane & 7), n16 - 1)) * a.b_stride + h));
     float c0[2], c1[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         c0[i] = FORM == kCrGated ? expf(a.c0[h]) : a.c0[h * D + d + i];
         c1[i] = a.c1[h * D + d + i];
     }
-    CrElem el[8][2];
+    // Per token and channel: decay, and what else is not the raw projection itself (write: q; general: a k).
+    float w[N][2], made[FORM == kCrGated ? 1 : N][2];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
+    for (int t = 0; t < N; ++t) {
+#pragma unroll
+        for (int j = 0; j < NX; ++j)
+            if (HAS_K && j < 2) raw[j][t].keep(t < n && in_row);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             float in[4];
 #pragma unroll
-            for (int j = 0; j < NX; ++j) {
-                in[j] = raw[j][t].value(i);
-                odd[t] += in[j] * 0.f;
-            }
-            el[t][i] = cr_elem<FORM>(in, c0[i], c1[i], a.p0);
-            if (t >= n || !in_row) el[t][i] = CrElem{1.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < NX; ++j) in[j] = raw[j][t].value(i);
+            const CrElem el = cr_elem<FORM>(in, c0[i], c1[i], a.p0);
+            const bool live = t < n && in_row;
+            w[t][i] = live ? el.w : 1.f;
+            if constexpr (FORM == kCrWrite) made[t][i] = live ? el.q : 0.f;
+            if constexpr (FORM == kCrGeneral) made[t][i] = live ? el.a : 0.f;
+            odd[t & 3] = fmaf(w[t][i], 0.f, odd[t & 3]);
+            if constexpr (FORM != kCrGated) odd[t & 3] = fmaf(made[t][i], 0.f, odd[t & 3]);
+            if constexpr (FORM == kCrGeneral) odd[t & 3] = fmaf(raw[0][t].value(i), 0.f, odd[t & 3]);
         }
     }
-    const float sum_odd = ((odd[0] + odd[1]) + (odd[2] + odd[3])) + ((odd[4] + odd[5]) + (odd[6] + odd[7])) + beta * 0.f;
-    const bool any_odd = __any(sum_odd != 0.f);
-    if (lane == 0) a.odd[h * a.records + rec] = any_odd;
-    float kk = 0.f, qq = 0.f;                         // sums of squares of token lane % 8
-    if constexpr (FORM != kCrWrite) {
+    auto kf = [&](int t, int i) { return FORM == kCrWrite ? 1.f - w[t][i] : raw[1][t].value(i); };
+    auto qf = [&](int t, int i) { return FORM == kCrWrite ? made[FORM == kCrGated ? 0 : t][i] : raw[0][t].value(i); };
+    auto af = [&](int t, int i) { return made[FORM == kCrGated ? 0 : t][i]; };
+    // 1 / |k| and 1 / |q| of token lane % 8 (where the form takes them)
+    float kn = 1.f, qn = 1.f;
+    if constexpr (HAS_K) {
         auto squares = [&](auto of) {                 // 8 tokens' sums over 64 lanes: halved three times over the lanes, then summed
             float s[8];
 #pragma unroll
             for (int t = 0; t < 8; ++t) s[t] = of(t);
             const bool o1 = lane & 1, o2 = lane & 2, o4 = lane & 4;
-            float u[4], w[2];
+            float u[4], x[2];
 #pragma unroll
             for (int t = 0; t < 4; ++t) u[t] = (o1 ? s[2 * t + 1] : s[2 * t]) + dpp_f32<0xB1>(o1 ? s[2 * t] : s[2 * t + 1]);
 #pragma unroll
-            for (int t = 0; t < 2; ++t) w[t] = (o2 ? u[2 * t + 1] : u[2 * t]) + dpp_f32<0x4E>(o2 ? u[2 * t] : u[2 * t + 1]);
-            float r = (o4 ? w[1] : w[0]) + __shfl_xor(o4 ? w[0] : w[1], 4);
+            for (int t = 0; t < 2; ++t) x[t] = (o2 ? u[2 * t + 1] : u[2 * t]) + dpp_f32<0x4E>(o2 ? u[2 * t] : u[2 * t + 1]);
+            float r = (o4 ? x[1] : x[0]) + __shfl_xor(o4 ? x[0] : x[1], 4);
             r += __shfl_xor(r, 8);
             r += __shfl_xor(r, 16);
             return r + __shfl_xor(r, 32);
         };
-        kk = squares([&](int t) { return el[t][0].k * el[t][0].k + el[t][1].k * el[t][1].k; });
-        if constexpr (FORM == kCrGated) qq = squares([&](int t) { return el[t][0].q * el[t][0].q + el[t][1].q * el[t][1].q; });
-    }
-    // ---- pair products: entry (row 4 g + e, column l16): rows k | q, columns k | a k
-    f32x4 p = {0.f, 0.f, 0.f, 0.f};
-    auto products = [&] {                             // of the operands in LDS
-        cr_wave_sync();
-        f32x4 p0 = {0.f, 0.f, 0.f, 0.f}, p1 = p0, p2 = p0, p3 = p0;
-        const int lrow = FORM == kCrWrite ? (8 + (l16 & 7)) : l16;
-        const float* lf = lds.left + lrow * ROW + 4 * g;
-        const float* rt = lds.right + (Lds::kRight == 16 ? l16 : (l16 & 7)) * ROW + 4 * g;
-#pragma unroll
-        for (int m = 0; m < NM; ++m) {
-            const f32x4 x = *(const f32x4*)(lf + 16 * m), y = *(const f32x4*)(rt + 16 * m);
-            p0 = cr_mfma(x[0], y[0], p0);
-            p1 = cr_mfma(x[1], y[1], p1);
-            p2 = cr_mfma(x[2], y[2], p2);
-            p3 = cr_mfma(x[3], y[3], p3);
+        const bool in = (lane & 7) < n;
+        const float ss = squares([&](int t) { return kf(t, 0) * kf(t, 0) + kf(t, 1) * kf(t, 1); });     // (all lanes take part)
+        odd[0] += ss * 0.f;
+        kn = in ? 1.0f / sqrtf(ss + a.p1) : 0.f;
+        if constexpr (FORM == kCrGated) {
+            const float qq = squares([&](int t) { return qf(t, 0) * qf(t, 0) + qf(t, 1) * qf(t, 1); });
+            odd[1] += qq * 0.f + beta * 0.f;
+            qn = 1.0f / sqrtf((qq + a.p1) * (float)D);
+            beta = in ? cr_sigmoid(beta) : 0.f;
         }
-        return (p0 + p1) + (p2 + p3);
-    };
-    // relative to the middle: left sides G_t / G_4, right sides G_4 / G_t
-    float side[2][8];
-    bool near = true;                                 // (false with a decay that is not a number)
+        if (lane < 8) {
+            lds.kn[th + lane] = kn;
+            lds.qn[th + lane] = qn;
+            lds.beta[th + lane] = beta;
+        }
+    }
+    // decays from the half's first token through t, and behind t to the half's end
+    float pre[2][N], suf[2][N];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        side[i][3] = 1.f;                             // of tokens 0 .. 3: products behind the token; 4 .. 7: through the token
+        pre[i][0] = w[0][i];
+        suf[i][N - 1] = 1.f;
 #pragma unroll
-        for (int t = 2; t >= 0; --t) side[i][t] = side[i][t + 1] * el[t + 1][i].w;
-        side[i][4] = el[4][i].w;
-#pragma unroll
-        for (int t = 5; t < 8; ++t) side[i][t] = side[i][t - 1] * el[t][i].w;
-        near = near && side[i][0] * el[0][i].w >= kCrNear && side[i][7] >= kCrNear;
+        for (int t = 1; t < N; ++t) {
+            pre[i][t] = pre[i][t - 1] * w[t][i];
+            suf[i][N - 1 - t] = suf[i][N - t] * w[N - t][i];
+        }
     }
-    if (__all(near)) {
+    {
+        const bool near = pre[0][N - 1] >= kCrNear && pre[1][N - 1] >= kCrNear;          // (false with a decay that is not a number)
+        const bool any_far = !__all(near), any_odd = __any((odd[0] + odd[1]) + (odd[2] + odd[3]) != 0.f);
+        if (lane == 0) {
+            lds.far[half] = any_far;
+            lds.odd[half] = any_odd;
+        }
+        if (in_row) *(float2*)(lds.total[half] + d) = make_float2(pre[0][N - 1], pre[1][N - 1]);
+    }
+    auto put = [&](float* rows, auto of) {            // this wave's 8 rows of this lane's two channels
         if (in_row) {
 #pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                float lv[2], rv[2], hb[2];
+            for (int t = 0; t < N; ++t) *(float2*)(rows + (th + t) * ROW + d) = make_float2(of(t, 0), of(t, 1));
+        }
+    };
+    __syncthreads();
+    if (half == 0 && lane == 0) a.odd[h * a.records + rec] = lds.odd[0] | lds.odd[1];
+    const bool near = (lds.far[0] | lds.far[1]) == 0;
+    // ---- pair products: entry (row 4 g + e, column l16), rows k (first wave) or q (second), columns k or a k
+    f32x4 pk = {0.f, 0.f, 0.f, 0.f}, pa = pk;
+    {
+        auto product = [&] {                          // of the operands in LDS
+            f32x4 p0 = {0.f, 0.f, 0.f, 0.f}, p1 = p0, p2 = p0, p3 = p0;
+            const float* lf = (half ? lds.q : lds.k) + l16 * ROW + 4 * g;
+            const float* rt = lds.right + l16 * ROW + 4 * g;
+#pragma unroll
+            for (int m = 0; m < NM; ++m) {
+                const f32x4 x = *(const f32x4*)(lf + 16 * m), y = *(const f32x4*)(rt + 16 * m);
+                p0 = cr_mfma(x[0], y[0], p0);
+                p1 = cr_mfma(x[1], y[1], p1);
+                p2 = cr_mfma(x[2], y[2], p2);
+                p3 = cr_mfma(x[3], y[3], p3);
+            }
+            return (p0 + p1) + (p2 + p3);
+        };
+        // Relative to the middle: left sides G_t / G_8, right sides G_8 / G_t.  Otherwise part 8, 4, 2, 1 (0: s = t) one after the
+        // other: left sides from the start of the part through the token, right sides behind the token to the end of its part.
+#pragma unroll 1
+        for (int part = 8; part >= 0; part = near ? -1 : part == 1 ? 0 : part == 0 ? -1 : part / 2) {
+            float lv[2][N], rv[2][N], first[2] = {1.f, 1.f};      // (first: left side of the first token's key, general)
+            if (part == 8) {
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
-                    const float inv = __builtin_amdgcn_rcpf(side[i][t]);
-                    lv[i] = t < 4 ? inv : side[i][t];
-                    rv[i] = t < 4 ? side[i][t] : inv;
-                    if constexpr (FORM == kCrGeneral) // the old state: through the token before
-                        hb[i] = t == 0 ? __builtin_amdgcn_rcpf(side[i][0] * el[0][i].w)
-                                       : t < 4 ? __builtin_amdgcn_rcpf(side[i][t - 1]) : t == 4 ? 1.f : side[i][t - 1];
-                    else hb[i] = lv[i];
+#pragma unroll
+                    for (int t = 0; t < N; ++t) {
+                        lv[i][t] = near && half == 0 ? __builtin_amdgcn_rcpf(suf[i][t]) : pre[i][t];
+                        rv[i][t] = near && half == 1 ? __builtin_amdgcn_rcpf(pre[i][t]) : suf[i][t];
+                    }
+                    if (near && half == 0) first[i] = __builtin_amdgcn_rcpf(pre[i][N - 1]);
                 }
-                if constexpr (FORM != kCrWrite) *(float2*)(lds.left + t * ROW + d) = make_float2(el[t][0].k * hb[0], el[t][1].k * hb[1]);
-                *(float2*)(lds.left + (8 + t) * ROW + d) = make_float2(el[t][0].q * lv[0], el[t][1].q * lv[1]);
-                *(float2*)(lds.right + t * ROW + d) = make_float2(el[t][0].k * rv[0], el[t][1].k * rv[1]);
-                if constexpr (FORM == kCrGeneral)
-                    *(float2*)(lds.right + (8 + t) * ROW + d) = make_float2(el[t][0].a * rv[0], el[t][1].a * rv[1]);
-            }
-        }
-        p = products();
-    } else {
-#pragma unroll 1
-        for (int part = 4; part >= 0; part = part == 1 ? 0 : part == 0 ? -1 : part / 2) {       // 4, 2, 1; 0: s = t
-            if (in_row) {
-                float lv[2] = {1.f, 1.f}, rv[2] = {1.f, 1.f};
+            } else {
 #pragma unroll
-                for (int t = 0; t < 8; ++t) {         // from the start of its part through the token
-                    if ((t & (part - 1)) == 0) lv[0] = lv[1] = 1.f;
-                    const float before[2] = {lv[0], lv[1]};
+                for (int i = 0; i < 2; ++i) {
+                    float f = 1.f;
 #pragma unroll
-                    for (int i = 0; i < 2; ++i) lv[i] *= part ? el[t][i].w : 1.f;
-                    const float* kv = FORM == kCrGeneral ? before : lv;
-                    if constexpr (FORM != kCrWrite) *(float2*)(lds.left + t * ROW + d) = make_float2(el[t][0].k * kv[0], el[t][1].k * kv[1]);
-                    *(float2*)(lds.left + (8 + t) * ROW + d) = make_float2(el[t][0].q * lv[0], el[t][1].q * lv[1]);
-                }
+                    for (int t = 0; t < N; ++t) {
+                        if ((t & (part - 1)) == 0) f = 1.f;
+                        f *= part ? w[t][i] : 1.f;
+                        lv[i][t] = f;
+                    }
 #pragma unroll
-                for (int t = 7; t >= 0; --t) {        // behind the token to the end of its part
-                    if (((t + 1) & (part - 1)) == 0) rv[0] = rv[1] = 1.f;
-                    *(float2*)(lds.right + t * ROW + d) = make_float2(el[t][0].k * rv[0], el[t][1].k * rv[1]);
-                    if constexpr (FORM == kCrGeneral)
-                        *(float2*)(lds.right + (8 + t) * ROW + d) = make_float2(el[t][0].a * rv[0], el[t][1].a * rv[1]);
-#pragma unroll
-                    for (int i = 0; i < 2; ++i) rv[i] *= part ? el[t][i].w : 1.f;
+                    for (int t = N - 1; t >= 0; --t) {
+                        if (((t + 1) & (part - 1)) == 0) f = 1.f;
+                        rv[i][t] = part ? f : 1.f;
+                        f *= w[t][i];
+                    }
                 }
             }
-            const f32x4 of = products();
+            if constexpr (HAS_K)
+                put(lds.k, [&](int t, int i) {        // (general: through the token before)
+                    if constexpr (FORM != kCrGeneral) return kf(t, i) * lv[i][t];
+                    return kf(t, i) * (t == 0 ? first[i] : (t & (part - 1)) == 0 ? 1.f : lv[i][t ? t - 1 : 0]);
+                });
+            put(lds.q, [&](int t, int i) { return qf(t, i) * lv[i][t]; });
+            put(lds.right, [&](int t, int i) { return kf(t, i) * rv[i][t]; });
+            // pairs whose tokens part at this part (one compare and a select: branches here have come out of the compiler without
+            // their assignments)
+            const uint32_t from = near ? 0 : part, many = near ? 16 : part ? part : 1;
+            auto take = [&](f32x4& to, f32x4 of) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int apart = ((4 * g + e) & 7) ^ (l16 & 7);
-                if (part ? apart >= part && apart < 2 * part : apart == 0) p[e] = of[e];
+                for (int e = 0; e < 4; ++e) to[e] = (uint32_t)((4 * g + e) ^ l16) - from < many ? of[e] : to[e];
+            };
+            __syncthreads();
+            if (HAS_K || half) take(pk, product());
+            __syncthreads();
+            if constexpr (FORM == kCrGeneral) {
+                put(lds.right, [&](int t, int i) { return af(t, i) * rv[i][t]; });
+                __syncthreads();
+                take(pa, product());
+                __syncthreads();
             }
-            cr_wave_sync();
         }
     }
-    // ---- [K; Q], K^, X^ and the chunk's decay
-    float G[2][8], F[2][8];
+    // ---- [K; Q] (through LDS), K^, X^ and the chunk's decay; k and q are unit vectors from here on (gated)
+    auto ku = [&](int t, int i) { return FORM == kCrGated ? kf(t, i) * cr_lane(kn, t) : kf(t, i); };
+    auto qu = [&](int t, int i) { return FORM == kCrGated ? qf(t, i) * cr_lane(qn, t) : qf(t, i); };
+    const float2 front = half ? *(const float2*)(lds.total[0] + d) : make_float2(1.f, 1.f);           // decays of the other half, in front
+    const float2 behind = half ? make_float2(1.f, 1.f) : *(const float2*)(lds.total[1] + d);          // and behind
+    const float fr[2] = {front.x, front.y}, be[2] = {behind.x, behind.y};
+    if constexpr (FORM == kCrGated) put(lds.k, [&](int t, int i) { return ku(t, i) * (fr[i] * pre[i][t]); });
+    if constexpr (FORM == kCrGeneral) put(lds.k, [&](int t, int i) { return ku(t, i) * (t ? fr[i] * pre[i][t ? t - 1 : 0] : fr[i]); });
+    put(lds.q, [&](int t, int i) { return qu(t, i) * (fr[i] * pre[i][t]); });
+    auto put_update = [&](int which, auto of) {       // lane (g, channel) of a tile: tokens 4 g .. 4 g + 3
+        if (in_row) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        G[i][0] = el[0][i].w;
-        F[i][7] = 1.f;
+            for (int gg = 0; gg < 2; ++gg) {
+                float* to = out + Rec::upd + which * 16 * D + (((d >> 4) * 4 + half * 2 + gg) * 16 + (d & 15)) * 4;
 #pragma unroll
-        for (int t = 1; t < 8; ++t) {
-            G[i][t] = G[i][t - 1] * el[t][i].w;
-            F[i][7 - t] = F[i][8 - t] * el[8 - t][i].w;
-        }
-    }
-    cr_wave_sync();
-    if (in_row) {
+                for (int i = 0; i < 2; ++i) {
+                    f32x4 r;
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            if constexpr (FORM == kCrGated)
-                *(float2*)(lds.left + t * ROW + d) = make_float2(el[t][0].k * G[0][t], el[t][1].k * G[1][t]);
-            if constexpr (FORM == kCrGeneral)
-                *(float2*)(lds.left + t * ROW + d) = make_float2(t ? el[t][0].k * G[0][t ? t - 1 : 0] : el[t][0].k,
-                                                                 t ? el[t][1].k * G[1][t ? t - 1 : 0] : el[t][1].k);
-            *(float2*)(lds.left + (8 + t) * ROW + d) = make_float2(el[t][0].q * G[0][t], el[t][1].q * G[1][t]);
-        }
-        *(float2*)(out + Rec::decay + d) = make_float2(G[0][7], G[1][7]);
-        // token pairs in the order of the lane groups that supply them: of V 0 1 | 2 3 | 4 5 | 6 7, of U 0 1 | 4 5 | 2 3 | 6 7
-        auto store = [&](int which, auto of, bool u) {
-#pragma unroll
-            for (int pos = 0; pos < 4; ++pos) {
-                const int t = u ? (pos == 1 ? 4 : pos == 2 ? 2 : 2 * pos) : 2 * pos;
-                float* to = out + Rec::upd + which * 8 * D + (((d >> 4) * 4 + pos) * 16 + (d & 15)) * 2;
-                *(f32x4*)to = f32x4{of(t, 0) * F[0][t], of(t + 1, 0) * F[0][t + 1], of(t, 1) * F[1][t], of(t + 1, 1) * F[1][t + 1]};
+                    for (int e = 0; e < 4; ++e) r[e] = of(4 * gg + e, i) * (suf[i][4 * gg + e] * be[i]);
+                    *(f32x4*)(to + 4 * i) = r;
+                }
             }
-        };
-        if constexpr (FORM == kCrGated) store(0, [&](int t, int i) { return el[t][i].k; }, true);
-        else store(0, [&](int t, int i) { return el[t][i].k; }, false);
-        if constexpr (FORM == kCrGeneral) store(1, [&](int t, int i) { return el[t][i].a; }, true);
+        }
+    };
+    if constexpr (FORM == kCrGated) put_update(0, ku); else put_update(0, kf);
+    if constexpr (FORM == kCrGeneral) put_update(1, af);
+    if (half == 0 && in_row) *(float2*)(out + Rec::decay + d) = make_float2(pre[0][N - 1] * be[0], pre[1][N - 1] * be[1]);
+    __syncthreads();
+    if (HAS_K || half) {
+        const float* rows = (half ? lds.q : lds.k) + l16 * ROW + 4 * g;
+        const int tile = HAS_K && half ? NM : 0;
+#pragma unroll
+        for (int m = 0; m < NM; ++m) *(f32x4*)(out + Rec::kq + ((tile + m) * 64 + lane) * 4) = *(const f32x4*)(rows + 16 * m);
     }
-    cr_wave_sync();
+    // ---- T, and what the tokens' writes bring the read-outs
+    float* mat = out + Rec::m;
+    auto put_matrix = [&](int which, f32x4 p, int strict) {                   // s <= t (strict: s < t), zeros elsewhere
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mat[which * 256 + (4 * g + e) * 16 + l16] = l16 + strict <= 4 * g + e ? p[e] : 0.f;
+    };
     if constexpr (FORM == kCrWrite) {
-        // lanes: (tile, g, row) of 8 rows, 16 bytes each
-#pragma unroll
-        for (int i = 0; i < NM / 2; ++i) {
-            const int at = i * 64 + lane;             // tile at / 32, g (at / 8) % 4, row at % 8
-            *(f32x4*)(out + Rec::kq + at * 4) = *(const f32x4*)(lds.left + (8 + (at & 7)) * ROW + 16 * (at >> 5) + 4 * ((at >> 3) & 3));
-        }
-    } else {
-#pragma unroll
-        for (int m = 0; m < NM; ++m) *(f32x4*)(out + Rec::kq + (m * 64 + lane) * 4) = *(const f32x4*)(lds.left + l16 * ROW + 16 * m + 4 * g);
-    }
-    // ---- M and M2
-    float* m = out + Rec::m;
-    float* m2 = out + Rec::m2;
-    if constexpr (FORM == kCrWrite) {
-        if (g < 2 && l16 < 8) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) m2[(4 * g + e) * 8 + l16] = l16 <= 4 * g + e ? p[e] : 0.f;
-        }
+        if (half) put_matrix(0, pk, 0);
         return;
     }
-    const int j = lane & 7;
-    const bool in = j < n;
-    const float kn = in ? 1.0f / sqrtf(kk + a.p1) : 0.f;                               // of token lane % 8
-    const float qn = FORM == kCrGated ? 1.0f / sqrtf((qq + a.p1) * (float)D) : 1.0f;
-    // Lanes 0 - 7: columns of M for the rows K; lanes 8 - 15: columns of M2; lanes 16 - 23: columns of M for the rows Q.
-    const int kind = lane >> 3;
-    float y[8], o[8];
-    if constexpr (FORM == kCrGated) {
-        // u = T beta (v - kn K^T S), T = (I + A)^-1, A_ts = beta_t kn_t kn_s P_ts (s < t);  y_t = kn_t u_t is what X^ = k G_8 / G_t
-        // takes, o_t = qn_t (Q^T S + sum_(s <= t) P'_ts y_s)
-        beta = in ? cr_sigmoid(beta) : 0.f;
-        const float rhs = kind == 0 ? -beta * kn * kn : kind == 1 ? beta * kn : 0.f;
-        const float scale = beta * kn * kn;
+    // gated: u = T (v - K^T S), T = (I + A)^-1 diag(beta), A_ts = beta_t kn_t kn_s P_ts (s < t);  o_t = Q^T S + qn_t kn_s P_ts u_s
+    // general: x = (I + A)^-1 diag(kn) (K^T S + PK v), A_ts = kn_t kn_s P_ts(k, a k), PK_ts = P_ts(k, k) (s < t); the writes along a k
+    //          take u_s = -kn_s x_s, which T makes at once;  o_t = Q^T S + P_ts(r, k) v_s + P_ts(r, a k) u_s
+    const float kc = lds.kn[l16];
+    f32x4 rows, p = FORM == kCrGated ? pk : pa;
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            float s = 0.f;
-#pragma unroll
-            for (int i = 0; i < t; ++i) s += cr_lane(p[t & 3], (t >> 2) * 16 + i) * y[i];
-            y[t] = (t == j ? rhs : 0.f) - cr_lane(scale, t) * s;
-        }
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            float s = (kind == 2 && t == j) ? 1.f : 0.f;
-#pragma unroll
-            for (int i = 0; i <= t; ++i) s += cr_lane(p[t & 3], (2 + (t >> 2)) * 16 + i) * y[i];
-            o[t] = s * cr_lane(qn, t);
-        }
-    } else {
-        // x_t = u_t^T S_(t-1) = kn_t (K^T S + sum_(s < t) P_ts(k, k) v_s - P_ts(k, a k) kn_s x_s);  y_t = kn_t x_t, taken with
-        // a minus sign by X^ = a k G_8 / G_t;  o_t = Q^T S + sum_(s <= t) P_ts(r, k) v_s - P_ts(r, a k) y_s
-        const float kn2 = kn * kn;
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const float nt = __shfl(p[t & 3], (t >> 2) * 16 + j);
-            float s = kind == 0 ? (t == j ? 1.f : 0.f) : kind == 1 ? (t > j ? nt : 0.f) : 0.f;
-#pragma unroll
-            for (int i = 0; i < t; ++i) s -= cr_lane(p[t & 3], (t >> 2) * 16 + 8 + i) * y[i];
-            y[t] = cr_lane(kn2, t) * s;
-        }
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const float bt = __shfl(p[t & 3], (2 + (t >> 2)) * 16 + j);
-            float s = kind == 2 ? (t == j ? 1.f : 0.f) : kind == 1 ? (t >= j ? bt : 0.f) : 0.f;
-#pragma unroll
-            for (int i = 0; i <= t; ++i) s -= cr_lane(p[t & 3], (2 + (t >> 2)) * 16 + 8 + i) * y[i];
-            o[t] = s;
-        }
+    for (int e = 0; e < 4; ++e) rows[e] = half ? (FORM == kCrGated ? lds.qn[4 * g + e] : 0.f) : lds.kn[4 * g + e];
+    if (half) {
+        if constexpr (FORM == kCrGated) p *= rows * kc;
+        put_matrix(1, p, 0);
+        if constexpr (FORM == kCrGeneral) put_matrix(2, pk, 0);
+        return;
     }
-    if (kind < 3) {
-        float* to = kind == 1 ? m2 + j : m + (kind == 2 ? 8 : 0) + j;
-        const int ld = kind == 1 ? 8 : 16;
+    if constexpr (FORM == kCrGeneral) put_matrix(3, pk, 1);
+    const float bc = FORM == kCrGated ? lds.beta[l16] : kc;
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            to[t * ld] = FORM == kCrGeneral ? -y[t] : y[t];
-            to[(8 + t) * ld] = o[t];
+    for (int e = 0; e < 4; ++e) p[e] *= (FORM == kCrGated ? rows[e] * lds.beta[4 * g + e] : rows[e]) * kc;
+    float y[L];                                       // column l16 of T
+#pragma unroll
+    for (int t = 0; t < L; ++t) {
+        float s0 = t == l16 ? bc : 0.f, s1 = 0.f;
+#pragma unroll
+        for (int i = 0; i < t; ++i) {
+            const float f = cr_lane(p[t & 3], (t >> 2) * 16 + i);
+            if (i & 1) s1 -= f * y[i]; else s0 -= f * y[i];
         }
+        y[t] = s0 + s1;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float lo2 = g & 1 ? y[4 + e] : y[e], hi2 = g & 1 ? y[12 + e] : y[8 + e];
+        mat[(4 * g + e) * 16 + l16] = (g & 2 ? hi2 : lo2) * (FORM == kCrGeneral ? -rows[e] : 1.f);
     }
 }
 
 // ------------------------------------------------------------------------------------------------ second launch
 // RS waves per (sequence, head, 16 value columns), each with D / RS key channels of the state in MFMA accumulators; RS = 2: the
-// waves' parts of [K; Q] S are exchanged through LDS.  A workgroup has four of these waves, one on each SIMD of a CU, and four that
-// do nothing but move: records and columns of V four chunks ahead into registers and two ahead into LDS (three slots), read-outs from LDS to
-// memory.  One barrier a chunk.  The products alone are bound by their chain (product, exchange, M, update); with the loads and
-// stores in the same waves every chunk also paid for their issue (gated, 4 x 1501 .. 2048 tokens, 16 heads: 264 us instead of 219).
+// waves' parts of K S are exchanged through LDS while Q S is multiplied, and each takes half of what is added to Q S, which the movers
+// add up.  A workgroup has four of these waves, one on each SIMD of a CU, and four that do nothing but move: records and columns of V four
+// chunks ahead into registers and two ahead into LDS (three slots), read-outs from LDS to memory.  One barrier a chunk.  With the loads
+// and stores in the products' waves every chunk also paid for their issue (chunks of 8: 264 us instead of 219).
 template <typename T, int FORM, int D, int RS>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void recurrence_states_kernel(
     const ChunkRecurrenceArgs a, const int first_seq) {
     constexpr int NM = D / 16 / RS;                   // tiles of a wave
+    constexpr int L = kCrChunk;
     typedef CrRecord<FORM, D> Rec;
     constexpr int ROUNDS = (Rec::words + 1023) / 1024;
-    constexpr int COLS = 64 / RS, PER = 2 / RS;       // value columns of the workgroup; elements of a row of V a thread moves
+    constexpr int COLS = 64 / RS, PER = 4 / RS;       // value columns of the workgroup; elements of a row of V a thread moves
     __shared__ __attribute__((aligned(16))) float slots[3][Rec::words];
-    __shared__ __attribute__((aligned(8))) float vs[3][kCrChunk][COLS], os[2][kCrChunk][COLS];
+    __shared__ __attribute__((aligned(16))) float vs[3][L][COLS], os[2][RS][L][COLS];
     __shared__ f32x4 part[RS == 1 ? 1 : 2][4][64];
     // Workgroups go to the eight XCDs in turn: an XCD takes neighbouring heads.
     const int pair = gridDim.x % 8 == 0 ? (int)(blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8) : (int)blockIdx.x;
@@ -528,16 +551,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int q0 = a.cu_q[b], len = a.cu_q[b + 1] - q0;
     if (len < 2) return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int chunks = (len + kCrChunk - 1) / kCrChunk, Dv = a.Dv;
+    const int chunks = (len + L - 1) / L, Dv = a.Dv;
 
     if (wave >= 4) {
         // ---------------------------------------------------------------- the movers
         const int tid = threadIdx.x - 256;
         const int64_t first = (int64_t)h * a.records + cr_first_record(q0 - a.cu_q[first_seq], b - first_seq);
         const float* rec = a.chunks + first * Rec::words;
-        const int tok = tid >> 5, col = (tid & 31) * PER, col_all = blockIdx.y * COLS + col;
+        const int tok = tid >> 4, col = (tid & 15) * PER, col_all = blockIdx.y * COLS + col;
         // (columns past the end: the last ones, used by waves that write nothing)
-        const T* v = (const T*)a.columns + first * 8 * Dv + tok * Dv + min(col_all, Dv - PER);
+        const T* v = (const T*)a.columns + first * L * Dv + tok * Dv + min(col_all, Dv - PER);
         float* o = a.raw + ((int64_t)h * a.T + q0 + tok) * Dv + col_all;
         struct Staged {
             f32x4 r[ROUNDS];
@@ -546,7 +569,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         auto fetch = [&](int c, Staged& st) {
             c = min(c, chunks - 1);
             const float* rc = rec + (int64_t)c * Rec::words;
-            st.v.load(v + (int64_t)c * 8 * Dv);
+            st.v.load(v + (int64_t)c * L * Dv);
 #pragma unroll
             for (int i = 0; i < ROUNDS; ++i)
                 if ((i + 1) * 1024 <= Rec::words || i * 1024 + tid * 4 < Rec::words) st.r[i] = *(const f32x4*)(rc + (uint32_t)(i * 1024 + tid * 4));
@@ -559,9 +582,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 if ((i + 1) * 1024 <= Rec::words || i * 1024 + tid * 4 < Rec::words) *(f32x4*)(slots[at] + i * 1024 + tid * 4) = st.r[i];
         };
         auto store = [&](int c) {
-            if (c * kCrChunk + tok < len && col_all < Dv) {
-#pragma unroll
-                for (int e = 0; e < PER; ++e) o[(int64_t)c * kCrChunk * Dv + e] = os[c & 1][tok][col + e];
+            if (c * L + tok < len && col_all < Dv) {
+                float* to = o + (int64_t)c * L * Dv;
+                if constexpr (RS == 1) *(f32x4*)to = *(const f32x4*)&os[c & 1][0][tok][col];
+                else {
+                    const float2 x = *(const float2*)&os[c & 1][0][tok][col], y = *(const float2*)&os[c & 1][RS - 1][tok][col];
+                    *(float2*)to = make_float2(x.x + y.x, x.y + y.y);
+                }
             }
         };
         Staged s0, s1;
@@ -609,54 +636,116 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int c = lane; c < chunks; c += 64) odd |= flags[c];
         odd = __any(odd != 0);
     }
-    const int at_kq = Rec::kq + (FORM == kCrWrite ? (g * 8 + (l16 & 7)) * 4 + d0 * 8 : lane * 4 + d0 * 16);
-    constexpr int kq_tile = 16 * Rec::kRows;
-    const int at_upd = Rec::upd + lane * 2 + d0 * 8, at_dec = Rec::decay + d0 + ((l16 + 4 * g) & 15), at_m = Rec::m + l16 * 16 + 4 * g;
-    const int at_m2 = Rec::m2 + (FORM == kCrWrite ? l16 & 7 : l16) * 8 + 2 * g;
-    f32x4 x[NM];
+    const int at_x = Rec::kq + lane * 4 + d0 * 16, at_upd = Rec::upd + lane * 4 + d0 * 16;
+    const int at_dec = Rec::decay + d0 + ((l16 + 4 * g) & 15), at_m = Rec::m + l16 * 16 + 4 * g;
+    constexpr bool HAS_K = FORM != kCrWrite, HAS_V = FORM != kCrGated;
+    constexpr int MV = FORM == kCrGeneral ? 512 : 0;  // the matrix that takes V to the read-outs
+    constexpr f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 x[NM];                                      // the first rows that a chunk multiplies: read behind the barrier in front of it
     auto read_x = [&](int at) {
 #pragma unroll
-        for (int m = 0; m < NM; ++m) x[m] = *(const f32x4*)(slots[at] + kq_tile * m + at_kq);
+        for (int m = 0; m < NM; ++m) x[m] = *(const f32x4*)(slots[at] + 256 * m + at_x);
+    };
+    // Rows of a lower triangular matrix times 16 rows of values, the wave's share of the 16; ODD: a zero above the diagonal keeps a later
+    // token out only while that token's value is finite, so token by token, each from rows that end with it.
+    constexpr int E0 = 4 / RS;
+    auto triangle = [&](auto odd_tag, auto all_tag, f32x4 mt, f32x4 x, f32x4 onto) {
+        constexpr bool ODD = decltype(odd_tag)::value, ALL = decltype(all_tag)::value || RS == 1;
+        auto sum = [&](int t, f32x4 c0) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (!ALL && e >= E0) continue;
+                const float me = ALL ? mt[e] : rp ? mt[(E0 + e) & 3] : mt[e], xe = ALL ? x[e] : rp ? x[(E0 + e) & 3] : x[e];
+                const int row = 4 * g + (ALL ? e : rp * E0 + e);
+                c0 = cr_mfma(me, ODD ? (row <= t ? xe : 0.f) : xe, c0);       // (a sum that goes on costs a product no wait)
+            }
+            return c0;
+        };
+        if constexpr (!ODD) return sum(0, onto);
+        f32x4 rows = zero;
+#pragma unroll 1
+        for (int t = 0; t < L; ++t) {
+            const f32x4 r = sum(t, onto);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (4 * g + e == t) rows[e] = r[e];
+        }
+        return rows;
     };
     cr_group_barrier();
     read_x(0);
     int at = 0;
     auto chunk = [&](auto odd_tag, int c) {           // chunk c from slot `at`
-        constexpr bool ODD = decltype(odd_tag)::value;
+        constexpr std::false_type share{};
+        constexpr std::true_type whole{};
         const float* rc = slots[at];
-        f32x4 y;
         float dec[NM];                                // lane e of group g: the decay of row 4 g + e of the tile
-        float2 uk[NM], ux[NM];
-        float vv[2];
-        const float2 y2 = *(const float2*)(rc + at_m2);
+        f32x4 xq[NM], up[NM], ux[NM], vv, mt, mq, mv, mk;
 #pragma unroll
-        for (int e = 0; e < 2; ++e) vv[e] = vs[at][2 * g + e][in_group];
-        if constexpr (FORM != kCrWrite) y = *(const f32x4*)(rc + at_m);
+        for (int m = 0; m < NM; ++m) xq[m] = HAS_K ? *(const f32x4*)(rc + 16 * D + 256 * m + at_x) : x[m];
 #pragma unroll
-        for (int m = 0; m < NM; ++m) {
-            dec[m] = rc[16 * m + at_dec];
-            if constexpr (FORM != kCrGated) uk[m] = *(const float2*)(rc + 128 * m + at_upd);
-            if constexpr (FORM != kCrWrite) ux[m] = *(const float2*)(rc + (Rec::kUpd - 1) * 8 * D + 128 * m + at_upd);
+        for (int e = 0; e < 4; ++e) vv[e] = vs[at][4 * g + e][in_group];
+        if constexpr (FORM == kCrGeneral) mk = *(const f32x4*)(rc + 768 + at_m);
+        if constexpr (HAS_V) mv = *(const f32x4*)(rc + MV + at_m);
+        if constexpr (HAS_K) {
+            mt = *(const f32x4*)(rc + at_m);
+            mq = *(const f32x4*)(rc + 256 + at_m);
         }
-        f32x4 c0 = {0.f, 0.f, 0.f, 0.f}, d = c0, c1 = c0, c2 = c0, c3 = c0;   // (four sums: a quarter of the roundings one after the other)
         __builtin_amdgcn_sched_barrier(0);            // the reads are on their way before the products
+        auto read_update = [&] {
 #pragma unroll
-        for (int m = 0; m < NM; ++m) {
-            c0 = cr_mfma(x[m][0], S[m][0], c0);
-            c1 = cr_mfma(x[m][1], S[m][1], c1);
-            c2 = cr_mfma(x[m][2], S[m][2], c2);
-            c3 = cr_mfma(x[m][3], S[m][3], c3);
+            for (int m = 0; m < NM; ++m) {
+                dec[m] = rc[16 * m + at_dec];
+                if constexpr (HAS_V) up[m] = *(const f32x4*)(rc + 256 * m + at_upd);
+                if constexpr (HAS_K) ux[m] = *(const f32x4*)(rc + (Rec::kUpd - 1) * 16 * D + 256 * m + at_upd);
+            }
+        };
+        // (four sums: a quarter of the roundings one after the other)
+        f32x4 ck = zero, other = zero, o0 = zero, o1 = zero, o2 = zero, o3 = zero;
+        auto q_tile = [&](int m) {
+            o0 = cr_mfma(xq[m][0], S[m][0], o0);
+            o1 = cr_mfma(xq[m][1], S[m][1], o1);
+            o2 = cr_mfma(xq[m][2], S[m][2], o2);
+            o3 = cr_mfma(xq[m][3], S[m][3], o3);
+        };
+        constexpr int QF = NM > 2 ? (NM + 1) / 2 : 1; // tiles of Q S in front of the barrier: while the parts of K S are written
+        if constexpr (HAS_K) {
+            f32x4 k1 = zero, k2 = zero, k3 = zero;
+#pragma unroll
+            for (int m = 0; m < NM; ++m) {
+                ck = cr_mfma(x[m][0], S[m][0], ck);
+                k1 = cr_mfma(x[m][1], S[m][1], k1);
+                k2 = cr_mfma(x[m][2], S[m][2], k2);
+                k3 = cr_mfma(x[m][3], S[m][3], k3);
+            }
+            f32x4 pk = zero;
+            if constexpr (FORM == kCrGeneral) pk = triangle(odd_tag, share, mk, vv, zero);
+            __builtin_amdgcn_sched_barrier(0);
+            read_update();
+            q_tile(0);
+            __builtin_amdgcn_sched_barrier(0);
+            ck = (ck + k1) + (k2 + k3);
+            if constexpr (FORM == kCrGeneral) ck += pk;
+            if constexpr (RS > 1) part[c & 1][wave][lane] = ck;
+        } else {
+            read_update();
+            q_tile(0);
         }
-        d = cr_mfma(y2.x, vv[0], d);
-        d = cr_mfma(y2.y, vv[1], d);
-        __builtin_amdgcn_sched_barrier(0);            // (d's products run while the last of C comes out: 298 -> 286 us, gated)
-        c0 = (c0 + c1) + (c2 + c3);
-        if constexpr (RS > 1) part[c & 1][wave][lane] = c0;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = 1; m < QF; ++m) q_tile(m);
+        __builtin_amdgcn_sched_barrier(0);
         cr_group_barrier();                           // chunk c + 1 is in its slot; chunk c - 1's slot is free
-        f32x4 other;
-        if constexpr (RS > 1) other = part[c & 1][wave ^ 1][lane];
+        if constexpr (HAS_K && RS > 1) other = part[c & 1][wave ^ 1][lane];
         at = at == 2 ? 0 : at + 1;
         read_x(at);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = QF; m < NM; ++m) q_tile(m);
+        f32x4 o = zero;
+        if constexpr (HAS_V) o = triangle(odd_tag, share, mv, vv, zero);
+        __builtin_amdgcn_sched_barrier(0);
+        o += (o0 + o1) + (o2 + o3);
         // the state moves on: rows 4 g + e of tile m decay, then take the chunk's writes
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
@@ -665,57 +754,23 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             S[m][2] *= dpp_f32<0x152>(dec[m]);
             S[m][3] *= dpp_f32<0x153>(dec[m]);
         }
-        if constexpr (FORM != kCrGated) {
+        if constexpr (HAS_V) {
 #pragma unroll
-            for (int m = 0; m < NM; ++m) S[m] = cr_mfma(uk[m].x, vv[0], S[m]);
+            for (int e = 0; e < 4; ++e)
 #pragma unroll
-            for (int m = 0; m < NM; ++m) S[m] = cr_mfma(uk[m].y, vv[1], S[m]);
+                for (int m = 0; m < NM; ++m) S[m] = cr_mfma(up[m][e], vv[e], S[m]);
         }
-        if constexpr (RS > 1) c0 += other;
-        if constexpr (!ODD) {
-            if constexpr (FORM != kCrWrite) {
+        if constexpr (HAS_K) {
+            ck += other;
+            const f32x4 u = triangle(odd_tag, whole, mt, FORM == kCrGated ? vv - ck : ck, zero);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) d = cr_mfma(y[e], c0[e], d);
-            }
-        } else {
-            // A zero above the diagonal keeps a later token out only while that token's value is finite: token by token, each
-            // from operands that end with it; a row of Q counts for its own read-out alone.
-            f32x4 rows = d;
-#pragma unroll 1
-            for (int t = 0; t < kCrChunk; ++t) {
-                f32x4 u = {0.f, 0.f, 0.f, 0.f};
-                u = cr_mfma(y2.x, 2 * g <= t ? vv[0] : 0.f, u);
-                u = cr_mfma(y2.y, 2 * g + 1 <= t ? vv[1] : 0.f, u);
-                f32x4 o = u;
-                if constexpr (FORM != kCrWrite) {
+            for (int e = 0; e < 4; ++e)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int at = (4 * g + e) & 7;
-                        u = cr_mfma(y[e], g < 2 && at <= t ? c0[e] : 0.f, u);
-                        o = cr_mfma(y[e], (g < 2 ? at <= t : at == t) ? c0[e] : 0.f, o);
-                    }
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (((4 * g + e) & 7) == t) rows[e] = g < 2 ? u[e] : o[e];
-            }
-            d = rows;
+                for (int m = 0; m < NM; ++m) S[m] = cr_mfma(ux[m][e], u[e], S[m]);
+            o += triangle(odd_tag, share, mq, u, zero);
         }
-        if constexpr (FORM == kCrWrite) {
-            d += c0;
-        } else {
-            // tokens 0, 1 | 4, 5 of U sit in groups 0 | 1, tokens 2, 3 | 6, 7 move to groups 2 | 3
-            const float u0 = cr_spread(d[0], d[2]), u1 = cr_spread(d[1], d[3]);
 #pragma unroll
-            for (int m = 0; m < NM; ++m) S[m] = cr_mfma(ux[m].x, u0, S[m]);
-#pragma unroll
-            for (int m = 0; m < NM; ++m) S[m] = cr_mfma(ux[m].y, u1, S[m]);
-        }
-        // write: rows 0 - 7 of the products are the read-outs (8 - 15 repeat them), else rows 8 - 15
-        if (rp == 0 && (FORM == kCrWrite ? g < 2 : g >= 2)) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) os[c & 1][4 * (g & 1) + e][in_group] = d[e];
-        }
+        for (int e = 0; e < 4; ++e) os[c & 1][rp][4 * g + e][in_group] = o[e];
     };
     if (odd == 0) {
         for (int c = 0; c < chunks; ++c) chunk(std::false_type{}, c);
@@ -921,11 +976,11 @@ static bool recurrence_built(int D, int Dv) {
 struct CrWorkspace {
     int64_t records, chunks, columns, raw, odd;       // how many (per head); bytes of the parts
     CrWorkspace(int form, int64_t T, int H, int D, int Dv, int seqs, int dtype) {
-        const int rows = form == kCrWrite ? 8 : 16;
-        const int words = rows * D + (form == kCrGeneral ? 2 : 1) * 8 * D + D + (form == kCrWrite ? 0 : 256) + 8 * rows;
+        const int words = (form == kCrWrite ? 16 : 32) * D + (form == kCrGeneral ? 2 : 1) * 16 * D + D +
+                          (form == kCrWrite ? 256 : form == kCrGated ? 512 : 1024);
         records = cr_first_record(T, seqs) + 1;
         chunks = records * H * words * 4;
-        columns = records * H * 8 * Dv * (dtype == NV_DTYPE_BF16 ? 2 : 4);
+        columns = records * H * kCrChunk * Dv * (dtype == NV_DTYPE_BF16 ? 2 : 4);
         raw = T * H * Dv * 4;
         odd = records * H * 4;
     }
@@ -935,12 +990,12 @@ struct CrWorkspace {
 template <typename T, int FORM, int D>
 static void chunks_of_size(const ChunkRecurrenceArgs& a, int first_seq, hipStream_t s) {
     const int seqs = a.num_seqs - first_seq;
-    const dim3 prep((unsigned)a.records, (unsigned)((a.H + 3) / 4)), pairs((unsigned)(seqs * a.H));
+    const dim3 prep((unsigned)a.records, (unsigned)a.H), pairs((unsigned)(seqs * a.H));
     const uintptr_t piece = 2 * sizeof(T) - 1;        // two channels by one load
     const bool vec = a.sv % 2 == 0 && a.s0 % 2 == 0 && a.s1 % 2 == 0 && a.s2 % 2 == 0 && a.s3 % 2 == 0 &&
                      (((uintptr_t)a.v | (uintptr_t)a.x0 | (uintptr_t)a.x1 | (uintptr_t)a.x2 | (uintptr_t)a.x3) & piece) == 0;
-    if (vec) hipLaunchKernelGGL((recurrence_chunks_kernel<T, FORM, D, true>), prep, dim3(256), 0, s, a, first_seq);
-    else hipLaunchKernelGGL((recurrence_chunks_kernel<T, FORM, D, false>), prep, dim3(256), 0, s, a, first_seq);
+    if (vec) hipLaunchKernelGGL((recurrence_chunks_kernel<T, FORM, D, true>), prep, dim3(128), 0, s, a, first_seq);
+    else hipLaunchKernelGGL((recurrence_chunks_kernel<T, FORM, D, false>), prep, dim3(128), 0, s, a, first_seq);
     // Two waves for a state's 16 columns while that leaves every workgroup (one a CU, two tiles of columns) a CU of its own.  Whole
     // calls, one against two waves, sequences of 768 rows, 16 heads: gated 128 x 128, 128 tiles 136 -> 99 us, 512: 160 -> 123,
     // 640: 170 -> 205, 1024: 202 -> 235; gated 64 x 64, 512: 121 -> 108, 640: 137 -> 175; write 128 x 128, 512: 138 -> 104, 640: 144 -> 174.

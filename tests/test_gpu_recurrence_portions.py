@@ -318,3 +318,23 @@ def test_read_outs_keep_their_precision():
     torch.cuda.synchronize()
     off = [((x.double() - want).norm() / want.norm()).item() for x in (got, tokens)]
     assert off[0] <= 1.35 * off[1], off
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("form,D,Dv", [("gated", 128, 128), ("gated", 96, 48), ("gated", 32, 80), ("general", 128, 128), ("general", 96, 96),
+                                       ("write", 96, 144), ("write", 64, 16)])
+@pytest.mark.parametrize("rows", [[15, 16, 17, 31, 32, 33, 48], [24] * 40], ids=["edges", "many"])   # (many: one wave for a state's columns)
+def test_chunks_of_16(form, D, Dv, rows, dtype):
+    """Around the chunk of 16 tokens and its halves, carried and fresh states, both splits of a state over waves.  The bounds are those
+    of test_portions: the same sums, of up to 128 products and 16 tokens, in another order."""
+    before = [5 * (i % 3) for i in range(len(rows))]
+    a, r, x, state = _operands(form, rows, before, 4, D, Dv, dtype, 11)
+    nv.set_context(_context(rows, before, False))
+    want_state = state.clone()
+    want = _forward(form, r, x, want_state)
+    nv.set_context(_context(rows, before, True))
+    got = _forward(form, a, x, state)
+    nv.set_context(None)
+    tol = dict(rtol=5e-5, atol=5e-5) if dtype == torch.float32 else dict(rtol=1e-2, atol=2e-2)
+    torch.testing.assert_close(got.float(), want.float(), **tol)
+    torch.testing.assert_close(state, want_state, rtol=2e-5, atol=2e-6 * want_state.abs().max().item())
