@@ -22,7 +22,7 @@ struct ChunkRecurrenceArgs {
     void* out;                                 // [T, H * Dv]
     int64_t out_stride;
     float* chunks;                             // the chunks' operands: [H, records, ..]
-    void* columns;                             // their rows of V: [H, records, 8, Dv]
+    void* columns;                             // their rows of V: [H, records, 16, Dv]
     float* raw;                                // [H, T, Dv]: read-outs in front of their norm
     uint32_t* odd;                             // [H, records]: some value of the chunk is not finite
     int64_t records;
