@@ -997,8 +997,9 @@ static void chunks_of_size(const ChunkRecurrenceArgs& a, int first_seq, hipStrea
     if (vec) hipLaunchKernelGGL((recurrence_chunks_kernel<T, FORM, D, true>), prep, dim3(128), 0, s, a, first_seq);
     else hipLaunchKernelGGL((recurrence_chunks_kernel<T, FORM, D, false>), prep, dim3(128), 0, s, a, first_seq);
     // Two waves for a state's 16 columns while that leaves every workgroup (one a CU, two tiles of columns) a CU of its own.  Whole
-    // calls, one against two waves, sequences of 768 rows, 16 heads: gated 128 x 128, 128 tiles 136 -> 99 us, 512: 160 -> 123,
-    // 640: 170 -> 205, 1024: 202 -> 235; gated 64 x 64, 512: 121 -> 108, 640: 137 -> 175; write 128 x 128, 512: 138 -> 104, 640: 144 -> 174.
+    // calls, one against two waves, sequences of 768 rows, 16 heads: gated 128 x 128, 128 tiles 114 -> 78 us, 512: 147 -> 113,
+    // 640: 158 -> 175, 1024: 190 -> 208; gated 64 x 64, 512: 122 -> 106, 640: 135 -> 155; general, 512: 188 -> 141, 640: 201 -> 223;
+    // write 128 x 128, 512: 100 -> 73, 640: 110 -> 118.
     const int tiles = a.Dv / 16;
     if ((int64_t)pairs.x * ((tiles + 1) / 2) <= 256)
         hipLaunchKernelGGL((recurrence_states_kernel<T, FORM, D, 2>), dim3(pairs.x, (unsigned)((tiles + 1) / 2)), dim3(512), 0, s, a, first_seq);

@@ -17,8 +17,9 @@ _workspaces: dict[tuple[int, int], torch.Tensor] = {}
 _retired: list[torch.Tensor] = []   # outgrown workspaces stay alive: captured graphs may point at them
 
 
-# The helpers below run several times a call, and a call of one token is bound by them (paged attention of one sequence: 28 us of host
-# work before, 20 now; attention with modified scores 37 and 30, experts 32 and 27): the raw stream without a Stream object around it, messages only where they are raised.
+# The helpers below run several times a call, and a call of one token is bound by them: the raw stream without a Stream object around
+# it, messages only where they are raised.  Host time a call, before and after: paged attention of one sequence 28 and 20 us,
+# attention with modified scores 37 and 30, routed experts 32 and 27.
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)      # (not in builds of torch without a GPU)
 
 
