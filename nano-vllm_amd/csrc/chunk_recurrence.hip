@@ -511,6 +511,7 @@ __global__ __launch_bounds__(128, FORM == kCrGeneral ? 2 : 3) void recurrence_ch
 #pragma unroll
     for (int e = 0; e < 4; ++e) p[e] *= (FORM == kCrGated ? rows[e] * lds.beta[4 * g + e] : rows[e]) * kc;
     float y[L];                                       // column l16 of T
+    f32x4 mine = {0.f, 0.f, 0.f, 0.f};                // its rows 4 g + e (an index by g into y would put y into memory)
 #pragma unroll
     for (int t = 0; t < L; ++t) {
         float s0 = t == l16 ? bc : 0.f, s1 = 0.f;
@@ -520,12 +521,10 @@ __global__ __launch_bounds__(128, FORM == kCrGeneral ? 2 : 3) void recurrence_ch
             if (i & 1) s1 -= f * y[i]; else s0 -= f * y[i];
         }
         y[t] = s0 + s1;
+        mine[t & 3] = g == (t >> 2) ? y[t] : mine[t & 3];
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const float lo2 = g & 1 ? y[4 + e] : y[e], hi2 = g & 1 ? y[12 + e] : y[8 + e];
-        mat[(4 * g + e) * 16 + l16] = (g & 2 ? hi2 : lo2) * (FORM == kCrGeneral ? -rows[e] : 1.f);
-    }
+    for (int e = 0; e < 4; ++e) mat[(4 * g + e) * 16 + l16] = mine[e] * (FORM == kCrGeneral ? -rows[e] : 1.f);
 }
 
 // ------------------------------------------------------------------------------------------------ second launch
@@ -673,16 +672,23 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         return rows;
     };
     cr_group_barrier();
-    read_x(0);
+    if (!HAS_K || odd == 0) read_x(0);
     int at = 0;
-    auto chunk = [&](auto odd_tag, int c) {           // chunk c from slot `at`
+    // Chunk c from slot `at`.  LATE: operands when they are needed, since the triangles' loops take registers of their own (read
+    // ahead there too, the kernels of a whole state a wave spilled and all their calls paid for it, 2 to 4 %).
+    auto chunk = [&](auto odd_tag, int c) {
+        constexpr bool LATE = HAS_K && decltype(odd_tag)::value;
         constexpr std::false_type share{};
         constexpr std::true_type whole{};
         const float* rc = slots[at];
         float dec[NM];                                // lane e of group g: the decay of row 4 g + e of the tile
         f32x4 xq[NM], up[NM], ux[NM], vv, mt, mq, mv, mk;
+        if constexpr (LATE) read_x(at);
+        auto read_xq = [&] {
 #pragma unroll
-        for (int m = 0; m < NM; ++m) xq[m] = HAS_K ? *(const f32x4*)(rc + 16 * D + 256 * m + at_x) : x[m];
+            for (int m = 0; m < NM; ++m) xq[m] = HAS_K ? *(const f32x4*)(rc + 16 * D + 256 * m + at_x) : x[m];
+        };
+        if constexpr (!LATE) read_xq();
 #pragma unroll
         for (int e = 0; e < 4; ++e) vv[e] = vs[at][4 * g + e][in_group];
         if constexpr (FORM == kCrGeneral) mk = *(const f32x4*)(rc + 768 + at_m);
@@ -721,7 +727,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             f32x4 pk = zero;
             if constexpr (FORM == kCrGeneral) pk = triangle(odd_tag, share, mk, vv, zero);
             __builtin_amdgcn_sched_barrier(0);
-            read_update();
+            if constexpr (LATE) read_xq(); else read_update();
             q_tile(0);
             __builtin_amdgcn_sched_barrier(0);
             ck = (ck + k1) + (k2 + k3);
@@ -733,15 +739,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int m = 1; m < QF; ++m) q_tile(m);
+        for (int m = 1; m < (LATE ? NM : QF); ++m) q_tile(m);
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (LATE) read_update();
         cr_group_barrier();                           // chunk c + 1 is in its slot; chunk c - 1's slot is free
         if constexpr (HAS_K && RS > 1) other = part[c & 1][wave ^ 1][lane];
         at = at == 2 ? 0 : at + 1;
-        read_x(at);
+        if constexpr (!LATE) read_x(at);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int m = QF; m < NM; ++m) q_tile(m);
+        for (int m = LATE ? NM : QF; m < NM; ++m) q_tile(m);
         f32x4 o = zero;
         if constexpr (HAS_V) o = triangle(odd_tag, share, mv, vv, zero);
         __builtin_amdgcn_sched_barrier(0);

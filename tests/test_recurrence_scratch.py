@@ -1,4 +1,9 @@
 """Scratch memory of the recurrent layers: asked for only by steps that use it, and set aside when the caches are sized."""
+import re
+import shutil
+import struct
+import subprocess
+
 import pytest
 import torch
 import torch.nn as nn
@@ -45,3 +50,27 @@ def test_sizes_without_a_launch_in_chunks_need_none():
 def test_single_tokens_allocate_nothing(max_rows, lead, portions):
     """All sequences of one row each, known as such by any of the step's three hints."""
     assert ops._portions(None, 0, None, 3, H, D, D, 3, max_rows, lead, portions)[2] is None
+
+
+READELF = shutil.which("llvm-readelf", path="/opt/rocm/llvm/bin")
+
+
+@pytest.mark.skipif(READELF is None, reason="no llvm-readelf")
+def test_kernels_keep_their_registers(tmp_path):
+    """No kernel of the recurrences in chunks has private memory: none spills, and none indexes an array by a lane's number."""
+    data = open(_lib.MIXERS_LIB_PATH, "rb").read()
+    magic, at, sizes = b"__CLANG_OFFLOAD_BUNDLE__", 0, {}
+    while (at := data.find(magic, at)) >= 0:           # one bundle per source file: code objects by target
+        (entries,), p = struct.unpack_from("<Q", data, at + 24), at + 32
+        for _ in range(entries):
+            off, size, chars = struct.unpack_from("<QQQ", data, p)
+            target, p = data[p + 24:p + 24 + chars], p + 24 + chars
+            code = data[at + off:at + off + size]
+            if target.endswith(b"gfx950") and b"recurrence_states_kernel" in code:
+                (tmp_path / "code").write_bytes(code)
+                notes = subprocess.run([READELF, "--notes", tmp_path / "code"], capture_output=True, text=True, check=True).stdout
+                for name, n in re.findall(r"\.name: +(\S*recurrence\S*)\n.*?\.private_segment_fixed_size: (\d+)", notes, re.S):
+                    sizes[name] = int(n)
+        at += 24
+    assert len(sizes) > 100
+    assert not {name: n for name, n in sizes.items() if n}
