@@ -50,11 +50,14 @@
 // as six bf16 products of three parts each, split by the movers (198 us for the second launch: the LDS traffic of the parts; 144 without
 // them), the same for the updates alone (176), four waves a state on eight product waves (180).
 //
-// Against 64 bits (float32 rows, 1 to 300 tokens a sequence): states 0.9 to 1.5 times the token-by-token launch's error, all below
-// 3.3e-7; read-outs 1.0 to 1.24 times (1.2e-7 to 2.4e-7), because a chunk's sums are taken in another order: C and the pair products
-// are four sums each, since one sum over all key channels has its roundings one after the other (1.6 times the error).  Chunks of 16
-// against chunks of 8, 30 to 900 tokens: read-outs 0.99 to 1.02 times the error, states 0.99 to 1.00 (general 1.04 to 1.10).  Of bf16
-// read-outs, which are 1.7e-3 off by their own rounding, neither shows.
+// Against 64 bits (float32 rows, 64 and 128 channels, 8 to 1000 tokens a sequence, fresh and carried states), relative to the
+// token-by-token launch: states gated 0.88 to 0.96 times its error, general 1.03 to 1.13, write 0.99 to 1.00; read-outs 0.91 to 1.06,
+// 0.98 to 1.08 and 1.01 to 1.09 (a read-out near zero aside, which its norm blows up in either).  Three things keep them there.
+// Decays are multiplied in 64 bits and each product is rounded once, where 15 roundings in a row are 15 factors of one channel's error.
+// Sums over all key channels have their roundings one after the other, so C is four sums and a pair product eight (four: read-outs 2 to
+// 5 % further off).  The removals of the general form are summed by themselves: on top of the state each of 16 terms is rounded at
+// the state's size (states 1.35 to 1.67 times the token-by-token launch's error).  Of bf16 read-outs, which are 1.7e-3 off by their own
+// rounding, none of it shows.
 //
 // The read-outs go to a scratch of fp32 rows, because a row's norm spans the workgroups of its value columns; a last launch
 // norms, weights and gates them.  Single tokens run in a launch of their own that streams every state once.
@@ -164,8 +167,7 @@ __device__ __forceinline__ f32x4 cr_mfma(float a, float b, f32x4 c) { return __b
 __device__ __forceinline__ float cr_lane(float x, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
 }
-// LDS writes of this wave / of the workgroup's waves are done; loads from memory stay in flight.
-__device__ __forceinline__ void cr_wave_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+// LDS writes of the workgroup's waves are done; loads from memory stay in flight.
 __device__ __forceinline__ void cr_group_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
@@ -213,8 +215,8 @@ __device__ __host__ __forceinline__ int64_t cr_first_record(int64_t first_row, i
 template <int D>
 struct CrPrepLds {
     static constexpr int kRow = D + 4;                            // rows of D channels start on different banks
-    float k[16 * kRow], q[16 * kRow], right[16 * kRow];           // left sides, then [K; Q]; right sides
-    float total[2][D], kn[16], qn[16], beta[16];
+    float k[16 * kRow], q[16 * kRow], right[16 * kRow];           // left sides, then [K; Q]; right sides, then the halves' decays
+    float kn[16], qn[16], beta[16];
     uint32_t odd[2], far[2];
 };
 
@@ -363,7 +365,6 @@ __global__ __launch_bounds__(128, FORM == kCrGeneral ? 2 : 3) void recurrence_ch
             lds.far[half] = any_far;
             lds.odd[half] = any_odd;
         }
-        if (in_row) *(float2*)(lds.total[half] + d) = make_float2(pre[0][N - 1], pre[1][N - 1]);
     }
     auto put = [&](float* rows, auto of) {            // this wave's 8 rows of this lane's two channels
         if (in_row) {
@@ -378,18 +379,16 @@ __global__ __launch_bounds__(128, FORM == kCrGeneral ? 2 : 3) void recurrence_ch
     f32x4 pk = {0.f, 0.f, 0.f, 0.f}, pa = pk;
     {
         auto product = [&] {                          // of the operands in LDS
-            f32x4 p0 = {0.f, 0.f, 0.f, 0.f}, p1 = p0, p2 = p0, p3 = p0;
+            f32x4 p[8] = {};
             const float* lf = (half ? lds.q : lds.k) + l16 * ROW + 4 * g;
             const float* rt = lds.right + l16 * ROW + 4 * g;
 #pragma unroll
             for (int m = 0; m < NM; ++m) {
                 const f32x4 x = *(const f32x4*)(lf + 16 * m), y = *(const f32x4*)(rt + 16 * m);
-                p0 = cr_mfma(x[0], y[0], p0);
-                p1 = cr_mfma(x[1], y[1], p1);
-                p2 = cr_mfma(x[2], y[2], p2);
-                p3 = cr_mfma(x[3], y[3], p3);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) p[4 * (m & 1) + e] = cr_mfma(x[e], y[e], p[4 * (m & 1) + e]);
             }
-            return (p0 + p1) + (p2 + p3);
+            return ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
         };
         // Relative to the middle: left sides G_t / G_8, right sides G_8 / G_t.  Otherwise part 8, 4, 2, 1 (0: s = t) one after the
         // other: left sides from the start of the part through the token, right sides behind the token to the end of its part.
@@ -449,15 +448,41 @@ __global__ __launch_bounds__(128, FORM == kCrGeneral ? 2 : 3) void recurrence_ch
             }
         }
     }
-    // ---- [K; Q] (through LDS), K^, X^ and the chunk's decay; k and q are unit vectors from here on (gated)
+    // ---- [K; Q] (through LDS), K^, X^ and the chunk's decay; k and q are unit vectors from here on (gated).  Decays from the chunk's
+    // start through a token (G) and behind it to the chunk's end (F).
     auto ku = [&](int t, int i) { return FORM == kCrGated ? kf(t, i) * cr_lane(kn, t) : kf(t, i); };
     auto qu = [&](int t, int i) { return FORM == kCrGated ? qf(t, i) * cr_lane(qn, t) : qf(t, i); };
-    const float2 front = half ? *(const float2*)(lds.total[0] + d) : make_float2(1.f, 1.f);           // decays of the other half, in front
-    const float2 behind = half ? make_float2(1.f, 1.f) : *(const float2*)(lds.total[1] + d);          // and behind
-    const float fr[2] = {front.x, front.y}, be[2] = {behind.x, behind.y};
-    if constexpr (FORM == kCrGated) put(lds.k, [&](int t, int i) { return ku(t, i) * (fr[i] * pre[i][t]); });
-    if constexpr (FORM == kCrGeneral) put(lds.k, [&](int t, int i) { return ku(t, i) * (t ? fr[i] * pre[i][t ? t - 1 : 0] : fr[i]); });
-    put(lds.q, [&](int t, int i) { return qu(t, i) * (fr[i] * pre[i][t]); });
+    float G[2][N], F[2][N], lead[2], all[2];
+    {
+        double2* const totals = (double2*)lds.right;
+        double total[2] = {1.0, 1.0};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+#pragma unroll
+            for (int t = 0; t < N; ++t) total[i] *= (double)w[t][i];
+        }
+        if (in_row) totals[half * (D / 2) + d / 2] = make_double2(total[0], total[1]);
+        __syncthreads();
+        const double2 other = totals[(half ^ 1) * (D / 2) + d / 2];
+        const double ot[2] = {other.x, other.y};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            double f = half ? ot[i] : 1.0;
+            lead[i] = (float)f;
+#pragma unroll
+            for (int t = 0; t < N; ++t) G[i][t] = (float)(f *= (double)w[t][i]);
+            f = half ? 1.0 : ot[i];
+#pragma unroll
+            for (int t = N - 1; t >= 0; --t) {
+                F[i][t] = (float)f;
+                f *= (double)w[t][i];
+            }
+            all[i] = (float)f;
+        }
+    }
+    if constexpr (FORM == kCrGated) put(lds.k, [&](int t, int i) { return ku(t, i) * G[i][t]; });
+    if constexpr (FORM == kCrGeneral) put(lds.k, [&](int t, int i) { return ku(t, i) * (t ? G[i][t ? t - 1 : 0] : lead[i]); });
+    put(lds.q, [&](int t, int i) { return qu(t, i) * G[i][t]; });
     auto put_update = [&](int which, auto of) {       // lane (g, channel) of a tile: tokens 4 g .. 4 g + 3
         if (in_row) {
 #pragma unroll
@@ -467,7 +492,7 @@ __global__ __launch_bounds__(128, FORM == kCrGeneral ? 2 : 3) void recurrence_ch
                 for (int i = 0; i < 2; ++i) {
                     f32x4 r;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) r[e] = of(4 * gg + e, i) * (suf[i][4 * gg + e] * be[i]);
+                    for (int e = 0; e < 4; ++e) r[e] = of(4 * gg + e, i) * F[i][4 * gg + e];
                     *(f32x4*)(to + 4 * i) = r;
                 }
             }
@@ -475,7 +500,7 @@ __global__ __launch_bounds__(128, FORM == kCrGeneral ? 2 : 3) void recurrence_ch
     };
     if constexpr (FORM == kCrGated) put_update(0, ku); else put_update(0, kf);
     if constexpr (FORM == kCrGeneral) put_update(1, af);
-    if (half == 0 && in_row) *(float2*)(out + Rec::decay + d) = make_float2(pre[0][N - 1] * be[0], pre[1][N - 1] * be[1]);
+    if (half == 0 && in_row) *(float2*)(out + Rec::decay + d) = make_float2(all[0], all[1]);
     __syncthreads();
     if (HAS_K || half) {
         const float* rows = (half ? lds.q : lds.k) + l16 * ROW + 4 * g;
@@ -648,15 +673,22 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // Rows of a lower triangular matrix times 16 rows of values, the wave's share of the 16; ODD: a zero above the diagonal keeps a later
     // token out only while that token's value is finite, so token by token, each from rows that end with it.
     constexpr int E0 = 4 / RS;
-    auto triangle = [&](auto odd_tag, auto all_tag, f32x4 mt, f32x4 x, f32x4 onto) {
-        constexpr bool ODD = decltype(odd_tag)::value, ALL = decltype(all_tag)::value || RS == 1;
+    typedef CrRow<E0> Share;
+    const int at_share = at_m + rp * E0;
+    auto share = [&](f32x4 x) {
+        Share r;
+#pragma unroll
+        for (int e = 0; e < E0; ++e) r[e] = rp ? x[(E0 + e) & 3] : x[e];
+        return r;
+    };
+    auto triangle = [&](auto odd_tag, auto mt, auto x, f32x4 onto) {
+        constexpr bool ODD = decltype(odd_tag)::value;
+        constexpr int E = sizeof(x) / sizeof(float);  // 4: all of the 16 rows
         auto sum = [&](int t, f32x4 c0) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if (!ALL && e >= E0) continue;
-                const float me = ALL ? mt[e] : rp ? mt[(E0 + e) & 3] : mt[e], xe = ALL ? x[e] : rp ? x[(E0 + e) & 3] : x[e];
-                const int row = 4 * g + (ALL ? e : rp * E0 + e);
-                c0 = cr_mfma(me, ODD ? (row <= t ? xe : 0.f) : xe, c0);       // (a sum that goes on costs a product no wait)
+            for (int e = 0; e < E; ++e) {
+                const int row = 4 * g + (E == 4 ? e : rp * E0 + e);
+                c0 = cr_mfma(mt[e], ODD ? (row <= t ? x[e] : 0.f) : x[e], c0);        // (a sum that goes on costs a product no wait)
             }
             return c0;
         };
@@ -671,6 +703,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
         return rows;
     };
+    // General: a chunk's removals, summed by themselves and added where the next products hide it (which costs 5 us of 227, one prompt of
+    // 2048 tokens).
+    f32x4 moved[FORM == kCrGeneral ? NM : 1] = {};
     cr_group_barrier();
     if (!HAS_K || odd == 0) read_x(0);
     int at = 0;
@@ -678,11 +713,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // ahead there too, the kernels of a whole state a wave spilled and all their calls paid for it, 2 to 4 %).
     auto chunk = [&](auto odd_tag, int c) {
         constexpr bool LATE = HAS_K && decltype(odd_tag)::value;
-        constexpr std::false_type share{};
-        constexpr std::true_type whole{};
         const float* rc = slots[at];
         float dec[NM];                                // lane e of group g: the decay of row 4 g + e of the tile
-        f32x4 xq[NM], up[NM], ux[NM], vv, mt, mq, mv, mk;
+        f32x4 xq[NM], up[NM], ux[NM], vv, mt;
+        Share mq, mv, mk;
         if constexpr (LATE) read_x(at);
         auto read_xq = [&] {
 #pragma unroll
@@ -691,11 +725,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if constexpr (!LATE) read_xq();
 #pragma unroll
         for (int e = 0; e < 4; ++e) vv[e] = vs[at][4 * g + e][in_group];
-        if constexpr (FORM == kCrGeneral) mk = *(const f32x4*)(rc + 768 + at_m);
-        if constexpr (HAS_V) mv = *(const f32x4*)(rc + MV + at_m);
+        if constexpr (FORM == kCrGeneral) mk = *(const Share*)(rc + 768 + at_share);
+        if constexpr (HAS_V) mv = *(const Share*)(rc + MV + at_share);
         if constexpr (HAS_K) {
             mt = *(const f32x4*)(rc + at_m);
-            mq = *(const f32x4*)(rc + 256 + at_m);
+            mq = *(const Share*)(rc + 256 + at_share);
         }
         __builtin_amdgcn_sched_barrier(0);            // the reads are on their way before the products
         auto read_update = [&] {
@@ -719,13 +753,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             f32x4 k1 = zero, k2 = zero, k3 = zero;
 #pragma unroll
             for (int m = 0; m < NM; ++m) {
+                if constexpr (FORM == kCrGeneral) S[m] += moved[m];
                 ck = cr_mfma(x[m][0], S[m][0], ck);
                 k1 = cr_mfma(x[m][1], S[m][1], k1);
                 k2 = cr_mfma(x[m][2], S[m][2], k2);
                 k3 = cr_mfma(x[m][3], S[m][3], k3);
             }
             f32x4 pk = zero;
-            if constexpr (FORM == kCrGeneral) pk = triangle(odd_tag, share, mk, vv, zero);
+            if constexpr (FORM == kCrGeneral) pk = triangle(odd_tag, mk, share(vv), zero);
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (LATE) read_xq(); else read_update();
             q_tile(0);
@@ -750,7 +785,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int m = LATE ? NM : QF; m < NM; ++m) q_tile(m);
         f32x4 o = zero;
-        if constexpr (HAS_V) o = triangle(odd_tag, share, mv, vv, zero);
+        if constexpr (HAS_V) o = triangle(odd_tag, mv, share(vv), zero);
         __builtin_amdgcn_sched_barrier(0);
         o += (o0 + o1) + (o2 + o3);
         // the state moves on: rows 4 g + e of tile m decay, then take the chunk's writes
@@ -767,14 +802,24 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
                 for (int m = 0; m < NM; ++m) S[m] = cr_mfma(up[m][e], vv[e], S[m]);
         }
+        if constexpr (FORM == kCrGeneral) __builtin_amdgcn_sched_barrier(0);      // (they run while the other wave's part comes)
         if constexpr (HAS_K) {
             ck += other;
-            const f32x4 u = triangle(odd_tag, whole, mt, FORM == kCrGated ? vv - ck : ck, zero);
+            const f32x4 u = triangle(odd_tag, mt, FORM == kCrGated ? vv - ck : ck, zero);
+            if constexpr (FORM == kCrGated) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
+                for (int e = 0; e < 4; ++e)
 #pragma unroll
-                for (int m = 0; m < NM; ++m) S[m] = cr_mfma(ux[m][e], u[e], S[m]);
-            o += triangle(odd_tag, share, mq, u, zero);
+                    for (int m = 0; m < NM; ++m) S[m] = cr_mfma(ux[m][e], u[e], S[m]);
+            } else {
+#pragma unroll
+                for (int m = 0; m < NM; ++m) moved[m] = cr_mfma(ux[m][0], u[0], zero);
+#pragma unroll
+                for (int e = 1; e < 4; ++e)
+#pragma unroll
+                    for (int m = 0; m < NM; ++m) moved[m] = cr_mfma(ux[m][e], u[e], moved[m]);
+            }
+            o += triangle(odd_tag, mq, share(u), zero);
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) os[c & 1][rp][4 * g + e][in_group] = o[e];
@@ -788,6 +833,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (!live) return;
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
+        if constexpr (FORM == kCrGeneral) S[m] += moved[m];
 #pragma unroll
         for (int e = 0; e < 4; ++e) slot[(int64_t)(16 * m + e) * Dv] = S[m][e];
     }
