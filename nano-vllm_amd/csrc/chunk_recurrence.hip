@@ -26,9 +26,11 @@
 //
 // G_t / G_s does not factor through one reference without overflow when a channel decays fast.  Both sides are taken relative to
 // the middle of the chunk, eight factors on either side, where no channel of the chunk has eight that multiply to less than 2^-80 (a
-// right side then keeps its 24 bits down to 2^-46 of the raw key).  Other chunks take the pairs in five sets by where s and t part:
-// in halves, quarters, eighths or neighbours of the chunk, each relative to the boundary between the two, where every factor is a decay
-// and nothing is divided, and s = t.  A chunk and head decide by themselves.
+// right side then keeps its 24 bits down to 2^-46 of the raw key).  Other chunks take the pairs in sets by where s and t part: in
+// halves, quarters, eighths or neighbours of the chunk, each relative to the boundary between the two, where every factor is a decay
+// and nothing is divided, and s = t; two sets, pairs across the halves and within a half relative to the half's middle, where no four
+// factors multiply to less than 2^-80.  A chunk and head decide by themselves.  Gated, 16 prompts of 300 .. 500 tokens, 16 heads
+// 128 x 128, a channel of every head at exp(-8) a token: 222 us with one set for all, 228 with two, 258 with five.
 //
 // Two launches: the first makes every chunk's operands (two waves per chunk and head, all chunks at once), the second walks the
 // chunks of a (sequence, head, 16 value columns) with the state in MFMA accumulators (128 channels: 32 registers) and reads the
@@ -359,10 +361,13 @@ __global__ __launch_bounds__(128, FORM == kCrGeneral ? 2 : 3) void recurrence_ch
         }
     }
     {
-        const bool near = pre[0][N - 1] >= kCrNear && pre[1][N - 1] >= kCrNear;          // (false with a decay that is not a number)
-        const bool any_far = !__all(near), any_odd = __any((odd[0] + odd[1]) + (odd[2] + odd[3]) != 0.f);
+        // (false with a decay that is not a number)
+        const bool near = __all(pre[0][N - 1] >= kCrNear && pre[1][N - 1] >= kCrNear);
+        const bool near4 = __all(pre[0][N / 2 - 1] >= kCrNear && pre[1][N / 2 - 1] >= kCrNear &&
+                                 suf[0][N / 2 - 1] >= kCrNear && suf[1][N / 2 - 1] >= kCrNear);
+        const bool any_odd = __any((odd[0] + odd[1]) + (odd[2] + odd[3]) != 0.f);
         if (lane == 0) {
-            lds.far[half] = any_far;
+            lds.far[half] = near ? 0 : near4 ? 1 : 2;
             lds.odd[half] = any_odd;
         }
     }
@@ -374,7 +379,7 @@ __global__ __launch_bounds__(128, FORM == kCrGeneral ? 2 : 3) void recurrence_ch
     };
     __syncthreads();
     if (half == 0 && lane == 0) a.odd[h * a.records + rec] = lds.odd[0] | lds.odd[1];
-    const bool near = (lds.far[0] | lds.far[1]) == 0;
+    const uint32_t far = __builtin_amdgcn_readfirstlane(max(lds.far[0], lds.far[1]));     // 0, 1, 2: one set of pairs, two, five
     // ---- pair products: entry (row 4 g + e, column l16), rows k (first wave) or q (second), columns k or a k
     f32x4 pk = {0.f, 0.f, 0.f, 0.f}, pa = pk;
     {
@@ -391,19 +396,20 @@ __global__ __launch_bounds__(128, FORM == kCrGeneral ? 2 : 3) void recurrence_ch
             return ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
         };
         // Relative to the middle: left sides G_t / G_8, right sides G_8 / G_t.  Otherwise part 8, 4, 2, 1 (0: s = t) one after the
-        // other: left sides from the start of the part through the token, right sides behind the token to the end of its part.
+        // other: left sides from the start of the part through the token, right sides behind the token to the end of its part; two
+        // sets: part 4 relative to the half's middle.
 #pragma unroll 1
-        for (int part = 8; part >= 0; part = near ? -1 : part == 1 ? 0 : part == 0 ? -1 : part / 2) {
+        for (int part = 8; part >= 0; part = far == 0 || part == 0 || (far == 1 && part == 4) ? -1 : part / 2) {
             float lv[2][N], rv[2][N], first[2] = {1.f, 1.f};      // (first: left side of the first token's key, general)
             if (part == 8) {
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
 #pragma unroll
                     for (int t = 0; t < N; ++t) {
-                        lv[i][t] = near && half == 0 ? __builtin_amdgcn_rcpf(suf[i][t]) : pre[i][t];
-                        rv[i][t] = near && half == 1 ? __builtin_amdgcn_rcpf(pre[i][t]) : suf[i][t];
+                        lv[i][t] = far == 0 && half == 0 ? __builtin_amdgcn_rcpf(suf[i][t]) : pre[i][t];
+                        rv[i][t] = far == 0 && half == 1 ? __builtin_amdgcn_rcpf(pre[i][t]) : suf[i][t];
                     }
-                    if (near && half == 0) first[i] = __builtin_amdgcn_rcpf(pre[i][N - 1]);
+                    if (far == 0 && half == 0) first[i] = __builtin_amdgcn_rcpf(pre[i][N - 1]);
                 }
             } else {
 #pragma unroll
@@ -421,6 +427,13 @@ __global__ __launch_bounds__(128, FORM == kCrGeneral ? 2 : 3) void recurrence_ch
                         rv[i][t] = part ? f : 1.f;
                         f *= w[t][i];
                     }
+                    if (far == 1) {
+                        first[i] = __builtin_amdgcn_rcpf(lv[i][N / 2 - 1]);
+#pragma unroll
+                        for (int t = 0; t < N / 2; ++t) lv[i][t] = __builtin_amdgcn_rcpf(rv[i][t]);
+#pragma unroll
+                        for (int t = N / 2; t < N; ++t) rv[i][t] = __builtin_amdgcn_rcpf(lv[i][t]);
+                    }
                 }
             }
             if constexpr (HAS_K)
@@ -432,7 +445,8 @@ __global__ __launch_bounds__(128, FORM == kCrGeneral ? 2 : 3) void recurrence_ch
             put(lds.right, [&](int t, int i) { return kf(t, i) * rv[i][t]; });
             // pairs whose tokens part at this part (one compare and a select: branches here have come out of the compiler without
             // their assignments)
-            const uint32_t from = near ? 0 : part, many = near ? 16 : part ? part : 1;
+            const bool middle = far == 0 || (far == 1 && part == 4);
+            const uint32_t from = middle ? 0 : part, many = middle ? 2 * part : part ? part : 1;
             auto take = [&](f32x4& to, f32x4 of) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) to[e] = (uint32_t)((4 * g + e) ^ l16) - from < many ? of[e] : to[e];

@@ -414,3 +414,30 @@ def test_long_portions_keep_their_precision(monkeypatch, form, B, rows):
     nv.set_context(None)
     ratio = [c / t for c, t in zip(*off)]
     assert all(r <= bound for r, bound in zip(ratio, OFF[form])), (ratio, off)
+
+
+@pytest.mark.parametrize("rate", [6.5, 7.5, 13.0, 14.5])
+@pytest.mark.parametrize("form", ["gated", "general", "write"])
+def test_fast_decays(form, rate):
+    """Channels that decay by about exp(-rate) a token beside slow ones, on both sides of where eight (6.9) and four (13.9) factors
+    multiply to 2^-80 and the chunk's pairs are taken in more sets."""
+    H, D, rows, before = 4, 128, [33, 40], [0, 3]
+    a, r, x, state = _operands(form, rows, before, H, D, D, torch.float32, 17)
+    fast = (torch.arange(H * D, device=DEV) % 5 == 0).float() * rate
+    for m in (a, r):
+        if form == "gated":
+            m.A_log.data.zero_()
+            m.dt_bias.data.copy_(torch.expm1(fast + 0.02).log())
+        elif form == "general":
+            m.decay_rate = rate
+            m.w_bias.data.copy_(torch.where(fast > 0, 20.0, -8.0))
+        else:
+            m.lower.data.zero_()
+            m.f_bias.data.copy_(3.0 - fast)
+    x["k" if form == "write" else "w"].mul_(0.02)
+    got_state, want_state = state.clone(), state.clone()
+    nv.set_context(_context(rows, before, True))
+    want, got = _forward(form, r, x, want_state), _forward(form, a, x, got_state)
+    nv.set_context(None)
+    torch.testing.assert_close(got, want, rtol=5e-5, atol=5e-5)          # (the bounds of test_portions)
+    torch.testing.assert_close(got_state, want_state, rtol=2e-5, atol=2e-6 * want_state.abs().max().item())
