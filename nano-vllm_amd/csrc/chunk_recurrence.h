@@ -1,5 +1,6 @@
 // Launchers of the recurrences with a decay per head and key channel, [D, Dv] states in fp32 per sequence and head:
-// portions in chunks on the matrix cores, single tokens as one pass over the state (chunk_recurrence.hip).
+// portions in chunks of 16 or 8 tokens on the matrix cores, single tokens as one pass over the state (chunk_recurrence.hip,
+// chunk_recurrence_short.hip).
 #pragma once
 #include "nv_common.h"
 
@@ -22,7 +23,7 @@ struct ChunkRecurrenceArgs {
     void* out;                                 // [T, H * Dv]
     int64_t out_stride;
     float* chunks;                             // the chunks' operands: [H, records, ..]
-    void* columns;                             // their rows of V: [H, records, 16, Dv]
+    void* columns;                             // their rows of V: [H, records, tokens of a chunk, Dv]
     float* raw;                                // [H, T, Dv]: read-outs in front of their norm
     uint32_t* odd;                             // [H, records]: some value of the chunk is not finite
     int64_t records;
@@ -32,10 +33,11 @@ struct ChunkRecurrenceArgs {
     float eps, p0, p1;                         // gated: -, key_eps; general: decay_rate, key_eps
 };
 
-// Sequences first_seq .. with at least two rows (the first_seq in front have one row each, singles_behind says whether others
-// may) / sequences with exactly one row (the others are passed over).
-int launch_chunk_recurrence(int form, const ChunkRecurrenceArgs& a, int first_seq, bool singles_behind, int dtype, hipStream_t s);
-int launch_single_recurrence(int form, const ChunkRecurrenceArgs& a, int dtype, hipStream_t s);
+// Chunks of 8 tokens (chunk_recurrence_short.hip): records of `rows` rows in `seqs` sequences, words of a record, and both launches
+// for the sequences first_seq .. with at least two rows (vec: two channels by one load; waves: for a state's 16 columns).
+int64_t short_recurrence_records(int64_t rows, int seqs);
+int short_recurrence_words(int form, int D);
+void launch_short_recurrence(int form, const ChunkRecurrenceArgs& a, int first_seq, bool vec, int waves, int dtype, hipStream_t s);
 
 // The launches of a step by what is known of its portions; false, with *rc NV_OK and nothing launched, when the sizes, the rows, a
 // missing workspace or an unknown number of rows (T = 0) leave a step that may hold longer portions to the token-by-token launch.

@@ -8,7 +8,7 @@
 //   write    (x0 = q, x1 = f_raw)   w = c1 + (1 - c1) sigmoid(x1 + c0);  k = 1 - w;  S <- diag(w) S + k v^T;  o = S^T silu(q)
 //
 // A token-by-token loop is bound by its serial chain (one pass over the state a token and the LDS reads of the token's vectors
-// by every lane), so portions run in CHUNKS of 16 tokens.  With G_t the product of the decays from the chunk's start through
+// by every lane), so portions run in CHUNKS, of 16 tokens here.  With G_t the product of the decays from the chunk's start through
 // token t, and S the state in front of the chunk, each form is
 //
 //   C = K S, Q S         what the tokens' k and q (r) find in S: K_t = k_t G_t (general: k_t G_(t-1)), Q_t = q_t G_t, 16 rows each
@@ -40,17 +40,16 @@
 // MFMA e of a tile contracts the four rows {4 g + e}, and the other operand is read in that order (16 bytes a lane); U, 16 rows, fills
 // all four groups.  The chunk takes 104 (gated) / 144 (general) / 68 (write) MFMAs of 32 cycles per 16 columns of 128 channels.
 //
-// Why 16 tokens: the products per token are those of chunks of 8, but a chunk's chain of exchange, triangle and update is paid half as
-// often, and Q S, which no other product waits for, is multiplied while the parts of K S are exchanged.  Whole calls, chunks of 8 against
-// 16, 16 heads 128 x 128, bf16 rows: gated, 4 prompts of 1501 .. 2048 tokens 285 -> 254 us (second launch 204 -> 166); general, 3 prompts
-// of 700 .. 2000: 285 -> 261; write, 8 portions of 509 over carried states: 115 -> 94, one prompt of 2048: 197 -> 118.  Where every SIMD
-// has a whole state's columns (general, 16 prompts of 300 .. 500) it is the products that count: 283 and 290; the shortest portions pay
-// for rows that are not there (general, 8 of 17: 28 and 33).  Token by token: gated 3123, general 3645, write 431; gated, 256 single
+// Why 16 tokens: the products per token are those of chunks of 8 (chunk_recurrence_short.hip, which short portions and full grids still
+// take: `cr_chunk_tokens`), but a chunk's chain of exchange, triangle and update is paid half as often, and Q S, which no other product
+// waits for, is multiplied while the parts of K S are exchanged.  Whole calls, chunks of 8 against 16, 16 heads 128 x 128, bf16 rows:
+// gated, 4 prompts of 1501 .. 2048 tokens 285 -> 248 us; general, 3 prompts of 700 .. 2000: 286 -> 266; write, 8 portions of 509 over
+// carried states: 114 -> 96, one prompt of 2048: 197 -> 119.  Token by token: gated 3123, general 3645, write 431; gated, 256 single
 // tokens: 393 -> 113 (4.8 TB/s of states, what a large copy reaches).
-// Of the 254 us the first launch is 83 (instructions: some 1700 a wave, half of them decays), the second 166, 129 chunks in a row at
-// 1.28 us: 0.83 us of MFMAs (15.3 ns each, back to back), the rest LDS latency and the chain.  Tried and slower: all large products
-// as six bf16 products of three parts each, split by the movers (198 us for the second launch: the LDS traffic of the parts; 144 without
-// them), the same for the updates alone (176), four waves a state on eight product waves (180).
+// In a profile of the 248-us call (286 us there) the first launch is 82 us, the second 177, 128 chunks in a row at 1.38 us: 0.83 us of MFMAs
+// (15.3 ns each, back to back), the rest LDS latency and the chain; the read-outs' norm is 26.  Tried and slower: all large products as six bf16 products of three parts each, split by the
+// movers (198 us for the second launch: the LDS traffic of the parts; 144 without them), the same for the updates alone (176), four
+// waves a state on eight product waves (180).
 //
 // Against 64 bits (float32 rows, 64 and 128 channels, 8 to 1000 tokens a sequence, fresh and carried states), relative to the
 // token-by-token launch: states gated 0.88 to 0.96 times its error, general 1.03 to 1.13, write 0.99 to 1.00; read-outs 0.91 to 1.06,
@@ -63,136 +62,18 @@
 //
 // The read-outs go to a scratch of fp32 rows, because a row's norm spans the workgroups of its value columns; a last launch
 // norms, weights and gates them.  Single tokens run in a launch of their own that streams every state once.
-#include <type_traits>
+#include <algorithm>
 
-#include "chunk_recurrence.h"
-#include "row_pieces.h"
+#include "chunk_recurrence_parts.h"
 #include "../../include/nanovllm_hip_mixers.h"
 
 namespace nv {
 
 constexpr int kCrChunk = 16;
-constexpr float kCrNear = 8.27180613e-25f;            // 2^-80
-
-__device__ __forceinline__ float cr_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
-// log(1 + exp(x)) = max(x, 0) + log(1 + u), u = exp(-|x|) <= 1; log(1 + u) = 2 atanh(s), s = u / (2 + u) <= 1/3, by its series
-// (the first term left out is below 2^-26 of the sum).  s carries the roundings of 2 + u and of the reciprocal.  Within 4 % of
-// log1pf's error, and 7 instead of 19 us of a 285 us call (gated prompts below); the hardware's logarithm and exponential took none of
-// these, with 1.35 times the error in a decay.
-__device__ __forceinline__ float cr_softplus(float x) {
-    const float u = expf(-fabsf(x)), n = 2.0f + u, lost = u - (n - 2.0f), r = __builtin_amdgcn_rcpf(n);
-    float s = u * r;
-    s = fmaf(fmaf(-s, lost, fmaf(-s, n, u)), r, s);
-    const float z = s * s;
-    float p = 1.0f / 15.0f;
-    p = fmaf(p, z, 1.0f / 13.0f);
-    p = fmaf(p, z, 1.0f / 11.0f);
-    p = fmaf(p, z, 1.0f / 9.0f);
-    p = fmaf(p, z, 1.0f / 7.0f);
-    p = fmaf(p, z, 1.0f / 5.0f);
-    p = fmaf(p, z, 1.0f / 3.0f);
-    return fmaxf(x, 0.f) + fmaf(2.0f * s * z, p, 2.0f * s);
-}
-
-// Decay and vectors of one token and channel from its raw projections (x: in the order of x0 .. x3).
-struct CrElem {
-    float w, k, q, a;                                 // decay; k (raw scale); q / r; removal rate times k (general)
-};
-template <int FORM>
-__device__ __forceinline__ CrElem cr_elem(const float* x, float c0, float c1, float p0) {
-    CrElem e;
-    if constexpr (FORM == kCrGated) {
-        e.w = expf(-c0 * cr_softplus(x[2] + c1));     // c0: exp(A_log)
-        e.k = x[1];
-        e.q = x[0];
-        e.a = 0.f;
-    } else if constexpr (FORM == kCrGeneral) {
-        e.w = expf(-p0 * cr_sigmoid(x[2] + c0));
-        e.k = x[1];
-        e.q = x[0];
-        e.a = cr_sigmoid(x[3] + c1) * x[1];
-    } else {
-        e.w = c1 + (1.0f - c1) * cr_sigmoid(x[1] + c0);
-        e.k = 1.0f - e.w;
-        e.q = x[0] * cr_sigmoid(x[0]);
-        e.a = 0.f;
-    }
-    return e;
-}
-
-// An element on its way from memory in a register of its own: packed halves would make every load wait for the one before.
-template <typename T> struct CrRaw;
-template <> struct CrRaw<__bf16> {
-    typedef uint32_t type;
-    static __device__ __forceinline__ uint32_t load(const __bf16* p) { return *(const uint16_t*)p; }
-    static __device__ __forceinline__ float value(uint32_t r) { return __builtin_bit_cast(float, r << 16); }
-};
-// Two neighbouring elements by one load (VEC) or two.
-template <typename T, bool VEC> struct CrPair;
-template <> struct CrPair<__bf16, true> {
-    uint32_t r;
-    __device__ __forceinline__ void load(const __bf16* p) { r = *(const uint32_t*)p; }
-    __device__ __forceinline__ float value(int i) const { return i ? bf16_hi(r) : bf16_lo(r); }
-    __device__ __forceinline__ void keep(bool in) { r = in ? r : 0u; }
-    __device__ __forceinline__ void store(__bf16* p) const { *(uint32_t*)p = r; }
-};
-template <> struct CrPair<float, true> {
-    float2 r;
-    __device__ __forceinline__ void load(const float* p) { r = *(const float2*)p; }
-    __device__ __forceinline__ float value(int i) const { return i ? r.y : r.x; }
-    __device__ __forceinline__ void keep(bool in) { r = in ? r : make_float2(0.f, 0.f); }
-    __device__ __forceinline__ void store(float* p) const { *(float2*)p = r; }
-};
-template <typename T> struct CrPair<T, false> {
-    typename CrRaw<T>::type r[2];
-    __device__ __forceinline__ void load(const T* p) {
-        r[0] = CrRaw<T>::load(p);
-        r[1] = CrRaw<T>::load(p + 1);
-    }
-    __device__ __forceinline__ float value(int i) const { return CrRaw<T>::value(r[i]); }
-    __device__ __forceinline__ void keep(bool in) {
-        r[0] = in ? r[0] : 0;
-        r[1] = in ? r[1] : 0;
-    }
-    __device__ __forceinline__ void store(T* p) const {
-        p[0] = (T)value(0);
-        p[1] = (T)value(1);
-    }
-};
-template <> struct CrRaw<float> {
-    typedef float type;
-    static __device__ __forceinline__ float load(const float* p) { return *p; }
-    static __device__ __forceinline__ float value(float r) { return r; }
-};
-
-__device__ __forceinline__ f32x4 cr_mfma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-__device__ __forceinline__ float cr_lane(float x, int lane) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
-}
-// LDS writes of the workgroup's waves are done; loads from memory stay in flight.
-__device__ __forceinline__ void cr_group_barrier() {
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-template <int N> using CrRow = __attribute__((ext_vector_type(N))) float;
-// PER neighbouring elements of a row of V by one load.
-template <typename T, int PER> struct CrColumns : CrPair<T, true> {};
-template <> struct CrColumns<__bf16, 4> {
-    uint2 r;
-    __device__ __forceinline__ void load(const __bf16* p) { r = *(const uint2*)p; }
-    __device__ __forceinline__ float value(int i) const { return i & 1 ? bf16_hi(i < 2 ? r.x : r.y) : bf16_lo(i < 2 ? r.x : r.y); }
-};
-template <> struct CrColumns<float, 4> {
-    f32x4 r;
-    __device__ __forceinline__ void load(const float* p) { r = *(const f32x4*)p; }
-    __device__ __forceinline__ float value(int i) const { return r[i]; }
-};
-
 // Where a chunk's operands lie in the workspace: one record per (head, chunk), in the order in which the lanes of the second
 // launch read them, a head's chunks one after the other, beside them the chunks' rows of V ([head][record][16][Dv], zeros past the
 // sequence's end); read-outs are [head][row][Dv] too.  The second launch has few loads in flight, so streams that stay within a page
-// for several chunks matter to it (heads side by side, every chunk on pages of its own: 302 us instead of 264, chunks of 8).  Records of a
-// sequence start at (first row + 15 x its number) / 16: enough for the chunks in front, whatever the lengths, without a scan over them.
+// for several chunks matter to it (heads side by side, every chunk on pages of its own: 302 us instead of 264, chunks of 8).
 template <int FORM, int D>
 struct CrRecord {
     static constexpr int kRows = FORM == kCrWrite ? 16 : 32;      // of [K; Q]: write has no K
@@ -204,11 +85,6 @@ struct CrRecord {
     static constexpr int m = decay + D;                           // [matrix][16][16]
     static constexpr int words = m + kMat * 256;
 };
-// (rows and numbers counted from the first sequence of the launch)
-__device__ __host__ __forceinline__ int64_t cr_first_record(int64_t first_row, int seq) {
-    return (first_row + (int64_t)(kCrChunk - 1) * seq) / kCrChunk;
-}
-
 // ------------------------------------------------------------------------------------------------ first launch
 // Two waves per (chunk, head), eight tokens each; a lane owns two neighbouring channels of its eight tokens, so running products need
 // no exchange but of the halves' totals.  LDS turns the pair products' operands, K and Q into the order of the matrix cores; one wave
@@ -238,10 +114,10 @@ __global__ __launch_bounds__(128, FORM == kCrGeneral ? 2 : 3) void recurrence_ch
     int lo = first_seq, hi = a.num_seqs;              // the last sequence whose records start at or in front of this one
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
-        if (cr_first_record(a.cu_q[mid] - row0, mid - first_seq) <= rec) lo = mid; else hi = mid;
+        if (cr_first_record<kCrChunk>(a.cu_q[mid] - row0, mid - first_seq) <= rec) lo = mid; else hi = mid;
     }
     const int b = lo, q0 = a.cu_q[b], len = a.cu_q[b + 1] - q0;
-    const int64_t c64 = rec - cr_first_record(q0 - row0, b - first_seq);
+    const int64_t c64 = rec - cr_first_record<kCrChunk>(q0 - row0, b - first_seq);
     if (len < 2 || c64 * L >= len) return;            // (for the whole workgroup)
     const int t0 = q0 + (int)c64 * L, n16 = min(L, q0 + len - t0), n = min(N, max(n16 - half * N, 0)), th = half * N;
     float* out = a.chunks + (h * a.records + rec) * Rec::words;
@@ -466,36 +342,37 @@ __global__ __launch_bounds__(128, FORM == kCrGeneral ? 2 : 3) void recurrence_ch
     // start through a token (G) and behind it to the chunk's end (F).
     auto ku = [&](int t, int i) { return FORM == kCrGated ? kf(t, i) * cr_lane(kn, t) : kf(t, i); };
     auto qu = [&](int t, int i) { return FORM == kCrGated ? qf(t, i) * cr_lane(qn, t) : qf(t, i); };
-    float G[2][N], F[2][N], lead[2], all[2];
+    float G[2][N], F[2][N];
+    double end[2] = {1.0, 1.0}, other[2];             // decays of this half, then of the chunk; of the other half
     {
-        double2* const totals = (double2*)lds.right;
-        double total[2] = {1.0, 1.0};
+        auto forward = [&](double (&f)[2]) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+            for (int i = 0; i < 2; ++i) {
 #pragma unroll
-            for (int t = 0; t < N; ++t) total[i] *= (double)w[t][i];
-        }
-        if (in_row) totals[half * (D / 2) + d / 2] = make_double2(total[0], total[1]);
-        __syncthreads();
-        const double2 other = totals[(half ^ 1) * (D / 2) + d / 2];
-        const double ot[2] = {other.x, other.y};
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            double f = half ? ot[i] : 1.0;
-            lead[i] = (float)f;
-#pragma unroll
-            for (int t = 0; t < N; ++t) G[i][t] = (float)(f *= (double)w[t][i]);
-            f = half ? 1.0 : ot[i];
-#pragma unroll
-            for (int t = N - 1; t >= 0; --t) {
-                F[i][t] = (float)f;
-                f *= (double)w[t][i];
+                for (int t = 0; t < N; ++t) G[i][t] = (float)(f[i] *= (double)w[t][i]);
             }
-            all[i] = (float)f;
-        }
+        };
+        auto backward = [&](double (&f)[2]) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+#pragma unroll
+                for (int t = N - 1; t >= 0; --t) {
+                    F[i][t] = (float)f[i];
+                    f[i] *= (double)w[t][i];
+                }
+            }
+        };
+        double2* const totals = (double2*)lds.right;
+        if (half) backward(end); else forward(end);
+        if (in_row) totals[half * (D / 2) + d / 2] = make_double2(end[0], end[1]);
+        __syncthreads();
+        const double2 o = totals[(half ^ 1) * (D / 2) + d / 2];
+        other[0] = end[0] = o.x;
+        other[1] = end[1] = o.y;
+        if (half) forward(end); else backward(end);
     }
     if constexpr (FORM == kCrGated) put(lds.k, [&](int t, int i) { return ku(t, i) * G[i][t]; });
-    if constexpr (FORM == kCrGeneral) put(lds.k, [&](int t, int i) { return ku(t, i) * (t ? G[i][t ? t - 1 : 0] : lead[i]); });
+    if constexpr (FORM == kCrGeneral) put(lds.k, [&](int t, int i) { return ku(t, i) * (t ? G[i][t ? t - 1 : 0] : half ? (float)other[i] : 1.f); });
     put(lds.q, [&](int t, int i) { return qu(t, i) * G[i][t]; });
     auto put_update = [&](int which, auto of) {       // lane (g, channel) of a tile: tokens 4 g .. 4 g + 3
         if (in_row) {
@@ -514,7 +391,7 @@ __global__ __launch_bounds__(128, FORM == kCrGeneral ? 2 : 3) void recurrence_ch
     };
     if constexpr (FORM == kCrGated) put_update(0, ku); else put_update(0, kf);
     if constexpr (FORM == kCrGeneral) put_update(1, af);
-    if (half == 0 && in_row) *(float2*)(out + Rec::decay + d) = make_float2(all[0], all[1]);
+    if (half == 0 && in_row) *(float2*)(out + Rec::decay + d) = make_float2((float)end[0], (float)end[1]);
     __syncthreads();
     if (HAS_K || half) {
         const float* rows = (half ? lds.q : lds.k) + l16 * ROW + 4 * g;
@@ -594,7 +471,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (wave >= 4) {
         // ---------------------------------------------------------------- the movers
         const int tid = threadIdx.x - 256;
-        const int64_t first = (int64_t)h * a.records + cr_first_record(q0 - a.cu_q[first_seq], b - first_seq);
+        const int64_t first = (int64_t)h * a.records + cr_first_record<kCrChunk>(q0 - a.cu_q[first_seq], b - first_seq);
         const float* rec = a.chunks + first * Rec::words;
         const int tok = tid >> 4, col = (tid & 15) * PER, col_all = blockIdx.y * COLS + col;
         // (columns past the end: the last ones, used by waves that write nothing)
@@ -670,7 +547,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     uint32_t odd = 0;                                 // some chunk of the sequence and head holds a value that is not finite
     {
-        const uint32_t* flags = a.odd + (int64_t)h * a.records + cr_first_record(q0 - a.cu_q[first_seq], b - first_seq);
+        const uint32_t* flags = a.odd + (int64_t)h * a.records + cr_first_record<kCrChunk>(q0 - a.cu_q[first_seq], b - first_seq);
         for (int c = lane; c < chunks; c += 64) odd |= flags[c];
         odd = __any(odd != 0);
     }
@@ -1038,16 +915,40 @@ static bool recurrence_built(int D, int Dv) {
     return (D == 32 || D == 64 || D == 96 || D == 128) && Dv % 16 == 0 && Dv <= 256 && D * Dv <= 128 * 128;
 }
 
+// Two waves for a state's 16 columns while that leaves every workgroup (one a CU, two tiles of columns) a CU of its own.  Whole
+// calls, one against two waves, sequences of 768 rows, 16 heads: gated 128 x 128, 128 tiles 114 -> 78 us, 512: 147 -> 113,
+// 640: 158 -> 175, 1024: 190 -> 208; gated 64 x 64, 512: 122 -> 106, 640: 135 -> 155; general, 512: 188 -> 141, 640: 201 -> 223;
+// write 128 x 128, 512: 100 -> 73, 640: 110 -> 118.
+static bool cr_two_waves(int64_t seqs, int H, int Dv) { return seqs * H * ((Dv / 16 + 1) / 2) <= 256; }
+
+// Tokens of a chunk, from the mean portion of the sequences behind the leading single tokens.  A chunk of 16 halves the serial chain but
+// takes more products and registers a token, and a portion's last chunk is as dear half empty.  So it pays in long portions, later where the
+// grid fills the chip by itself (one wave a state), later the more products the form has, and sooner where every workgroup of the
+// first launch has a CU to itself.  Whole calls, 16 heads, chunks of 16 against 8, lines from 16 .. 2048 rows in 1 .. 128
+// sequences:  write, 128 x 128: 8 of 64 rows 0.96, 32 of 64 0.92, 8 of 17 1.18, 64 x 64: 16 of 128 0.99, 32 of 72 1.10, 1 of 33 0.95;
+// gated, 128 x 128: 4 of 192 0.94, 8 of 256 1.00, 16 of 256 0.96, 256 of 2 1.43, 64 x 64: 16 of 256 1.03, of 512 0.99, 32 x 32: 16 of 512
+// 1.05, 1 of 128 0.95; general, 128 x 128: 2 of 512 0.94, 4 of 256 1.05, 16 of 512 1.03, 256 of 2 1.58, 1 of 192 0.96.
+static int cr_chunk_tokens(int form, int64_t rows, int64_t seqs, int H, int D, int Dv) {
+    const bool alone = (cr_first_record<kCrChunk>(rows, (int)seqs) + 1) * H <= 256, two = cr_two_waves(seqs, H, Dv);
+    if (form == kCrGeneral && !two) return 8;
+    const int64_t from = form == kCrWrite ? (alone ? 25 : D >= 128 ? 64 : 128)
+                                          : form == kCrGated ? (alone ? 96 : two ? 192 : 128 * 256 / D) : (alone ? 128 : 512);
+    return rows >= from * seqs ? kCrChunk : 8;
+}
+
 // The workspace of T rows in seqs sequences: records, their rows of V, read-outs, flags; the parts in front of the flags are whole
 // 16-byte pieces.
 struct CrWorkspace {
+    int tokens;                                       // of a chunk
     int64_t records, chunks, columns, raw, odd;       // how many (per head); bytes of the parts
-    CrWorkspace(int form, int64_t T, int H, int D, int Dv, int seqs, int dtype) {
-        const int words = (form == kCrWrite ? 16 : 32) * D + (form == kCrGeneral ? 2 : 1) * 16 * D + D +
-                          (form == kCrWrite ? 256 : form == kCrGated ? 512 : 1024);
-        records = cr_first_record(T, seqs) + 1;
+    CrWorkspace(int form, int chunk, int64_t T, int H, int D, int Dv, int seqs, int dtype) {
+        tokens = chunk;
+        const int words = tokens != kCrChunk ? short_recurrence_words(form, D)
+                                             : (form == kCrWrite ? 16 : 32) * D + (form == kCrGeneral ? 2 : 1) * 16 * D + D +
+                                                   (form == kCrWrite ? 256 : form == kCrGated ? 512 : 1024);
+        records = tokens != kCrChunk ? short_recurrence_records(T, seqs) : cr_first_record<kCrChunk>(T, seqs) + 1;
         chunks = records * H * words * 4;
-        columns = records * H * kCrChunk * Dv * (dtype == NV_DTYPE_BF16 ? 2 : 4);
+        columns = records * H * tokens * Dv * (dtype == NV_DTYPE_BF16 ? 2 : 4);
         raw = T * H * Dv * 4;
         odd = records * H * 4;
     }
@@ -1055,32 +956,35 @@ struct CrWorkspace {
 };
 
 template <typename T, int FORM, int D>
-static void chunks_of_size(const ChunkRecurrenceArgs& a, int first_seq, hipStream_t s) {
-    const int seqs = a.num_seqs - first_seq;
-    const dim3 prep((unsigned)a.records, (unsigned)a.H), pairs((unsigned)(seqs * a.H));
-    const uintptr_t piece = 2 * sizeof(T) - 1;        // two channels by one load
-    const bool vec = a.sv % 2 == 0 && a.s0 % 2 == 0 && a.s1 % 2 == 0 && a.s2 % 2 == 0 && a.s3 % 2 == 0 &&
-                     (((uintptr_t)a.v | (uintptr_t)a.x0 | (uintptr_t)a.x1 | (uintptr_t)a.x2 | (uintptr_t)a.x3) & piece) == 0;
+static void chunks_of_size(const ChunkRecurrenceArgs& a, int first_seq, bool vec, int waves, hipStream_t s) {
+    const dim3 prep((unsigned)a.records, (unsigned)a.H), block(512);
+    const unsigned pairs = (unsigned)((a.num_seqs - first_seq) * a.H), tiles = (unsigned)(a.Dv / 16);
     if (vec) hipLaunchKernelGGL((recurrence_chunks_kernel<T, FORM, D, true>), prep, dim3(128), 0, s, a, first_seq);
     else hipLaunchKernelGGL((recurrence_chunks_kernel<T, FORM, D, false>), prep, dim3(128), 0, s, a, first_seq);
-    // Two waves for a state's 16 columns while that leaves every workgroup (one a CU, two tiles of columns) a CU of its own.  Whole
-    // calls, one against two waves, sequences of 768 rows, 16 heads: gated 128 x 128, 128 tiles 114 -> 78 us, 512: 147 -> 113,
-    // 640: 158 -> 175, 1024: 190 -> 208; gated 64 x 64, 512: 122 -> 106, 640: 135 -> 155; general, 512: 188 -> 141, 640: 201 -> 223;
-    // write 128 x 128, 512: 100 -> 73, 640: 110 -> 118.
-    const int tiles = a.Dv / 16;
-    if ((int64_t)pairs.x * ((tiles + 1) / 2) <= 256)
-        hipLaunchKernelGGL((recurrence_states_kernel<T, FORM, D, 2>), dim3(pairs.x, (unsigned)((tiles + 1) / 2)), dim3(512), 0, s, a, first_seq);
-    else
-        hipLaunchKernelGGL((recurrence_states_kernel<T, FORM, D, 1>), dim3(pairs.x, (unsigned)((tiles + 3) / 4)), dim3(512), 0, s, a, first_seq);
+    if constexpr (FORM != kCrGeneral) {               // (general: steps of two waves only)
+        if (waves == 1) {
+            hipLaunchKernelGGL((recurrence_states_kernel<T, FORM, D, 1>), dim3(pairs, (tiles + 3) / 4), block, 0, s, a, first_seq);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((recurrence_states_kernel<T, FORM, D, 2>), dim3(pairs, (tiles + 1) / 2), block, 0, s, a, first_seq);
 }
 
 template <typename T, int FORM>
-static int chunks_of(const ChunkRecurrenceArgs& a, int first_seq, bool singles_behind, hipStream_t s) {
-    switch (a.D) {
-        case 32: chunks_of_size<T, FORM, 32>(a, first_seq, s); break;
-        case 64: chunks_of_size<T, FORM, 64>(a, first_seq, s); break;
-        case 96: chunks_of_size<T, FORM, 96>(a, first_seq, s); break;
-        default: chunks_of_size<T, FORM, 128>(a, first_seq, s); break;
+static int chunks_of(const ChunkRecurrenceArgs& a, int first_seq, int tokens, bool singles_behind, int dtype, hipStream_t s) {
+    const uintptr_t piece = 2 * sizeof(T) - 1;        // two channels by one load
+    const bool pairs = a.sv % 2 == 0 && a.s0 % 2 == 0 && a.s1 % 2 == 0 && a.s2 % 2 == 0 && a.s3 % 2 == 0 &&
+                       (((uintptr_t)a.v | (uintptr_t)a.x0 | (uintptr_t)a.x1 | (uintptr_t)a.x2 | (uintptr_t)a.x3) & piece) == 0;
+    const int waves = cr_two_waves(a.num_seqs - first_seq, a.H, a.Dv) ? 2 : 1;
+    if (tokens != kCrChunk) {
+        launch_short_recurrence(FORM, a, first_seq, pairs, waves, dtype, s);
+    } else {
+        switch (a.D) {
+            case 32: chunks_of_size<T, FORM, 32>(a, first_seq, pairs, waves, s); break;
+            case 64: chunks_of_size<T, FORM, 64>(a, first_seq, pairs, waves, s); break;
+            case 96: chunks_of_size<T, FORM, 96>(a, first_seq, pairs, waves, s); break;
+            default: chunks_of_size<T, FORM, 128>(a, first_seq, pairs, waves, s); break;
+        }
     }
     const dim3 rows((unsigned)a.T);
     const bool vec = a.gate_stride % 4 == 0 && a.out_stride % 4 == 0 &&
@@ -1111,10 +1015,11 @@ static int singles_of(const ChunkRecurrenceArgs& a, hipStream_t s) {
     return form == kCrGated ? FN<float, kCrGated>(__VA_ARGS__)                                                        \
                             : form == kCrGeneral ? FN<float, kCrGeneral>(__VA_ARGS__) : FN<float, kCrWrite>(__VA_ARGS__)
 
-int launch_chunk_recurrence(int form, const ChunkRecurrenceArgs& a, int first_seq, bool singles_behind, int dtype, hipStream_t s) {
-    NV_CR_DISPATCH(chunks_of, a, first_seq, singles_behind, s);
+static int launch_chunk_recurrence(int form, const ChunkRecurrenceArgs& a, int first_seq, int tokens, bool singles_behind, int dtype,
+                                   hipStream_t s) {
+    NV_CR_DISPATCH(chunks_of, a, first_seq, tokens, singles_behind, dtype, s);
 }
-int launch_single_recurrence(int form, const ChunkRecurrenceArgs& a, int dtype, hipStream_t s) {
+static int launch_single_recurrence(int form, const ChunkRecurrenceArgs& a, int dtype, hipStream_t s) {
     NV_CR_DISPATCH(singles_of, a, s);
 }
 #undef NV_CR_DISPATCH
@@ -1129,7 +1034,7 @@ bool run_recurrence_portions(int form, ChunkRecurrenceArgs a, int lead, int port
     if (!recurrence_built(a.D, a.Dv) || (uintptr_t)a.state % 16 != 0 || a.T >= (1LL << 31) || (int64_t)a.num_seqs * a.H >= (1LL << 31) ||
         (rest && (workspace == nullptr || a.T <= 0)))
         return false;
-    const CrWorkspace ws(form, a.T, a.H, a.D, a.Dv, a.num_seqs - lead, dtype);
+    const CrWorkspace ws(form, cr_chunk_tokens(form, a.T - lead, a.num_seqs - lead, a.H, a.D, a.Dv), a.T, a.H, a.D, a.Dv, a.num_seqs - lead, dtype);
     const int64_t need = ws.bytes();
     if (rest && workspace_bytes < need) {
         set_error("recurrence: workspace of %lld bytes, need %lld", (long long)workspace_bytes, (long long)need);
@@ -1147,7 +1052,7 @@ bool run_recurrence_portions(int form, ChunkRecurrenceArgs a, int lead, int port
     a.raw = (float*)((char*)a.columns + ws.columns);
     a.odd = (uint32_t*)((char*)a.raw + ws.raw);
     a.records = ws.records;
-    if (rest) *rc = launch_chunk_recurrence(form, a, lead, singles_behind, dtype, s);
+    if (rest) *rc = launch_chunk_recurrence(form, a, lead, ws.tokens, singles_behind, dtype, s);
     return true;
 }
 
@@ -1158,5 +1063,10 @@ extern "C" int64_t nv_recurrence_workspace_bytes(int form, int64_t T, int H, int
     if (form < 0 || form > 2 || T <= 0 || H <= 0 || D <= 0 || Dv <= 0 || leading_singles < 0 || num_seqs <= leading_singles ||
         !nv::recurrence_built(D, Dv))
         return 0;
-    return nv::CrWorkspace(form, T, H, D, Dv, num_seqs - leading_singles, dtype).bytes();
+    // (never less than chunks of 8 would need: more rows in as many sequences need no less, whichever they are taken in)
+    const int seqs = num_seqs - leading_singles;
+    int64_t need = nv::CrWorkspace(form, 8, T, H, D, Dv, seqs, dtype).bytes();
+    if (nv::cr_chunk_tokens(form, T - leading_singles, seqs, H, D, Dv) == nv::kCrChunk)
+        need = std::max(need, nv::CrWorkspace(form, nv::kCrChunk, T, H, D, Dv, seqs, dtype).bytes());
+    return need;
 }

@@ -15,8 +15,8 @@
 //                          channel, and the read-out normalised: o / rms(o) * norm_w * sigmoid(gate_raw).
 //                          Everything after the raw projections is fp32.
 //
-// With a workspace and head sizes in steps of 32 up to 128 the recurrence runs in chunks of 8 tokens on the matrix cores
-// (chunk_recurrence.hip).  What follows is the launch for the other sizes and for calls without a workspace.
+// With a workspace and head sizes in steps of 32 up to 128 portions run in chunks on the matrix cores, single tokens in one pass
+// over their states (chunk_recurrence.hip).  What follows is the launch for the other sizes and for calls without a workspace.
 //
 // Layout of the recurrence: one workgroup per (sequence, head).  A lane owns one value column and a quarter of the
 // key rows (a contiguous run: its quad index r owns rows r * RPL .. r * RPL + RPL - 1, read from LDS four at a time; the

@@ -573,8 +573,8 @@ def _portions(dll, form: int, rows: torch.Tensor, T: int, H: int, D: int, Dv: in
 def recurrence_scratch_bytes(form: int, rows: int, H: int, D: int, Dv: int, seqs: int, dtype: torch.dtype) -> int:
     """The most bytes a recurrent layer allocates for a step of up to `rows` rows in up to `seqs` sequences (form: 0 gated delta
     rule, 1 generalized delta rule, 2 gated write)."""
-    return int(_lib.mixers().nv_recurrence_workspace_bytes(form, rows, H, D, Dv, seqs, 0,
-                                                           _lib.DTYPE_BF16 if dtype == _BF16 else _lib.DTYPE_F32))
+    need, dt = _lib.mixers().nv_recurrence_workspace_bytes, _lib.DTYPE_BF16 if dtype == _BF16 else _lib.DTYPE_F32
+    return max((int(need(form, rows, H, D, Dv, n, 0, dt)) for n in range(1, seqs + 1)), default=0)       # (fewer sequences may take larger chunks)
 
 
 def gated_delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a_raw: torch.Tensor, b_raw: torch.Tensor,

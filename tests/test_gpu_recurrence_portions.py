@@ -1,5 +1,5 @@
 """GPU: the recurrences with a decay per head and key channel against the eager stand-ins of the same layers, at the sizes where
-their launches change: around the chunk of 8 tokens, single tokens in front of, between and beside longer portions, fresh and
+their launches change: around the chunks of 8 and of 16 tokens, single tokens in front of, between and beside longer portions, fresh and
 carried states, every built number of key channels, value columns that do not fill a workgroup, decays from none to total."""
 import pytest
 import torch
@@ -162,11 +162,30 @@ def test_entries_without_workspace(form, entry):
 def test_values_that_are_not_finite(form, name, value, dtype, Dv):
     """What is not finite in one token's row reaches that row and what comes after it, as token by token: no row in front of it,
     no other head, no other sequence; and what it makes finite (a gate fully open or closed) is finite."""
-    H, D, at = 4, 128, 11                  # token 3 of the second chunk of the first sequence
-    Dv = D if form == "general" else Dv
+    Dv = 128 if form == "general" else Dv
     rows, before = [21, 9, 13], [0, 5, 0]
     if Dv == 128:
         rows, before = rows * 16, before * 16
+    _strike(form, name, value, dtype, Dv, rows, before, 11)              # token 3 of the second chunk of 8 of the first sequence
+
+
+@pytest.mark.parametrize("at", [0, 3, 7, 8, 15, 16])
+@pytest.mark.parametrize("value", [float("nan"), float("-inf")])
+@pytest.mark.parametrize("form,name", [("gated", "q"), ("gated", "k"), ("gated", "v"), ("gated", "w"), ("gated", "b"), ("general", "q"),
+                                       ("general", "k"), ("general", "v"), ("general", "w"), ("general", "a"), ("write", "q"),
+                                       ("write", "k"), ("write", "v")])
+def test_values_that_are_not_finite_in_chunks_of_16(form, name, value, at):
+    """The same in both halves of a chunk, at its ends and in front of the next one, for portions that run in chunks of 16."""
+    _strike(form, name, value, torch.float32, 128, [130, 129, 128], [0, 5, 0], at)
+
+
+@pytest.mark.parametrize("form,name,rows", [("gated", "k", 257), ("gated", "w", 257), ("write", "k", 130), ("write", "v", 130)])
+def test_values_that_are_not_finite_in_chunks_of_16_one_wave(form, name, rows):
+    _strike(form, name, float("nan"), torch.bfloat16, 128, [rows] * 17, [0, 5] * 8 + [0], 8)
+
+
+def _strike(form, name, value, dtype, Dv, rows, before, at):
+    H, D = 4, 128
     n, ctx = rows[0], _context(rows, before, True)
     a, r, x, state = _operands(form, rows, before, H, D, Dv, dtype, 9)
     nv.set_context(ctx)
@@ -207,14 +226,14 @@ def test_values_that_are_not_finite(form, name, value, dtype, Dv):
         torch.testing.assert_close(g[ok], w[ok], **tol)
 
 
-@pytest.mark.parametrize("rows", [1, 8])
-def test_decays_keep_their_precision(rows):
+@pytest.mark.parametrize("rows,B", [(1, 32), (8, 32), (100, 2), (257, 32)])    # (the last two: chunks of 16, two waves and one)
+def test_decays_keep_their_precision(rows, B):
     """A state that nothing is written to is its decays' product.  Against 64 bits the launches for known portions are no further off
     than the token-by-token entry: each decay is the rounding of its exponent's two sums and products, and of the exponential, on
     both sides, so their root-mean-square errors over 65536 channels agree within a few percent (softplus and exponential of
     single instructions: 1.35 and 1.24 times as far off)."""
     from nanovllm_amd import _lib
-    B, H, D, Dv = 32, 16, 128, 16
+    H, D, Dv = 16, 128, 16
     T = B * rows
     g = torch.Generator(device=DEV).manual_seed(3)
     zero, v = torch.zeros(T, H, D, device=DEV), torch.zeros(T, H, Dv, device=DEV)
@@ -252,7 +271,17 @@ def test_decays_keep_their_precision(rows):
 def test_total_decay_behind_large_values(form, at):
     """A token whose decays forget everything sees nothing of what was written before it, also within its chunk and however large
     that was: its factors are below any that the pair products could divide by."""
-    H, D, rows, before = 4, 128, [24, 13], [0, 3]
+    _forget(form, at, [24, 13])
+
+
+@pytest.mark.parametrize("at", [3, 7, 8, 15, 16, 17])
+@pytest.mark.parametrize("form", ["gated", "general", "write"])
+def test_total_decay_behind_large_values_in_chunks_of_16(form, at):
+    _forget(form, at, [130, 129])
+
+
+def _forget(form, at, rows):
+    H, D, before = 4, 128, [0, 3]
     a, r, x, state = _operands(form, rows, before, H, D, D, torch.float32, 13)
     for m in (a, r):
         if form == "gated":
@@ -275,7 +304,9 @@ def test_total_decay_behind_large_values(form, at):
     want, got = _forward(form, r, x, want_state), _forward(form, a, x, got_state)
     nv.set_context(None)
     torch.testing.assert_close(got, want, rtol=5e-5, atol=5e-5)          # (the bounds of test_portions)
-    torch.testing.assert_close(got_state, want_state, rtol=2e-5, atol=2e-6 * state.abs().max().item())
+    # (about 110 writes behind it add up to more than the states before: each is rounded at the sum's size, as in test_portions)
+    scale = max(state.abs().max().item(), want_state.abs().max().item() if max(rows) > 100 else 0.0)
+    torch.testing.assert_close(got_state, want_state, rtol=2e-5, atol=2e-6 * scale)
 
 
 def test_read_outs_keep_their_precision():
@@ -323,12 +354,24 @@ def test_read_outs_keep_their_precision():
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("form,D,Dv", [("gated", 128, 128), ("gated", 96, 48), ("gated", 32, 80), ("general", 128, 128), ("general", 96, 96),
                                        ("write", 96, 144), ("write", 64, 16)])
-@pytest.mark.parametrize("rows", [[15, 16, 17, 31, 32, 33, 48], [24] * 40], ids=["edges", "many"])   # (many: one wave for a state's columns)
+@pytest.mark.parametrize("rows", [[900, 15, 16, 17, 31, 32, 33, 48], [15, 16, 17, 31, 32, 33, 48], [24] * 40], ids=["edges", "edges_of_8", "many"])
 def test_chunks_of_16(form, D, Dv, rows, dtype):
-    """Around the chunk of 16 tokens and its halves, carried and fresh states, both splits of a state over waves.  The bounds are those
-    of test_portions: the same sums, of up to 128 products and 16 tokens, in another order."""
+    """Around the chunk of 16 tokens and its halves (edges; the long portion makes it the step's chunk), and at the same rows in chunks of
+    8, carried and fresh states.  The bounds are those of test_portions: the same sums, of up to 128 products and 16 tokens, in another
+    order."""
+    _compare_portions(form, D, Dv, rows, 2 if rows[0] == 900 else 4, dtype)
+
+
+@pytest.mark.parametrize("form,D,Dv,rows", [("gated", 128, 128, [300, 220] * 10), ("gated", 96, 48, [400, 300] * 18), ("write", 128, 128, [150, 129] * 9),
+                                            ("write", 64, 16, [150, 129] * 33)])
+def test_chunks_of_16_one_wave(form, D, Dv, rows):
+    """Steps that fill the chip: one wave for a state's columns."""
+    _compare_portions(form, D, Dv, rows, 4, torch.bfloat16)
+
+
+def _compare_portions(form, D, Dv, rows, H, dtype):
     before = [5 * (i % 3) for i in range(len(rows))]
-    a, r, x, state = _operands(form, rows, before, 4, D, Dv, dtype, 11)
+    a, r, x, state = _operands(form, rows, before, H, D, Dv, dtype, 11)
     nv.set_context(_context(rows, before, False))
     want_state = state.clone()
     want = _forward(form, r, x, want_state)
@@ -374,14 +417,14 @@ def _in_64_bits(form, m, x, state, B, rows):
     return (o / torch.sqrt((o * o).mean(-1, keepdim=True) + 1e-5) * weight * gate).view(B * rows, H * Dv), S
 
 
-# Bounds of (read-outs, states).  Measured: 0.96 to 1.03 and 0.89 to 0.92 (gated), 1.00 to 1.02 and 0.91 to 0.95 (general), 0.99 to 1.02 and
-# 0.99 (write); with decays multiplied in 32 bits, pair products in four sums and removals on top of the state, 1.09 and 0.97, 1.16 and 1.30,
-# 1.05 and 1.005.
-OFF = {"gated": (1.05, 0.95), "general": (1.05, 1.0), "write": (1.035, 1.0)}
+# Bounds of (read-outs, states).  Measured at 33 .. 257 rows: 0.95 to 1.03 and 0.89 to 0.96 (gated), 0.98 to 1.02 and 0.90 to 0.95 (general),
+# 0.99 to 1.02 and 0.99 (write); at 33 and 70 rows with decays multiplied in 32 bits, pair products in four sums and removals on top of the
+# state: up to 1.09 and 0.97, 1.16 and 1.30, 1.05 and 1.005.
+OFF = {"gated": (1.05, 1.0), "general": (1.05, 1.0), "write": (1.035, 1.0)}
 
 
-@pytest.mark.parametrize("rows", [33, 70])
-@pytest.mark.parametrize("form,B", [("gated", 2), ("gated", 16), ("general", 2), ("write", 2), ("write", 16)])   # two waves for a state's columns and one
+@pytest.mark.parametrize("form,B,rows", [("gated", 2, 97), ("gated", 16, 257), ("general", 2, 129), ("general", 2, 144), ("write", 2, 33),
+                                         ("write", 16, 129)])          # two waves for a state's columns and (B = 16) one
 def test_long_portions_keep_their_precision(monkeypatch, form, B, rows):
     """Float32 rows over carried states against 64 bits, relative to the token-by-token launch: a chunk takes the same sums in another
     order."""
@@ -417,11 +460,12 @@ def test_long_portions_keep_their_precision(monkeypatch, form, B, rows):
 
 
 @pytest.mark.parametrize("rate", [6.5, 7.5, 13.0, 14.5])
+@pytest.mark.parametrize("rows", [[130, 129], [17, 8]], ids=["chunks_of_16", "chunks_of_8"])
 @pytest.mark.parametrize("form", ["gated", "general", "write"])
-def test_fast_decays(form, rate):
+def test_fast_decays(form, rows, rate):
     """Channels that decay by about exp(-rate) a token beside slow ones, on both sides of where eight (6.9) and four (13.9) factors
     multiply to 2^-80 and the chunk's pairs are taken in more sets."""
-    H, D, rows, before = 4, 128, [33, 40], [0, 3]
+    H, D, before = 4, 128, [0, 3]
     a, r, x, state = _operands(form, rows, before, H, D, D, torch.float32, 17)
     fast = (torch.arange(H * D, device=DEV) % 5 == 0).float() * rate
     for m in (a, r):

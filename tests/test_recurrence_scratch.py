@@ -52,6 +52,45 @@ def test_single_tokens_allocate_nothing(max_rows, lead, portions):
     assert ops._portions(None, 0, None, 3, H, D, D, 3, max_rows, lead, portions)[2] is None
 
 
+def _need(form, T, seqs, lead=0, heads=16, d=D):
+    return _lib.mixers().nv_recurrence_workspace_bytes(form, T, heads, d, d, seqs, lead, _lib.DTYPE_BF16)
+
+
+def _bytes(form, tokens, T, seqs, heads=16, d=D):
+    """Records of `tokens` tokens with their rows of V, read-outs and flags of a step."""
+    words = (1 if form == 2 else 2) * tokens * d + (2 if form == 1 else 1) * tokens * d + d
+    words += {8: (384, 384, 64), 16: (512, 1024, 256)}[tokens][form]
+    records = (T + (tokens - 1) * seqs) // tokens + 1
+    return heads * (records * (words * 4 + tokens * d * 2 + 4) + T * d * 4)
+
+
+@pytest.mark.parametrize("form", range(3))
+@pytest.mark.parametrize("seqs,rows", [(256, 2), (256, 5), (8, 17), (64, 24)])
+def test_short_portions_take_small_records(form, seqs, rows):
+    """A record of 16 tokens for a portion of a few is twice the memory and, for many of them, up to 1.6 times the time."""
+    assert _need(form, seqs * rows, seqs) == _bytes(form, 8, seqs * rows, seqs)
+    assert _need(form, seqs * rows + 7, seqs + 7, 7) == _bytes(form, 8, seqs * rows + 7, seqs)        # single tokens in front
+
+
+@pytest.mark.parametrize("form,seqs,rows,tokens", [(0, 4, 191, 8), (0, 4, 192, 16), (0, 16, 255, 8), (0, 16, 256, 16), (0, 1, 96, 16), (1, 4, 511, 8),
+                                                   (1, 4, 512, 16), (1, 16, 512, 8), (1, 1, 128, 16), (2, 8, 63, 8), (2, 8, 64, 16), (2, 1, 25, 16)])
+def test_long_portions_take_chunks_of_16(form, seqs, rows, tokens):
+    T = seqs * rows
+    assert _need(form, T, seqs) == max(_bytes(form, 8, T, seqs), _bytes(form, tokens, T, seqs))
+
+
+@pytest.mark.parametrize("form", range(3))
+@pytest.mark.parametrize("d", [64, 128])
+def test_no_step_needs_more_than_the_layers_say(form, d):
+    most = {n: ops.recurrence_scratch_bytes(form, 4096, 16, d, d, n, torch.bfloat16) for n in (1, 5, 40)}
+    for n, bound in most.items():
+        for seqs in range(1, n + 1):
+            for T in (seqs, 2 * seqs, 33, 95 * seqs, 128 * seqs - 1, 255 * seqs, 256 * seqs, 511 * seqs, 4095, 4096):
+                if seqs <= T <= 4096:
+                    assert _need(form, T, seqs, heads=16, d=d) <= bound, (seqs, T)
+    assert ops.recurrence_scratch_bytes(form, 4096, 16, d, d, 0, torch.bfloat16) == 0
+
+
 READELF = shutil.which("llvm-readelf", path="/opt/rocm/llvm/bin")
 
 
