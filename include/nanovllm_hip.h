@@ -189,6 +189,8 @@ NV_API int nv_attn_decode_paged_static(const void* q, const void* k_cache, const
  */
 NV_API int64_t nv_attn_prefill_workspace_bytes(int B, int total_q, int max_seqlen_q, int max_seqlen_k,
                                         int H_q, int H_kv, int D);
+/* The plan of such a call: query tiles of a workgroup of the hand-scheduled kernel; 0: the other kernel, or no call. */
+NV_API int nv_attn_prefill_query_tiles(int B, int total_q, int max_seqlen_q, int max_seqlen_k, int H_q, int H_kv);
 NV_API int nv_attn_prefill_varlen(const void* q, const void* k_cache, const void* v_cache, void* o,
                            const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
                            const int32_t* block_tables, int B, int max_blocks,

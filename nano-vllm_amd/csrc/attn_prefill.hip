@@ -451,21 +451,29 @@ static void prefill_grid(PrefillShape& sh, int B, int H_q, int H_kv, int max_seq
     prefill_set_grid(sh);
 }
 
-// Several query tiles a workgroup make all workgroups of a sequence equal, so that whole rounds of them are paid: 528 on 256 CUs are
-// three rounds, the last one nearly empty, where single tiles, heaviest first, fill the chip to the end.  In key tiles of one CU, for
-// sequences of the mean length: the rounds, or all the work and the fixed cost of every single tile, with 5 % to spare (uneven
-// sequences end a round of shares earlier than their mean says).
-// 32 / 8 heads, prompts, two tiles against one: 3 of 1999 .. 3500 tokens 221 -> 199 us, 6 of 1365 148 -> 122; two full rounds stay as they
-// are (4 of 2048 tokens, 1 of 8192).
-static bool prefill_shares_pay(const PrefillShape& sh, int B, int items, int groups, int total_q, int max_seqlen_q, int max_seqlen_k) {
-    constexpr int64_t kFixed = 8;                     // a workgroup's fixed cost (about 12 us) in key tiles of 1.5 us
-    const int64_t mean = std::max<int64_t>(1, std::min<int64_t>(max_seqlen_q, total_q / B));
-    const int64_t n = (mean + sh.rows_per_wg - 1) / sh.rows_per_wg, slots = (n + items - 1) / items;
-    const int64_t cached = std::max(0, max_seqlen_k - max_seqlen_q) / kBN;
-    const int64_t pair = n * (n + 1) / 2 * (sh.rows_per_wg / kBN) + n * cached;       // key tiles of a sequence and head group
-    const int64_t all = (int64_t)sh.n_pairs * groups, rounds = (all * slots + 255) / 256;
-    const int64_t shares = rounds * (pair / slots + kFixed), singles = all * (pair + n * kFixed) / 256;
-    return shares * 20 <= singles * 21;
+// What a launch with m query tiles a workgroup takes, in key tiles of one CU times 256 CUs, for one sequence of the most rows and others
+// that share the rest.  Several tiles (shares) make all workgroups of a sequence equal and pay the fixed cost once, but whole rounds of them
+// are paid: 528 on 256 CUs are three rounds, the last one nearly empty, where single tiles, heaviest first, fill the chip to the end.
+// On 153 steps of 8/1, 16/8, 32/8 and 64/8 heads (equal, uneven, one long among short ones, cached chunks) the cheapest of the plans by
+// this cost is 1.6 % slower on average than the best one, 19 % at most; the largest shares that leave 512 workgroups were 11 and 140 %.
+static int64_t prefill_cost(const PrefillShape& sh, int B, int m, int groups, int total_q, int max_seqlen_q, int max_seqlen_k) {
+    constexpr int64_t kFixed = 11;                    // a workgroup's start and end in key tiles of 1.5 us
+    const int64_t per = (int64_t)sh.n_pairs / B * groups, tile = sh.rows_per_wg / kBN, cached = std::max(0, max_seqlen_k - max_seqlen_q) / kBN;
+    struct { int64_t wgs, each, work; } kind[2] = {};
+    for (int i = 0; i < (B > 1 ? 2 : 1); ++i) {
+        const int64_t rest = i ? ((int64_t)total_q - max_seqlen_q + B - 2) / (B - 1) : max_seqlen_q;
+        const int64_t n = (std::min<int64_t>(max_seqlen_q, std::max<int64_t>(1, rest)) + sh.rows_per_wg - 1) / sh.rows_per_wg;
+        const int64_t slots = (n + m - 1) / m, tiles = n * (n + 1) / 2 * tile + n * cached, all = i ? per * (B - 1) : per;
+        kind[i] = {all * slots, tiles / slots + kFixed, all * (tiles + slots * kFixed)};
+    }
+    if (m == 1) return std::max(kind[0].work + kind[1].work, 256 * (sh.n_qtiles * tile + cached + kFixed));
+    // the long sequence's rounds; the others beside its last one, then in rounds of their own
+    const int64_t over = kind[0].wgs % 256, left = 256 - over, full = kind[0].wgs / 256 * kind[0].each, c0 = kind[0].each, c1 = kind[1].each;
+    const int64_t beside = over ? c0 / std::max<int64_t>(c1, 1) * left : 0;
+    int64_t t = full + (over ? c0 : 0);
+    if (kind[1].wgs > beside) t += (kind[1].wgs - beside + 255) / 256 * c1;
+    else if (kind[1].wgs > 0) t = std::max(t, full + (kind[1].wgs + left - 1) / left * c1);
+    return 256 * t;
 }
 
 static PrefillShape prefill_shape(int B, int total_q, int H_q, int H_kv, int max_seqlen_q, int max_seqlen_k) {
@@ -504,19 +512,22 @@ static PrefillShape prefill_shape(int B, int total_q, int H_q, int H_kv, int max
         sh.nsplit = ns_asm > 1 ? (tiles + sh.tiles_per_split - 1) / sh.tiles_per_split : 1;
         // several query tiles per workgroup (equal work for all workgroups of a sequence, a half or a quarter
         // of the fixed per-workgroup cost: about 6 us until the first MFMA) while that still leaves two
-        // workgroups per CU
+        // workgroups per CU: the cheapest plan (single tiles only where a grid can hold them)
         if (sh.nsplit == 1) {
             const int groups = sh.wg_per_pair / sh.n_qtiles;
-            for (int m = kMaxItemsPerWg; m >= 2; m /= 2) {
-                const int slots = (sh.n_qtiles + m - 1) / m;
-                if ((int64_t)sh.n_pairs * slots * groups >= 512) {
-                    if (!prefill_shares_pay(sh, B, m, groups, total_q, max_seqlen_q, max_seqlen_k)) break;
+            int64_t least = sh.grid_base < (1LL << 31) ? prefill_cost(sh, B, 1, groups, total_q, max_seqlen_q, max_seqlen_k) : INT64_MAX;
+            for (int m = 2; m <= kMaxItemsPerWg; m *= 2) {
+                if ((int64_t)sh.n_pairs * ((sh.n_qtiles + m - 1) / m) * groups < 512) break;
+                const int64_t cost = prefill_cost(sh, B, m, groups, total_q, max_seqlen_q, max_seqlen_k);
+                if (cost < least || (cost == least && sh.items_per_wg > 1)) {
+                    least = cost;
                     sh.items_per_wg = m;
-                    sh.wg_per_pair = slots * groups;
-                    sh.n_qtiles = slots;
-                    prefill_set_grid(sh);
-                    break;
                 }
+            }
+            if (sh.items_per_wg > 1) {
+                sh.n_qtiles = (sh.n_qtiles + sh.items_per_wg - 1) / sh.items_per_wg;
+                sh.wg_per_pair = sh.n_qtiles * groups;
+                prefill_set_grid(sh);
             }
         }
         return sh;
@@ -552,6 +563,13 @@ extern "C" int64_t nv_attn_prefill_workspace_bytes(int B, int total_q, int max_s
     if (sh.nsplit == 1) return 16;
     if (sh.hand_scheduled) return prefill_asm_state_bytes(sh.grid_base, sh.nsplit);
     return (int64_t)total_q * H_q * sh.nsplit * kPartStride * (int64_t)sizeof(float);
+}
+
+extern "C" int nv_attn_prefill_query_tiles(int B, int total_q, int max_seqlen_q, int max_seqlen_k, int H_q, int H_kv) {
+    using namespace nv;
+    if (B <= 0 || total_q <= 0 || max_seqlen_q <= 0 || max_seqlen_k < 0 || H_q <= 0 || H_kv <= 0 || H_q % H_kv != 0) return 0;
+    const PrefillShape sh = prefill_shape(B, total_q, H_q, H_kv, max_seqlen_q, max_seqlen_k);
+    return sh.hand_scheduled ? sh.items_per_wg : 0;
 }
 
 extern "C" int nv_attn_prefill_varlen(const void* q, const void* k_cache, const void* v_cache,
