@@ -319,8 +319,7 @@ __global__ __launch_bounds__(128, FORM == kCrGeneral ? 2 : 3) void recurrence_ch
                 });
             put(lds.q, [&](int t, int i) { return qf(t, i) * lv[i][t]; });
             put(lds.right, [&](int t, int i) { return kf(t, i) * rv[i][t]; });
-            // pairs whose tokens part at this part (one compare and a select: branches here have come out of the compiler without
-            // their assignments)
+            // pairs whose tokens part at this part
             const bool middle = far == 0 || (far == 1 && part == 4);
             const uint32_t from = middle ? 0 : part, many = middle ? 2 * part : part ? part : 1;
             auto take = [&](f32x4& to, f32x4 of) {
