@@ -205,6 +205,10 @@ NV_API int nv_moe_tile_rows_for(int64_t pairs, int E, int width, int ff, const v
 NV_API int64_t nv_moe_max_tiles(int64_t pairs, int E, int tile_rows);
 NV_API int nv_moe_align(const int32_t* ids, int32_t* sorted_pairs, int32_t* meta, int64_t pairs, int E,
                         int tile_rows, void* stream);
+/* nv_moe_route and nv_moe_align together, counts: nv_moe_route_sort_words ints of scratch (NULL where that is 0). */
+NV_API int64_t nv_moe_route_sort_words(int64_t T, int E);
+NV_API int nv_moe_route_sort(const float* logits, int32_t* ids, float* weights, int32_t* sorted_pairs, int32_t* meta,
+                             int32_t* counts, int64_t T, int E, int top, int tile_rows, void* stream);
 NV_API int nv_moe_gate_up(const void* h, int64_t h_stride, const void* gate_up, const int32_t* sorted_pairs,
                           const int32_t* meta, void* y, int dtype, int64_t pairs, int E, int top, int width, int ff,
                           float limit, float alpha, int tile_rows, void* stream);

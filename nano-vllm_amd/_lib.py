@@ -96,6 +96,8 @@ MIXERS_PROTOTYPES = {
     "nv_moe_tile_rows": (_i32, [_i64, _i32]),
     "nv_moe_max_tiles": (_i64, [_i64, _i32, _i32]),
     "nv_moe_align": (_i32, [_vp, _vp, _vp, _i64, _i32, _i32, _vp]),
+    "nv_moe_route_sort_words": (_i64, [_i64, _i32]),
+    "nv_moe_route_sort": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp]),
     "nv_moe_gate_up": (_i32, [_vp, _i64, _vp, _vp, _vp, _vp, _i32, _i64, _i32, _i32, _i32, _i32, _f32, _f32, _i32, _vp]),
     "nv_moe_down": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _i32, _i32, _i32, _i32, _vp]),
     "nv_moe_gate_up_act": (_i32, [_vp, _i64, _vp, _vp, _vp, _vp, _i32, _i64, _i32, _i32, _i32, _i32, _f32, _f32, _f32, _i32,

@@ -823,13 +823,13 @@ def moe_experts(h: torch.Tensor, logits: torch.Tensor, gate_up: torch.Tensor, do
         return out
     hp, gp, dp = h.data_ptr(), gate_up.data_ptr(), down.data_ptr()
     rows = dll.nv_moe_tile_rows_for(P, E, W, ff, hp, h.stride(0), gp, dp, dt)
-    # ids, weights, sorted pairs and the table of tiles (words, each part on a cache line of its own) in one allocation
-    part = (P + 63) // 64 * 64
-    scratch = torch.empty(3 * part + 1 + 3 * dll.nv_moe_max_tiles(P, E, rows), dtype=torch.int32, device=dev)
+    # ids, weights, sorted pairs, the sort's counts and the table of tiles (words, each part on a cache line of its own) in one allocation
+    part, counted = (P + 63) // 64 * 64, (dll.nv_moe_route_sort_words(T, E) + 63) // 64 * 64
+    scratch = torch.empty(3 * part + counted + 1 + 3 * dll.nv_moe_max_tiles(P, E, rows), dtype=torch.int32, device=dev)
     ids = scratch.data_ptr()
-    wgt, sorted_pairs, meta = ids + 4 * part, ids + 8 * part, ids + 12 * part
-    _lib.check(dll.nv_moe_route(logits.data_ptr(), ids, wgt, T, E, int(top), s), "nv_moe_route", dll)
-    _lib.check(dll.nv_moe_align(ids, sorted_pairs, meta, P, E, rows, s), "nv_moe_align", dll)
+    wgt, sorted_pairs, counts = ids + 4 * part, ids + 8 * part, ids + 12 * part
+    meta = counts + 4 * counted
+    _lib.check(dll.nv_moe_route_sort(logits.data_ptr(), ids, wgt, sorted_pairs, meta, counts, T, E, int(top), rows, s), "nv_moe_route_sort", dll)
     y = torch.empty((P, ff), dtype=h.dtype, device=dev)
     yp = y.data_ptr()
     _lib.check(dll.nv_moe_gate_up(hp, h.stride(0), gp, sorted_pairs, meta, yp, dt, P, E, int(top), W, ff, float(limit), float(alpha), rows, s),
