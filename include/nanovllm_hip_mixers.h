@@ -190,16 +190,16 @@ NV_API int nv_latent_prep_store(const void* q, int64_t q_stride, int Dq, const v
 /*
  * Routed experts.  nv_moe_route: the `top` largest of every row of logits [T, E] (fp32), weights = softmax over the
  * chosen; ids / weights: [T, top].  nv_moe_align: sorted_pairs [pairs] = the (token, choice) pairs ordered by expert,
- * meta = [number of row tiles, then (expert, first position, rows) per tile], tiles of at most tile_rows (16, 64 or 128,
- * nv_moe_tile_rows suggests one) rows of one expert; meta holds 1 + 3 * nv_moe_max_tiles ints.  nv_moe_gate_up:
+ * meta = [number of row tiles, then (expert, first position, rows) per tile], tiles of at most tile_rows (16, 32, 64 or
+ * 128, nv_moe_tile_rows suggests one) rows of one expert; meta holds 1 + 3 * nv_moe_max_tiles ints.  nv_moe_gate_up:
  * y[position] = g * sigmoid(alpha g) * (u + 1), g = min(G_e h, limit), u = clamp(U_e h, -limit, limit), with
  * gate_up: [E, 2 ff, width] (gate rows, then up rows), y: [pairs, ff] of dtype.  nv_moe_down: out[pair] =
  * pair_weights[pair] * (D_e y[position]), down: [E, width, ff], out: [pairs, width] fp32.
  */
 NV_API int nv_moe_route(const float* logits, int32_t* ids, float* weights, int64_t T, int E, int top, void* stream);
 NV_API int nv_moe_tile_rows(int64_t pairs, int E);
-/* The same with 128 as a further answer, for bf16 rows and weights that the 128-row launches take (16-byte pieces, widths of
- * whole 64-deep slices); tile_rows = 128 is refused by the products otherwise.  up: the gate-up or up weights. */
+/* The same with 32 and 128 as further answers, for bf16 rows and weights in 16-byte pieces and widths of whole 64-deep slices;
+ * tile_rows = 32 and 128 are refused by the products otherwise.  up: the gate-up or up weights. */
 NV_API int nv_moe_tile_rows_for(int64_t pairs, int E, int width, int ff, const void* h, int64_t h_stride, const void* up,
                                 const void* down, int dtype);
 NV_API int64_t nv_moe_max_tiles(int64_t pairs, int E, int tile_rows);

@@ -14,7 +14,7 @@
 //                       the `top` rows of a token in a fixed order (no atomics, bitwise reproducible).
 //
 // Both products are one grouped matrix product on the matrix cores: a workgroup of four waves takes one row tile
-// (16 or 64 rows of ONE expert) and 64 or 128 output columns, stages 64-deep (fp32: 32-deep) slices of the rows and of the
+// (16 to 128 rows of ONE expert) and 64 or 128 output columns, stages 64-deep (fp32: 32-deep) slices of the rows and of the
 // expert's weight rows through LDS, the next slices already on their way into registers, and issues v_mfma_f32_16x16x32_bf16 (bfloat16) or v_mfma_f32_16x16x4_f32 (true fp32) on them; a
 // wave owns 16 or 32 columns and all row sub-tiles.  Weights are
 // [E, rows_out, rows_in] with the contraction index contiguous, as stored.  The launch is sized for the most tiles any
@@ -652,6 +652,138 @@ __global__ __launch_bounds__(256, 2) void moe_big_kernel(
     }
 }
 
+// Few rows per expert, bf16: bound by the expert's weights, which stream from memory straight into the operands of the matrix cores, past LDS.
+// A workgroup takes a tile of at most 16 MT rows and 64 weight rows (gate and up: 32 columns of both); its four waves take a quarter of the
+// contraction each and add their sums up in LDS, so that every wave has 16 KiB of weights on their way and a CU that holds two to
+// four workgroups 128 to 256 (the kernel below has 16 a workgroup).  Top 4 of 32 experts, width 2048, ff 1024, 32 tokens: gate and up 66 -> 48.5 us
+// (5.5 TB/s), down 28 -> 26.5 (5.1); the call with 1 token 47 -> 23.  Steps 32 deep for 64 rows, three workgroups a CU: 64 -> 75 us at 256 tokens.  Rows past the tile repeat its first one, weight rows past N the
+// last one; neither is written.
+template <int MODE, int MT>
+__global__ __launch_bounds__(256, MT == 1 ? 4 : MT == 2 ? 3 : 2) void moe_rows_kernel(
+    const __bf16* __restrict__ a, int64_t a_stride, const __bf16* __restrict__ w, const int* __restrict__ sorted_pairs,
+    const int* __restrict__ meta, const float* __restrict__ pair_w, __bf16* __restrict__ y, float* __restrict__ out, int top, int N,
+    int K, float limit, float alpha, float up_shift) {
+    constexpr bool GATE_UP = MODE == 1, GATHER = MODE != 0;
+    constexpr int NB = 4, COLS = GATE_UP ? 32 : 64;
+    __shared__ f32x4 part[MT > 1 ? 2 : 1][4][NB][64];
+    // An XCD takes a run of the items, the tiles of an expert next to each other: they read its weights once from memory.
+    const int tiles = meta[0], n_cols = (N + COLS - 1) / COLS, items = tiles * n_cols, per_xcd = (items + 7) / 8, at = blockIdx.x / 8;
+    const int item = (blockIdx.x & 7) * per_xcd + at;
+    if (at >= per_xcd || item >= items) return;
+    const int tile = item % tiles, n0 = (item / tiles) * COLS;
+    const int e = meta[1 + 3 * tile], row0 = meta[2 + 3 * tile], rows = meta[3 + 3 * tile];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, g = lane >> 4;
+    const int steps = K / 64, per = (steps + 3) / 4, s0 = min(wave * per, steps), s1 = min(s0 + per, steps);
+    const __bf16* we = w + (int64_t)e * ((GATE_UP ? 2 : 1) * (int64_t)N) * K + s0 * 64 + 8 * g;
+    const __bf16 *wp[NB], *xp[MT];
+    int src[MT];                                      // on its way in front of the weights, which do not need it
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        src[m] = row0 + (m * 16 + l16 < rows ? m * 16 + l16 : 0);
+        if constexpr (GATHER) src[m] = sorted_pairs[src[m]];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        const int64_t n = GATE_UP ? (j >> 1) * (int64_t)N + min(n0 + (j & 1) * 16 + l16, N - 1) : min(n0 + j * 16 + l16, N - 1);
+        wp[j] = we + n * K;
+    }
+    f32x4 acc[MT][NB];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[m][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int D = 2;                              // a step: 64 deep, whole cache lines of every row
+    struct Step {
+        bf16x8 w[NB][D], x[MT][D];
+    };
+    auto load_w = [&](Step& f) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+#pragma unroll
+            for (int i = 0; i < D; ++i) f.w[j][i] = *(const bf16x8*)(wp[j] + i * 32);
+            wp[j] += 32 * D;
+        }
+    };
+    auto load_x = [&](Step& f) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+#pragma unroll
+            for (int i = 0; i < D; ++i) f.x[m][i] = *(const bf16x8*)(xp[m] + i * 32);
+            xp[m] += 32 * D;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto load = [&](Step& f) {
+        load_w(f);
+        load_x(f);
+    };
+    auto multiply = [&](const Step& f) {
+#pragma unroll
+        for (int i = 0; i < D; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+#pragma unroll
+                for (int m = 0; m < MT; ++m) acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[j][i], f.x[m][i], acc[m][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    Step f0, f1;
+    int n = (s1 - s0) * (2 / D);
+    if (n > 0) load_w(f0);
+    if (n > 1) load_w(f1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) xp[m] = a + (int64_t)(GATHER ? src[m] / top : src[m]) * a_stride + s0 * 64 + 8 * g;
+    if (n > 0) load_x(f0);
+    if (n > 1) load_x(f1);
+#pragma unroll 1
+    for (; n > 3; n -= 2) {
+        multiply(f0);
+        load(f0);
+        multiply(f1);
+        load(f1);
+    }
+    if (n > 0) multiply(f0);
+    if (n > 2) load(f0);
+    if (n > 1) multiply(f1);
+    if (n > 2) multiply(f0);
+    // lane (l16, g) holds of row 16 m + l16 the weight rows 4 g + i of each block
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        if (m > 0 && m * 16 >= rows) break;           // (for the whole workgroup)
+        auto& p = part[MT > 1 ? m & 1 : 0];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) p[wave][j][lane] = acc[m][j];
+        __syncthreads();                              // (the buffer's last reads lie in front of the barrier before)
+        auto sum = [&](int j) { return (p[0][j][lane] + p[1][j][lane]) + (p[2][j][lane] + p[3][j][lane]); };
+        const int r = m * 16 + l16, c = n0 + (GATE_UP ? wave & 1 : wave) * 16 + 4 * g;
+        const bool live = r < rows && c < N && (!GATE_UP || wave < 2);
+        if (!live) {
+        } else if constexpr (GATE_UP) {
+            const f32x4 gs = sum(wave), us = sum(wave + 2);
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float gg = fminf(gs[i], limit), u = fminf(fmaxf(us[i], -limit), limit);
+                v[i] = gg / (1.0f + expf(-alpha * gg)) * (u + up_shift);
+            }
+            *(uint2*)(y + (int64_t)(row0 + r) * N + c) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+        } else if constexpr (MODE == 2) {
+            const f32x4 us = sum(wave);
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float u = fmaxf(us[i], 0.f);
+                v[i] = u * u;
+            }
+            *(uint2*)(y + (int64_t)(row0 + r) * N + c) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+        } else {
+            const int pair = sorted_pairs[row0 + r];
+            *(f32x4*)(out + (int64_t)pair * N + c) = sum(wave) * pair_w[pair];
+        }
+    }
+}
+
 // MODE 1 (gate and up): A rows are gathered token rows, B holds the expert's gate rows and up rows, the epilogue is the
 //         gated activation.
 // MODE 2 (up alone):   A rows are gathered token rows, B the expert's up rows, the epilogue is max(x, 0)^2.
@@ -762,6 +894,14 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(
     }
 }
 
+// Tiles of 128 rows and of few rows take whole 64-deep slices and 16-byte pieces of both operands' rows, and of the result's.
+static bool moe_big_ok(int dtype, const void* a, int64_t a_stride, const void* w, int N, int K) {
+    return dtype == NV_DTYPE_BF16 && K % 64 == 0 && N % 8 == 0 && a_stride % 8 == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0;
+}
+static bool moe_rows_ok(const void* result, const void* a, int64_t a_stride, const void* w, int N, int K) {
+    return (uintptr_t)result % 16 == 0 && moe_big_ok(NV_DTYPE_BF16, a, a_stride, w, N, K);
+}
+
 template <typename T, int MODE>
 static void launch_grouped(const void* a, int64_t a_stride, const void* w, const int* sorted_pairs, const int* meta,
                            const float* pair_w, void* y, float* out, int top, int N, int K, float limit, float alpha,
@@ -771,6 +911,19 @@ static void launch_grouped(const void* a, int64_t a_stride, const void* w, const
             constexpr int cols = MODE == 1 ? 128 : 256;
             hipLaunchKernelGGL(moe_big_kernel<MODE>, dim3((unsigned)(((int64_t)max_tiles * ((N + cols - 1) / cols) + 7) / 8 * 8)), dim3(256), 0, s,
                                (const T*)a, a_stride, (const T*)w, sorted_pairs, meta, pair_w, (T*)y, out, top, N, K, limit, alpha, up_shift);
+            return;
+        }
+    }
+    if constexpr (sizeof(T) == 2) {
+        if (moe_rows_ok(MODE == 0 ? (const void*)out : y, a, a_stride, w, N, K)) {
+            const int64_t items = (int64_t)max_tiles * ((N + (MODE == 1 ? 31 : 63)) / (MODE == 1 ? 32 : 64));
+#define NV_MOE_ROWS(MT)                                                                                                              \
+    hipLaunchKernelGGL((moe_rows_kernel<MODE, MT>), dim3((unsigned)((items + 7) / 8 * 8)), dim3(256), 0, s, (const T*)a, a_stride, (const T*)w, \
+                       sorted_pairs, meta, pair_w, (T*)y, out, top, N, K, limit, alpha, up_shift)
+            if (tile_rows == 64) NV_MOE_ROWS(4);
+            else if (tile_rows == 32) NV_MOE_ROWS(2);
+            else NV_MOE_ROWS(1);
+#undef NV_MOE_ROWS
             return;
         }
     }
@@ -806,25 +959,29 @@ extern "C" int nv_moe_route(const float* logits, int32_t* ids, float* weights, i
 
 extern "C" int nv_moe_tile_rows(int64_t pairs, int E) { return pairs >= 32 * (int64_t)E ? 64 : 16; }
 
-// Rows of 128 take pairs of whole 32-deep slices and 16-byte pieces of both products' rows.
-static bool moe_big_ok(int dtype, const void* a, int64_t a_stride, const void* w, int N, int K) {
-    return dtype == NV_DTYPE_BF16 && K % 64 == 0 && N % 8 == 0 && a_stride % 8 == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0;
-}
-
-// 128 rows from 96 per expert on, where they win at every size measured.  Whole calls, top 4 of 32 experts, tiles of 64 against
-// 128 rows: width 2048, ff 1024: 48 pairs an expert 128 / 123 us, 80: 137 / 130, 96: 141 / 128, 112: 173 / 172, 192: 217 / 160;
-// width 1024, ff 2048: 48: 119 / 123, 64: 127 / 124, 96: 145 / 128, 112: 153 / 144, 192: 195 / 157.
+// By pairs per expert: tiles of 16 rows below 8, of 32 below 24, of 64 (all of these stream the weights past LDS, which costs little more with
+// more rows a tile and saves the second reading of an expert that has more), then of 128 staged through LDS, which wants enough of its
+// 128 x 256 blocks to fill the chip.  Whole calls, us, tiles of 16 / 32 / 64 / 128 rows:
+//   top 4 of 32 experts, width 2048, ff 1024:  6 pairs an expert 83 / 86 / 89 / 108, 16: 107 / 96 / 101 / 113, 24: 134 / 107 / 108 / 115,
+//   32: 149 / 121 / 113 / 116, 40: 174 / 142 / 118 / 119, 64: 252 / 178 / 156 / 122 (blocks of 64 x 128 through LDS took 117 to 141 for all of these)
+//   top 2 of 32, 1024, 1024:  16: 53 / 48 / 51 / 54, 32: 78 / 63 / 57 / 56, 48: 105 / 79 / 65 / 59
+//   top 2 of 16, 1024, 512:  6: 18 / 18 / 20 / 38, 24: 27 / 29 / 25 / 42, 64: 47 / 39 / 38 / 46, 96: 61 / 52 / 40 / 47, 128: 73 / 58 / 59 / 49
+//   top 4 of 16, 2048, 512:  12: 36 / 30 / 30 / 53, 48: 66 / 51 / 39 / 59, 96: 104 / 83 / 64 / 63
+// tiles of 64 / 128 rows:  top 2 of 16, 2048, 1024:  48: 60 / 67, 64: 94 / 68;  top 4 of 32, 1024, 512:  40: 42 / 47, 48: 51 / 47
 extern "C" int nv_moe_tile_rows_for(int64_t pairs, int E, int width, int ff, const void* h, int64_t h_stride, const void* up,
                                     const void* down, int dtype) {
-    const bool big = pairs >= 96 * (int64_t)E && moe_big_ok(dtype, h, h_stride, up, ff, width) && moe_big_ok(dtype, down, ff, down, width, ff);
-    return big ? nv::kMoeBigRows : nv_moe_tile_rows(pairs, E);
+    using namespace nv;
+    if (!moe_big_ok(dtype, h, h_stride, up, ff, width) || !moe_big_ok(dtype, down, ff, down, width, ff)) return nv_moe_tile_rows(pairs, E);
+    const int64_t blocks = (int64_t)E * ((ff + 127) / 128);           // of the first product, a tile an expert
+    if (pairs >= (blocks >= 256 ? 40 : blocks >= 128 ? 48 : 96) * (int64_t)E) return kMoeBigRows;
+    return pairs >= 24 * (int64_t)E ? 64 : pairs >= 8 * (int64_t)E ? 32 : 16;
 }
 
 extern "C" int64_t nv_moe_max_tiles(int64_t pairs, int E, int tile_rows) {
     return pairs / tile_rows + std::min<int64_t>(pairs, E);
 }
 
-static bool moe_tile_ok(int rows) { return rows == 16 || rows == 64 || rows == 128; }
+static bool moe_tile_ok(int rows) { return rows == 16 || rows == 32 || rows == 64 || rows == 128; }
 
 extern "C" int nv_moe_align(const int32_t* ids, int32_t* sorted_pairs, int32_t* meta, int64_t pairs, int E,
                             int tile_rows, void* stream) {
@@ -857,7 +1014,7 @@ extern "C" int nv_moe_route_sort(const float* logits, int32_t* ids, float* weigh
                                  int64_t T, int E, int top, int tile_rows, void* stream) {
     using namespace nv;
     NV_REQUIRE(T >= 0 && E > 0 && top >= 1 && top <= E && top <= kMoeMaxTop && moe_tile_ok(tile_rows), NV_ERR_INVALID_ARG,
-               "nv_moe_route_sort: top=%d must lie in 1 .. min(E=%d, %d), tiles have 16, 64 or 128 rows", top, E, kMoeMaxTop);
+               "nv_moe_route_sort: top=%d must lie in 1 .. min(E=%d, %d), tiles have 16, 32, 64 or 128 rows", top, E, kMoeMaxTop);
     if (T == 0 || E > kMoeSortMaxE) {
         const int rc = nv_moe_route(logits, ids, weights, T, E, top, stream);
         return rc != NV_OK ? rc : nv_moe_align(ids, sorted_pairs, meta, T * top, E, tile_rows, stream);
@@ -900,8 +1057,8 @@ extern "C" int nv_moe_gate_up_act(const void* h, int64_t h_stride, const void* g
     if (pairs == 0) return NV_OK;
     NV_REQUIRE(h && gate_up && sorted_pairs && meta && y, NV_ERR_INVALID_ARG, "nv_moe_gate_up: null pointer");
     NV_REQUIRE(dtype == NV_DTYPE_BF16 || dtype == NV_DTYPE_F32, NV_ERR_INVALID_ARG, "nv_moe_gate_up: bad dtype");
-    NV_REQUIRE(tile_rows != 128 || ((uintptr_t)y % 16 == 0 && moe_big_ok(dtype, h, h_stride, gate_up, ff, width)), NV_ERR_UNSUPPORTED,
-               "nv_moe_gate_up: tiles of 128 rows take bf16 rows in whole pieces");
+    NV_REQUIRE((tile_rows != 128 && tile_rows != 32) || ((uintptr_t)y % 16 == 0 && moe_big_ok(dtype, h, h_stride, gate_up, ff, width)), NV_ERR_UNSUPPORTED,
+               "nv_moe_gate_up: tiles of 32 or 128 rows take bf16 rows in whole pieces");
     const int64_t tiles = nv_moe_max_tiles(pairs, E, tile_rows);
     NV_REQUIRE(tiles * ((ff + kMoeBN - 1) / kMoeBN) < (1LL << 31), NV_ERR_UNSUPPORTED, "nv_moe_gate_up: launch too large");
     hipStream_t s = (hipStream_t)stream;
@@ -923,8 +1080,8 @@ extern "C" int nv_moe_down(const void* y, const void* down, const int32_t* sorte
     if (pairs == 0) return NV_OK;
     NV_REQUIRE(y && down && sorted_pairs && meta && pair_weights && out, NV_ERR_INVALID_ARG, "nv_moe_down: null pointer");
     NV_REQUIRE(dtype == NV_DTYPE_BF16 || dtype == NV_DTYPE_F32, NV_ERR_INVALID_ARG, "nv_moe_down: bad dtype");
-    NV_REQUIRE(tile_rows != 128 || ((uintptr_t)out % 16 == 0 && moe_big_ok(dtype, y, ff, down, width, ff)), NV_ERR_UNSUPPORTED,
-               "nv_moe_down: tiles of 128 rows take bf16 rows in whole pieces");
+    NV_REQUIRE((tile_rows != 128 && tile_rows != 32) || ((uintptr_t)out % 16 == 0 && moe_big_ok(dtype, y, ff, down, width, ff)), NV_ERR_UNSUPPORTED,
+               "nv_moe_down: tiles of 32 or 128 rows take bf16 rows in whole pieces");
     const int64_t tiles = nv_moe_max_tiles(pairs, E, tile_rows);
     NV_REQUIRE(tiles * ((width + kMoeBN - 1) / kMoeBN) < (1LL << 31), NV_ERR_UNSUPPORTED, "nv_moe_down: launch too large");
     hipStream_t s = (hipStream_t)stream;
@@ -963,8 +1120,8 @@ extern "C" int nv_moe_up_relu2(const void* h, int64_t h_stride, const void* up, 
     if (pairs == 0) return NV_OK;
     NV_REQUIRE(h && up && sorted_pairs && meta && y, NV_ERR_INVALID_ARG, "nv_moe_up_relu2: null pointer");
     NV_REQUIRE(dtype == NV_DTYPE_BF16 || dtype == NV_DTYPE_F32, NV_ERR_INVALID_ARG, "nv_moe_up_relu2: bad dtype");
-    NV_REQUIRE(tile_rows != 128 || ((uintptr_t)y % 16 == 0 && moe_big_ok(dtype, h, h_stride, up, ff, width)), NV_ERR_UNSUPPORTED,
-               "nv_moe_up_relu2: tiles of 128 rows take bf16 rows in whole pieces");
+    NV_REQUIRE((tile_rows != 128 && tile_rows != 32) || ((uintptr_t)y % 16 == 0 && moe_big_ok(dtype, h, h_stride, up, ff, width)), NV_ERR_UNSUPPORTED,
+               "nv_moe_up_relu2: tiles of 32 or 128 rows take bf16 rows in whole pieces");
     const int64_t tiles = nv_moe_max_tiles(pairs, E, tile_rows);
     NV_REQUIRE(tiles * ((ff + kMoeBN - 1) / kMoeBN) < (1LL << 31), NV_ERR_UNSUPPORTED, "nv_moe_up_relu2: launch too large");
     hipStream_t s = (hipStream_t)stream;
