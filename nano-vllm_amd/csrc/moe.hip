@@ -466,27 +466,36 @@ __global__ __launch_bounds__(256) void moe_place_kernel(const int* __restrict__ 
 
 // Many rows per expert, bf16: a workgroup of four waves takes 128 rows of one expert and 256 weight rows (gate and up: 128 columns of
 // both), a wave 64 x 128 of it on v_mfma_f32_32x32x16_bf16 (weights as the first operand, so that a lane holds four neighbouring
-// columns of a row).  Slices 32 deep go straight into LDS (LDS-DMA, chunks swizzled by row so that the 16-byte operand reads are free
-// of bank conflicts); two workgroups share a CU, so that one's products cover the other's barrier, first loads and epilogue.
-// 64 x 128 a wave, because LDS reads come next: 6 KiB for 8 MFMAs of 32 cycles, three quarters of what a CU's LDS delivers; 64 x 64
-// would take all of it.  Rows past the tile repeat its first one, weight rows past N the last one; neither is written.
-// What bounds it: the latency of the slices.  Three buffers, two slices in flight, and one LDS object per buffer: with one array the
-// compiler waits for the loads just issued before it reads another buffer (656 us for the whole call below with two halves of one
-// array, 619 with two objects, 590 .. 605 with three).  Slices 64 deep, one workgroup a CU: 642 us.
-// 8192 tokens, top 4 of 32 experts, width 2048, ff 1024: gate and up 433 -> 338 us, down 354 -> 240 us (the tiles of 64 x 128 below,
-// which other sizes still take, against these); the call 780 -> 600 us.
+// columns of a row).  Slices 64 deep, whole cache lines of every row, go straight into LDS (LDS-DMA, chunks swizzled by row so that the
+// 16-byte operand reads are free of bank conflicts).  A wave reads all operands of its slice into registers; the next slice then goes into the same
+// 48 KiB while it multiplies, and the other workgroup of the CU has its turn at LDS.  Rows past the tile repeat its first one, weight rows past N the last
+// ones; neither is written.
+// What bounds it: the way of the slices from L2 (11 TB/s through the CUs' vector caches).  Slices 32 deep take half a cache line of every row
+// and the same line again for the next slice: 340 and 240 us for both products of the call below, with three buffers and two slices in
+// flight.  Without any loads behind the first slice it is 217 and 136 us, with all of them in the vector caches 226 and 145, in L2 263 and 160.
+// Buffer loads, because the compiler waits for all LDS reads behind a global load into LDS (and has no 64-bit addresses to add up): 336 -> 281
+// us; the products at a higher priority than the other workgroup's reads: 299 -> 281.  256 x 256 by one workgroup a CU, two buffers: four
+// waves of 128 x 128 319 and 211 us, eight of 64 x 128 349 and 220; a load of the lines two slices ahead into L2: no gain.
+// 8192 tokens, top 4 of 32 experts, width 2048, ff 1024: gate and up 340 -> 281 us, down 240 -> 187; the call 583 -> 497.
 constexpr int kMoeBigRows = 128;
-__device__ __forceinline__ int big_off(int row, int ch) { return row * 64 + ((ch ^ ((row >> 2) & 3)) * 16); }
 
+// g * sigmoid(alpha g) * (u + shift) on the hardware's exponential and reciprocal (one unit in the last place each, in front of a rounding to
+// bf16): expf and a division are 45 instructions a value, 10 us a 256 x 256 block.
+__device__ __forceinline__ float moe_glu(float g, float u, float alpha, float shift) {
+    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * (-1.4426950408889634f * alpha))) * (u + shift);
+}
+
+__device__ __forceinline__ int big_off(int row, int ch) { return row * 128 + ((ch ^ ((row >> 1) & 7)) * 16); }
 template <int MODE>
 __global__ __launch_bounds__(256, 2) void moe_big_kernel(
     const __bf16* __restrict__ a, int64_t a_stride, const __bf16* __restrict__ w, const int* __restrict__ sorted_pairs,
     const int* __restrict__ meta, const float* __restrict__ pair_w, __bf16* __restrict__ y, float* __restrict__ out, int top, int N,
     int K, float limit, float alpha, float up_shift) {
     constexpr bool GATE_UP = MODE == 1, GATHER = MODE != 0;
-    constexpr int COLS = GATE_UP ? 128 : 256, XB = kMoeBigRows * 64, BUF = XB + 256 * 64;       // bytes: rows' slice, both slices
-    __shared__ __attribute__((aligned(16))) unsigned char buf0[BUF], buf1[BUF], buf2[BUF];
+    constexpr int COLS = GATE_UP ? 128 : 256, XB = kMoeBigRows * 128;       // bytes: rows' slice
+    __shared__ __attribute__((aligned(16))) unsigned char buf[XB + 256 * 128];
     __shared__ int src_row[kMoeBigRows];
+    __shared__ float weight[MODE == 0 ? kMoeBigRows : 1];
     // Workgroups go to the eight XCDs in turn; an XCD takes a run of the tiles that there are, all column blocks of a tile next to each
     // other: its L2 then holds a tile's rows for all of them and an expert's weights for its tiles (tiles next to each other instead:
     // no difference at the call above).
@@ -497,37 +506,39 @@ __global__ __launch_bounds__(256, 2) void moe_big_kernel(
     const int e = meta[1 + 3 * tile], row0 = meta[2 + 3 * tile], rows = meta[3 + 3 * tile];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, hh = lane >> 5, wr = wave >> 1, wc = wave & 1;
-    for (int i = tid; i < kMoeBigRows; i += 256) src_row[i] = sorted_pairs[row0 + min(i, rows - 1)];
+    for (int i = tid; i < kMoeBigRows; i += 256) {
+        src_row[i] = sorted_pairs[row0 + min(i, rows - 1)];
+        if constexpr (MODE == 0) weight[i] = pair_w[src_row[i]];
+    }
     __syncthreads();
     const __bf16* we = w + (int64_t)e * ((GATE_UP ? 2 : 1) * (int64_t)N) * K;
-    // a piece of 1 KiB: 16 rows of 64 bytes, lane l fills bytes 16 l .. of it
-    const int p_row = lane >> 2, p_ch = (lane & 3) ^ ((p_row >> 2) & 3);
-    const char *xp[2], *wp[4];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int r = (wave * 2 + i) * 16 + p_row;
-        const int64_t at = GATHER ? (int64_t)(src_row[r] / top) : row0 + min(r, rows - 1);
-        xp[i] = (const char*)(a + at * a_stride + p_ch * 8);
-    }
+    // a piece of 1 KiB: 8 rows of 128 bytes, lane l fills bytes 16 l .. of it; a wave takes four of the rows and eight of the weight rows
+    const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(GATHER ? a : a + (int64_t)row0 * a_stride), 0, -1, 0x00020000);
+    const auto wr_ = __builtin_amdgcn_make_buffer_rsrc((void*)we, 0, -1, 0x00020000);
+    const int p_row = lane >> 3;
+    uint32_t x_lane[4], w_lane[2], w_piece[8];        // (the launch keeps all offsets below 4 GiB)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int lr = (wave * 4 + i) * 16 + p_row;   // weight row of the workgroup: gate rows, then up rows
-        const int64_t n = GATE_UP ? (lr >> 7) * (int64_t)N + min(n0 + (lr & 127), N - 1) : min(n0 + lr, N - 1);
-        wp[i] = (const char*)(we + n * K + p_ch * 8);
+        const int r = (wave * 4 + i) * 8 + p_row;
+        x_lane[i] = ((uint32_t)(GATHER ? src_row[r] / top : min(r, rows - 1)) * (uint32_t)a_stride + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2u;
     }
-    auto stage = [&](unsigned char* dst) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)xp[i],
-                                             (__attribute__((address_space(3))) void*)(dst + (wave * 2 + i) * 1024), 16, 0, 0);
-            xp[i] += 64;
-        }
+    for (int i = 0; i < 2; ++i) w_lane[i] = (uint32_t)(p_row * K + ((lane & 7) ^ (i * 4 + (p_row >> 1))) * 8) * 2u;
+    // (N is a multiple of 8: a piece's weight rows are all there or none of them is)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)wp[i],
-                                             (__attribute__((address_space(3))) void*)(dst + XB + (wave * 4 + i) * 1024), 16, 0, 0);
-            wp[i] += 64;
-        }
+    for (int i = 0; i < 8; ++i) {
+        const int lr = (wave * 8 + i) * 8;            // first weight row of the piece: gate rows, then up rows
+        w_piece[i] = (uint32_t)(GATE_UP ? (lr >> 7) * N + min(n0 + (lr & 127), N - 8) : min(n0 + lr, N - 8)) * (uint32_t)K * 2u;
+    }
+    auto stage = [&](int t) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(wr_, (__attribute__((address_space(3))) void*)(buf + XB + (wave * 8 + i) * 1024), 16,
+                                                     w_lane[i & 1], w_piece[i] + t * 128, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(buf + (wave * 4 + i) * 1024), 16, x_lane[i],
+                                                     t * 128, 0, 0);
     };
     f32x16 acc[4][2];                                 // [weight block: gate 0, 1, up 0, 1 | 0 .. 3][row block]
 #pragma unroll
@@ -536,60 +547,52 @@ __global__ __launch_bounds__(256, 2) void moe_big_kernel(
         for (int x = 0; x < 2; ++x)
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[j][x][i] = 0.f;
-    auto multiply = [&](const unsigned char* xs) {
-        const unsigned char* ws = xs + XB;
-        bf16x8 xf[2][2], wf[2][4];                    // all operands of the slice are on their way before the first product
+    bf16x8 xf[4][2], wf[4][4];                        // operands of the four 16-deep steps of a slice
+    auto read = [&](int s) {
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
+        for (int x = 0; x < 2; ++x) xf[s][x] = *(const bf16x8*)(buf + big_off(wr * 64 + x * 32 + l32, 2 * s + hh));
 #pragma unroll
-            for (int x = 0; x < 2; ++x) xf[s][x] = *(const bf16x8*)(xs + big_off(wr * 64 + x * 32 + l32, 2 * s + hh));
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int lr = GATE_UP ? (j >> 1) * 128 + wc * 64 + (j & 1) * 32 : wc * 128 + j * 32;
-                wf[s][j] = *(const bf16x8*)(ws + big_off(lr + l32, 2 * s + hh));
-            }
+        for (int j = 0; j < 4; ++j) {
+            const int lr = GATE_UP ? (j >> 1) * 128 + wc * 64 + (j & 1) * 32 : wc * 128 + j * 32;
+            wf[s][j] = *(const bf16x8*)(buf + XB + big_off(lr + l32, 2 * s + hh));
         }
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int x = 0; x < 2; ++x) acc[j][x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[s][j], xf[s][x], acc[j][x], 0, 0, 0);
     };
-    // One slice: this wave's part of it has landed (all but the newest `flying` loads have) and the wave is done reading the one
-    // before; past the barrier so it is for all waves, and the slice after the next one goes where the one before was.
-    // (The builtin, which the compiler's own count of loads in flight follows; __syncthreads would wait for all of them.)
-    auto step = [&](bool more, bool stages, const unsigned char* now, unsigned char* after_next) {
+    auto multiply = [&](int s) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int x = 0; x < 2; ++x) acc[j][x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[s][j], xf[s][x], acc[j][x], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const int slices = K / 64;
+    stage(0);
+    for (int t = 0; t < slices; ++t) {
         asm volatile("" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);            // (nor may the products sink below the wait)
-        if (more) __builtin_amdgcn_s_waitcnt(0x76);   // vmcnt(6) lgkmcnt(0): the six of the next slice stay in flight
-        else __builtin_amdgcn_s_waitcnt(0x70);        // vmcnt(0) lgkmcnt(0)
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0x70);             // vmcnt(0) lgkmcnt(0): this wave's part of the slice has landed
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (stages) stage(after_next);
-        __builtin_amdgcn_sched_barrier(0);            // (the compiler would start the loads behind the products)
-        multiply(now);
-    };
-    const int slices = K / 32;                        // at least 2 (K is a multiple of 64)
-    stage(buf0);
-    stage(buf1);
-    int t = 0;
-    for (; t + 4 < slices; t += 3) {
-        step(true, true, buf0, buf2);
-        step(true, true, buf1, buf0);
-        step(true, true, buf2, buf1);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) read(s);
+        if (t + 1 < slices) {
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0xc07f);       // lgkmcnt(0): the wave has read the slice
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            stage(t + 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) multiply(s);
+        __builtin_amdgcn_s_setprio(0);
     }
-    const int left = slices - t;                      // 2 .. 4
-    step(true, left > 2, buf0, buf2);
-    step(left > 2, left > 3, buf1, buf0);
-    if (left > 2) step(left > 3, false, buf2, buf1);
-    if (left > 3) step(false, false, buf0, buf2);
     __syncthreads();                                  // the slices are done with: each wave turns its blocks through LDS of its own
     // lane (l32, hh) holds of row 64 wr + 32 x + l32 the weight rows 8 (i >> 2) + 4 hh + (i & 3) of each block
     if constexpr (MODE != 0) {
         constexpr int CW = GATE_UP ? 64 : 128, LD = CW * 2 + 16;       // columns of the wave; bytes of a staged row
-        unsigned char* st = (wave < 2 ? buf0 : buf1) + (wave & 1) * 32 * LD;
+        unsigned char* st = buf + wave * 32 * LD;
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
 #pragma unroll
@@ -602,7 +605,7 @@ __global__ __launch_bounds__(256, 2) void moe_big_kernel(
                         if constexpr (GATE_UP) {
                             const float g = fminf(acc[j][x][i + t], limit);
                             const float u = fminf(fmaxf(acc[j + 2][x][i + t], -limit), limit);
-                            v[t] = g / (1.0f + expf(-alpha * g)) * (u + up_shift);
+                            v[t] = moe_glu(g, u, alpha, up_shift);
                         } else {
                             const float u = fmaxf(acc[j][x][i + t], 0.f);
                             v[t] = u * u;
@@ -622,7 +625,7 @@ __global__ __launch_bounds__(256, 2) void moe_big_kernel(
         }
     } else {
         constexpr int LD = 64 * 4 + 16;
-        unsigned char* st = (wave < 2 ? buf0 : buf1) + (wave & 1) * 32 * LD;
+        unsigned char* st = buf + wave * 32 * LD;
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
 #pragma unroll
@@ -641,7 +644,7 @@ __global__ __launch_bounds__(256, 2) void moe_big_kernel(
                     float4 v = *(const float4*)(st + rr * LD + c * 4);
                     if (r < rows && n < N) {
                         const int pair = src_row[r];
-                        const float f = pair_w[pair];
+                        const float f = weight[r];
                         v.x *= f; v.y *= f; v.z *= f; v.w *= f;
                         *(float4*)(out + (int64_t)pair * N + n) = v;
                     }
@@ -902,12 +905,18 @@ static bool moe_rows_ok(const void* result, const void* a, int64_t a_stride, con
     return (uintptr_t)result % 16 == 0 && moe_big_ok(NV_DTYPE_BF16, a, a_stride, w, N, K);
 }
 
+// A block's offsets from the first row and from the expert's first weight row, in bytes, are 32 bits (tiles of 128 rows beyond that, an input or an
+// expert's matrix of 4 GiB, take the general launch).
+static bool moe_offsets_ok(int64_t a_rows, int64_t a_stride, int64_t w_rows, int K) {
+    return a_rows * a_stride < (1LL << 31) - K && w_rows * K < (1LL << 31) - K;
+}
+
 template <typename T, int MODE>
 static void launch_grouped(const void* a, int64_t a_stride, const void* w, const int* sorted_pairs, const int* meta,
                            const float* pair_w, void* y, float* out, int top, int N, int K, float limit, float alpha,
-                           float up_shift, int max_tiles, int tile_rows, hipStream_t s) {
+                           float up_shift, int max_tiles, int tile_rows, int64_t a_rows, hipStream_t s) {
     if constexpr (sizeof(T) == 2) {
-        if (tile_rows == kMoeBigRows) {               // (the caller has checked sizes and alignment)
+        if (tile_rows == kMoeBigRows && moe_offsets_ok(MODE == 0 ? kMoeBigRows : a_rows, a_stride, (MODE == 1 ? 2 : 1) * (int64_t)N, K)) {               // (the caller has checked sizes and alignment)
             constexpr int cols = MODE == 1 ? 128 : 256;
             hipLaunchKernelGGL(moe_big_kernel<MODE>, dim3((unsigned)(((int64_t)max_tiles * ((N + cols - 1) / cols) + 7) / 8 * 8)), dim3(256), 0, s,
                                (const T*)a, a_stride, (const T*)w, sorted_pairs, meta, pair_w, (T*)y, out, top, N, K, limit, alpha, up_shift);
@@ -915,7 +924,7 @@ static void launch_grouped(const void* a, int64_t a_stride, const void* w, const
         }
     }
     if constexpr (sizeof(T) == 2) {
-        if (moe_rows_ok(MODE == 0 ? (const void*)out : y, a, a_stride, w, N, K)) {
+        if (tile_rows < kMoeBigRows && moe_rows_ok(MODE == 0 ? (const void*)out : y, a, a_stride, w, N, K)) {
             const int64_t items = (int64_t)max_tiles * ((N + (MODE == 1 ? 31 : 63)) / (MODE == 1 ? 32 : 64));
 #define NV_MOE_ROWS(MT)                                                                                                              \
     hipLaunchKernelGGL((moe_rows_kernel<MODE, MT>), dim3((unsigned)((items + 7) / 8 * 8)), dim3(256), 0, s, (const T*)a, a_stride, (const T*)w, \
@@ -935,6 +944,12 @@ static void launch_grouped(const void* a, int64_t a_stride, const void* w, const
     hipLaunchKernelGGL((moe_grouped_kernel<T, MT, NT, MODE>), dim3((unsigned)(max_tiles * ((N + 64 * NT - 1) / (64 * NT)))), \
                        dim3(256), 0, s, (const T*)a, a_stride, (const T*)w, sorted_pairs, meta, pair_w, (T*)y, out, top, N, K,  \
                        limit, alpha, up_shift, vec_ok, max_tiles)
+    if constexpr (sizeof(T) == 2) {
+        if (tile_rows == kMoeBigRows) {
+            NV_MOE_LAUNCH(8, 1);
+            return;
+        }
+    }
     if (tile_rows == 64 && sizeof(T) == 2) NV_MOE_LAUNCH(4, 2);
     else if (tile_rows == 64) NV_MOE_LAUNCH(4, 1);
     else NV_MOE_LAUNCH(1, 1);
@@ -962,18 +977,18 @@ extern "C" int nv_moe_tile_rows(int64_t pairs, int E) { return pairs >= 32 * (in
 // By pairs per expert: tiles of 16 rows below 8, of 32 below 24, of 64 (all of these stream the weights past LDS, which costs little more with
 // more rows a tile and saves the second reading of an expert that has more), then of 128 staged through LDS, which wants enough of its
 // 128 x 256 blocks to fill the chip.  Whole calls, us, tiles of 16 / 32 / 64 / 128 rows:
-//   top 4 of 32 experts, width 2048, ff 1024:  6 pairs an expert 83 / 86 / 89 / 108, 16: 107 / 96 / 101 / 113, 24: 134 / 107 / 108 / 115,
-//   32: 149 / 121 / 113 / 116, 40: 174 / 142 / 118 / 119, 64: 252 / 178 / 156 / 122 (blocks of 64 x 128 through LDS took 117 to 141 for all of these)
+//   top 4 of 32 experts, width 2048, ff 1024:  6 pairs an expert 83 / 86 / 89 / 108, 16: 107 / 96 / 101 / 113, 24: 134 / 107 / 105 / 115,
+//   32: 149 / 121 / 112 / 116, 40: 174 / 142 / 118 / 117, 64: 252 / 178 / 156 / 123 (blocks of 64 x 128 through LDS took 117 to 141 for all of these)
 //   top 2 of 32, 1024, 1024:  16: 53 / 48 / 51 / 54, 32: 78 / 63 / 57 / 56, 48: 105 / 79 / 65 / 59
-//   top 2 of 16, 1024, 512:  6: 18 / 18 / 20 / 38, 24: 27 / 29 / 25 / 42, 64: 47 / 39 / 38 / 46, 96: 61 / 52 / 40 / 47, 128: 73 / 58 / 59 / 49
-//   top 4 of 16, 2048, 512:  12: 36 / 30 / 30 / 53, 48: 66 / 51 / 39 / 59, 96: 104 / 83 / 64 / 63
-// tiles of 64 / 128 rows:  top 2 of 16, 2048, 1024:  48: 60 / 67, 64: 94 / 68;  top 4 of 32, 1024, 512:  40: 42 / 47, 48: 51 / 47
+//   top 2 of 16, 1024, 512:  6: 18 / 18 / 20 / 38, 24: 27 / 29 / 25 / 40, 64: 47 / 39 / 39 / 42, 96: 61 / 52 / 40 / 42, 128: 73 / 58 / 59 / 45
+//   top 4 of 16, 2048, 512:  12: 36 / 30 / 30 / 53, 48: 66 / 51 / 39 / 57, 96: 104 / 83 / 64 / 59
+// tiles of 64 / 128 rows:  top 2 of 16, 2048, 1024:  48: 60 / 69, 64: 94 / 70;  top 4 of 32, 1024, 512:  40: 42 / 45, 48: 51 / 45
 extern "C" int nv_moe_tile_rows_for(int64_t pairs, int E, int width, int ff, const void* h, int64_t h_stride, const void* up,
                                     const void* down, int dtype) {
     using namespace nv;
     if (!moe_big_ok(dtype, h, h_stride, up, ff, width) || !moe_big_ok(dtype, down, ff, down, width, ff)) return nv_moe_tile_rows(pairs, E);
     const int64_t blocks = (int64_t)E * ((ff + 127) / 128);           // of the first product, a tile an expert
-    if (pairs >= (blocks >= 256 ? 40 : blocks >= 128 ? 48 : 96) * (int64_t)E) return kMoeBigRows;
+    if (pairs >= (blocks >= 256 ? 40 : blocks >= 128 ? 48 : 84) * (int64_t)E) return kMoeBigRows;
     return pairs >= 24 * (int64_t)E ? 64 : pairs >= 8 * (int64_t)E ? 32 : 16;
 }
 
@@ -1064,10 +1079,10 @@ extern "C" int nv_moe_gate_up_act(const void* h, int64_t h_stride, const void* g
     hipStream_t s = (hipStream_t)stream;
     if (dtype == NV_DTYPE_BF16)
         launch_grouped<__bf16, 1>(h, h_stride, gate_up, sorted_pairs, meta, nullptr, y, nullptr, top, ff, width, limit,
-                                     alpha, up_shift, (int)tiles, tile_rows, s);
+                                     alpha, up_shift, (int)tiles, tile_rows, pairs / top, s);
     else
         launch_grouped<float, 1>(h, h_stride, gate_up, sorted_pairs, meta, nullptr, y, nullptr, top, ff, width, limit,
-                                    alpha, up_shift, (int)tiles, tile_rows, s);
+                                    alpha, up_shift, (int)tiles, tile_rows, pairs / top, s);
     return check_launch("nv_moe_gate_up");
 }
 
@@ -1087,10 +1102,10 @@ extern "C" int nv_moe_down(const void* y, const void* down, const int32_t* sorte
     hipStream_t s = (hipStream_t)stream;
     if (dtype == NV_DTYPE_BF16)
         launch_grouped<__bf16, 0>(y, ff, down, sorted_pairs, meta, pair_weights, nullptr, out, 1, width, ff, 0.f, 0.f, 0.f,
-                                      (int)tiles, tile_rows, s);
+                                      (int)tiles, tile_rows, pairs, s);
     else
         launch_grouped<float, 0>(y, ff, down, sorted_pairs, meta, pair_weights, nullptr, out, 1, width, ff, 0.f, 0.f, 0.f,
-                                     (int)tiles, tile_rows, s);
+                                     (int)tiles, tile_rows, pairs, s);
     return check_launch("nv_moe_down");
 }
 
@@ -1127,10 +1142,10 @@ extern "C" int nv_moe_up_relu2(const void* h, int64_t h_stride, const void* up, 
     hipStream_t s = (hipStream_t)stream;
     if (dtype == NV_DTYPE_BF16)
         launch_grouped<__bf16, 2>(h, h_stride, up, sorted_pairs, meta, nullptr, y, nullptr, top, ff, width, 0.f, 0.f, 0.f,
-                                  (int)tiles, tile_rows, s);
+                                  (int)tiles, tile_rows, pairs / top, s);
     else
         launch_grouped<float, 2>(h, h_stride, up, sorted_pairs, meta, nullptr, y, nullptr, top, ff, width, 0.f, 0.f, 0.f,
-                                 (int)tiles, tile_rows, s);
+                                 (int)tiles, tile_rows, pairs / top, s);
     return check_launch("nv_moe_up_relu2");
 }
 

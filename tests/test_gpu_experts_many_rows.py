@@ -46,3 +46,16 @@ def test_many_rows(form, E, T, top, W, ff):
     got, want = a(h, ids, weights, gate_up, down), r(f(h), ids, weights, f(gate_up), f(down))
     live = (ids < E)[..., None].expand_as(got)
     torch.testing.assert_close(got[live], want[live], **_tol())
+
+
+def test_rows_far_apart():
+    """Rows whose byte offsets do not fit 32 bits: another launch takes the same tiles."""
+    E, T, top, W, ff = 2, 300, 1, 128, 64
+    g = torch.Generator(device=DEV).manual_seed(3)
+    h = torch.empty(T, (1 << 31) // T // 8 * 8 + 8, dtype=torch.bfloat16, device=DEV)[:, :W]
+    near = torch.randn(T, W, generator=g, device=DEV).to(torch.bfloat16)
+    h.copy_(near)
+    mk = lambda *s, scale=1.0: (torch.randn(*s, generator=g, device=DEV) * scale).to(torch.bfloat16)
+    gate_up, down, logits = mk(E, 2 * ff, W, scale=W ** -0.5), mk(E, W, ff, scale=ff ** -0.5), torch.randn(T, E, generator=g, device=DEV)
+    a = moe.MoEExperts(top, 1.5)
+    torch.testing.assert_close(a(h, logits, gate_up, down), a(near, logits, gate_up, down), **_tol())
