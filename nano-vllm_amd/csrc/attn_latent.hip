@@ -37,6 +37,7 @@ constexpr float kLatRunInit = -1.0e30f;        // finite initial running maximum
 constexpr float kLatRaise = 8.0f;              // log2 units: weights stay below 2^8 between raises
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kLatRows = 32;                   // rows of a wave
+constexpr int64_t kLatHeader = 64;             // bytes of the workspace in front of the states
 constexpr int kLatStageRow = 144;              // bytes per row of the output staging area (128 + 16: spreads the banks)
 
 struct LatentParams {
@@ -53,7 +54,9 @@ struct LatentParams {
                                  // columns beside the queries would not fit the registers)
     int row_tiles;               // rows kernel: 128-row tiles of the longest sequence
     int head_groups;             // single kernel: groups of 32 heads
-    int nsplit, tiles_per_split;
+    int nsplit, tiles_per_split; // rows kernel: the most ranges a row can have, and the fewest tiles of one
+    int slots;                   // rows kernel: workgroups that the chip holds at a time; 0: the launch is no larger than that
+    int* share;                  // [1]: tiles of a range of the rows kernel, where slots > 0
 };
 
 __device__ __forceinline__ float lat_max_xor32(float x) {
@@ -217,7 +220,27 @@ __device__ __forceinline__ float lat_finish(float m, float l, const float* sink,
 }
 
 // ------------------------------------------------------------------------------------------------ several tokens
-template <int D32, int DV32, int KB, int OCC>
+// Key tiles of a range: what the step has for every slot, not less than the launch has room for.  All row tiles get a whole range
+// first, longest first, and what is left of the long ones goes to the slots whose row tile was short: 16 heads, 256 columns, 1024 rows
+// of each of 2 sequences of 3000 and 6001 keys take 63 tiles the longest way, where ranges of half the longest sequence take 94: with the order
+// of the workgroups 220 -> 164 us a call; 500 rows of each of 4 sequences of 1000 .. 3000 keys 138 -> 106, 16 prompts of 200 .. 512 tokens
+// 67 -> 53 (device times, 256 columns; rows of one range write no state).
+template <int KT>
+__device__ __forceinline__ int lat_share(const LatentParams& p, int lane) {
+    int64_t total = 0;
+    for (int b = lane; b < p.B; b += 64) {
+        const int n_q = p.cu_q[b + 1] - p.cu_q[b], n_k = p.cu_k[b + 1] - p.cu_k[b];
+        if (n_q <= 1) continue;
+        const int64_t tiles = ((int64_t)n_q * p.H + 4 * kLatRows - 1) / (4 * kLatRows);
+        total += tiles * (n_k - n_q / 2) / KT + tiles;
+    }
+    for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o);
+    const int64_t share = (total + p.slots - 1) / p.slots;
+    return (int)min(max(share, (int64_t)p.tiles_per_split), (int64_t)1 << 24);
+}
+
+// EVEN: the launch is more than the chip holds at a time, so the order and the ranges of its workgroups matter.
+template <int D32, int DV32, int KB, int OCC, bool EVEN>
 __global__ __launch_bounds__(256, OCC) void attn_latent_rows_kernel(const LatentParams p) {
     constexpr int D = 32 * D32, KT = 32 * KB, kTile = KT * D * 2, kPieces = D32 * KB / 2;
     static_assert(D32 * KB % 2 == 0, "a wave stages whole pieces");
@@ -228,18 +251,27 @@ __global__ __launch_bounds__(256, OCC) void attn_latent_rows_kernel(const Latent
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int split = blockIdx.y, dv0 = blockIdx.z * DV32, Dv = p.Dv;
-    const int b = blockIdx.x % p.B, qt = p.row_tiles - 1 - blockIdx.x / p.B;     // the latest (heaviest) tiles first
+    // The latest (heaviest) tiles first, the sequences in turn.  A workgroup's index gives its XCD (of eight) and there its shader engine
+    // (of four, eight CUs each), and it waits for that one, others idle or not.  So a launch of more than one round turns every 32
+    // workgroups by another amount, or two sequences would keep to half of the engines each; with key ranges, which come
+    // in rounds of their own, it takes the sequences one after the other.
+    const int first = blockIdx.x & ~31, x = EVEN && first + 32 <= (int)gridDim.x ? first + ((blockIdx.x + 13 * (first >> 5)) & 31) : (int)blockIdx.x;
+    const bool one_by_one = EVEN && p.nsplit > 1;
+    const int b = one_by_one ? x / p.row_tiles : x % p.B, qt = p.row_tiles - 1 - (one_by_one ? x % p.row_tiles : x / p.B);
     const int q_begin = p.cu_q[b], n_q = p.cu_q[b + 1] - q_begin, n_k = p.cu_k[b + 1] - p.cu_k[b];
     const int rows = n_q * p.H, row0 = qt * 4 * kLatRows;
+    const int share = EVEN && p.nsplit > 1 ? __builtin_amdgcn_readfirstlane(lat_share<KT>(p, lane)) : p.tiles_per_split;
+    if (EVEN && p.nsplit > 1 && blockIdx.x == 0 && split == 0 && blockIdx.z == 0 && tid == 0) *p.share = share;        // (for the merge)
     if (n_q <= 1 || row0 >= rows) return;                    // (single tokens belong to the other kernel)
     const int start = n_k - n_q;
     const int rw0 = row0 + wave * kLatRows;                  // the wave's first row
     const bool wave_live = rw0 < rows;
     const int my_row = min(rw0 + r, rows - 1);
     const int qpos = start + my_row / p.H;
+    const int tiles = (start + (min(row0 + 4 * kLatRows, rows) - 1) / p.H) / KT + 1;
+    const int t_begin = split * share, t_end = min(tiles, t_begin + share);
+    if (EVEN && split > 0 && t_begin >= tiles) return;
     const int wave_first_pos = start + min(rw0, rows - 1) / p.H, wave_last_pos = start + min(rw0 + kLatRows - 1, rows - 1) / p.H;
-    const int last_key = start + (min(row0 + 4 * kLatRows, rows) - 1) / p.H;
-    const int t_begin = split * p.tiles_per_split, t_end = min(last_key / KT + 1, t_begin + p.tiles_per_split);
 
     LatentWave<D32, DV32, KB> w;
     w.init(p.q + ((int64_t)q_begin * p.H + my_row) * D, h);
@@ -285,14 +317,14 @@ __global__ __launch_bounds__(256, OCC) void attn_latent_rows_kernel(const Latent
     unsigned char* stg = (wave < 2 ? buf0 : buf1) + (wave & 1) * (kLatRows * kLatStageRow);
     const int rows_here = rows - rw0;
     const int64_t grow = (int64_t)q_begin * p.H + rw0;
-    if (p.nsplit > 1) {
+    if (EVEN ? tiles > share : p.nsplit > 1) {
         float* dst = p.part + (grow * p.nsplit + split) * (Dv + 2);
         const int64_t ld = (int64_t)p.nsplit * (Dv + 2);
         if (dv0 == 0 && h == 0 && r < rows_here) {
             dst[r * ld + Dv] = w.m_run;
             dst[r * ld + Dv + 1] = l_tot;
         }
-        if (t_begin >= t_end) return;                        // no keys in this range: l = 0 says so
+        if (!EVEN && t_begin >= t_end) return;               // no keys in this range: l = 0 says so
 #pragma unroll
         for (int d = 0; d < DV32; ++d) {
 #pragma unroll
@@ -433,21 +465,29 @@ __global__ __launch_bounds__(256, OCC) void attn_latent_single_kernel(const Late
 }
 
 // Joins the key ranges of a row (token, head): one wave per row.  only: 1 = rows of single-token sequences, 2 = the others.
-__global__ __launch_bounds__(256) void attn_latent_merge_kernel(const LatentParams p, int Dv, int64_t total_rows, int only) {
+__global__ __launch_bounds__(256) void attn_latent_merge_kernel(const LatentParams p, int Dv, int64_t total_rows, int only, int tile_keys) {
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= total_rows) return;
     const int lane = threadIdx.x & 63;
-    const int t = (int)(row / p.H);
+    const int t = (int)(row / p.H), even = only == 2 && p.slots > 0, share = even ? *p.share : 0;
     int lo = 0, hi = p.B;
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
         if (p.cu_q[mid] <= t) lo = mid; else hi = mid;
     }
-    if ((p.cu_q[lo + 1] - p.cu_q[lo] == 1) != (only == 1)) return;
+    const int q_begin = p.cu_q[lo], n_q = p.cu_q[lo + 1] - q_begin;
+    if ((n_q == 1) != (only == 1)) return;
+    int ranges = p.nsplit;
+    if (even) {                                              // (a row of one range has its output already)
+        const int n_k = p.cu_k[lo + 1] - p.cu_k[lo], end = (int)((row - (int64_t)q_begin * p.H) / (4 * kLatRows) + 1) * (4 * kLatRows);
+        const int tiles = (n_k - n_q + (min(end, n_q * p.H) - 1) / p.H) / tile_keys + 1;
+        if (tiles <= share) return;
+        ranges = (tiles + share - 1) / share;
+    }
     const float* base = p.part + row * p.nsplit * (Dv + 2);
     // lane s holds range s (at most 32 of them): its share of the denominator and the factor of its accumulators
     float m = kLatRunInit, l = 0.f;
-    if (lane < p.nsplit) {
+    if (lane < ranges) {
         const float2 ml = *(const float2*)(base + lane * (Dv + 2) + Dv);
         l = ml.y;
         if (l > 0.f) m = ml.x;
@@ -461,7 +501,7 @@ __global__ __launch_bounds__(256) void attn_latent_merge_kernel(const LatentPara
     for (int c = 2 * lane; c < Dv; c += 128) {               // (Dv is even)
         float ox = 0.f, oy = 0.f;
 #pragma unroll 8
-        for (int s = 0; s < p.nsplit; ++s) {
+        for (int s = 0; s < ranges; ++s) {
             const float fs = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f), s));   // (some lanes may sit this out)
             const float2 v = *(const float2*)(base + s * (Dv + 2) + c);
             ox += fs > 0.f ? fs * v.x : 0.f;
@@ -499,7 +539,7 @@ static LatentPlan latent_single_plan(int B, int H, int max_k) {
 }
 
 template <int D32, int DV32>
-static int launch_latent_rows(LatentParams p, int max_q, int max_k, hipStream_t s) {
+static int launch_latent_rows(LatentParams& p, int max_q, int max_k, hipStream_t s) {
     constexpr int KB = D32 <= 8 ? 2 : 1, OCC = D32 <= 5 || (D32 == 6 && DV32 == 4) ? 2 : 1, D = 32 * D32;
     const LatentPlan plan = latent_rows_plan(p.B, p.H, max_q, max_k, D);
     p.nsplit = plan.nsplit;
@@ -507,8 +547,11 @@ static int launch_latent_rows(LatentParams p, int max_q, int max_k, hipStream_t 
     p.row_tiles = (int)(((int64_t)max_q * p.H + 127) / 128);
     p.tiles_per_block = p.block_size / (32 * KB);
     p.dv_groups = p.Dv / (32 * DV32);
-    hipLaunchKernelGGL((attn_latent_rows_kernel<D32, DV32, KB, OCC>),
-                       dim3((unsigned)(p.B * p.row_tiles), (unsigned)p.nsplit, (unsigned)p.dv_groups), dim3(256), 0, s, p);
+    const int slots = std::max(1, 256 * OCC / p.dv_groups);
+    p.slots = (int64_t)p.B * p.row_tiles * p.nsplit > slots ? slots : 0;
+    const dim3 grid((unsigned)(p.B * p.row_tiles), (unsigned)p.nsplit, (unsigned)p.dv_groups);
+    if (p.slots > 0) hipLaunchKernelGGL((attn_latent_rows_kernel<D32, DV32, KB, OCC, true>), grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((attn_latent_rows_kernel<D32, DV32, KB, OCC, false>), grid, dim3(256), 0, s, p);
     return check_launch("nv_attn_latent_paged (rows kernel)");
 }
 template <int D32, int DV32>
@@ -544,7 +587,7 @@ extern "C" int64_t nv_attn_latent_workspace_bytes(int num_seqs, int64_t T, int H
     if (num_seqs <= 0 || T <= 0 || H <= 0 || Dv <= 0 || max_seqlen_k <= 0) return 0;
     int n = latent_single_plan(num_seqs, H, max_seqlen_k).nsplit;
     if (max_seqlen_q > 1) n = std::max(n, latent_rows_plan(num_seqs, H, max_seqlen_q, max_seqlen_k, D).nsplit);
-    return n > 1 ? T * H * n * (int64_t)(Dv + 2) * (int64_t)sizeof(float) : 0;
+    return n > 1 ? kLatHeader + T * H * n * (int64_t)(Dv + 2) * (int64_t)sizeof(float) : 0;
 }
 
 extern "C" int nv_attn_latent_paged(const void* q, const void* cache, void* out, const int32_t* cu_seqlens_q,
@@ -575,7 +618,8 @@ extern "C" int nv_attn_latent_paged(const void* q, const void* cache, void* out,
     p.q = (const __bf16*)q;
     p.cache = (const __bf16*)cache;
     p.out = (__bf16*)out;
-    p.part = (float*)workspace;
+    p.share = (int*)workspace;
+    p.part = workspace ? (float*)((char*)workspace + kLatHeader) : nullptr;
     p.cu_q = cu_seqlens_q;
     p.cu_k = cu_seqlens_k;
     p.block_tables = block_tables;
@@ -591,7 +635,7 @@ extern "C" int nv_attn_latent_paged(const void* q, const void* cache, void* out,
     const auto merge = [&](const LatentPlan& plan, int only) {
         if (plan.nsplit <= 1) return (int)NV_OK;
         p.nsplit = plan.nsplit;
-        hipLaunchKernelGGL(attn_latent_merge_kernel, dim3((unsigned)((T * H + 3) / 4)), dim3(256), 0, s, p, Dv, T * H, only);
+        hipLaunchKernelGGL(attn_latent_merge_kernel, dim3((unsigned)((T * H + 3) / 4)), dim3(256), 0, s, p, Dv, T * H, only, latent_tile_keys(D));
         return check_launch("nv_attn_latent_paged (merge)");
     };
     int rc = NV_ERR_UNSUPPORTED;

@@ -1,0 +1,34 @@
+"""GPU: latent attention launches of more workgroups than the chip holds at a time (key ranges by what the step has for every slot, rows of one
+range without a state): sequences of very different lengths, single tokens between them, row tiles that are not full, one range alone."""
+import pytest
+import torch
+
+from nanovllm_amd import ops
+from buvalix_util import paged_context
+from test_gpu_nekodra_layers import DEV, reference_rows, rn
+
+pytestmark = pytest.mark.gpu
+
+STEPS = {"far_apart": ([150, 1, 150, 150], [2500, 90, 150, 700]), "one_long": ([260, 5], [3000, 64]), "prompts": ([500, 300, 1, 77], [500, 300, 1, 77]),
+         "equal": ([200, 200], [1600, 1600])}
+
+
+@pytest.mark.parametrize("H", [16, 13])
+@pytest.mark.parametrize("D,Dv", [(256, 256), (160, 128), (320, 320)])
+@pytest.mark.parametrize("step", list(STEPS))
+def test_even_shares(D, Dv, H, step):
+    n_q, n_k = STEPS[step]
+    bs, nb = 64, sum(-(-n // 64) for n in n_k) + 3
+    ctx, _ = paged_context(n_q, n_k, bs, nb, D, DEV)
+    H *= 4                                 # (rows are tokens times heads)
+    g = torch.Generator().manual_seed(D + H)
+    q = rn(g, sum(n_q), H, D, std=3.0 / D ** 0.5).to(torch.bfloat16)
+    cache = rn(g, nb, bs, 1, D).to(torch.bfloat16)
+    sink = torch.linspace(-3.0, 6.0, H, device=DEV)
+    got = [ops.attn_latent_paged(q, cache, cache[..., :Dv], ctx.cu_seqlens_q, ctx.cu_seqlens_k, ctx.block_tables, 0.9, sink, max(n_q), max(n_k), -1)
+           for _ in range(2)]
+    want = reference_rows(q, cache, ctx, 0.9, sink, Dv)
+    assert torch.equal(got[0], got[1]) and torch.isfinite(got[0]).all()
+    # (the bound of the other launches' test: probabilities and outputs are rounded to bf16, 2^-9 each)
+    err = (got[0].float() - want).view(sum(n_q), -1).norm(dim=-1) / want.norm(dim=-1)
+    assert err.max().item() < 1.2e-2, (int(err.argmax()), err.max().item())
