@@ -14,6 +14,7 @@ struct ScoremodRowsParams {
     int v_ld, n_dist, H, G, block_size, max_blocks, max_block;
     float softcap, scale_log2, cap_in;         // cap_in: a raw score's factor to the exponent of tanh
     int hpw, n_qtiles, wg_per_pair, n_pairs, xs_shift, slots_per_pair, grid_base, nsplit, tiles_per_split;
+    int rounds, there_and_back;                // pairs of an XCD; all workgroups run at a time
 };
 struct ScoremodRowsPlan {
     int hpw;                                   // heads of a kv head's group that a workgroup takes (1, 2 or 4)

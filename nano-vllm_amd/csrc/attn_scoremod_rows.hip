@@ -14,8 +14,8 @@
 //
 // What bounds it: the vector units.  64 soft-capped scores cost a SIMD two exponentials and a reciprocal at quarter rate, about 70
 // cycles with what is around them, beside 32 cycles of matrix products.  Measured (4 prompts of 1777 .. 2048 tokens, 16 / 8 heads of 128,
-// soft cap and sink, the call with its preparation of 21 us): 127 us (129 with the denominator as a product of rounded weights with
-// ones); with the launch on 16 x 16 tiles, values transposed through registers, which other sizes still take, 496 us (44 of them
+// soft cap and sink, the call with its preparation of 21 us): 116 us (127 with an XCD's pairs one after the other, see there; 129 with the
+// denominator as a product of rounded weights with ones, 3 us more with a polynomial in place of the cap's exponential and reciprocal); with the launch on 16 x 16 tiles, values transposed through registers, which other sizes still take, 496 us (44 of them
 // preparation).
 #include <algorithm>
 #include <type_traits>
@@ -56,11 +56,19 @@ __global__ __launch_bounds__(256, 2) void scoremod_rows_kernel(const ScoremodRow
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, hh = lane >> 5;
 
-    // workgroup -> (sequence, kv head, head group, query tile): workgroups that read the same keys share an XCD
+    // Workgroup -> (sequence, kv head, head group, query tile): workgroups that read the same keys share an XCD.  An XCD takes its pairs
+    // (of sequence and kv head) four together, the heaviest query tiles of all first; pair after pair, a CU's workgroups were heavy or light
+    // together and the last pair's heaviest tile began half way.  Workgroups one after the other run on the XCD's four shader engines, so
+    // the pairs turn by one every time.  Where all workgroups are there from the start, 32 (one for each CU) go there and the next 32
+    // back instead, so that a CU that has a heavy one gets a light one with it (one heavy after the other is better where
+    // CUs that have ended take the next).
     const int split = blockIdx.x / p.grid_base, bid = blockIdx.x - split * p.grid_base;
-    const int xcd = bid & 7, slot = bid >> 3, round = slot / p.slots_per_pair;
-    const int pair = round * (8 >> p.xs_shift) + (xcd >> p.xs_shift);
-    const int widx = ((slot - round * p.slots_per_pair) << p.xs_shift) + (xcd & ((1 << p.xs_shift) - 1));
+    const int xcd = bid & 7, slot = bid >> 3, four = slot / (4 * p.slots_per_pair), together = min(4, p.rounds - 4 * four);
+    int at = slot - four * 4 * p.slots_per_pair;
+    if (p.there_and_back && (at & 32) && (at | 31) < together * p.slots_per_pair) at ^= 31;
+    const int rank = at / together, one = at - rank * together + (p.there_and_back ? 0 : rank);
+    const int pair = (4 * four + one % together) * (8 >> p.xs_shift) + (xcd >> p.xs_shift);
+    const int widx = (rank << p.xs_shift) + (xcd & ((1 << p.xs_shift) - 1));
     if (pair >= p.n_pairs || widx >= p.wg_per_pair) return;
     const int groups = p.wg_per_pair / p.n_qtiles, hg = widx % groups, qt = p.n_qtiles - 1 - widx / groups;   // heaviest first
     const int b = pair / p.G, g = pair - b * p.G;
@@ -345,6 +353,8 @@ int launch_scoremod_rows(ScoremodRowsParams p, const ScoremodRowsPlan& f, int D,
     p.n_pairs = f.n_pairs;
     p.xs_shift = f.xs_shift;
     p.slots_per_pair = f.slots_per_pair;
+    p.rounds = (int)(f.grid_base / (8 * (int64_t)f.slots_per_pair));
+    p.there_and_back = f.grid_base * f.nsplit <= 256 * (D + Dv == 128 ? 4 : D + Dv == 192 ? 3 : 2);       // (workgroups that a CU holds)
     p.grid_base = (int)f.grid_base;
     p.nsplit = f.nsplit;
     p.tiles_per_split = f.tiles_per_split;

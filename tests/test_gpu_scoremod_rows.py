@@ -160,3 +160,16 @@ def test_values_as_columns_of_the_keys(D, Dv, at, softcap, step):
     got, want = (ops.attn_scoremod_paged(q, kc, x, ctx.cu_seqlens_q, ctx.cu_seqlens_k, ctx.block_tables, D ** -0.5, softcap, None, None,
                                          max(n_qs), max(n_ks)) for x in (values, values.contiguous()))
     assert got.isfinite().all() and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("H,G,n_qs", [(16, 16, [700] * 11 + [90]), (8, 8, [300, 40, 129, 257, 300, 2, 64, 299, 31]), (4, 1, [1500, 700, 900]), (8, 4, [640])])
+def test_every_row_whatever_the_order(H, G, n_qs):
+    """Launches of more and of fewer workgroups than the chip holds, numbers of sequences and kv heads that leave the last group of an XCD's
+    pairs short, pairs spread over XCDs: every row is written once, by the workgroup that has its keys."""
+    a, r, ctx, pos, q, k, v, kc, vc = _step(H, G, 64, 64, 64, n_qs, n_qs, softcap=25.0)
+    kc_r, vc_r = kc.clone(), vc.clone()
+    nv.set_context(ctx)
+    o, o_r = a(q, k, v, pos, kc, vc), r(q, k, v, pos, kc_r, vc_r)
+    nv.set_context(None)
+    # (as in test_portions)
+    torch.testing.assert_close(o.float(), o_r.float(), rtol=2e-2, atol=2e-2)
