@@ -6,7 +6,10 @@ into ``nano-vllm_amd/lib/``.  There is no fallback: if it cannot be loaded, ``li
 from __future__ import annotations
 
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
+import sysconfig
 import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -178,6 +181,17 @@ class NanoVllmHipError(RuntimeError):
     """A C-ABI call returned a non-zero status."""
 
 
+def _native_calls():
+    """The module of csrc/calls.cpp, or None where it is not built (no Python headers): every call goes through ctypes then."""
+    path = os.path.join(_HERE, "lib", "nv_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
+    if not os.path.exists(path):
+        return None
+    loader = importlib.machinery.ExtensionFileLoader("nv_calls", path)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("nv_calls", path, loader=loader))
+    loader.exec_module(module)
+    return module
+
+
 def load(path: str | None = None, prototypes: dict | None = None) -> C.CDLL:
     """Load the shared library and attach prototypes.  Raises if it is missing or stale."""
     path = path or os.environ.get("NANOVLLM_HIP_LIB", LIB_PATH)
@@ -194,6 +208,13 @@ def load(path: str | None = None, prototypes: dict | None = None) -> C.CDLL:
     got = dll.nv_abi_version()
     if got != ABI_VERSION:
         raise RuntimeError(f"{path}: ABI version {got}, bindings expect {ABI_VERSION}; rebuild the library")
+    calls = _native_calls()
+    if calls is not None:
+        for name in (prototypes if prototypes is not None else PROTOTYPES):
+            fn = getattr(dll, name)
+            quick = calls.bind(name, C.cast(fn, C.c_void_p).value, fn)
+            if quick is not None:
+                setattr(dll, name, quick)
     return dll
 
 
