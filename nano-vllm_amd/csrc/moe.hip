@@ -464,6 +464,14 @@ __global__ __launch_bounds__(256) void moe_place_kernel(const int* __restrict__ 
     }
 }
 
+// The gated unit of all three kernels below.  (On the hardware's exponential and reciprocal the tiles of 128 rows would save 17 of
+// the 497 us of the call measured there, at one or two units in the last place more and with nothing left of a denormal reciprocal.)
+__device__ __forceinline__ float moe_glu(float g, float u, float limit, float alpha, float shift) {
+    g = fminf(g, limit);
+    u = fminf(fmaxf(u, -limit), limit);
+    return g / (1.0f + expf(-alpha * g)) * (u + shift);
+}
+
 // Many rows per expert, bf16: a workgroup of four waves takes 128 rows of one expert and 256 weight rows (gate and up: 128 columns of
 // both), a wave 64 x 128 of it on v_mfma_f32_32x32x16_bf16 (weights as the first operand, so that a lane holds four neighbouring
 // columns of a row).  Slices 64 deep, whole cache lines of every row, go straight into LDS (LDS-DMA, chunks swizzled by row so that the
@@ -476,14 +484,8 @@ __global__ __launch_bounds__(256) void moe_place_kernel(const int* __restrict__ 
 // Buffer loads, because the compiler waits for all LDS reads behind a global load into LDS (and has no 64-bit addresses to add up): 336 -> 281
 // us; the products at a higher priority than the other workgroup's reads: 299 -> 281.  256 x 256 by one workgroup a CU, two buffers: four
 // waves of 128 x 128 319 and 211 us, eight of 64 x 128 349 and 220; a load of the lines two slices ahead into L2: no gain.
-// 8192 tokens, top 4 of 32 experts, width 2048, ff 1024: gate and up 340 -> 281 us, down 240 -> 187; the call 583 -> 497.
+// 8192 tokens, top 4 of 32 experts, width 2048, ff 1024: gate and up 340 -> 297 us, down 240 -> 187; the call 604 -> 497.
 constexpr int kMoeBigRows = 128;
-
-// g * sigmoid(alpha g) * (u + shift) on the hardware's exponential and reciprocal (one unit in the last place each, in front of a rounding to
-// bf16): expf and a division are 45 instructions a value, 10 us a 256 x 256 block.
-__device__ __forceinline__ float moe_glu(float g, float u, float alpha, float shift) {
-    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * (-1.4426950408889634f * alpha))) * (u + shift);
-}
 
 __device__ __forceinline__ int big_off(int row, int ch) { return row * 128 + ((ch ^ ((row >> 1) & 7)) * 16); }
 template <int MODE>
@@ -603,9 +605,7 @@ __global__ __launch_bounds__(256, 2) void moe_big_kernel(
 #pragma unroll
                     for (int t = 0; t < 4; ++t) {
                         if constexpr (GATE_UP) {
-                            const float g = fminf(acc[j][x][i + t], limit);
-                            const float u = fminf(fmaxf(acc[j + 2][x][i + t], -limit), limit);
-                            v[t] = moe_glu(g, u, alpha, up_shift);
+                            v[t] = moe_glu(acc[j][x][i + t], acc[j + 2][x][i + t], limit, alpha, up_shift);
                         } else {
                             const float u = fmaxf(acc[j][x][i + t], 0.f);
                             v[t] = u * u;
@@ -766,10 +766,7 @@ __global__ __launch_bounds__(256, MT == 1 ? 4 : MT == 2 ? 3 : 2) void moe_rows_k
             const f32x4 gs = sum(wave), us = sum(wave + 2);
             float v[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float gg = fminf(gs[i], limit), u = fminf(fmaxf(us[i], -limit), limit);
-                v[i] = gg / (1.0f + expf(-alpha * gg)) * (u + up_shift);
-            }
+            for (int i = 0; i < 4; ++i) v[i] = moe_glu(gs[i], us[i], limit, alpha, up_shift);
             *(uint2*)(y + (int64_t)(row0 + r) * N + c) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
         } else if constexpr (MODE == 2) {
             const f32x4 us = sum(wave);
@@ -882,9 +879,7 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(
                 const int r = m * 16 + 4 * lg + i;
                 if (r >= rows) continue;
                 if constexpr (GATE_UP) {
-                    const float g = fminf(acc[nt][m][i], limit);
-                    const float u = fminf(fmaxf(acc[NT + nt][m][i], -limit), limit);
-                    y[(int64_t)(row0 + r) * N + n] = (T)(g / (1.0f + expf(-alpha * g)) * (u + up_shift));
+                    y[(int64_t)(row0 + r) * N + n] = (T)moe_glu(acc[nt][m][i], acc[NT + nt][m][i], limit, alpha, up_shift);
                 } else if constexpr (MODE == 2) {
                     const float u = fmaxf(acc[nt][m][i], 0.f);
                     y[(int64_t)(row0 + r) * N + n] = (T)(u * u);
