@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "launch_order.h"
 #include "nv_common.h"
 #include "../../include/nanovllm_hip_mixers.h"
 
@@ -235,8 +236,7 @@ __device__ __forceinline__ int lat_share(const LatentParams& p, int lane) {
         total += tiles * (n_k - n_q / 2) / KT + tiles;
     }
     for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o);
-    const int64_t share = (total + p.slots - 1) / p.slots;
-    return (int)min(max(share, (int64_t)p.tiles_per_split), (int64_t)1 << 24);
+    return latent_share(total, p.slots, p.tiles_per_split);
 }
 
 // EVEN: the launch is more than the chip holds at a time, so the order and the ranges of its workgroups matter.
@@ -268,9 +268,10 @@ __global__ __launch_bounds__(256, OCC) void attn_latent_rows_kernel(const Latent
     const bool wave_live = rw0 < rows;
     const int my_row = min(rw0 + r, rows - 1);
     const int qpos = start + my_row / p.H;
-    const int tiles = (start + (min(row0 + 4 * kLatRows, rows) - 1) / p.H) / KT + 1;
+    const int tiles = latent_tiles(start + (min(row0 + 4 * kLatRows, rows) - 1) / p.H, KT, p.nsplit, p.tiles_per_split);
     const int t_begin = split * share, t_end = min(tiles, t_begin + share);
-    if (EVEN && split > 0 && t_begin >= tiles) return;
+    const int ranges = EVEN ? latent_ranges(tiles, share) : p.nsplit;
+    if (split >= ranges) return;
     const int wave_first_pos = start + min(rw0, rows - 1) / p.H, wave_last_pos = start + min(rw0 + kLatRows - 1, rows - 1) / p.H;
 
     LatentWave<D32, DV32, KB> w;
@@ -317,7 +318,7 @@ __global__ __launch_bounds__(256, OCC) void attn_latent_rows_kernel(const Latent
     unsigned char* stg = (wave < 2 ? buf0 : buf1) + (wave & 1) * (kLatRows * kLatStageRow);
     const int rows_here = rows - rw0;
     const int64_t grow = (int64_t)q_begin * p.H + rw0;
-    if (EVEN ? tiles > share : p.nsplit > 1) {
+    if (ranges > 1) {
         float* dst = p.part + (grow * p.nsplit + split) * (Dv + 2);
         const int64_t ld = (int64_t)p.nsplit * (Dv + 2);
         if (dv0 == 0 && h == 0 && r < rows_here) {
@@ -480,9 +481,8 @@ __global__ __launch_bounds__(256) void attn_latent_merge_kernel(const LatentPara
     int ranges = p.nsplit;
     if (even) {                                              // (a row of one range has its output already)
         const int n_k = p.cu_k[lo + 1] - p.cu_k[lo], end = (int)((row - (int64_t)q_begin * p.H) / (4 * kLatRows) + 1) * (4 * kLatRows);
-        const int tiles = (n_k - n_q + (min(end, n_q * p.H) - 1) / p.H) / tile_keys + 1;
-        if (tiles <= share) return;
-        ranges = (tiles + share - 1) / share;
+        ranges = latent_ranges(latent_tiles(n_k - n_q + (min(end, n_q * p.H) - 1) / p.H, tile_keys, p.nsplit, p.tiles_per_split), share);
+        if (ranges == 1) return;
     }
     const float* base = p.part + row * p.nsplit * (Dv + 2);
     // lane s holds range s (at most 32 of them): its share of the denominator and the factor of its accumulators

@@ -1,0 +1,43 @@
+"""Index arithmetic of launches that choose their order or key ranges on the device, over many launch shapes with a host compiler."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SHIM = r"""
+#include "launch_order.h"
+using namespace nv;
+extern "C" int latent(int64_t total, int slots, int last_key, int tile_keys, int nsplit, int fewest, int* share, int* tiles) {
+    *share = latent_share(total, slots, fewest);
+    *tiles = latent_tiles(last_key, tile_keys, nsplit, fewest);
+    return latent_ranges(*tiles, *share);
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def order(tmp_path_factory):
+    d = tmp_path_factory.mktemp("launch_order")
+    src, lib = d / "shim.cpp", d / "shim.so"
+    src.write_text(SHIM)
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Werror", "-shared", "-fPIC", "-I", os.path.join(ROOT, "nano-vllm_amd", "csrc"),
+                    str(src), "-o", str(lib)], check=True)
+    dll = C.CDLL(str(lib))
+    dll.latent.argtypes = [C.c_int64] + [C.c_int] * 5 + [C.POINTER(C.c_int)] * 2
+    return dll
+
+
+def test_latent_ranges_stay_within_what_was_stated(order):
+    """Whatever a sequence's true length: no state beyond the workspace (none at all where there is one range), no key beyond the stated
+    length's ranges, and every key tile within them in one range."""
+    share, tiles = C.c_int(), C.c_int()
+    for nsplit, fewest in ((1, 1), (1, 7), (1, 40), (2, 8), (3, 9), (7, 8), (32, 8), (32, 30)):
+        for last_key in list(range(0, 64 * (nsplit * fewest + 3), 61)) + [10 ** 5, 10 ** 7]:
+            for total in (0, 1, 100, 5000, 10 ** 6, 10 ** 12):
+                n = order.latent(total, 256, last_key, 64, nsplit, fewest, C.byref(share), C.byref(tiles))
+                assert share.value >= fewest and 1 <= n <= nsplit
+                assert tiles.value == min(last_key // 64 + 1, nsplit * fewest)
+                assert (n - 1) * share.value < tiles.value <= n * share.value
