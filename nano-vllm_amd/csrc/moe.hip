@@ -892,12 +892,9 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(
     }
 }
 
-// Tiles of 128 rows and of few rows take whole 64-deep slices and 16-byte pieces of both operands' rows, and of the result's.
-static bool moe_big_ok(int dtype, const void* a, int64_t a_stride, const void* w, int N, int K) {
+// Tiles of 32 and 128 rows are for whole 64-deep slices and 16-byte pieces of the rows and weights that they are suggested for.
+static bool moe_pieces_ok(int dtype, const void* a, int64_t a_stride, const void* w, int N, int K) {
     return dtype == NV_DTYPE_BF16 && K % 64 == 0 && N % 8 == 0 && a_stride % 8 == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0;
-}
-static bool moe_rows_ok(const void* result, const void* a, int64_t a_stride, const void* w, int N, int K) {
-    return (uintptr_t)result % 16 == 0 && moe_big_ok(NV_DTYPE_BF16, a, a_stride, w, N, K);
 }
 
 // A block's offsets from the first row and from the expert's first weight row, in bytes, are 32 bits (tiles of 128 rows beyond that, an input or an
@@ -910,8 +907,10 @@ template <typename T, int MODE>
 static void launch_grouped(const void* a, int64_t a_stride, const void* w, const int* sorted_pairs, const int* meta,
                            const float* pair_w, void* y, float* out, int top, int N, int K, float limit, float alpha,
                            float up_shift, int max_tiles, int tile_rows, int64_t a_rows, hipStream_t s) {
+    // activations and outputs that do not start on 16 bytes take the general launch, in tiles of any size
+    const bool pieces = sizeof(T) == 2 && (MODE == 0 ? (uintptr_t)out : (uintptr_t)y) % 16 == 0 && moe_pieces_ok(NV_DTYPE_BF16, a, a_stride, w, N, K);
     if constexpr (sizeof(T) == 2) {
-        if (tile_rows == kMoeBigRows && moe_offsets_ok(MODE == 0 ? kMoeBigRows : a_rows, a_stride, (MODE == 1 ? 2 : 1) * (int64_t)N, K)) {               // (the caller has checked sizes and alignment)
+        if (pieces && tile_rows == kMoeBigRows && moe_offsets_ok(MODE == 0 ? kMoeBigRows : a_rows, a_stride, (MODE == 1 ? 2 : 1) * (int64_t)N, K)) {
             constexpr int cols = MODE == 1 ? 128 : 256;
             hipLaunchKernelGGL(moe_big_kernel<MODE>, dim3((unsigned)(((int64_t)max_tiles * ((N + cols - 1) / cols) + 7) / 8 * 8)), dim3(256), 0, s,
                                (const T*)a, a_stride, (const T*)w, sorted_pairs, meta, pair_w, (T*)y, out, top, N, K, limit, alpha, up_shift);
@@ -919,7 +918,7 @@ static void launch_grouped(const void* a, int64_t a_stride, const void* w, const
         }
     }
     if constexpr (sizeof(T) == 2) {
-        if (tile_rows < kMoeBigRows && moe_rows_ok(MODE == 0 ? (const void*)out : y, a, a_stride, w, N, K)) {
+        if (pieces && tile_rows < kMoeBigRows) {
             const int64_t items = (int64_t)max_tiles * ((N + (MODE == 1 ? 31 : 63)) / (MODE == 1 ? 32 : 64));
 #define NV_MOE_ROWS(MT)                                                                                                              \
     hipLaunchKernelGGL((moe_rows_kernel<MODE, MT>), dim3((unsigned)((items + 7) / 8 * 8)), dim3(256), 0, s, (const T*)a, a_stride, (const T*)w, \
@@ -940,8 +939,9 @@ static void launch_grouped(const void* a, int64_t a_stride, const void* w, const
                        dim3(256), 0, s, (const T*)a, a_stride, (const T*)w, sorted_pairs, meta, pair_w, (T*)y, out, top, N, K,  \
                        limit, alpha, up_shift, vec_ok, max_tiles)
     if constexpr (sizeof(T) == 2) {
-        if (tile_rows == kMoeBigRows) {
-            NV_MOE_LAUNCH(8, 1);
+        if (tile_rows == kMoeBigRows || tile_rows == 32) {
+            if (tile_rows == 32) NV_MOE_LAUNCH(2, 1);
+            else NV_MOE_LAUNCH(8, 1);
             return;
         }
     }
@@ -981,7 +981,7 @@ extern "C" int nv_moe_tile_rows(int64_t pairs, int E) { return pairs >= 32 * (in
 extern "C" int nv_moe_tile_rows_for(int64_t pairs, int E, int width, int ff, const void* h, int64_t h_stride, const void* up,
                                     const void* down, int dtype) {
     using namespace nv;
-    if (!moe_big_ok(dtype, h, h_stride, up, ff, width) || !moe_big_ok(dtype, down, ff, down, width, ff)) return nv_moe_tile_rows(pairs, E);
+    if (!moe_pieces_ok(dtype, h, h_stride, up, ff, width) || !moe_pieces_ok(dtype, nullptr, ff, down, width, ff)) return nv_moe_tile_rows(pairs, E);
     const int64_t blocks = (int64_t)E * ((ff + 127) / 128);           // of the first product, a tile an expert
     if (pairs >= (blocks >= 256 ? 40 : blocks >= 128 ? 48 : 84) * (int64_t)E) return kMoeBigRows;
     return pairs >= 24 * (int64_t)E ? 64 : pairs >= 8 * (int64_t)E ? 32 : 16;
@@ -1067,7 +1067,7 @@ extern "C" int nv_moe_gate_up_act(const void* h, int64_t h_stride, const void* g
     if (pairs == 0) return NV_OK;
     NV_REQUIRE(h && gate_up && sorted_pairs && meta && y, NV_ERR_INVALID_ARG, "nv_moe_gate_up: null pointer");
     NV_REQUIRE(dtype == NV_DTYPE_BF16 || dtype == NV_DTYPE_F32, NV_ERR_INVALID_ARG, "nv_moe_gate_up: bad dtype");
-    NV_REQUIRE((tile_rows != 128 && tile_rows != 32) || ((uintptr_t)y % 16 == 0 && moe_big_ok(dtype, h, h_stride, gate_up, ff, width)), NV_ERR_UNSUPPORTED,
+    NV_REQUIRE((tile_rows != 128 && tile_rows != 32) || moe_pieces_ok(dtype, h, h_stride, gate_up, ff, width), NV_ERR_UNSUPPORTED,
                "nv_moe_gate_up: tiles of 32 or 128 rows take bf16 rows in whole pieces");
     const int64_t tiles = nv_moe_max_tiles(pairs, E, tile_rows);
     NV_REQUIRE(tiles * ((ff + kMoeBN - 1) / kMoeBN) < (1LL << 31), NV_ERR_UNSUPPORTED, "nv_moe_gate_up: launch too large");
@@ -1090,7 +1090,7 @@ extern "C" int nv_moe_down(const void* y, const void* down, const int32_t* sorte
     if (pairs == 0) return NV_OK;
     NV_REQUIRE(y && down && sorted_pairs && meta && pair_weights && out, NV_ERR_INVALID_ARG, "nv_moe_down: null pointer");
     NV_REQUIRE(dtype == NV_DTYPE_BF16 || dtype == NV_DTYPE_F32, NV_ERR_INVALID_ARG, "nv_moe_down: bad dtype");
-    NV_REQUIRE((tile_rows != 128 && tile_rows != 32) || ((uintptr_t)out % 16 == 0 && moe_big_ok(dtype, y, ff, down, width, ff)), NV_ERR_UNSUPPORTED,
+    NV_REQUIRE((tile_rows != 128 && tile_rows != 32) || moe_pieces_ok(dtype, nullptr, ff, down, width, ff), NV_ERR_UNSUPPORTED,
                "nv_moe_down: tiles of 32 or 128 rows take bf16 rows in whole pieces");
     const int64_t tiles = nv_moe_max_tiles(pairs, E, tile_rows);
     NV_REQUIRE(tiles * ((width + kMoeBN - 1) / kMoeBN) < (1LL << 31), NV_ERR_UNSUPPORTED, "nv_moe_down: launch too large");
@@ -1130,7 +1130,7 @@ extern "C" int nv_moe_up_relu2(const void* h, int64_t h_stride, const void* up, 
     if (pairs == 0) return NV_OK;
     NV_REQUIRE(h && up && sorted_pairs && meta && y, NV_ERR_INVALID_ARG, "nv_moe_up_relu2: null pointer");
     NV_REQUIRE(dtype == NV_DTYPE_BF16 || dtype == NV_DTYPE_F32, NV_ERR_INVALID_ARG, "nv_moe_up_relu2: bad dtype");
-    NV_REQUIRE((tile_rows != 128 && tile_rows != 32) || ((uintptr_t)y % 16 == 0 && moe_big_ok(dtype, h, h_stride, up, ff, width)), NV_ERR_UNSUPPORTED,
+    NV_REQUIRE((tile_rows != 128 && tile_rows != 32) || moe_pieces_ok(dtype, h, h_stride, up, ff, width), NV_ERR_UNSUPPORTED,
                "nv_moe_up_relu2: tiles of 32 or 128 rows take bf16 rows in whole pieces");
     const int64_t tiles = nv_moe_max_tiles(pairs, E, tile_rows);
     NV_REQUIRE(tiles * ((ff + kMoeBN - 1) / kMoeBN) < (1LL << 31), NV_ERR_UNSUPPORTED, "nv_moe_up_relu2: launch too large");
