@@ -1,5 +1,4 @@
-// Index arithmetic of launches whose workgroups choose their order or their key ranges on the device: plain functions of integers, so that
-// a host compiler can check them over every launch shape.
+// Rules and index arithmetic of launches as plain functions of integers, so that a host compiler can check them over every launch shape.
 #pragma once
 #include <stdint.h>
 
@@ -24,5 +23,16 @@ NV_HD int latent_tiles(int last_key, int tile_keys, int nsplit, int fewest) {
 }
 // Its ranges: at most nsplit, since a share is never below `fewest`.
 NV_HD int latent_ranges(int tiles, int share) { return tiles <= share ? 1 : (tiles - 1) / share + 1; }
+
+// Tiles of 128 rows, no more blocks than CUs: slices 32 deep, since nothing else runs on a CU while its one workgroup waits for a slice.  Tiles of an
+// expert: one, from 100 pairs on as many as its pairs fill and a half.  First / second product of 16 or 32 experts, us, 64 and 32 deep:
+//   128 blocks   width 2048, ff 1024: 41.5 and 36.7 / 23.9 and 21.8;  width 1024, ff 512: 25.7 and 23.0 / 15.7 and 15.3
+//   256          2048, 1024: 50.5 and 46.8 / 30.2 and 27.3;  1024, 1024: 31.9 and 27.8 / (128) 24.3 and 22.1
+//   192, 256     2048, 1024, 128 and 192 pairs an expert: 46.6 and 38.9 / 27.2 and 23.9, 42.9 and 41.0 / 25.5 and 25.4
+//   320, 384     2048, 1024: 50.7 and 68.5 / 32.0 and 39.7, 68.0 and 83.0 / 34.6 and 42.1
+// (the same order with weights that come from memory instead of the last cache: 51.9 and 47.0 / 27.4 and 25.1 for the first)
+NV_HD bool moe_few_blocks(int64_t pairs, int E, int n_cols) {
+    return (pairs <= 100 * (int64_t)E ? E : pairs / 128 + E / 2) * n_cols <= 256;
+}
 
 }  // namespace nv

@@ -22,6 +22,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "launch_order.h"
 #include "mfma_tile.h"
 #include "../../include/nanovllm_hip_mixers.h"
 
@@ -478,24 +479,28 @@ __device__ __forceinline__ float moe_glu(float g, float u, float limit, float al
 // 16-byte operand reads are free of bank conflicts).  A wave reads all operands of its slice into registers; the next slice then goes into the same
 // 48 KiB while it multiplies, and the other workgroup of the CU has its turn at LDS.  Rows past the tile repeat its first one, weight rows past N the last
 // ones; neither is written.
+// Launches that leave a CU one workgroup, and rows or weights 4 GiB apart, take slices 32 deep by address, three buffers and two slices in flight.
 // What bounds it: the way of the slices from L2 (11 TB/s through the CUs' vector caches).  Slices 32 deep take half a cache line of every row
-// and the same line again for the next slice: 340 and 240 us for both products of the call below, with three buffers and two slices in
-// flight.  Without any loads behind the first slice it is 217 and 136 us, with all of them in the vector caches 226 and 145, in L2 263 and 160.
+// and the same line again for the next slice: 340 and 240 us for both products of the call below.  Without any loads behind the first slice it is 217 and 136 us, with all of them in the vector caches 226 and 145, in L2 263 and 160.
 // Buffer loads, because the compiler waits for all LDS reads behind a global load into LDS (and has no 64-bit addresses to add up): 336 -> 281
 // us; the products at a higher priority than the other workgroup's reads: 299 -> 281.  256 x 256 by one workgroup a CU, two buffers: four
 // waves of 128 x 128 319 and 211 us, eight of 64 x 128 349 and 220; a load of the lines two slices ahead into L2: no gain.
 // 8192 tokens, top 4 of 32 experts, width 2048, ff 1024: gate and up 340 -> 297 us, down 240 -> 187; the call 604 -> 497.
 constexpr int kMoeBigRows = 128;
 
-__device__ __forceinline__ int big_off(int row, int ch) { return row * 128 + ((ch ^ ((row >> 1) & 7)) * 16); }
-template <int MODE>
+// D: depth of a slice, 64 or 32.  A piece of 1 KiB is 512 / D rows of 2 D bytes, lane l fills bytes 16 l .. of it.
+template <int D>
+__device__ __forceinline__ int big_off(int row, int ch) {
+    return row * 2 * D + ((ch ^ (D == 64 ? (row >> 1) & 7 : (row >> 2) & 3)) * 16);
+}
+template <int MODE, int D>
 __global__ __launch_bounds__(256, 2) void moe_big_kernel(
     const __bf16* __restrict__ a, int64_t a_stride, const __bf16* __restrict__ w, const int* __restrict__ sorted_pairs,
     const int* __restrict__ meta, const float* __restrict__ pair_w, __bf16* __restrict__ y, float* __restrict__ out, int top, int N,
     int K, float limit, float alpha, float up_shift) {
     constexpr bool GATE_UP = MODE == 1, GATHER = MODE != 0;
-    constexpr int COLS = GATE_UP ? 128 : 256, XB = kMoeBigRows * 128;       // bytes: rows' slice
-    __shared__ __attribute__((aligned(16))) unsigned char buf[XB + 256 * 128];
+    constexpr int COLS = GATE_UP ? 128 : 256, XB = kMoeBigRows * 2 * D, BUF = XB + 256 * 2 * D;       // bytes: rows' slice, both slices
+    __shared__ __attribute__((aligned(16))) unsigned char buf[BUF], buf1[D == 64 ? 16 : BUF], buf2[D == 64 ? 16 : BUF];
     __shared__ int src_row[kMoeBigRows];
     __shared__ float weight[MODE == 0 ? kMoeBigRows : 1];
     // Workgroups go to the eight XCDs in turn; an XCD takes a run of the tiles that there are, all column blocks of a tile next to each
@@ -514,33 +519,67 @@ __global__ __launch_bounds__(256, 2) void moe_big_kernel(
     }
     __syncthreads();
     const __bf16* we = w + (int64_t)e * ((GATE_UP ? 2 : 1) * (int64_t)N) * K;
-    // a piece of 1 KiB: 8 rows of 128 bytes, lane l fills bytes 16 l .. of it; a wave takes four of the rows and eight of the weight rows
+    // a wave stages XP pieces of the rows and WP of the weight rows
+    constexpr int PR = 512 / D, XP = kMoeBigRows / PR / 4, WP = 256 / PR / 4;
+    const int p_row = lane / (D / 8), p_ch = lane % (D / 8);
+    // 64 deep: 32-bit offsets from the first row and from the expert's first weight row (the launch sees to it that they fit)
     const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(GATHER ? a : a + (int64_t)row0 * a_stride), 0, -1, 0x00020000);
     const auto wr_ = __builtin_amdgcn_make_buffer_rsrc((void*)we, 0, -1, 0x00020000);
-    const int p_row = lane >> 3;
-    uint32_t x_lane[4], w_lane[2], w_piece[8];        // (the launch keeps all offsets below 4 GiB)
+    uint32_t x_lane[4], w_lane[2], w_piece[8];
+    const char *xp[2], *wp[4];                        // 32 deep: addresses
+    if constexpr (D == 64) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int r = (wave * 4 + i) * 8 + p_row;
-        x_lane[i] = ((uint32_t)(GATHER ? src_row[r] / top : min(r, rows - 1)) * (uint32_t)a_stride + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2u;
+        for (int i = 0; i < XP; ++i) {
+            const int r = (wave * XP + i) * PR + p_row;
+            x_lane[i] = ((uint32_t)(GATHER ? src_row[r] / top : min(r, rows - 1)) * (uint32_t)a_stride + (p_ch ^ ((r >> 1) & 7)) * 8) * 2u;
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) w_lane[i] = (uint32_t)(p_row * K + (p_ch ^ (i * 4 + (p_row >> 1))) * 8) * 2u;
+        // (N is a multiple of 8: a piece's weight rows are all there or none of them is)
+#pragma unroll
+        for (int i = 0; i < WP; ++i) {
+            const int lr = (wave * WP + i) * PR;      // first weight row of the piece: gate rows, then up rows
+            w_piece[i] = (uint32_t)(GATE_UP ? (lr >> 7) * N + min(n0 + (lr & 127), N - 8) : min(n0 + lr, N - 8)) * (uint32_t)K * 2u;
+        }
+    } else {
+        const int ch = p_ch ^ ((p_row >> 2) & 3);
+#pragma unroll
+        for (int i = 0; i < XP; ++i) {
+            const int r = (wave * XP + i) * PR + p_row;
+            const int64_t at = GATHER ? (int64_t)(src_row[r] / top) : row0 + min(r, rows - 1);
+            xp[i] = (const char*)(a + at * a_stride + ch * 8);
+        }
+#pragma unroll
+        for (int i = 0; i < WP; ++i) {
+            const int lr = (wave * WP + i) * PR + p_row;
+            const int64_t n = GATE_UP ? (lr >> 7) * (int64_t)N + min(n0 + (lr & 127), N - 1) : min(n0 + lr, N - 1);
+            wp[i] = (const char*)(we + n * K + ch * 8);
+        }
     }
+    auto stage = [&](unsigned char* dst, int t) {     // (32 deep: the slices one after the other)
+        if constexpr (D == 64) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) w_lane[i] = (uint32_t)(p_row * K + ((lane & 7) ^ (i * 4 + (p_row >> 1))) * 8) * 2u;
-    // (N is a multiple of 8: a piece's weight rows are all there or none of them is)
+            for (int i = 0; i < WP; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(wr_, (__attribute__((address_space(3))) void*)(dst + XB + (wave * WP + i) * 1024), 16,
+                                                         w_lane[i & 1], w_piece[i] + t * 128, 0, 0);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int lr = (wave * 8 + i) * 8;            // first weight row of the piece: gate rows, then up rows
-        w_piece[i] = (uint32_t)(GATE_UP ? (lr >> 7) * N + min(n0 + (lr & 127), N - 8) : min(n0 + lr, N - 8)) * (uint32_t)K * 2u;
-    }
-    auto stage = [&](int t) {
+            for (int i = 0; i < XP; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(dst + (wave * XP + i) * 1024), 16, x_lane[i],
+                                                         t * 128, 0, 0);
+        } else {
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(wr_, (__attribute__((address_space(3))) void*)(buf + XB + (wave * 8 + i) * 1024), 16,
-                                                     w_lane[i & 1], w_piece[i] + t * 128, 0, 0);
+            for (int i = 0; i < XP; ++i) {
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)xp[i],
+                                                 (__attribute__((address_space(3))) void*)(dst + (wave * XP + i) * 1024), 16, 0, 0);
+                xp[i] += 64;
+            }
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(buf + (wave * 4 + i) * 1024), 16, x_lane[i],
-                                                     t * 128, 0, 0);
+            for (int i = 0; i < WP; ++i) {
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)wp[i],
+                                                 (__attribute__((address_space(3))) void*)(dst + XB + (wave * WP + i) * 1024), 16, 0, 0);
+                wp[i] += 64;
+            }
+        }
     };
     f32x16 acc[4][2];                                 // [weight block: gate 0, 1, up 0, 1 | 0 .. 3][row block]
 #pragma unroll
@@ -549,14 +588,14 @@ __global__ __launch_bounds__(256, 2) void moe_big_kernel(
         for (int x = 0; x < 2; ++x)
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[j][x][i] = 0.f;
-    bf16x8 xf[4][2], wf[4][4];                        // operands of the four 16-deep steps of a slice
-    auto read = [&](int s) {
+    bf16x8 xf[D / 16][2], wf[D / 16][4];              // operands of the 16-deep steps of a slice
+    auto read = [&](const unsigned char* src, int s) {
 #pragma unroll
-        for (int x = 0; x < 2; ++x) xf[s][x] = *(const bf16x8*)(buf + big_off(wr * 64 + x * 32 + l32, 2 * s + hh));
+        for (int x = 0; x < 2; ++x) xf[s][x] = *(const bf16x8*)(src + big_off<D>(wr * 64 + x * 32 + l32, 2 * s + hh));
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int lr = GATE_UP ? (j >> 1) * 128 + wc * 64 + (j & 1) * 32 : wc * 128 + j * 32;
-            wf[s][j] = *(const bf16x8*)(buf + XB + big_off(lr + l32, 2 * s + hh));
+            wf[s][j] = *(const bf16x8*)(src + XB + big_off<D>(lr + l32, 2 * s + hh));
         }
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -567,34 +606,67 @@ __global__ __launch_bounds__(256, 2) void moe_big_kernel(
             for (int x = 0; x < 2; ++x) acc[j][x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[s][j], xf[s][x], acc[j][x], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
     };
-    const int slices = K / 64;
-    stage(0);
-    for (int t = 0; t < slices; ++t) {
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(0x70);             // vmcnt(0) lgkmcnt(0): this wave's part of the slice has landed
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int s = 0; s < 4; ++s) read(s);
-        if (t + 1 < slices) {
+    const int slices = K / D;
+    if constexpr (D == 64) {
+        stage(buf, 0);
+        for (int t = 0; t < slices; ++t) {
             asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_waitcnt(0xc07f);       // lgkmcnt(0): the wave has read the slice
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_waitcnt(0x70);         // vmcnt(0) lgkmcnt(0): this wave's part of the slice has landed
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
-            stage(t + 1);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) multiply(s);
-        __builtin_amdgcn_s_setprio(0);
+            for (int s = 0; s < 4; ++s) read(buf, s);
+            if (t + 1 < slices) {
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the wave has read the slice
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                stage(buf, t + 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) multiply(s);
+            __builtin_amdgcn_s_setprio(0);
+        }
+    } else {
+        // One slice: this wave's part of it has landed (all but the newest six loads have) and the wave is done reading the one before;
+        // past the barrier so it is for all waves, and the slice after the next one goes where the one before was.  An LDS object per buffer and
+        // no condition inside the loop: the compiler waits for the loads just issued in front of every read otherwise (36 -> 48 us).
+        auto step = [&](bool more, bool stages, const unsigned char* now, unsigned char* after_next) {
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);        // (nor may the products sink below the wait)
+            if (more) __builtin_amdgcn_s_waitcnt(0x76);       // vmcnt(6) lgkmcnt(0): the six of the next slice stay in flight
+            else __builtin_amdgcn_s_waitcnt(0x70);    // vmcnt(0) lgkmcnt(0)
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            if (stages) stage(after_next, 0);
+            __builtin_amdgcn_sched_barrier(0);        // (the compiler would start the loads behind the products)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) read(now, s);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) multiply(s);
+        };
+        stage(buf, 0);                                // (at least 2 slices: K is a multiple of 64)
+        stage(buf1, 0);
+        int t = 0;
+        for (; t + 4 < slices; t += 3) {
+            step(true, true, buf, buf2);
+            step(true, true, buf1, buf);
+            step(true, true, buf2, buf1);
+        }
+        const int left = slices - t;                  // 2 .. 4
+        step(true, left > 2, buf, buf2);
+        step(left > 2, left > 3, buf1, buf);
+        if (left > 2) step(left > 3, false, buf2, buf1);
+        if (left > 3) step(false, false, buf, buf2);
     }
     __syncthreads();                                  // the slices are done with: each wave turns its blocks through LDS of its own
     // lane (l32, hh) holds of row 64 wr + 32 x + l32 the weight rows 8 (i >> 2) + 4 hh + (i & 3) of each block
     if constexpr (MODE != 0) {
         constexpr int CW = GATE_UP ? 64 : 128, LD = CW * 2 + 16;       // columns of the wave; bytes of a staged row
-        unsigned char* st = buf + wave * 32 * LD;
+        unsigned char* st = D == 64 ? buf + wave * 32 * LD : (wave < 2 ? buf : buf1) + (wave & 1) * 32 * LD;
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
 #pragma unroll
@@ -625,7 +697,7 @@ __global__ __launch_bounds__(256, 2) void moe_big_kernel(
         }
     } else {
         constexpr int LD = 64 * 4 + 16;
-        unsigned char* st = buf + wave * 32 * LD;
+        unsigned char* st = D == 64 ? buf + wave * 32 * LD : (wave < 2 ? buf : buf1) + (wave & 1) * 32 * LD;
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
 #pragma unroll
@@ -906,14 +978,21 @@ static bool moe_offsets_ok(int64_t a_rows, int64_t a_stride, int64_t w_rows, int
 template <typename T, int MODE>
 static void launch_grouped(const void* a, int64_t a_stride, const void* w, const int* sorted_pairs, const int* meta,
                            const float* pair_w, void* y, float* out, int top, int N, int K, float limit, float alpha,
-                           float up_shift, int max_tiles, int tile_rows, int64_t a_rows, hipStream_t s) {
+                           float up_shift, int64_t pairs, int E, int tile_rows, int64_t a_rows, hipStream_t s) {
+    const int max_tiles = (int)nv_moe_max_tiles(pairs, E, tile_rows);
     // activations and outputs that do not start on 16 bytes take the general launch, in tiles of any size
     const bool pieces = sizeof(T) == 2 && (MODE == 0 ? (uintptr_t)out : (uintptr_t)y) % 16 == 0 && moe_pieces_ok(NV_DTYPE_BF16, a, a_stride, w, N, K);
     if constexpr (sizeof(T) == 2) {
         if (pieces && tile_rows == kMoeBigRows && moe_offsets_ok(MODE == 0 ? kMoeBigRows : a_rows, a_stride, (MODE == 1 ? 2 : 1) * (int64_t)N, K)) {
             constexpr int cols = MODE == 1 ? 128 : 256;
-            hipLaunchKernelGGL(moe_big_kernel<MODE>, dim3((unsigned)(((int64_t)max_tiles * ((N + cols - 1) / cols) + 7) / 8 * 8)), dim3(256), 0, s,
-                               (const T*)a, a_stride, (const T*)w, sorted_pairs, meta, pair_w, (T*)y, out, top, N, K, limit, alpha, up_shift);
+            const int n_cols = (N + cols - 1) / cols;
+            const dim3 grid((unsigned)(((int64_t)max_tiles * n_cols + 7) / 8 * 8));
+            if (moe_few_blocks(pairs, E, n_cols))
+                hipLaunchKernelGGL((moe_big_kernel<MODE, 32>), grid, dim3(256), 0, s, (const T*)a, a_stride, (const T*)w, sorted_pairs, meta, pair_w,
+                                   (T*)y, out, top, N, K, limit, alpha, up_shift);
+            else
+                hipLaunchKernelGGL((moe_big_kernel<MODE, 64>), grid, dim3(256), 0, s, (const T*)a, a_stride, (const T*)w, sorted_pairs, meta, pair_w,
+                                   (T*)y, out, top, N, K, limit, alpha, up_shift);
             return;
         }
     }
@@ -1074,10 +1153,10 @@ extern "C" int nv_moe_gate_up_act(const void* h, int64_t h_stride, const void* g
     hipStream_t s = (hipStream_t)stream;
     if (dtype == NV_DTYPE_BF16)
         launch_grouped<__bf16, 1>(h, h_stride, gate_up, sorted_pairs, meta, nullptr, y, nullptr, top, ff, width, limit,
-                                     alpha, up_shift, (int)tiles, tile_rows, pairs / top, s);
+                                     alpha, up_shift, pairs, E, tile_rows, pairs / top, s);
     else
         launch_grouped<float, 1>(h, h_stride, gate_up, sorted_pairs, meta, nullptr, y, nullptr, top, ff, width, limit,
-                                    alpha, up_shift, (int)tiles, tile_rows, pairs / top, s);
+                                    alpha, up_shift, pairs, E, tile_rows, pairs / top, s);
     return check_launch("nv_moe_gate_up");
 }
 
@@ -1097,10 +1176,10 @@ extern "C" int nv_moe_down(const void* y, const void* down, const int32_t* sorte
     hipStream_t s = (hipStream_t)stream;
     if (dtype == NV_DTYPE_BF16)
         launch_grouped<__bf16, 0>(y, ff, down, sorted_pairs, meta, pair_weights, nullptr, out, 1, width, ff, 0.f, 0.f, 0.f,
-                                      (int)tiles, tile_rows, pairs, s);
+                                      pairs, E, tile_rows, pairs, s);
     else
         launch_grouped<float, 0>(y, ff, down, sorted_pairs, meta, pair_weights, nullptr, out, 1, width, ff, 0.f, 0.f, 0.f,
-                                     (int)tiles, tile_rows, pairs, s);
+                                     pairs, E, tile_rows, pairs, s);
     return check_launch("nv_moe_down");
 }
 
@@ -1137,10 +1216,10 @@ extern "C" int nv_moe_up_relu2(const void* h, int64_t h_stride, const void* up, 
     hipStream_t s = (hipStream_t)stream;
     if (dtype == NV_DTYPE_BF16)
         launch_grouped<__bf16, 2>(h, h_stride, up, sorted_pairs, meta, nullptr, y, nullptr, top, ff, width, 0.f, 0.f, 0.f,
-                                  (int)tiles, tile_rows, pairs / top, s);
+                                  pairs, E, tile_rows, pairs / top, s);
     else
         launch_grouped<float, 2>(h, h_stride, up, sorted_pairs, meta, nullptr, y, nullptr, top, ff, width, 0.f, 0.f, 0.f,
-                                 (int)tiles, tile_rows, pairs / top, s);
+                                 pairs, E, tile_rows, pairs / top, s);
     return check_launch("nv_moe_up_relu2");
 }
 

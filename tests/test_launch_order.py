@@ -1,4 +1,4 @@
-"""Index arithmetic of launches that choose their order or key ranges on the device, over many launch shapes with a host compiler."""
+"""Rules and index arithmetic of launches, over many launch shapes with a host compiler."""
 import ctypes as C
 import os
 import subprocess
@@ -15,6 +15,7 @@ extern "C" int latent(int64_t total, int slots, int last_key, int tile_keys, int
     *tiles = latent_tiles(last_key, tile_keys, nsplit, fewest);
     return latent_ranges(*tiles, *share);
 }
+extern "C" int few_blocks(int64_t pairs, int E, int n_cols) { return moe_few_blocks(pairs, E, n_cols); }
 """
 
 
@@ -27,6 +28,7 @@ def order(tmp_path_factory):
                     str(src), "-o", str(lib)], check=True)
     dll = C.CDLL(str(lib))
     dll.latent.argtypes = [C.c_int64] + [C.c_int] * 5 + [C.POINTER(C.c_int)] * 2
+    dll.few_blocks.argtypes = [C.c_int64, C.c_int, C.c_int]
     return dll
 
 
@@ -41,3 +43,10 @@ def test_latent_ranges_stay_within_what_was_stated(order):
                 assert share.value >= fewest and 1 <= n <= nsplit
                 assert tiles.value == min(last_key // 64 + 1, nsplit * fewest)
                 assert (n - 1) * share.value < tiles.value <= n * share.value
+
+
+def test_experts_one_workgroup_a_cu(order):
+    """Tiles of 128 rows: (pairs an expert, experts, column blocks) on either side of what was measured."""
+    for per, E, cols, few in ((40, 16, 8, 1), (96, 16, 8, 1), (96, 32, 8, 1), (100, 32, 8, 1), (112, 32, 8, 0), (192, 16, 8, 1), (256, 16, 8, 0),
+                              (256, 16, 4, 1), (512, 16, 4, 0), (40, 64, 8, 0), (1024, 32, 8, 0), (1024, 1, 16, 1)):
+        assert order.few_blocks(per * E, E, cols) == few, (per, E, cols)
