@@ -969,8 +969,8 @@ static bool moe_pieces_ok(int dtype, const void* a, int64_t a_stride, const void
     return dtype == NV_DTYPE_BF16 && K % 64 == 0 && N % 8 == 0 && a_stride % 8 == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0;
 }
 
-// A block's offsets from the first row and from the expert's first weight row, in bytes, are 32 bits (tiles of 128 rows beyond that, an input or an
-// expert's matrix of 4 GiB, take the general launch).
+// Offsets from the first row and from the expert's first weight row are 32 bits in bytes, 64 deep; an input or an expert's matrix of 4 GiB takes
+// slices 32 deep by address.
 static bool moe_offsets_ok(int64_t a_rows, int64_t a_stride, int64_t w_rows, int K) {
     return a_rows * a_stride < (1LL << 31) - K && w_rows * K < (1LL << 31) - K;
 }
@@ -983,11 +983,11 @@ static void launch_grouped(const void* a, int64_t a_stride, const void* w, const
     // activations and outputs that do not start on 16 bytes take the general launch, in tiles of any size
     const bool pieces = sizeof(T) == 2 && (MODE == 0 ? (uintptr_t)out : (uintptr_t)y) % 16 == 0 && moe_pieces_ok(NV_DTYPE_BF16, a, a_stride, w, N, K);
     if constexpr (sizeof(T) == 2) {
-        if (pieces && tile_rows == kMoeBigRows && moe_offsets_ok(MODE == 0 ? kMoeBigRows : a_rows, a_stride, (MODE == 1 ? 2 : 1) * (int64_t)N, K)) {
+        if (pieces && tile_rows == kMoeBigRows) {
             constexpr int cols = MODE == 1 ? 128 : 256;
             const int n_cols = (N + cols - 1) / cols;
             const dim3 grid((unsigned)(((int64_t)max_tiles * n_cols + 7) / 8 * 8));
-            if (moe_few_blocks(pairs, E, n_cols))
+            if (moe_few_blocks(pairs, E, n_cols) || !moe_offsets_ok(MODE == 0 ? kMoeBigRows : a_rows, a_stride, (MODE == 1 ? 2 : 1) * (int64_t)N, K))
                 hipLaunchKernelGGL((moe_big_kernel<MODE, 32>), grid, dim3(256), 0, s, (const T*)a, a_stride, (const T*)w, sorted_pairs, meta, pair_w,
                                    (T*)y, out, top, N, K, limit, alpha, up_shift);
             else
