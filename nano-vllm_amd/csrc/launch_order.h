@@ -35,4 +35,17 @@ NV_HD bool moe_few_blocks(int64_t pairs, int E, int n_cols) {
     return (pairs <= 100 * (int64_t)E ? E : pairs / 128 + E / 2) * n_cols <= 256;
 }
 
+// Tiles of up to 64 rows past LDS, an expert's weights once for each of its tiles, or through it.  What pays depends on how many tiles read
+// the same weights, and where a whole tile an expert does, on how many blocks of 128 x 128 the first product has.  Both products, us, past / through LDS:
+//   tiles of 16: 32 experts, 2048, 1024: 8 pairs an expert 69 / 65 (weights from memory: 76 / 91), 12: 75 / 67 (83 / 92), 20: 108 / 71 (113 / 96);
+//     16 of 2048, 1024: 12: 49 / 45 (54 / 62), 16: 48 / 46 (52 / 64), 20: 59 / 46 (62 / 64)
+//   tiles of 64, 256 blocks: 32 of 2048, 1024: 32: 92 / 82 (98 / 100), 40: 99 / 85 (105 / 104), 64: 142 / 102, 1024: 1477 / 713
+//     128 blocks: 16 of 2048, 1024: 48: 54 / 74, 56: 73 / 75 (77 / 88), 64: 86 / 76;  32 of 1024, 512: 56: 44 / 47, 64: 54 / 47
+//     64 blocks: 16 of 1024, 512: 64: 32 / 44, 96: 33 / 44, 160: 53 / 46
+NV_HD bool moe_streams(int tile_rows, int64_t pairs, int E, int ff) {
+    const int64_t blocks = (int64_t)E * ((ff + 127) / 128);
+    const int line = tile_rows == 16 ? 16 : tile_rows == 32 ? 28 : tile_rows == 64 ? (blocks >= 256 ? 40 : blocks >= 128 ? 64 : 128) : 0;
+    return pairs < line * (int64_t)E;
+}
+
 }  // namespace nv

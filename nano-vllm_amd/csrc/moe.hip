@@ -997,7 +997,7 @@ static void launch_grouped(const void* a, int64_t a_stride, const void* w, const
         }
     }
     if constexpr (sizeof(T) == 2) {
-        if (pieces && tile_rows < kMoeBigRows) {
+        if (pieces && moe_streams(tile_rows, pairs, E, MODE == 0 ? K : N)) {
             const int64_t items = (int64_t)max_tiles * ((N + (MODE == 1 ? 31 : 63)) / (MODE == 1 ? 32 : 64));
 #define NV_MOE_ROWS(MT)                                                                                                              \
     hipLaunchKernelGGL((moe_rows_kernel<MODE, MT>), dim3((unsigned)((items + 7) / 8 * 8)), dim3(256), 0, s, (const T*)a, a_stride, (const T*)w, \

@@ -15,6 +15,7 @@ extern "C" int latent(int64_t total, int slots, int last_key, int tile_keys, int
     *tiles = latent_tiles(last_key, tile_keys, nsplit, fewest);
     return latent_ranges(*tiles, *share);
 }
+extern "C" int streams(int tile_rows, int64_t pairs, int E, int ff) { return moe_streams(tile_rows, pairs, E, ff); }
 extern "C" int few_blocks(int64_t pairs, int E, int n_cols) { return moe_few_blocks(pairs, E, n_cols); }
 """
 
@@ -29,6 +30,7 @@ def order(tmp_path_factory):
     dll = C.CDLL(str(lib))
     dll.latent.argtypes = [C.c_int64] + [C.c_int] * 5 + [C.POINTER(C.c_int)] * 2
     dll.few_blocks.argtypes = [C.c_int64, C.c_int, C.c_int]
+    dll.streams.argtypes = [C.c_int, C.c_int64, C.c_int, C.c_int]
     return dll
 
 
@@ -50,3 +52,15 @@ def test_experts_one_workgroup_a_cu(order):
     for per, E, cols, few in ((40, 16, 8, 1), (96, 16, 8, 1), (96, 32, 8, 1), (100, 32, 8, 1), (112, 32, 8, 0), (192, 16, 8, 1), (256, 16, 8, 0),
                               (256, 16, 4, 1), (512, 16, 4, 0), (40, 64, 8, 0), (1024, 32, 8, 0), (1024, 1, 16, 1)):
         assert order.few_blocks(per * E, E, cols) == few, (per, E, cols)
+
+
+def test_experts_weights_past_lds(order):
+    """The tiles of nv_moe_tile_rows (16 rows, 64 from 32 pairs an expert on) do not read an expert's weights once for each of many tiles."""
+    from nanovllm_amd import _lib
+    rows = _lib.mixers().nv_moe_tile_rows
+    for E, ff, past in ((32, 1024, (1, 8, 12, 32, 36)), (16, 1024, (1, 8, 12, 32, 48, 56)), (32, 512, (8, 32, 56)), (16, 512, (8, 32, 96))):
+        for per in past:
+            assert order.streams(rows(per * E, E), per * E, E, ff), (E, ff, per)
+        for per in (20, 24, 31, 160, 256, 1024, 10 ** 5):
+            assert not order.streams(rows(per * E, E), per * E, E, ff), (E, ff, per)
+    assert not any(order.streams(64, 64 * E, E, ff) for E, ff in ((32, 1024), (16, 1024), (32, 512)))
