@@ -1052,17 +1052,19 @@ extern "C" int nv_moe_tile_rows(int64_t pairs, int E) { return pairs >= 32 * (in
 // more rows a tile and saves the second reading of an expert that has more), then of 128 staged through LDS, which wants enough of its
 // 128 x 256 blocks to fill the chip.  Whole calls, us, tiles of 16 / 32 / 64 / 128 rows:
 //   top 4 of 32 experts, width 2048, ff 1024:  6 pairs an expert 83 / 86 / 89 / 108, 16: 107 / 96 / 101 / 113, 24: 134 / 107 / 105 / 115,
-//   32: 149 / 121 / 112 / 116, 40: 174 / 142 / 118 / 117, 64: 252 / 178 / 156 / 123 (blocks of 64 x 128 through LDS took 117 to 141 for all of these)
+//   32: 149 / 121 / 112 / 116, 40: 174 / 142 / 118 / 117, 64: 252 / 178 / 156 / 123
 //   top 2 of 32, 1024, 1024:  16: 53 / 48 / 51 / 54, 32: 78 / 63 / 57 / 56, 48: 105 / 79 / 65 / 59
 //   top 2 of 16, 1024, 512:  6: 18 / 18 / 20 / 38, 24: 27 / 29 / 25 / 40, 64: 47 / 39 / 39 / 42, 96: 61 / 52 / 40 / 42, 128: 73 / 58 / 59 / 45
 //   top 4 of 16, 2048, 512:  12: 36 / 30 / 30 / 53, 48: 66 / 51 / 39 / 57, 96: 104 / 83 / 64 / 59
-// tiles of 64 / 128 rows:  top 2 of 16, 2048, 1024:  48: 60 / 69, 64: 94 / 70;  top 4 of 32, 1024, 512:  40: 42 / 45, 48: 51 / 45
+// With 128 blocks it is the first expert that has more than 64 rows which decides, so routings differ.  Both products, tiles of 64 in four routings and of 128:
+//   top 2 of 16, 2048, 1024:  48: 53, 53, 52, 54 and 57, 52: 67, 54, 54, 70 and 57, 56: 69, 72, 73, 72 and 57 (weights from memory: 48: 59 and 73, 56: 77 and 74)
+//   top 4 of 32, 1024, 512:  48: 43, 34, 34, 41 and 37, 52: 44, 44, 35, 42 and 37 (48: 36 and 42, 52: 45 and 43)
 extern "C" int nv_moe_tile_rows_for(int64_t pairs, int E, int width, int ff, const void* h, int64_t h_stride, const void* up,
                                     const void* down, int dtype) {
     using namespace nv;
     if (!moe_pieces_ok(dtype, h, h_stride, up, ff, width) || !moe_pieces_ok(dtype, nullptr, ff, down, width, ff)) return nv_moe_tile_rows(pairs, E);
     const int64_t blocks = (int64_t)E * ((ff + 127) / 128);           // of the first product, a tile an expert
-    if (pairs >= (blocks >= 256 ? 40 : blocks >= 128 ? 48 : 84) * (int64_t)E) return kMoeBigRows;
+    if (pairs >= (blocks >= 256 ? 40 : blocks >= 128 ? 52 : 84) * (int64_t)E) return kMoeBigRows;
     return pairs >= 24 * (int64_t)E ? 64 : pairs >= 8 * (int64_t)E ? 32 : 16;
 }
 

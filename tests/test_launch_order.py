@@ -64,3 +64,11 @@ def test_experts_weights_past_lds(order):
         for per in (20, 24, 31, 160, 256, 1024, 10 ** 5):
             assert not order.streams(rows(per * E, E), per * E, E, ff), (E, ff, per)
     assert not any(order.streams(64, 64 * E, E, ff) for E, ff in ((32, 1024), (16, 1024), (32, 512)))
+
+
+def test_experts_tile_rows():
+    """Where tiles of 128 rows start, on either side of the lines: blocks of 128 x 128 of the first product, pairs an expert."""
+    from nanovllm_amd import _lib
+    rows_for = lambda E, W, ff, per: _lib.mixers().nv_moe_tile_rows_for(per * E, E, W, ff, 4096, W, 4096, 4096, 0)
+    for E, W, ff, line in ((32, 2048, 1024, 40), (64, 2048, 512, 40), (16, 2048, 1024, 52), (32, 1024, 512, 52), (16, 1024, 512, 84)):
+        assert [rows_for(E, W, ff, per) for per in (7, 8, 23, 24, line - 1, line)] == [16, 32, 32, 64, 64, 128], (E, W, ff)
