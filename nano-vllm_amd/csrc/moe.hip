@@ -38,7 +38,9 @@ constexpr int kMoeBN = 64;
 constexpr int kMoeRoutePerLane = 8;            // experts <= 512 stay in registers
 constexpr int kMoeNone = 0x7fffffff;
 __device__ __forceinline__ void moe_better(float& v, int& e, float ov, int oe) {
-    if (oe != kMoeNone && (e == kMoeNone || ov > v || (ov == v && oe < e))) { v = ov; e = oe; }
+    const bool take = (oe != kMoeNone) & ((e == kMoeNone) | (ov > v) | ((ov == v) & (oe < e)));      // (no branches)
+    v = take ? ov : v;
+    e = take ? oe : e;
 }
 template <int CTRL>
 __device__ __forceinline__ void moe_better_dpp(float& v, int& e) {
@@ -323,10 +325,16 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
 }
 
 // Routing and sort together.  Few tokens: one launch of one workgroup, the pairs' ids and places stay in registers.  More: the
-// first launch routes kMoeSortTokens or more tokens a workgroup and leaves every workgroup's counts per expert, the second one adds them up
-// and places the pairs; the single workgroup of moe_align_kernel spends its time on 32768 additions to LDS.  Top 4 of 32 experts, two
-// launches of their own against these: 8192 tokens 13 + 21 -> 7 + 5 us, 256 tokens 6.5 + 4.8 -> 4.7 + 4.6, 32 tokens 6.6 + 4.8 -> 5.
-constexpr int kMoeSortMaxE = 512, kMoeSortFew = 128, kMoeSortTokens = 16, kMoeSortGroups = 256;
+// first launch routes a few tokens a workgroup and leaves every workgroup's counts per expert, the second one adds them up
+// and places the pairs; the single workgroup of moe_align_kernel spends its time on 32768 additions to LDS.  Beyond 64 experts a token takes a
+// wave for a microsecond a choice, so that a wave has one as long as the counts of the workgroups stay few.
+// Two launches of their own against these, us:
+//   top 4 of 32 experts, 32 tokens 11.1 -> 4.7, 128: 11.5 -> 7.7, 256: 11.8 -> 7.4, 8192: 36.2 -> 12.8
+//   top 8 of 65: 8 tokens 17.6 -> 9.2, 128: 18.6 -> 12.1 (82 in one workgroup), 1024: 23.6 -> 17.4 (35 with four tokens a wave), 8192: 66.5 -> 60.9
+//   top 8 of 512: 8 tokens 45 -> 11.4, 128: 47 -> 16.9, 1024: 52 -> 32.5, 8192: 104 -> 84;  top 2 of 65, 4096 and 8192: 17.6 -> 18.4, 24.8 -> 25.5
+constexpr int kMoeSortMaxE = 512, kMoeSortGroups = 256;
+constexpr __host__ __device__ int moe_sort_few(int E) { return E <= 64 ? 128 : 16; }
+constexpr __host__ __device__ int moe_sort_least(int E) { return E <= 64 ? 16 : 4; }         // a token a wave, four side by side up to 64 experts
 
 // first / first_tile [E + 1] from the counts by one wave (in LDS)
 __device__ __forceinline__ void moe_scan(const int* counts, int* first, int* first_tile, int E, int tile_rows, int lane) {
@@ -370,7 +378,7 @@ __global__ __launch_bounds__(1024) void moe_route_sort_few_kernel(const float* _
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     for (int e = tid; e < E; e += 1024) counts[e] = 0;
     __syncthreads();
-    constexpr int G = PER == 1 ? 4 : 1, N = kMoeSortFew / (16 * G);      // tokens of a wave side by side; times
+    constexpr int G = PER == 1 ? 4 : 1, N = moe_sort_few(64 * PER) / (16 * G);       // tokens of a wave side by side; times
     const int at = lane & (64 / G - 1), mine = wave * G + lane / (64 / G);
     int id[N], place[N];
     float reg[PER == 1 ? N : 1][4];
@@ -1092,13 +1100,18 @@ extern "C" int nv_moe_align(const int32_t* ids, int32_t* sorted_pairs, int32_t* 
     return check_launch("nv_moe_align");
 }
 
-static int moe_sort_tokens(int64_t T) {               // of a workgroup of the first launch
-    const int64_t least = (T + nv::kMoeSortGroups - 1) / nv::kMoeSortGroups;
-    return (int)std::max<int64_t>(nv::kMoeSortTokens, (least + 15) / 16 * 16);
+// Tokens of a workgroup of the first launch.  Beyond 64 experts a wave's next token costs a microsecond a choice, and a workgroup more
+// costs every workgroup of the second launch E counts, about a microsecond for 5200.
+static int moe_sort_tokens(int64_t T, int E, int top) {
+    const int whole = nv::moe_sort_least(E);
+    int64_t n = (T + nv::kMoeSortGroups - 1) / nv::kMoeSortGroups;
+    n = (n + whole - 1) / whole * whole;
+    while (E > 64 && n * n * top * 1300 < T * E) n += whole;
+    return (int)n;
 }
 extern "C" int64_t nv_moe_route_sort_words(int64_t T, int E) {
-    if (T <= nv::kMoeSortFew || E > nv::kMoeSortMaxE) return 0;
-    const int tokens = moe_sort_tokens(T);
+    if (T <= nv::moe_sort_few(E) || E > nv::kMoeSortMaxE) return 0;
+    const int tokens = moe_sort_tokens(T, E, nv::kMoeMaxTop);         // (the most workgroups of any number of choices)
     return (T + tokens - 1) / tokens * E;
 }
 extern "C" int nv_moe_route_sort(const float* logits, int32_t* ids, float* weights, int32_t* sorted_pairs, int32_t* meta, int32_t* counts,
@@ -1110,10 +1123,10 @@ extern "C" int nv_moe_route_sort(const float* logits, int32_t* ids, float* weigh
         const int rc = nv_moe_route(logits, ids, weights, T, E, top, stream);
         return rc != NV_OK ? rc : nv_moe_align(ids, sorted_pairs, meta, T * top, E, tile_rows, stream);
     }
-    NV_REQUIRE(logits && ids && weights && sorted_pairs && meta && (counts || T <= kMoeSortFew), NV_ERR_INVALID_ARG, "nv_moe_route_sort: null pointer");
+    NV_REQUIRE(logits && ids && weights && sorted_pairs && meta && (counts || T <= moe_sort_few(E)), NV_ERR_INVALID_ARG, "nv_moe_route_sort: null pointer");
     NV_REQUIRE(T * top < (1LL << 31), NV_ERR_UNSUPPORTED, "nv_moe_route_sort: too many pairs");
     hipStream_t s = (hipStream_t)stream;
-    if (T <= kMoeSortFew) {
+    if (T <= moe_sort_few(E)) {
         if (E <= 64)
             hipLaunchKernelGGL(moe_route_sort_few_kernel<1>, dim3(1), dim3(1024), 0, s, logits, ids, weights, sorted_pairs, meta, (int)T, E, top, tile_rows);
         else
@@ -1121,7 +1134,7 @@ extern "C" int nv_moe_route_sort(const float* logits, int32_t* ids, float* weigh
                                (int)T, E, top, tile_rows);
         return check_launch("nv_moe_route_sort");
     }
-    const int tokens = moe_sort_tokens(T);
+    const int tokens = moe_sort_tokens(T, E, top);
     const unsigned groups = (unsigned)((T + tokens - 1) / tokens);
     int columns = 16;
     while (columns < E && columns < 256) columns *= 2;
