@@ -1043,7 +1043,7 @@ extern "C" int nv_attn_scoremod_paged_vld(const void* q, const void* k_cache, co
         rp.max_blocks = max_blocks_per_seq;
         rp.max_block = (int)std::max<int64_t>(0, std::min<int64_t>(num_blocks - 1, 0x7fffffff));
         rp.softcap = softcap;
-        const int rc = launch_scoremod_rows(rp, plan, D, Dv, num_seqs, max_seqlen_q, scale, s);
+        const int rc = launch_scoremod_rows(rp, plan, D, Dv, num_seqs, T, max_seqlen_q, max_seqlen_k, scale, s);
         if (rc != NV_OK) return rc;
     } else if (several && tile_ok) {
         const int tiles = (max_seqlen_q + kTileQ - 1) / kTileQ;

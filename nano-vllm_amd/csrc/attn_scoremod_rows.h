@@ -14,7 +14,7 @@ struct ScoremodRowsParams {
     int v_ld, n_dist, H, G, block_size, max_blocks, max_block;
     float softcap, scale_log2, cap_in;         // cap_in: a raw score's factor to the exponent of tanh
     int hpw, n_qtiles, wg_per_pair, n_pairs, xs_shift, slots_per_pair, grid_base, nsplit, tiles_per_split;
-    int rounds, there_and_back;                // pairs of an XCD; all workgroups run at a time
+    int rounds, even, there_and_back;          // pairs of an XCD; they are about as long (1, 0, or -1: see cu_k); all workgroups run at a time
 };
 struct ScoremodRowsPlan {
     int hpw;                                   // heads of a kv head's group that a workgroup takes (1, 2 or 4)
@@ -24,7 +24,7 @@ struct ScoremodRowsPlan {
 
 bool scoremod_rows_built(int D, int Dv, int block_size);
 ScoremodRowsPlan scoremod_rows_plan(int num_seqs, int64_t T, int H, int G, int Dv, int max_seqlen_q, int max_seqlen_k);
-int launch_scoremod_rows(ScoremodRowsParams p, const ScoremodRowsPlan& f, int D, int Dv, int num_seqs, int max_seqlen_q, float scale,
+int launch_scoremod_rows(ScoremodRowsParams p, const ScoremodRowsPlan& f, int D, int Dv, int num_seqs, int64_t total_q, int max_seqlen_q, int max_seqlen_k, float scale,
                          hipStream_t s);
 
 }  // namespace nv

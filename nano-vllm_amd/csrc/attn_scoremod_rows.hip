@@ -21,6 +21,7 @@
 #include <type_traits>
 
 #include "attn_scoremod_rows.h"
+#include "launch_order.h"
 
 namespace nv {
 
@@ -61,14 +62,27 @@ __global__ __launch_bounds__(256, 2) void scoremod_rows_kernel(const ScoremodRow
     // together and the last pair's heaviest tile began half way.  Workgroups one after the other run on the XCD's four shader engines, so
     // the pairs turn by one every time.  Where all workgroups are there from the start, 32 (one for each CU) go there and the next 32
     // back instead, so that a CU that has a heavy one gets a light one with it (one heavy after the other is better where
-    // CUs that have ended take the next).
+    // CUs that have ended take the next).  Pairs of very different lengths are no order of weight that way and go one after the other:
+    // 16 / 4 heads of 64, 16 chunks of 300 rows on 600 .. 4000 keys 121 us, together 145, 6 prompts of 300 .. 1300 50 and 57, 6 of 466 .. 862 50 and 37.
     const int split = blockIdx.x / p.grid_base, bid = blockIdx.x - split * p.grid_base;
-    const int xcd = bid & 7, slot = bid >> 3, four = slot / (4 * p.slots_per_pair), together = min(4, p.rounds - 4 * four);
-    int at = slot - four * 4 * p.slots_per_pair;
-    if (p.there_and_back && (at & 32) && (at | 31) < together * p.slots_per_pair) at ^= 31;
-    const int rank = at / together, one = at - rank * together + (p.there_and_back ? 0 : rank);
-    const int pair = (4 * four + one % together) * (8 >> p.xs_shift) + (xcd >> p.xs_shift);
-    const int widx = (rank << p.xs_shift) + (xcd & ((1 << p.xs_shift) - 1));
+    const PairGroup group = scoremod_group(bid, p.rounds, p.slots_per_pair, p.xs_shift);
+    bool even = p.even > 0;
+    if (p.even < 0) {                                 // (keys in front of the rows: the host does not know their number)
+        int longest = 0, keys = 0, n = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int pair = group.pair + i * group.step;
+            if (i < group.n && pair < p.n_pairs) {
+                const int b = pair / p.G, rows = p.cu_q[b + 1] - p.cu_q[b], n_k = rows > 1 ? p.cu_k[b + 1] - p.cu_k[b] : 0;
+                longest = max(longest, n_k);
+                keys += n_k;
+                n += rows > 1;
+            }
+        }
+        even = scoremod_even(keys, longest, n, 0);
+    }
+    const PairPlace at = scoremod_order(group, bid, p.slots_per_pair, p.xs_shift, even ? 4 : 1, even ? p.there_and_back : 0);
+    const int pair = at.pair, widx = at.place;
     if (pair >= p.n_pairs || widx >= p.wg_per_pair) return;
     const int groups = p.wg_per_pair / p.n_qtiles, hg = widx % groups, qt = p.n_qtiles - 1 - widx / groups;   // heaviest first
     const int b = pair / p.G, g = pair - b * p.G;
@@ -345,7 +359,7 @@ static void rows_by_mod(const ScoremodRowsParams& p, hipStream_t s) {
     else hipLaunchKernelGGL((scoremod_rows_kernel<D32, V32, kSrPlain>), grid, dim3(256), 0, s, p);
 }
 
-int launch_scoremod_rows(ScoremodRowsParams p, const ScoremodRowsPlan& f, int D, int Dv, int num_seqs, int max_seqlen_q, float scale,
+int launch_scoremod_rows(ScoremodRowsParams p, const ScoremodRowsPlan& f, int D, int Dv, int num_seqs, int64_t total_q, int max_seqlen_q, int max_seqlen_k, float scale,
                          hipStream_t s) {
     p.hpw = f.hpw;
     p.n_qtiles = f.n_qtiles;
@@ -354,6 +368,7 @@ int launch_scoremod_rows(ScoremodRowsParams p, const ScoremodRowsPlan& f, int D,
     p.xs_shift = f.xs_shift;
     p.slots_per_pair = f.slots_per_pair;
     p.rounds = (int)(f.grid_base / (8 * (int64_t)f.slots_per_pair));
+    p.even = max_seqlen_q != max_seqlen_k ? -1 : scoremod_even(total_q, max_seqlen_q, num_seqs, 1);
     p.there_and_back = f.grid_base * f.nsplit <= 256 * (D + Dv == 128 ? 4 : D + Dv == 192 ? 3 : 2);       // (workgroups that a CU holds)
     p.grid_base = (int)f.grid_base;
     p.nsplit = f.nsplit;

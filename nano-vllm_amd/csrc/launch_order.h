@@ -24,6 +24,35 @@ NV_HD int latent_tiles(int last_key, int tile_keys, int nsplit, int fewest) {
 // Its ranges: at most nsplit, since a share is never below `fewest`.
 NV_HD int latent_ranges(int tiles, int share) { return tiles <= share ? 1 : (tiles - 1) / share + 1; }
 
+// Score-modified attention, prompt portions: workgroup (of a key range) -> its pair of sequence and kv head and its place in the pair, heaviest query
+// tile first.  Workgroups go to the eight XCDs in turn; an XCD has `rounds` pairs (8 >> xs_shift of them a round over all XCDs), four to a group.
+// grid: 8 * rounds * slots_per_pair; places past a pair's workgroups and pairs past the last one are for the caller to leave out.
+struct PairGroup {
+    int pair, step, n;          // the group's first pair, from one pair to the next, how many there are
+    int at;                     // the workgroup's place in the group
+};
+struct PairPlace {
+    int pair, place;
+};
+NV_HD PairGroup scoremod_group(int index, int rounds, int slots_per_pair, int xs_shift) {
+    const int xcd = index & 7, slot = index >> 3, group = slot / (4 * slots_per_pair), left = rounds - 4 * group;
+    return {4 * group * (8 >> xs_shift) + (xcd >> xs_shift), 8 >> xs_shift, left < 4 ? left : 4, slot - group * 4 * slots_per_pair};
+}
+// Whether pairs are of about the same length: `n` of them (of a group of chunks; the sequences of a step of whole prompts) with `keys` keys in all.  In 170 steps of 2 to 16 sequences whole prompts gained from
+// an average of three quarters of the longest on, chunks, whose tiles are all about as heavy as their sequence is long, from eight ninths on.
+NV_HD bool scoremod_even(int64_t keys, int64_t longest, int n, int whole_prompts) {
+    return whole_prompts ? keys * 4 >= longest * n * 3 : keys * 9 >= longest * n * 8;
+}
+// together: the pairs of the group (four, or one) that are taken place by place, turning by one every time; the others one
+// after the other.  there_and_back: 32 workgroups of the XCD there and the next 32 back instead.
+NV_HD PairPlace scoremod_order(const PairGroup& g, int index, int slots_per_pair, int xs_shift, int together, int there_and_back) {
+    const int part = g.at / (together * slots_per_pair), left = g.n - part * together, n = together < left ? together : left;
+    int at = g.at - part * together * slots_per_pair;
+    if (there_and_back && (at & 32) && (at | 31) < n * slots_per_pair) at ^= 31;
+    const int rank = at / n, one = at - rank * n + (there_and_back ? 0 : rank);
+    return {g.pair + (part * together + one % n) * g.step, (rank << xs_shift) + (index & ((1 << xs_shift) - 1))};
+}
+
 // Tiles of 128 rows, no more blocks than CUs: slices 32 deep, since nothing else runs on a CU while its one workgroup waits for a slice.  Tiles of an
 // expert: one, from 100 pairs on as many as its pairs fill and a half.  First / second product of 16 or 32 experts, us, 64 and 32 deep:
 //   128 blocks   width 2048, ff 1024: 41.5 and 36.7 / 23.9 and 21.8;  width 1024, ff 512: 25.7 and 23.0 / 15.7 and 15.3

@@ -173,3 +173,21 @@ def test_every_row_whatever_the_order(H, G, n_qs):
     nv.set_context(None)
     # (as in test_portions)
     torch.testing.assert_close(o.float(), o_r.float(), rtol=2e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("H,G,n_qs,n_ks", [
+    (8, 8, [2500] * 4, None),                         # all resident, 4 rounds of 20: workgroups 32 .. 63 of an XCD's group go back
+    (16, 8, [900] * 9, None),                         # more than are resident, 9 rounds: the last group has one pair, the others turn
+    (16, 4, [300] * 6, [310, 330, 350, 340, 320, 300]),   # chunks of about the same length, a group of three pairs
+    (16, 4, [300] * 6, [2000, 330, 1200, 340, 700, 300]),  # and of very different ones: one after the other
+    (16, 4, [300, 1, 300, 40, 1], [1000, 3000, 980, 990, 64]),     # single rows between them
+    (16, 8, [700, 90, 350, 300, 410], None)])         # prompts of very different lengths
+def test_orders_of_pairs(H, G, n_qs, n_ks):
+    """Every order that the launch chooses from: every row is written once, by the workgroup that has its keys."""
+    a, r, ctx, pos, q, k, v, kc, vc = _step(H, G, 64, 64, 64, n_qs, n_ks or n_qs, softcap=25.0)
+    kc_r, vc_r = kc.clone(), vc.clone()
+    nv.set_context(ctx)
+    o, o_r = a(q, k, v, pos, kc, vc), r(q, k, v, pos, kc_r, vc_r)
+    nv.set_context(None)
+    # (as in test_portions)
+    torch.testing.assert_close(o.float(), o_r.float(), rtol=2e-2, atol=2e-2)

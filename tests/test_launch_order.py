@@ -15,6 +15,16 @@ extern "C" int latent(int64_t total, int slots, int last_key, int tile_keys, int
     *tiles = latent_tiles(last_key, tile_keys, nsplit, fewest);
     return latent_ranges(*tiles, *share);
 }
+// where every workgroup of a grid goes: pair and place, -1 for those that leave
+extern "C" void scored(int rounds, int slots, int xs_shift, int together, int there_and_back, int pairs, int places, int* pair, int* place) {
+    for (int i = 0; i < 8 * rounds * slots; ++i) {
+        const PairPlace at = scoremod_order(scoremod_group(i, rounds, slots, xs_shift), i, slots, xs_shift, together, there_and_back);
+        const bool there = at.pair < pairs && at.place < places;
+        pair[i] = there ? at.pair : -1;
+        place[i] = there ? at.place : -1;
+    }
+}
+extern "C" int even(int64_t keys, int64_t longest, int n, int whole_prompts) { return scoremod_even(keys, longest, n, whole_prompts); }
 extern "C" int streams(int tile_rows, int64_t pairs, int E, int ff) { return moe_streams(tile_rows, pairs, E, ff); }
 extern "C" int few_blocks(int64_t pairs, int E, int n_cols) { return moe_few_blocks(pairs, E, n_cols); }
 """
@@ -31,6 +41,7 @@ def order(tmp_path_factory):
     dll.latent.argtypes = [C.c_int64] + [C.c_int] * 5 + [C.POINTER(C.c_int)] * 2
     dll.few_blocks.argtypes = [C.c_int64, C.c_int, C.c_int]
     dll.streams.argtypes = [C.c_int, C.c_int64, C.c_int, C.c_int]
+    dll.even.argtypes = [C.c_int64, C.c_int64, C.c_int, C.c_int]
     return dll
 
 
@@ -72,3 +83,33 @@ def test_experts_tile_rows():
     rows_for = lambda E, W, ff, per: _lib.mixers().nv_moe_tile_rows_for(per * E, E, W, ff, 4096, W, 4096, 4096, 0)
     for E, W, ff, line in ((32, 2048, 1024, 40), (64, 2048, 512, 40), (16, 2048, 1024, 52), (32, 1024, 512, 52), (16, 1024, 512, 84)):
         assert [rows_for(E, W, ff, per) for per in (7, 8, 23, 24, line - 1, line)] == [16, 32, 32, 64, 64, 128], (E, W, ff)
+
+
+@pytest.mark.parametrize("there_and_back", [0, 1])
+@pytest.mark.parametrize("together", [1, 4])
+def test_scored_every_place_once(order, together, there_and_back):
+    """Every query tile of every pair of sequence and kv head is one workgroup's, whatever the order; and all pairs of an XCD's group stay there."""
+    for pairs in (1, 2, 3, 4, 7, 8, 9, 24, 33, 64, 72):
+        for xs_shift in ([0] if pairs > 4 else [0, 1, 2, 3]):
+            rounds = -(-pairs // (8 >> xs_shift))
+            for places in (1, 2, 5, 8, 20, 31, 32, 33, 64, 97):
+                slots = -(-places // (1 << xs_shift))
+                n = 8 * rounds * slots
+                pair, place = (C.c_int * n)(), (C.c_int * n)()
+                order.scored(rounds, slots, xs_shift, together, there_and_back, pairs, places, pair, place)
+                got = [(p, w) for p, w in zip(pair, place) if p >= 0]
+                assert sorted(got) == [(p, w) for p in range(pairs) for w in range(places)], (pairs, xs_shift, places)
+                # a pair's workgroups are on its 1 << xs_shift XCDs (index % 8)
+                assert all(i % 8 >> xs_shift == p % (8 >> xs_shift) for i, p in enumerate(pair) if p >= 0)
+                if there_and_back and together == 4 and rounds == 4 and places == 20 and not xs_shift:
+                    plain, at = (C.c_int * n)(), (C.c_int * n)()
+                    order.scored(rounds, slots, xs_shift, 4, 0, pairs, places, plain, at)
+                    assert list(plain) != list(pair)          # (places 32 .. 63 of the group go back)
+
+
+def test_scored_pairs_of_about_the_same_length(order):
+    """Steps measured on either side (16 / 4 heads of 64: an XCD has every other sequence)."""
+    for lengths, whole, even in (((2048, 1957, 1867, 1777), 1, 1), ((1000, 886, 771, 657), 1, 1), ((862, 783, 704, 625, 546, 466), 1, 1),
+                                 ((1300, 1100, 900, 700, 500, 300), 1, 0),
+                                 ((4000, 4000), 0, 1), ((5000, 4000, 3000), 0, 0), ((4000, 2666), 0, 0), ((3000, 2080, 1160), 0, 0), ((2400, 2300, 2200), 0, 1), ((), 0, 1)):
+        assert order.even(sum(lengths), max(lengths, default=0), len(lengths), whole) == even, lengths
