@@ -56,7 +56,7 @@ struct LatentParams {
     int row_tiles;               // rows kernel: 128-row tiles of the longest sequence
     int head_groups;             // single kernel: groups of 32 heads
     int nsplit, tiles_per_split; // rows kernel: the most ranges a row can have, and the fewest tiles of one
-    int slots;                   // rows kernel: workgroups that the chip holds at a time; 0: the launch is no larger than that
+    int slots;                   // rows kernel: workgroups that the chip holds at a time; 0: neither the order nor even ranges matter
     int* share;                  // [1]: tiles of a range of the rows kernel, where slots > 0
 };
 
@@ -253,8 +253,8 @@ __global__ __launch_bounds__(256, OCC) void attn_latent_rows_kernel(const Latent
     const int split = blockIdx.y, dv0 = blockIdx.z * DV32, Dv = p.Dv;
     // The latest (heaviest) tiles first, the sequences in turn.  A workgroup's index gives its XCD (of eight) and there its shader engine
     // (of four, eight CUs each), and it waits for that one, others idle or not.  So a launch of more than one round turns every 32
-    // workgroups by another amount, or two sequences would keep to half of the engines each; with key ranges, which come
-    // in rounds of their own, it takes the sequences one after the other.
+    // workgroups by another amount, or two sequences would keep to half of the engines each (without key ranges only where they would); with
+    // key ranges, which come in rounds of their own, it takes the sequences one after the other.
     const int first = blockIdx.x & ~31, x = EVEN && first + 32 <= (int)gridDim.x ? first + ((blockIdx.x + 13 * (first >> 5)) & 31) : (int)blockIdx.x;
     const bool one_by_one = EVEN && p.nsplit > 1;
     const int b = one_by_one ? x / p.row_tiles : x % p.B, qt = p.row_tiles - 1 - (one_by_one ? x % p.row_tiles : x / p.B);
@@ -539,7 +539,7 @@ static LatentPlan latent_single_plan(int B, int H, int max_k) {
 }
 
 template <int D32, int DV32>
-static int launch_latent_rows(LatentParams& p, int max_q, int max_k, hipStream_t s) {
+static int launch_latent_rows(LatentParams& p, int64_t total_q, int max_q, int max_k, hipStream_t s) {
     constexpr int KB = D32 <= 8 ? 2 : 1, OCC = D32 <= 5 || (D32 == 6 && DV32 == 4) ? 2 : 1, D = 32 * D32;
     const LatentPlan plan = latent_rows_plan(p.B, p.H, max_q, max_k, D);
     p.nsplit = plan.nsplit;
@@ -548,7 +548,7 @@ static int launch_latent_rows(LatentParams& p, int max_q, int max_k, hipStream_t
     p.tiles_per_block = p.block_size / (32 * KB);
     p.dv_groups = p.Dv / (32 * DV32);
     const int slots = std::max(1, 256 * OCC / p.dv_groups);
-    p.slots = (int64_t)p.B * p.row_tiles * p.nsplit > slots ? slots : 0;
+    p.slots = (int64_t)p.B * p.row_tiles * p.nsplit > slots && (p.nsplit > 1 || latent_turns(p.B, total_q, max_q, max_k)) ? slots : 0;
     const dim3 grid((unsigned)(p.B * p.row_tiles), (unsigned)p.nsplit, (unsigned)p.dv_groups);
     if (p.slots > 0) hipLaunchKernelGGL((attn_latent_rows_kernel<D32, DV32, KB, OCC, true>), grid, dim3(256), 0, s, p);
     else hipLaunchKernelGGL((attn_latent_rows_kernel<D32, DV32, KB, OCC, false>), grid, dim3(256), 0, s, p);
@@ -645,7 +645,7 @@ extern "C" int nv_attn_latent_paged(const void* q, const void* cache, void* out,
         X(5, 4, 4) X(6, 4, 4) X(8, 6, 6) X(10, 8, 8) X(18, 16, 8)
     if (several) {
         switch (D / 32 * 100 + Dv / 32) {
-#define NV_LAT_CASE(A, V, W) case A * 100 + V: rc = launch_latent_rows<A, W>(p, max_seqlen_q, max_seqlen_k, s); break;
+#define NV_LAT_CASE(A, V, W) case A * 100 + V: rc = launch_latent_rows<A, W>(p, T, max_seqlen_q, max_seqlen_k, s); break;
             NV_LAT_ALL(NV_LAT_CASE)
 #undef NV_LAT_CASE
         }

@@ -15,6 +15,13 @@ NV_HD int latent_share(int64_t total_tiles, int slots, int fewest) {
     const int64_t share = (total_tiles + slots - 1) / slots, most = (int64_t)1 << 24;
     return (int)(share < fewest ? fewest : share > most ? most : share);
 }
+// Launches of more than one round without key ranges: whether the order of workgroups is turned.  Their sequences come in turn, so each of 2, 4, 8 ..
+// keeps to some of the XCDs and shader engines, and those of the longest are what the launch waits for; any other number, and sequences
+// of about the same length, spread by themselves.  Rows of 320, us, as they come / turned: 4 prompts of 446 .. 931 101 / 78, 4 chunks of 456 rows on 865
+// 105 / 77, 13 prompts of 103 .. 164 28 / 35, 9 of 616 .. 805 144 / 158;  256: 8 of 318 .. 670 61 / 49, 8 of 1000 .. 1024 106 / 109, 7 of 309 .. 542 35 / 40.
+NV_HD bool latent_turns(int num_seqs, int64_t total_q, int max_q, int max_k) {
+    return num_seqs > 1 && (num_seqs & (num_seqs - 1)) == 0 && (max_q != max_k || total_q * 9 < (int64_t)num_seqs * max_q * 8);
+}
 // Key tiles of a row tile whose last row sees `last_key`.  Workspace and block tables hold what the caller's longest length has room for,
 // nsplit ranges of `fewest` tiles; keys beyond it, where that length was stated too small, are left out.
 NV_HD int latent_tiles(int last_key, int tile_keys, int nsplit, int fewest) {

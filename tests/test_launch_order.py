@@ -15,6 +15,7 @@ extern "C" int latent(int64_t total, int slots, int last_key, int tile_keys, int
     *tiles = latent_tiles(last_key, tile_keys, nsplit, fewest);
     return latent_ranges(*tiles, *share);
 }
+extern "C" int turns(int num_seqs, int64_t total_q, int max_q, int max_k) { return latent_turns(num_seqs, total_q, max_q, max_k); }
 // where every workgroup of a grid goes: pair and place, -1 for those that leave
 extern "C" void scored(int rounds, int slots, int xs_shift, int together, int there_and_back, int pairs, int places, int* pair, int* place) {
     for (int i = 0; i < 8 * rounds * slots; ++i) {
@@ -42,6 +43,7 @@ def order(tmp_path_factory):
     dll.few_blocks.argtypes = [C.c_int64, C.c_int, C.c_int]
     dll.streams.argtypes = [C.c_int, C.c_int64, C.c_int, C.c_int]
     dll.even.argtypes = [C.c_int64, C.c_int64, C.c_int, C.c_int]
+    dll.turns.argtypes = [C.c_int, C.c_int64, C.c_int, C.c_int]
     return dll
 
 
@@ -113,3 +115,10 @@ def test_scored_pairs_of_about_the_same_length(order):
                                  ((1300, 1100, 900, 700, 500, 300), 1, 0),
                                  ((4000, 4000), 0, 1), ((5000, 4000, 3000), 0, 0), ((4000, 2666), 0, 0), ((3000, 2080, 1160), 0, 0), ((2400, 2300, 2200), 0, 1), ((), 0, 1)):
         assert order.even(sum(lengths), max(lengths, default=0), len(lengths), whole) == even, lengths
+
+
+def test_latent_turned_order(order):
+    """Launches of more than one round without key ranges, on either side of what was measured."""
+    for n_qs, max_k, turned in (([931, 770, 608, 446], 931, 1), ([670 - 50 * i for i in range(8)], 670, 1), ([456] * 4, 865, 1), ([1024, 1000] * 4, 1024, 0),
+                                ([164, 103] * 6 + [130], 164, 0), ([805 - 23 * i for i in range(9)], 805, 0), ([542, 309, 425] * 2 + [400], 542, 0), ([900], 4000, 0)):
+        assert order.turns(len(n_qs), sum(n_qs), max(n_qs), max_k) == turned, n_qs
