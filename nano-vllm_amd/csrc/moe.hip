@@ -1056,7 +1056,7 @@ extern "C" int nv_moe_route(const float* logits, int32_t* ids, float* weights, i
 
 extern "C" int nv_moe_tile_rows(int64_t pairs, int E) { return pairs >= 32 * (int64_t)E ? 64 : 16; }
 
-// By pairs per expert: tiles of 16 rows below 8, of 32 below 24, of 64 (all of these stream the weights past LDS, which costs little more with
+// By pairs per expert: tiles of 16 rows below 8, of 32 below 21, of 64 (all of these stream the weights past LDS, which costs little more with
 // more rows a tile and saves the second reading of an expert that has more), then of 128 staged through LDS, which wants enough of its
 // 128 x 256 blocks to fill the chip.  Whole calls, us, tiles of 16 / 32 / 64 / 128 rows:
 //   top 4 of 32 experts, width 2048, ff 1024:  6 pairs an expert 83 / 86 / 89 / 108, 16: 107 / 96 / 101 / 113, 24: 134 / 107 / 105 / 115,
@@ -1064,16 +1064,19 @@ extern "C" int nv_moe_tile_rows(int64_t pairs, int E) { return pairs >= 32 * (in
 //   top 2 of 32, 1024, 1024:  16: 53 / 48 / 51 / 54, 32: 78 / 63 / 57 / 56, 48: 105 / 79 / 65 / 59
 //   top 2 of 16, 1024, 512:  6: 18 / 18 / 20 / 38, 24: 27 / 29 / 25 / 40, 64: 47 / 39 / 39 / 42, 96: 61 / 52 / 40 / 42, 128: 73 / 58 / 59 / 45
 //   top 4 of 16, 2048, 512:  12: 36 / 30 / 30 / 53, 48: 66 / 51 / 39 / 57, 96: 104 / 83 / 64 / 59
-// With 128 blocks it is the first expert that has more than 64 rows which decides, so routings differ.  Both products, tiles of 64 in four routings and of 128:
-//   top 2 of 16, 2048, 1024:  48: 53, 53, 52, 54 and 57, 52: 67, 54, 54, 70 and 57, 56: 69, 72, 73, 72 and 57 (weights from memory: 48: 59 and 73, 56: 77 and 74)
-//   top 4 of 32, 1024, 512:  48: 43, 34, 34, 41 and 37, 52: 44, 44, 35, 42 and 37 (48: 36 and 42, 52: 45 and 43)
+// It is the first expert with more rows than a tile that decides, so routings differ, and more experts have one earlier.  Both products, us:
+//   tiles of 32 / 64: 16 of 2048, 1024:  20: 41 / 44, 23 with one of 33 rows: 56 / 45
+//   tiles of 64 in four routings and of 128:  16 of 2048, 1024:  48: 53, 53, 52, 54 and 57, 52: 67, 54, 54, 70 and 57, 56: 69, 72, 73, 72 and 57
+//     32 of 1024, 512:  44: 34, 33, 34, 34 and 37, 48: 43, 34, 34, 41 and 37;  32 of 2048, 512:  48: 69, 57, 59, 68 and 56
+// Short rows of many blocks, from 21 to 31 pairs: 16-row tiles through LDS, 32 of 1024, 1024:  24: 40 us, tiles of 64 47 (weights from memory 50 and 51).
 extern "C" int nv_moe_tile_rows_for(int64_t pairs, int E, int width, int ff, const void* h, int64_t h_stride, const void* up,
                                     const void* down, int dtype) {
     using namespace nv;
     if (!moe_pieces_ok(dtype, h, h_stride, up, ff, width) || !moe_pieces_ok(dtype, nullptr, ff, down, width, ff)) return nv_moe_tile_rows(pairs, E);
     const int64_t blocks = (int64_t)E * ((ff + 127) / 128);           // of the first product, a tile an expert
-    if (pairs >= (blocks >= 256 ? 40 : blocks >= 128 ? 52 : 84) * (int64_t)E) return kMoeBigRows;
-    return pairs >= 24 * (int64_t)E ? 64 : pairs >= 8 * (int64_t)E ? 32 : 16;
+    if (pairs >= (blocks >= 256 ? 40 : blocks < 128 ? 84 : E < 32 ? 52 : 48) * (int64_t)E) return kMoeBigRows;
+    if (pairs >= 21 * (int64_t)E) return blocks >= 256 && width <= 1024 && pairs < 32 * (int64_t)E ? 16 : 64;
+    return pairs >= 8 * (int64_t)E ? 32 : 16;
 }
 
 extern "C" int64_t nv_moe_max_tiles(int64_t pairs, int E, int tile_rows) {

@@ -79,12 +79,14 @@ def test_experts_weights_past_lds(order):
     assert not any(order.streams(64, 64 * E, E, ff) for E, ff in ((32, 1024), (16, 1024), (32, 512)))
 
 
-def test_experts_tile_rows():
+def test_experts_tile_rows(order):
     """Where tiles of 128 rows start, on either side of the lines: blocks of 128 x 128 of the first product, pairs an expert."""
     from nanovllm_amd import _lib
     rows_for = lambda E, W, ff, per: _lib.mixers().nv_moe_tile_rows_for(per * E, E, W, ff, 4096, W, 4096, 4096, 0)
-    for E, W, ff, line in ((32, 2048, 1024, 40), (64, 2048, 512, 40), (16, 2048, 1024, 52), (32, 1024, 512, 52), (16, 1024, 512, 84)):
-        assert [rows_for(E, W, ff, per) for per in (7, 8, 23, 24, line - 1, line)] == [16, 32, 32, 64, 64, 128], (E, W, ff)
+    for E, W, ff, line in ((32, 2048, 1024, 40), (64, 2048, 512, 40), (16, 2048, 1024, 52), (32, 1024, 512, 48), (32, 2048, 512, 48), (16, 1024, 512, 84)):
+        assert [rows_for(E, W, ff, per) for per in (7, 8, 20, 21, line - 1, line)] == [16, 32, 32, 64, 64, 128], (E, W, ff)
+    assert [rows_for(32, 1024, 1024, per) for per in (7, 8, 20, 21, 31, 32, 39, 40)] == [16, 32, 32, 16, 16, 64, 64, 128]
+    assert not order.streams(16, 21 * 32, 32, 1024)                   # (those go through LDS)
 
 
 @pytest.mark.parametrize("there_and_back", [0, 1])
