@@ -9,6 +9,7 @@ import ctypes as C
 import importlib.machinery
 import importlib.util
 import os
+import sys
 import sysconfig
 import threading
 
@@ -192,6 +193,12 @@ def _native_calls():
     return module
 
 
+def _signature(restype, argtypes) -> str:
+    """The form that nv_calls.signature has: a letter for the result and for each argument."""
+    letters = {_i32: "i", _i64: "l", _f32: "f", C.c_double: "d"}
+    return "".join(letters.get(t, "p") for t in (restype, *argtypes))
+
+
 def load(path: str | None = None, prototypes: dict | None = None) -> C.CDLL:
     """Load the shared library and attach prototypes.  Raises if it is missing or stale."""
     path = path or os.environ.get("NANOVLLM_HIP_LIB", LIB_PATH)
@@ -209,12 +216,11 @@ def load(path: str | None = None, prototypes: dict | None = None) -> C.CDLL:
     if got != ABI_VERSION:
         raise RuntimeError(f"{path}: ABI version {got}, bindings expect {ABI_VERSION}; rebuild the library")
     calls = _native_calls()
-    if calls is not None:
-        for name in (prototypes if prototypes is not None else PROTOTYPES):
-            fn = getattr(dll, name)
-            quick = calls.bind(name, C.cast(fn, C.c_void_p).value, fn)
-            if quick is not None:
-                setattr(dll, name, quick)
+    if hasattr(calls, "signature"):          # (only what was built from a header that says the same; ctypes takes the others)
+        for name, prototype in (prototypes if prototypes is not None else PROTOTYPES).items():
+            if calls.signature(name) == _signature(*prototype):
+                fn = getattr(dll, name)
+                setattr(dll, name, calls.bind(name, C.cast(fn, C.c_void_p).value, fn))
     return dll
 
 
@@ -241,7 +247,7 @@ def build(target: str = "all") -> None:
     """Compile the in-tree libraries (`all`), or only the second one (`mixers`), with hipcc for gfx950."""
     import subprocess
     jobs = str(min(16, os.cpu_count() or 4))
-    subprocess.run(["make", "-C", os.path.join(_HERE, "csrc"), "-j", jobs, target], check=True,
+    subprocess.run(["make", "-C", os.path.join(_HERE, "csrc"), "-j", jobs, f"PYTHON={sys.executable}", target], check=True,
                    stdout=subprocess.DEVNULL)
 
 

@@ -51,9 +51,17 @@ bool take(PyObject* o, T& v) {
     return false;
 }
 
+template <typename T>
+constexpr char letter() {
+    if constexpr (std::is_pointer_v<T>) return 'p';
+    else if constexpr (std::is_floating_point_v<T>) return sizeof(T) == 4 ? 'f' : 'd';
+    else return sizeof(T) == 4 ? 'i' : 'l';
+}
+
 template <typename F> struct Entry;
 template <typename R, typename... A>
 struct Entry<R(A...)> {
+    static constexpr char signature[] = {letter<R>(), letter<A>()..., 0};          // result, arguments
     template <size_t... I>
     static bool all(PyObject* const* args, std::tuple<A...>& v, std::index_sequence<I...>) {
         return (take(args[I], std::get<I>(v)) && ...);
@@ -73,10 +81,10 @@ struct Entry<R(A...)> {
 };
 
 struct Known {
-    const char* name;
+    const char *name, *signature;
     vectorcallfunc call;
 };
-#define NV_ENTRY(NAME) {#NAME, &Entry<decltype(NAME)>::call},
+#define NV_ENTRY(NAME) {#NAME, Entry<decltype(NAME)>::signature, &Entry<decltype(NAME)>::call},
 const Known known[] = {
     NV_ENTRY(nv_store_kvcache) NV_ENTRY(nv_attn_decode_workspace_bytes) NV_ENTRY(nv_attn_decode_paged)
     NV_ENTRY(nv_attn_decode_suggest_chunk) NV_ENTRY(nv_attn_decode_workspace_bytes_chunked) NV_ENTRY(nv_attn_decode_paged_chunked)
@@ -137,7 +145,16 @@ PyObject* bind(PyObject*, PyObject* args) {
     Py_RETURN_NONE;
 }
 
-PyMethodDef methods[] = {{"bind", bind, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
+// signature(name) -> what the header that this was built from says: a letter for the result and for each argument, or None
+PyObject* signature(PyObject*, PyObject* name) {
+    const char* wanted = PyUnicode_AsUTF8(name);
+    if (wanted == nullptr) return nullptr;
+    for (const Known& k : known)
+        if (strcmp(k.name, wanted) == 0) return PyUnicode_FromString(k.signature);
+    Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {{"bind", bind, METH_VARARGS, nullptr}, {"signature", signature, METH_O, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "nv_calls", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

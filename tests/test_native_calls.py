@@ -52,3 +52,31 @@ def test_pointers_floats_and_error_codes(dll):
     with pytest.raises(_lib.NanoVllmHipError):
         _lib.check(fn(None, None, None, 4, 128, 128, 1e-6, None), "nv_rmsnorm")
     assert fn(None, None, None, 0, 128, 128, 1, None) == fn.otherwise(None, None, None, 0, 128, 128, 1, None)      # an integer for a float
+
+
+def test_only_callables_of_the_same_signature(dll, monkeypatch):
+    """A module that was built from another header, or before modules said what they were built from, takes no call."""
+    module = _lib._native_calls()
+    name = "nv_attn_decode_suggest_chunk"
+
+    class Other:
+        bind = staticmethod(module.bind)
+
+        @staticmethod
+        def signature(n):
+            s = module.signature(n)
+            return s[:-1] + "i" if n == name else s           # its last argument was 32 bits then
+
+    class Before:
+        bind = staticmethod(module.bind)
+
+    quick = lambda d, n: hasattr(getattr(d, n), "otherwise")
+    monkeypatch.setattr(_lib, "_native_calls", lambda: Other)
+    d = _lib.load()
+    assert not quick(d, name) and quick(d, "nv_rmsnorm")
+    monkeypatch.setattr(_lib, "_native_calls", lambda: Before)
+    assert not any(quick(_lib.load(), n) for n in _lib.PROTOTYPES)
+    monkeypatch.undo()
+    turned = dict(_lib.PROTOTYPES, nv_rmsnorm=(C.c_int, [C.c_void_p] * 4 + [C.c_int64] * 3 + [C.c_float]))
+    assert not quick(_lib.load(None, turned), "nv_rmsnorm")     # prototypes of the caller's own
+    assert module.signature("nv_rmsnorm") == "ippplilfp" and module.signature("nv_strerror") is None
