@@ -80,8 +80,8 @@ __device__ __forceinline__ void moe_route_token(const float* __restrict__ z, int
         moe_better_dpp<0x4E>(bv, be);
         moe_better_dpp<0x141>(bv, be);
         moe_better_dpp<0x140>(bv, be);
-        if (E > 16) moe_better(bv, be, __shfl_xor(bv, 16), __shfl_xor(be, 16));
-        if (E > 32) moe_better(bv, be, __shfl_xor(bv, 32), __shfl_xor(be, 32));
+        moe_better(bv, be, __shfl_xor(bv, 16), __shfl_xor(be, 16));
+        moe_better(bv, be, __shfl_xor(bv, 32), __shfl_xor(be, 32));
         be = __builtin_amdgcn_readfirstlane(be);
         bv = moe_first(bv);
         if ((be & 63) == lane && be < 64 * PER) taken |= 1u << (be >> 6);

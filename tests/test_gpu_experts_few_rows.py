@@ -47,3 +47,11 @@ def test_few_rows(form, E, T, top, W, ff, rows):
     got, want = a(h, ids, weights, gate_up, down), r(f(h), ids, weights, f(gate_up), f(down))
     live = (ids < E)[..., None].expand_as(got)
     torch.testing.assert_close(got[live], want[live], **_tol())
+
+
+# a wave's quarter of the contraction in 4, 5, 8 steps of 64 and, with the last wave short of steps or without any, 5 + 5 + 5 + 2 and 2 + 2 + 1 + 0
+@pytest.mark.parametrize("E,T,top,W,ff,rows", [(4, 6, 2, 1024, 1280, 16), (4, 25, 2, 1280, 1088, 32), (4, 60, 2, 1088, 2048, 64), (2, 17, 1, 2048, 320, 32),
+                                               (3, 90, 1, 2048, 1024, 64), (32, 40, 4, 1088, 1024, 16)])
+@pytest.mark.parametrize("form", ["clamped", "relu2", "silu"])
+def test_few_rows_long_contractions(form, E, T, top, W, ff, rows):
+    test_few_rows(form, E, T, top, W, ff, rows)

@@ -36,3 +36,33 @@ def test_route_sort(T, E, top):
         at += int(n[e])
     assert int(m[0]) == len(want_tiles) <= tiles
     assert torch.equal(m[1:1 + 3 * len(want_tiles)].view(-1, 3), torch.tensor(want_tiles, dtype=i32).view(-1, 3))
+
+
+# tokens on either side of one workgroup's (16 beyond 64 experts), a wave with more than one token, more workgroups than one for each 4 tokens
+@pytest.mark.parametrize("T", [16, 18, 513, 1025, 3001])
+@pytest.mark.parametrize("E,top", [(64, 8), (65, 16), (129, 1), (512, 2), (512, 16)])
+def test_route_sort_sizes(T, E, top):
+    test_route_sort(T, E, top)
+
+
+@pytest.mark.parametrize("T", [1, 3, 17, 1000])
+@pytest.mark.parametrize("E,top", [(4, 4), (16, 1), (33, 5), (64, 16), (65, 2), (512, 3), (520, 16)])
+def test_route(T, E, top):
+    """The choice alone (nv_moe_route): ties, equal logits, infinite ones and, in some tokens, logits that are not numbers."""
+    g = torch.Generator(device=DEV).manual_seed(T * E)
+    logits = torch.randn(T, E, generator=g, device=DEV)
+    logits[::3] = logits[::3].round()
+    logits[1::5] = 0.0
+    logits[2::7, ::2] = float("-inf")
+    dll, i32 = ops._lib.mixers(), torch.int32
+    ids, wgt = torch.full((T, top), -1, dtype=i32, device=DEV), torch.zeros(T, top, device=DEV)
+    run = lambda: ops._lib.check(dll.nv_moe_route(logits.data_ptr(), ids.data_ptr(), wgt.data_ptr(), T, E, top, torch.cuda.current_stream().cuda_stream),
+                                 "nv_moe_route", dll)
+    run()
+    val, want = logits.cpu().sort(dim=-1, descending=True, stable=True)
+    assert torch.equal(ids.cpu().long(), want[:, :top])
+    torch.testing.assert_close(wgt.cpu(), torch.softmax(val[:, :top], -1), rtol=1e-5, atol=1e-7)
+    logits[::2, E // 2] = float("nan")
+    run()
+    chosen = ids.cpu().long().sort(-1).values
+    assert chosen.min() >= 0 and chosen.max() < E and (chosen.diff(dim=-1) > 0).all()       # experts, none of them twice
