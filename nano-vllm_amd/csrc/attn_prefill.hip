@@ -25,6 +25,7 @@
 
 #include "nv_common.h"
 #include "attn_prefill_shared.h"
+#include "launch_order.h"
 
 #ifndef NV_PF_MAX_ITEMS
 #define NV_PF_MAX_ITEMS 4
@@ -632,13 +633,9 @@ extern "C" int nv_attn_prefill_varlen(const void* q, const void* k_cache, const 
     p.xs_shift = sh.xs_shift;
     p.slots_per_pair = sh.slots_per_pair;
     p.rounds = (int)(sh.grid_base / (8 * (int64_t)sh.slots_per_pair));
-    // Single query tiles of sequences of about the same length, about two rounds of them: an XCD takes several pairs together, the heaviest tiles
-    // of all first, as long as their keys and values stay within half its L2.  4 prompts of 2000 .. 2048 tokens, 16 / 8 heads: 101 -> 86 us, 8 of
-    // 900 .. 1024 68 -> 57, 6 of 1000 .. 1365 72 -> 64; 2 of 600 and 2048, 32 / 8 heads, 61 -> 66, and with more rounds the
-    // order counts for less than the L2 (32 / 8 heads, 7 of 600 .. 1100: 76 -> 81, 4 of 1000 new tokens on 3000: 107 -> 130).
-    const bool few = sh.hand_scheduled && sh.nsplit == 1 && sh.items_per_wg == 1 && (int64_t)sh.n_pairs * sh.wg_per_pair <= 576 &&
-                     (int64_t)total_q * 4 >= (int64_t)B * max_seqlen_q * 3;
-    p.together = few ? std::min(4, std::max(1, 4096 / std::max(max_seqlen_k, 1))) : 1;
+    p.together = sh.hand_scheduled && sh.nsplit == 1 && sh.items_per_wg == 1
+                     ? prefill_together((int64_t)sh.n_pairs * sh.wg_per_pair, total_q, B, max_seqlen_q, max_seqlen_k)
+                     : 1;
     p.fd_slots_per_pair = make_fastdiv((uint32_t)sh.slots_per_pair);
     p.pair_items = sh.items_per_wg;
     p.groups = sh.wg_per_pair / sh.n_qtiles;

@@ -31,6 +31,26 @@ NV_HD int latent_tiles(int last_key, int tile_keys, int nsplit, int fewest) {
 // Its ranges: at most nsplit, since a share is never below `fewest`.
 NV_HD int latent_ranges(int tiles, int share) { return tiles <= share ? 1 : (tiles - 1) / share + 1; }
 
+// Prompt attention, single query tiles a workgroup: how many pairs of sequence and kv head an XCD takes together, the heaviest tiles of all first.  For
+// sequences of about the same length and about two rounds of workgroups, as long as the pairs' keys and values stay within half its L2.  4 prompts of 2000 ..
+// 2048 tokens, 16 / 8 heads: 101 -> 86 us, 8 of 900 .. 1024 68 -> 57, 6 of 1000 .. 1365 72 -> 64; 2 of 600 and 2048, 32 / 8 heads, 61 -> 66, and with
+// more rounds the order counts for less than the L2 (32 / 8 heads, 7 of 600 .. 1100: 76 -> 81, 4 of 1000 new tokens on 3000: 107 -> 130).
+NV_HD int prefill_together(int64_t workgroups, int64_t total_q, int num_seqs, int max_q, int max_k) {
+    if (workgroups > 576 || total_q * 4 < (int64_t)num_seqs * max_q * 3) return 1;
+    const int fit = 4096 / (max_k > 1 ? max_k : 1);
+    return fit < 1 ? 1 : fit < 4 ? fit : 4;
+}
+// A workgroup's slot on its XCD -> round of pairs and place in the pair: `together` rounds place by place, turning by one every time.
+struct RoundPlace {
+    int round, place;
+};
+NV_HD RoundPlace prefill_order(int slot, int rounds, int slots_per_pair, int together) {
+    const int round = slot / slots_per_pair;
+    if (together <= 1) return {round, slot - round * slots_per_pair};
+    const int first = round - round % together, left = rounds - first, n = together < left ? together : left, at = slot - first * slots_per_pair;
+    return {first + (at + at / n) % n, at / n};
+}
+
 // Score-modified attention, prompt portions: workgroup (of a key range) -> its pair of sequence and kv head and its place in the pair, heaviest query
 // tile first.  Workgroups go to the eight XCDs in turn; an XCD has `rounds` pairs (8 >> xs_shift of them a round over all XCDs), four to a group.
 // grid: 8 * rounds * slots_per_pair; places past a pair's workgroups and pairs past the last one are for the caller to leave out.

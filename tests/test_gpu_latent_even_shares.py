@@ -32,3 +32,21 @@ def test_even_shares(D, Dv, H, step):
     # (the bound of the other launches' test: probabilities and outputs are rounded to bf16, 2^-9 each)
     err = (got[0].float() - want).view(sum(n_q), -1).norm(dim=-1) / want.norm(dim=-1)
     assert err.max().item() < 1.2e-2, (int(err.argmax()), err.max().item())
+
+
+@pytest.mark.parametrize("step,D,Dv,H,even", [("far_apart", 160, 128, 64, True), ("far_apart", 256, 256, 52, True), ("one_long", 256, 256, 64, True),
+                                              ("one_long", 320, 320, 52, True), ("equal", 256, 256, 64, True),
+                                              ("one_long", 160, 128, 64, True), ("equal", 160, 128, 64, False), ("one_long", 160, 128, 8, False)])
+def test_which_launches_have_even_ranges(step, D, Dv, H, even):
+    """The launch writes its share in front of the states in the workspace where ranges are sized on the device, and only there."""
+    n_q, n_k = STEPS[step]
+    ctx, _ = paged_context(n_q, n_k, 64, sum(-(-n // 64) for n in n_k) + 3, D, DEV)
+    g = torch.Generator().manual_seed(D + H)
+    q, cache = rn(g, sum(n_q), H, D).to(torch.bfloat16), rn(g, sum(-(-n // 64) for n in n_k) + 3, 64, 1, D).to(torch.bfloat16)
+    need = ops._lib.mixers().nv_attn_latent_workspace_bytes(len(n_q), sum(n_q), H, D, Dv, max(n_q), max(n_k))
+    assert need > 64
+    head = ops._workspace(q.device, need)[:4].view(torch.int32)
+    head.fill_(-7)
+    ops.attn_latent_paged(q, cache, cache[..., :Dv], ctx.cu_seqlens_q, ctx.cu_seqlens_k, ctx.block_tables, 0.9, None, max(n_q), max(n_k), -1)
+    tile, share = 64 if D <= 256 else 32, int(head.item())
+    assert (8 <= share <= -(-max(n_k) // tile)) if even else share == -7

@@ -5,6 +5,7 @@ import torch
 
 import nanovllm_amd as nv
 from nanovllm_amd import _lib, ops
+from test_launch_order import order                              # noqa: F401 (a fixture)
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -33,3 +34,11 @@ def test_together(H, G, lens):
         _lib.set_tuning()
     # (both round probabilities and outputs to bf16, 2^-9 each, outputs are at most of order one)
     torch.testing.assert_close(got.float(), want.float(), rtol=2e-2, atol=1e-2)
+
+
+@pytest.mark.parametrize("H,G,lens,together", [(16, 8, [1024] * 8, 4), (16, 8, [1300, 1299, 1200, 1100, 1000], 3), (16, 8, [2048, 1900, 1800], 2), (32, 8, [700, 700, 690, 650], 4),
+                                               (16, 8, [4000, 3900], 1)])
+def test_launches_above_take_several_pairs(order, H, G, lens, together):           # noqa: F811
+    """The launches of test_together are the ones that they are meant to be: single tiles, several pairs at a time."""
+    tiles = -(-max(lens) // (64 * 4 // (H // G)))
+    assert order.pairs_together(len(lens) * G * tiles, sum(lens), len(lens), max(lens), max(lens)) == together

@@ -25,6 +25,16 @@ extern "C" void scored(int rounds, int slots, int xs_shift, int together, int th
         place[i] = there ? at.place : -1;
     }
 }
+extern "C" int pairs_together(int64_t workgroups, int64_t total_q, int num_seqs, int max_q, int max_k) {
+    return prefill_together(workgroups, total_q, num_seqs, max_q, max_k);
+}
+extern "C" void prompt(int rounds, int slots, int together, int* round, int* place) {
+    for (int i = 0; i < rounds * slots; ++i) {
+        const RoundPlace at = prefill_order(i, rounds, slots, together);
+        round[i] = at.round;
+        place[i] = at.place;
+    }
+}
 extern "C" int even(int64_t keys, int64_t longest, int n, int whole_prompts) { return scoremod_even(keys, longest, n, whole_prompts); }
 extern "C" int streams(int tile_rows, int64_t pairs, int E, int ff) { return moe_streams(tile_rows, pairs, E, ff); }
 extern "C" int few_blocks(int64_t pairs, int E, int n_cols) { return moe_few_blocks(pairs, E, n_cols); }
@@ -44,6 +54,7 @@ def order(tmp_path_factory):
     dll.streams.argtypes = [C.c_int, C.c_int64, C.c_int, C.c_int]
     dll.even.argtypes = [C.c_int64, C.c_int64, C.c_int, C.c_int]
     dll.turns.argtypes = [C.c_int, C.c_int64, C.c_int, C.c_int]
+    dll.pairs_together.argtypes = [C.c_int64, C.c_int64] + [C.c_int] * 3
     return dll
 
 
@@ -124,3 +135,24 @@ def test_latent_turned_order(order):
     for n_qs, max_k, turned in (([931, 770, 608, 446], 931, 1), ([670 - 50 * i for i in range(8)], 670, 1), ([456] * 4, 865, 1), ([1024, 1000] * 4, 1024, 0),
                                 ([164, 103] * 6 + [130], 164, 0), ([805 - 23 * i for i in range(9)], 805, 0), ([542, 309, 425] * 2 + [400], 542, 0), ([900], 4000, 0)):
         assert order.turns(len(n_qs), sum(n_qs), max(n_qs), max_k) == turned, n_qs
+
+
+@pytest.mark.parametrize("together", [1, 2, 3, 4])
+def test_prompt_every_place_once(order, together):
+    for rounds in (1, 2, 3, 4, 5, 8, 9, 13):
+        for slots in (1, 2, 7, 8, 32, 33):
+            n = rounds * slots
+            round_, place = (C.c_int * n)(), (C.c_int * n)()
+            order.prompt(rounds, slots, together, round_, place)
+            assert sorted(zip(round_, place)) == [(r, s) for r in range(rounds) for s in range(slots)], (rounds, slots)
+            assert all(r // together == i // slots // together for i, r in enumerate(round_))          # within its group of pairs
+            if together == 1:
+                assert list(zip(round_, place)) == [(i // slots, i % slots) for i in range(n)]
+
+
+def test_prompt_pairs_together(order):
+    # (query tiles of 128 rows of two heads: 2 x 64 rows and, with 4 heads a kv head, 64 of four)
+    wgs = lambda lens, H, G: len(lens) * G * -(-max(lens) // (128 if H // G == 2 else 64))
+    for H, G, lens, max_k, want in ((16, 8, [2048] * 4, 2048, 2), (16, 8, [1024] * 8, 1024, 4), (16, 8, [1365, 1180, 1000] * 2, 1365, 3), (32, 8, [600, 2048], 2048, 1),
+                                    (32, 8, [1100, 850, 600] * 2, 1100, 1), (16, 8, [1000] * 4, 3000, 1), (32, 8, [2048] * 4, 2048, 1)):
+        assert order.pairs_together(wgs(lens, H, G), sum(lens), len(lens), max(lens), max_k) == want, (H, lens)
