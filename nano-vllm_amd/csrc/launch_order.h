@@ -32,7 +32,7 @@ NV_HD int latent_tiles(int last_key, int tile_keys, int nsplit, int fewest) {
 NV_HD int latent_ranges(int tiles, int share) { return tiles <= share ? 1 : (tiles - 1) / share + 1; }
 
 // Prompt attention, single query tiles a workgroup: how many pairs of sequence and kv head an XCD takes together, the heaviest tiles of all first.  For
-// sequences of about the same length and about two rounds of workgroups, as long as the pairs' keys and values stay within half its L2.  4 prompts of 2000 ..
+// sequences of about the same length and about two rounds of workgroups, as long as the pairs' keys and values stay within half its L2 (those of a larger set, below, within all of it).  4 prompts of 2000 ..
 // 2048 tokens, 16 / 8 heads: 101 -> 86 us, 8 of 900 .. 1024 68 -> 57, 6 of 1000 .. 1365 72 -> 64; 2 of 600 and 2048, 32 / 8 heads, 61 -> 66, and with
 // more rounds the order counts for less than the L2 (32 / 8 heads, 7 of 600 .. 1100: 76 -> 81, 4 of 1000 new tokens on 3000: 107 -> 130).
 NV_HD int prefill_together(int64_t workgroups, int64_t total_q, int num_seqs, int max_q, int max_k) {
@@ -40,14 +40,20 @@ NV_HD int prefill_together(int64_t workgroups, int64_t total_q, int num_seqs, in
     const int fit = 4096 / (max_k > 1 ? max_k : 1);
     return fit < 1 ? 1 : fit < 4 ? fit : 4;
 }
-// A workgroup's slot on its XCD -> round of pairs and place in the pair: `together` rounds place by place, turning by one every time.
+// An XCD's `rounds` pairs in sets of as many as that, or a few more: sets differ by a pair at most, because what is left over for a short last one begins with
+// its heaviest tile when the others end.  One after the other / in sets of four with the rest last / so: 9 prompts of 545 .. 793, 16 / 8 heads,
+// 48.8 / 51.8 / 44.7 us, 10 of 627 .. 654, 16 / 4, 45.0 / 46.4 / 39.7, 5 of 771 .. 1206, 16 / 16, 58.7 / 63.1 / 58.9; 90 launches of 257 to 576
+// workgroups 1 / 0.960 / 0.938 on average, 1.06 at most (1.07 with the rest last).
+NV_HD int prefill_sets(int rounds, int together) { return rounds > together ? rounds / together : 1; }
+// A workgroup's slot on its XCD -> round of pairs and place in the pair: the rounds of a set place by place, turning by one every time.
 struct RoundPlace {
     int round, place;
 };
-NV_HD RoundPlace prefill_order(int slot, int rounds, int slots_per_pair, int together) {
+NV_HD RoundPlace prefill_order(int slot, int rounds, int slots_per_pair, int sets) {
     const int round = slot / slots_per_pair;
-    if (together <= 1) return {round, slot - round * slots_per_pair};
-    const int first = round - round % together, left = rounds - first, n = together < left ? together : left, at = slot - first * slots_per_pair;
+    if (sets == rounds) return {round, slot - round * slots_per_pair};
+    const int least = rounds / sets, more = (rounds - least * sets) * (least + 1);         // rounds of the sets with one more, which are first
+    const int from = round < more ? 0 : more, n = round < more ? least + 1 : least, first = from + (round - from) / n * n, at = slot - first * slots_per_pair;
     return {first + (at + at / n) % n, at / n};
 }
 

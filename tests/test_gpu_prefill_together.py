@@ -42,3 +42,10 @@ def test_launches_above_take_several_pairs(order, H, G, lens, together):        
     """The launches of test_together are the ones that they are meant to be: single tiles, several pairs at a time."""
     tiles = -(-max(lens) // (64 * 4 // (H // G)))
     assert order.pairs_together(len(lens) * G * tiles, sum(lens), len(lens), max(lens), max(lens)) == together
+
+
+# numbers of pairs an XCD that sets of three or four leave a rest of: 5 in one set (the last XCDs have 4), 9 as 5 and 4, 10 as 4, 3 and 3, 5 spread over two XCDs each
+@pytest.mark.parametrize("H,G,lens", [(16, 4, [654 - 3 * i for i in range(9)]), (16, 8, [790 - 30 * i for i in range(9)]), (16, 16, [1206, 1100, 990, 880, 771]),
+                                      (16, 4, [943, 930, 915, 900, 885])])
+def test_uneven_numbers_of_pairs(H, G, lens):
+    test_together(H, G, lens)
