@@ -229,14 +229,21 @@ __device__ __forceinline__ float lat_finish(float m, float l, const float* sink,
 template <int KT>
 __device__ __forceinline__ int lat_share(const LatentParams& p, int lane) {
     int64_t total = 0;
+    int least = 0x7fffffff, longest = 0;                     // keys in front of a sequence's rows, keys of a sequence
     for (int b = lane; b < p.B; b += 64) {
         const int n_q = p.cu_q[b + 1] - p.cu_q[b], n_k = p.cu_k[b + 1] - p.cu_k[b];
         if (n_q <= 1) continue;
         const int64_t tiles = ((int64_t)n_q * p.H + 4 * kLatRows - 1) / (4 * kLatRows);
         total += tiles * (n_k - n_q / 2) / KT + tiles;
+        least = min(least, n_k - n_q);
+        longest = max(longest, n_k);
     }
-    for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o);
-    return latent_share(total, p.slots, p.tiles_per_split);
+    for (int o = 32; o > 0; o >>= 1) {
+        total += __shfl_xor(total, o);
+        least = min(least, __shfl_xor(least, o));
+        longest = max(longest, __shfl_xor(longest, o));
+    }
+    return latent_alike(least, longest) ? p.tiles_per_split : latent_share(total, p.slots, p.tiles_per_split);
 }
 
 // EVEN: the launch is more than the chip holds at a time, so the order and the ranges of its workgroups matter.

@@ -15,6 +15,11 @@ NV_HD int latent_share(int64_t total_tiles, int slots, int fewest) {
     const int64_t share = (total_tiles + slots - 1) / slots, most = (int64_t)1 << 24;
     return (int)(share < fewest ? fewest : share > most ? most : share);
 }
+// Chunks behind at least three quarters of the longest sequence: all row tiles are about as long, so equal ranges of each, as the host plans them, are
+// even already, and a share for every slot leaves whole row tiles over for a second round.  Share / equal ranges, 16 heads: 7 chunks of 290 rows
+// on 2966 .. 3257 keys, rows of 256, 199 / 181 us (174 where every row tile has all ranges), 9 of 161 on 3708 .. 3828, rows of 160, 100.2 / 99.6 (94.0).
+// With less in front: 8 of 256 on 3053 .. 4036, rows of 256, 147 / 166.
+NV_HD bool latent_alike(int least_in_front, int longest) { return (int64_t)least_in_front * 4 >= (int64_t)longest * 3; }
 // Launches of more than one round without key ranges: whether the order of workgroups is turned.  Their sequences come in turn, so each of 2, 4, 8 ..
 // keeps to some of the XCDs and shader engines, and those of the longest are what the launch waits for; any other number, and sequences
 // of about the same length, spread by themselves.  Rows of 320, us, as they come / turned: 4 prompts of 446 .. 931 101 / 78, 4 chunks of 456 rows on 865

@@ -50,3 +50,12 @@ def test_which_launches_have_even_ranges(step, D, Dv, H, even):
     ops.attn_latent_paged(q, cache, cache[..., :Dv], ctx.cu_seqlens_q, ctx.cu_seqlens_k, ctx.block_tables, 0.9, None, max(n_q), max(n_k), -1)
     tile, share = 64 if D <= 256 else 32, int(head.item())
     assert (8 <= share <= -(-max(n_k) // tile)) if even else share == -7
+
+
+@pytest.mark.parametrize("H", [16, 13])
+@pytest.mark.parametrize("D,Dv", [(256, 256), (160, 128), (320, 320)])
+@pytest.mark.parametrize("step", ["alike"])
+def test_alike(D, Dv, H, step, monkeypatch):
+    """Chunks behind most of their keys: the host's ranges, in the same launch."""
+    monkeypatch.setitem(STEPS, "alike", ([40, 1, 33, 40], [1900, 90, 1800, 1700]))
+    test_even_shares(D, Dv, H, step)

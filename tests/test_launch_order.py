@@ -15,6 +15,7 @@ extern "C" int latent(int64_t total, int slots, int last_key, int tile_keys, int
     *tiles = latent_tiles(last_key, tile_keys, nsplit, fewest);
     return latent_ranges(*tiles, *share);
 }
+extern "C" int alike(int least_in_front, int longest) { return latent_alike(least_in_front, longest); }
 extern "C" int turns(int num_seqs, int64_t total_q, int max_q, int max_k) { return latent_turns(num_seqs, total_q, max_q, max_k); }
 // where every workgroup of a grid goes: pair and place, -1 for those that leave
 extern "C" void scored(int rounds, int slots, int xs_shift, int together, int there_and_back, int pairs, int places, int* pair, int* place) {
@@ -129,6 +130,12 @@ def test_scored_pairs_of_about_the_same_length(order):
                                  ((1300, 1100, 900, 700, 500, 300), 1, 0),
                                  ((4000, 4000), 0, 1), ((5000, 4000, 3000), 0, 0), ((4000, 2666), 0, 0), ((3000, 2080, 1160), 0, 0), ((2400, 2300, 2200), 0, 1), ((), 0, 1)):
         assert order.even(sum(lengths), max(lengths, default=0), len(lengths), whole) == even, lengths
+
+
+def test_latent_chunks_of_about_the_same_keys(order):
+    """Row tiles of about the same length have the host's ranges: steps measured on either side (rows, keys of the sequences)."""
+    for rows, shortest, longest, alike in ((290, 2966, 3257, 1), (161, 3708, 3828, 1), (238, 1876, 2009, 1), (256, 3053, 4036, 0), (1024, 3000, 6001, 0), (900, 900, 900, 0)):
+        assert order.alike(shortest - rows, longest) == alike, (rows, shortest, longest)
 
 
 def test_latent_turned_order(order):
