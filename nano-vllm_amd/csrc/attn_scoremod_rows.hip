@@ -368,8 +368,7 @@ int launch_scoremod_rows(ScoremodRowsParams p, const ScoremodRowsPlan& f, int D,
     p.xs_shift = f.xs_shift;
     p.slots_per_pair = f.slots_per_pair;
     p.rounds = (int)(f.grid_base / (8 * (int64_t)f.slots_per_pair));
-    // (no more workgroups of a key range than CUs: the order hardly matters, and asking takes half a microsecond)
-    p.even = f.grid_base <= 256 ? 1 : max_seqlen_q != max_seqlen_k ? -1 : scoremod_even(total_q, max_seqlen_q, num_seqs, 1);
+    p.even = scoremod_pairs(f.grid_base, num_seqs, total_q, max_seqlen_q, max_seqlen_k);
     p.there_and_back = f.grid_base * f.nsplit <= 256 * (D + Dv == 128 ? 4 : D + Dv == 192 ? 3 : 2);       // (workgroups that a CU holds)
     p.grid_base = (int)f.grid_base;
     p.nsplit = f.nsplit;

@@ -81,6 +81,14 @@ NV_HD PairGroup scoremod_group(int index, int rounds, int slots_per_pair, int xs
 NV_HD bool scoremod_even(int64_t keys, int64_t longest, int n, int whole_prompts) {
     return whole_prompts ? keys * 4 >= longest * n * 3 : keys * 9 >= longest * n * 8;
 }
+// What a launch knows of that: 1 and 0, or -1 where a group of chunks is to look at its own lengths.  Chunks of no more workgroups of a key range than CUs
+// do not look, which takes half a microsecond of 13 to 21, and go one after the other: with several key ranges the order is not without
+// effect there, 5 of 230 rows on 2194 .. 3955 keys, 16 / 8 heads of 128, 83 us so and 96 together, 2 of 431 on 3229 .. 4093 73 and 84; 80 such
+// steps, from 0.90 to 1.14 of the time and 1.005 on average together, 0.997 looking first (7 of them 2 to 4 % slower for it).
+NV_HD int scoremod_pairs(int64_t grid_base, int num_seqs, int64_t total_q, int max_q, int max_k) {
+    if (max_q == max_k) return scoremod_even(total_q, max_q, num_seqs, 1);
+    return grid_base <= 256 ? 0 : -1;
+}
 // together: the pairs of the group (four, or one) that are taken place by place, turning by one every time; the others one
 // after the other.  there_and_back: 32 workgroups of the XCD there and the next 32 back instead.
 NV_HD PairPlace scoremod_order(const PairGroup& g, int index, int slots_per_pair, int xs_shift, int together, int there_and_back) {

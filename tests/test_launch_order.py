@@ -38,6 +38,9 @@ extern "C" void prompt(int rounds, int slots, int sets, int* round, int* place) 
     }
 }
 extern "C" int even(int64_t keys, int64_t longest, int n, int whole_prompts) { return scoremod_even(keys, longest, n, whole_prompts); }
+extern "C" int scored_pairs(int64_t grid_base, int num_seqs, int64_t total_q, int max_q, int max_k) {
+    return scoremod_pairs(grid_base, num_seqs, total_q, max_q, max_k);
+}
 extern "C" int streams(int tile_rows, int64_t pairs, int E, int ff) { return moe_streams(tile_rows, pairs, E, ff); }
 extern "C" int few_blocks(int64_t pairs, int E, int n_cols) { return moe_few_blocks(pairs, E, n_cols); }
 """
@@ -55,6 +58,7 @@ def order(tmp_path_factory):
     dll.few_blocks.argtypes = [C.c_int64, C.c_int, C.c_int]
     dll.streams.argtypes = [C.c_int, C.c_int64, C.c_int, C.c_int]
     dll.even.argtypes = [C.c_int64, C.c_int64, C.c_int, C.c_int]
+    dll.scored_pairs.argtypes = [C.c_int64, C.c_int, C.c_int64, C.c_int, C.c_int]
     dll.turns.argtypes = [C.c_int, C.c_int64, C.c_int, C.c_int]
     dll.pairs_together.argtypes = [C.c_int64, C.c_int64] + [C.c_int] * 3
     return dll
@@ -130,6 +134,13 @@ def test_scored_pairs_of_about_the_same_length(order):
                                  ((1300, 1100, 900, 700, 500, 300), 1, 0),
                                  ((4000, 4000), 0, 1), ((5000, 4000, 3000), 0, 0), ((4000, 2666), 0, 0), ((3000, 2080, 1160), 0, 0), ((2400, 2300, 2200), 0, 1), ((), 0, 1)):
         assert order.even(sum(lengths), max(lengths, default=0), len(lengths), whole) == even, lengths
+
+
+def test_scored_pairs_of_a_launch(order):
+    """Whole prompts by their rows, whatever the grid; chunks of a small grid one after the other, of a large one by what their groups see."""
+    for grid_base, lens, max_k, want in ((160, [230] * 5, 3955, 0), (256, [431] * 2, 4093, 0), (264, [300] * 8, 2696, -1), (160, [600, 590], 600, 1),
+                                         (160, [900, 300, 200], 900, 0), (2048, [2048, 1957, 1867, 1777], 2048, 1), (2048, [2048, 300, 300], 2048, 0)):
+        assert order.scored_pairs(grid_base, len(lens), sum(lens), max(lens), max_k) == want, (grid_base, lens)
 
 
 def test_latent_chunks_of_about_the_same_keys(order):
