@@ -1,5 +1,6 @@
 // The 32 x 32 tile launch for prompt portions of the score-modified attention (attn_scoremod_rows.hip).
 #pragma once
+#include "launch_order.h"
 #include "nv_common.h"
 
 namespace nv {
@@ -14,7 +15,8 @@ struct ScoremodRowsParams {
     int v_ld, n_dist, H, G, block_size, max_blocks, max_block;
     float softcap, scale_log2, cap_in;         // cap_in: a raw score's factor to the exponent of tanh
     int hpw, n_qtiles, wg_per_pair, n_pairs, xs_shift, slots_per_pair, grid_base, nsplit, tiles_per_split;
-    int rounds, even, there_and_back;          // pairs of an XCD; they are about as long (1, 0, or -1: see cu_k); all workgroups run at a time
+    PairSets sets;                             // of an XCD's pairs
+    int even, there_and_back;                  // the pairs of a set are about as long (1, 0, or -1: see cu_k); all workgroups run at a time
 };
 struct ScoremodRowsPlan {
     int hpw;                                   // heads of a kv head's group that a workgroup takes (1, 2 or 4)

@@ -21,7 +21,6 @@
 #include <type_traits>
 
 #include "attn_scoremod_rows.h"
-#include "launch_order.h"
 
 namespace nv {
 
@@ -58,19 +57,19 @@ __global__ __launch_bounds__(256, 2) void scoremod_rows_kernel(const ScoremodRow
     const int r = lane & 31, hh = lane >> 5;
 
     // Workgroup -> (sequence, kv head, head group, query tile): workgroups that read the same keys share an XCD.  An XCD takes its pairs
-    // (of sequence and kv head) four together, the heaviest query tiles of all first; pair after pair, a CU's workgroups were heavy or light
+    // (of sequence and kv head) about four together, the heaviest query tiles of all first; pair after pair, a CU's workgroups were heavy or light
     // together and the last pair's heaviest tile began half way.  Workgroups one after the other run on the XCD's four shader engines, so
     // the pairs turn by one every time.  Where all workgroups are there from the start, 32 (one for each CU) go there and the next 32
     // back instead, so that a CU that has a heavy one gets a light one with it (one heavy after the other is better where
     // CUs that have ended take the next).  Pairs of very different lengths are no order of weight that way and go one after the other:
     // 16 / 4 heads of 64, 16 chunks of 300 rows on 600 .. 4000 keys 121 us, together 145, 6 prompts of 300 .. 1300 50 and 57, 6 of 466 .. 862 50 and 37.
     const int split = blockIdx.x / p.grid_base, bid = blockIdx.x - split * p.grid_base;
-    const PairGroup group = scoremod_group(bid, p.rounds, p.slots_per_pair, p.xs_shift);
+    const PairGroup group = scoremod_group(bid, p.sets, p.slots_per_pair, p.xs_shift);
     bool even = p.even > 0;
     if (p.even < 0) {                                 // (keys in front of the rows: the host does not know their number)
         int longest = 0, keys = 0, n = 0;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < 5; ++i) {
             const int pair = group.pair + i * group.step;
             if (i < group.n && pair < p.n_pairs) {
                 const int b = pair / p.G, rows = p.cu_q[b + 1] - p.cu_q[b], n_k = rows > 1 ? p.cu_k[b + 1] - p.cu_k[b] : 0;
@@ -81,7 +80,7 @@ __global__ __launch_bounds__(256, 2) void scoremod_rows_kernel(const ScoremodRow
         }
         even = scoremod_even(keys, longest, n, 0);
     }
-    const PairPlace at = scoremod_order(group, bid, p.slots_per_pair, p.xs_shift, even ? 4 : 1, even ? p.there_and_back : 0);
+    const PairPlace at = scoremod_order(group, bid, p.slots_per_pair, p.xs_shift, even, p.there_and_back);
     const int pair = at.pair, widx = at.place;
     if (pair >= p.n_pairs || widx >= p.wg_per_pair) return;
     const int groups = p.wg_per_pair / p.n_qtiles, hg = widx % groups, qt = p.n_qtiles - 1 - widx / groups;   // heaviest first
@@ -367,7 +366,7 @@ int launch_scoremod_rows(ScoremodRowsParams p, const ScoremodRowsPlan& f, int D,
     p.n_pairs = f.n_pairs;
     p.xs_shift = f.xs_shift;
     p.slots_per_pair = f.slots_per_pair;
-    p.rounds = (int)(f.grid_base / (8 * (int64_t)f.slots_per_pair));
+    p.sets = scoremod_sets((int)(f.grid_base / (8 * (int64_t)f.slots_per_pair)));
     p.even = scoremod_pairs(f.grid_base, num_seqs, total_q, max_seqlen_q, max_seqlen_k);
     p.there_and_back = f.grid_base * f.nsplit <= 256 * (D + Dv == 128 ? 4 : D + Dv == 192 ? 3 : 2);       // (workgroups that a CU holds)
     p.grid_base = (int)f.grid_base;

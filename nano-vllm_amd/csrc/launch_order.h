@@ -36,6 +36,21 @@ NV_HD int latent_tiles(int last_key, int tile_keys, int nsplit, int fewest) {
 // Its ranges: at most nsplit, since a share is never below `fewest`.
 NV_HD int latent_ranges(int tiles, int share) { return tiles <= share ? 1 : (tiles - 1) / share + 1; }
 
+// An XCD's pairs in sets that differ by one at most: the first `more` pairs in sets of least + 1, the others in sets of `least`.
+struct PairSets {
+    int least, more;
+};
+NV_HD PairSets pair_sets(int pairs, int sets) { return {pairs / sets, pairs % sets * (pairs / sets + 1)}; }
+// A workgroup's slot on its XCD -> its set's first pair, how many there are, and its place among their workgroups.  (One division on the device.)
+struct SetPlace {
+    int first, n, at;
+};
+NV_HD SetPlace set_place(int slot, int slots_per_pair, const PairSets& s) {
+    const int front = s.more * slots_per_pair, n = slot < front ? s.least + 1 : s.least, rest = slot < front ? slot : slot - front;
+    const int set = rest / (n * slots_per_pair);
+    return {(slot < front ? 0 : s.more) + set * n, n, rest - set * n * slots_per_pair};
+}
+
 // Prompt attention, single query tiles a workgroup: how many pairs of sequence and kv head an XCD takes together, the heaviest tiles of all first.  For
 // sequences of about the same length and about two rounds of workgroups, as long as the pairs' keys and values stay within half its L2 (those of a larger set, below, within all of it).  4 prompts of 2000 ..
 // 2048 tokens, 16 / 8 heads: 101 -> 86 us, 8 of 900 .. 1024 68 -> 57, 6 of 1000 .. 1365 72 -> 64; 2 of 600 and 2048, 32 / 8 heads, 61 -> 66, and with
@@ -63,8 +78,12 @@ NV_HD RoundPlace prefill_order(int slot, int rounds, int slots_per_pair, int set
 }
 
 // Score-modified attention, prompt portions: workgroup (of a key range) -> its pair of sequence and kv head and its place in the pair, heaviest query
-// tile first.  Workgroups go to the eight XCDs in turn; an XCD has `rounds` pairs (8 >> xs_shift of them a round over all XCDs), four to a group.
+// tile first.  Workgroups go to the eight XCDs in turn; an XCD has `rounds` pairs (8 >> xs_shift of them a round over all XCDs) in sets of three to
+// five: what four at a time leave over begins with its heaviest tile when the others end.  One after the other / fours and the rest last /
+// so: 3 prompts of 1893 .. 2197, 16 heads of 128 each, 127 / 138 / 117 us, 12 of 444 .. 676, 16 / 4 of 64, 43.6 / 47.0 / 41.8; 70
+// launches of a number of pairs that fours do not divide 1 / 0.991 / 0.975 on average, 1.05 at most (1.08 with the rest last).
 // grid: 8 * rounds * slots_per_pair; places past a pair's workgroups and pairs past the last one are for the caller to leave out.
+NV_HD PairSets scoremod_sets(int rounds) { return pair_sets(rounds, rounds < 6 ? 1 : (rounds + 2) / 4); }
 struct PairGroup {
     int pair, step, n;          // the group's first pair, from one pair to the next, how many there are
     int at;                     // the workgroup's place in the group
@@ -72,9 +91,9 @@ struct PairGroup {
 struct PairPlace {
     int pair, place;
 };
-NV_HD PairGroup scoremod_group(int index, int rounds, int slots_per_pair, int xs_shift) {
-    const int xcd = index & 7, slot = index >> 3, group = slot / (4 * slots_per_pair), left = rounds - 4 * group;
-    return {4 * group * (8 >> xs_shift) + (xcd >> xs_shift), 8 >> xs_shift, left < 4 ? left : 4, slot - group * 4 * slots_per_pair};
+NV_HD PairGroup scoremod_group(int index, const PairSets& sets, int slots_per_pair, int xs_shift) {
+    const SetPlace at = set_place(index >> 3, slots_per_pair, sets);
+    return {at.first * (8 >> xs_shift) + ((index & 7) >> xs_shift), 8 >> xs_shift, at.n, at.at};
 }
 // Whether pairs are of about the same length: `n` of them (of a group of chunks; the sequences of a step of whole prompts) with `keys` keys in all.  In 170 steps of 2 to 16 sequences whole prompts gained from
 // an average of three quarters of the longest on, chunks, whose tiles are all about as heavy as their sequence is long, from eight ninths on.
@@ -89,14 +108,13 @@ NV_HD int scoremod_pairs(int64_t grid_base, int num_seqs, int64_t total_q, int m
     if (max_q == max_k) return scoremod_even(total_q, max_q, num_seqs, 1);
     return grid_base <= 256 ? 0 : -1;
 }
-// together: the pairs of the group (four, or one) that are taken place by place, turning by one every time; the others one
-// after the other.  there_and_back: 32 workgroups of the XCD there and the next 32 back instead.
-NV_HD PairPlace scoremod_order(const PairGroup& g, int index, int slots_per_pair, int xs_shift, int together, int there_and_back) {
-    const int part = g.at / (together * slots_per_pair), left = g.n - part * together, n = together < left ? together : left;
-    int at = g.at - part * together * slots_per_pair;
-    if (there_and_back && (at & 32) && (at | 31) < n * slots_per_pair) at ^= 31;
-    const int rank = at / n, one = at - rank * n + (there_and_back ? 0 : rank);
-    return {g.pair + (part * together + one % n) * g.step, (rank << xs_shift) + (index & ((1 << xs_shift) - 1))};
+// together: the pairs of the set place by place, turning by one every time, or one after the other.  there_and_back: 32 workgroups of the XCD there and the next 32 back instead.
+NV_HD PairPlace scoremod_order(const PairGroup& g, int index, int slots_per_pair, int xs_shift, bool together, int there_and_back) {
+    int at = g.at;
+    if (together && there_and_back && (at & 32) && (at | 31) < g.n * slots_per_pair) at ^= 31;
+    const int rank = together ? at / g.n : at % slots_per_pair;
+    const int one = together ? (at - rank * g.n + (there_and_back ? 0 : rank)) % g.n : at / slots_per_pair;
+    return {g.pair + one * g.step, (rank << xs_shift) + (index & ((1 << xs_shift) - 1))};
 }
 
 // Tiles of 128 rows, no more blocks than CUs: slices 32 deep, since nothing else runs on a CU while its one workgroup waits for a slice.  Tiles of an
