@@ -25,7 +25,6 @@
 
 #include "nv_common.h"
 #include "attn_prefill_shared.h"
-#include "launch_order.h"
 
 #ifndef NV_PF_MAX_ITEMS
 #define NV_PF_MAX_ITEMS 4
@@ -632,9 +631,9 @@ extern "C" int nv_attn_prefill_varlen(const void* q, const void* k_cache, const 
     p.grid_base = (int)sh.grid_base;
     p.xs_shift = sh.xs_shift;
     p.slots_per_pair = sh.slots_per_pair;
-    p.rounds = (int)(sh.grid_base / (8 * (int64_t)sh.slots_per_pair));
+    const int rounds = (int)(sh.grid_base / (8 * (int64_t)sh.slots_per_pair));
     const bool together = sh.hand_scheduled && sh.nsplit == 1 && sh.items_per_wg == 1;
-    p.sets = together ? prefill_sets(p.rounds, prefill_together((int64_t)sh.n_pairs * sh.wg_per_pair, total_q, B, max_seqlen_q, max_seqlen_k)) : p.rounds;
+    p.sets = prefill_sets(rounds, together ? prefill_together((int64_t)sh.n_pairs * sh.wg_per_pair, total_q, B, max_seqlen_q, max_seqlen_k) : 1);
     p.fd_slots_per_pair = make_fastdiv((uint32_t)sh.slots_per_pair);
     p.pair_items = sh.items_per_wg;
     p.groups = sh.wg_per_pair / sh.n_qtiles;

@@ -1,6 +1,7 @@
 // Declarations shared by the two prefill attention kernels (attn_prefill.hip, attn_prefill_asm.hip).
 #pragma once
 
+#include "launch_order.h"
 #include "nv_common.h"
 
 namespace nv {
@@ -46,7 +47,7 @@ struct PrefillParams {
     // pairs: then each pair is spread over 1 << xs_shift XCDs (2, 4 or 8), or most of the chip would idle
     // (one sequence on a one-kv-head shard ran on one XCD of eight).  slots_per_pair = ceil(wg_per_pair >> xs_shift).
     int xs_shift, slots_per_pair;
-    int rounds, sets;     // pairs of an XCD, and how many sets of them it takes one after the other, in each the heaviest query tiles of all first
+    PairSets sets;        // of an XCD's pairs, taken one set after the other, in each the heaviest query tiles of all first
     int pair_items;       // hand-scheduled kernel: query tiles per workgroup (1, 2 or 4; balanced over the sequence)
     // the block-index decomposition's divisors, prepared by the host (the merge launch is a few hundred instructions long)
     int groups;           // wg_per_pair / n_qtiles: head groups per kv head (G / hpw)

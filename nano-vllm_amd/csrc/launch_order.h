@@ -64,17 +64,16 @@ NV_HD int prefill_together(int64_t workgroups, int64_t total_q, int num_seqs, in
 // its heaviest tile when the others end.  One after the other / in sets of four with the rest last / so: 9 prompts of 545 .. 793, 16 / 8 heads,
 // 48.8 / 51.8 / 44.7 us, 10 of 627 .. 654, 16 / 4, 45.0 / 46.4 / 39.7, 5 of 771 .. 1206, 16 / 16, 58.7 / 63.1 / 58.9; 90 launches of 257 to 576
 // workgroups 1 / 0.960 / 0.938 on average, 1.06 at most (1.07 with the rest last).
-NV_HD int prefill_sets(int rounds, int together) { return rounds > together ? rounds / together : 1; }
+NV_HD PairSets prefill_sets(int rounds, int together) { return pair_sets(rounds, rounds > together ? rounds / together : 1); }
 // A workgroup's slot on its XCD -> round of pairs and place in the pair: the rounds of a set place by place, turning by one every time.
 struct RoundPlace {
     int round, place;
 };
-NV_HD RoundPlace prefill_order(int slot, int rounds, int slots_per_pair, int sets) {
-    const int round = slot / slots_per_pair;
-    if (sets == rounds) return {round, slot - round * slots_per_pair};
-    const int least = rounds / sets, more = (rounds - least * sets) * (least + 1);         // rounds of the sets with one more, which are first
-    const int from = round < more ? 0 : more, n = round < more ? least + 1 : least, first = from + (round - from) / n * n, at = slot - first * slots_per_pair;
-    return {first + (at + at / n) % n, at / n};
+NV_HD RoundPlace prefill_order(int slot, int slots_per_pair, const PairSets& sets) {
+    const SetPlace s = set_place(slot, slots_per_pair, sets);
+    if (s.n == 1) return {s.first, s.at};
+    const int place = s.at / s.n;
+    return {s.first + (s.at + place) % s.n, place};
 }
 
 // Score-modified attention, prompt portions: workgroup (of a key range) -> its pair of sequence and kv head and its place in the pair, heaviest query

@@ -29,10 +29,14 @@ extern "C" void scored(int rounds, int slots, int xs_shift, int together, int th
 extern "C" int pairs_together(int64_t workgroups, int64_t total_q, int num_seqs, int max_q, int max_k) {
     return prefill_together(workgroups, total_q, num_seqs, max_q, max_k);
 }
-extern "C" int sets(int rounds, int together) { return prefill_sets(rounds, together); }
-extern "C" void prompt(int rounds, int slots, int sets, int* round, int* place) {
+extern "C" void sets(int rounds, int together, int* least, int* more) {
+    const PairSets s = prefill_sets(rounds, together);
+    *least = s.least;
+    *more = s.more;
+}
+extern "C" void prompt(int rounds, int slots, int together, int* round, int* place) {
     for (int i = 0; i < rounds * slots; ++i) {
-        const RoundPlace at = prefill_order(i, rounds, slots, sets);
+        const RoundPlace at = prefill_order(i, slots, prefill_sets(rounds, together));
         round[i] = at.round;
         place[i] = at.place;
     }
@@ -159,14 +163,15 @@ def test_latent_turned_order(order):
 @pytest.mark.parametrize("together", [1, 2, 3, 4])
 def test_prompt_every_place_once(order, together):
     for rounds in (1, 2, 3, 4, 5, 8, 9, 13, 72):
-        sets = order.sets(rounds, together)
-        sizes = [rounds // sets + (i < rounds % sets) for i in range(sets)]
-        assert sum(sizes) == rounds and min(sizes) >= min(together, rounds) and max(sizes) <= min(sizes) + 1 <= 2 * together       # nothing is left over
+        least, more = C.c_int(), C.c_int()
+        order.sets(rounds, together, C.byref(least), C.byref(more))
+        sizes = [least.value + 1] * (more.value // (least.value + 1)) + [least.value] * ((rounds - more.value) // least.value)
+        assert sum(sizes) == rounds and least.value >= min(together, rounds) and max(sizes) <= 2 * together       # nothing is left over
         of = [s for s, n in enumerate(sizes) for _ in range(n)]
         for slots in (1, 2, 7, 8, 32, 33):
             n = rounds * slots
             round_, place = (C.c_int * n)(), (C.c_int * n)()
-            order.prompt(rounds, slots, sets, round_, place)
+            order.prompt(rounds, slots, together, round_, place)
             assert sorted(zip(round_, place)) == [(r, s) for r in range(rounds) for s in range(slots)], (rounds, slots)
             assert [of[r] for r in round_] == [of[i // slots] for i in range(n)]          # one set after the other
             for s in set(of):                                     # the heaviest tiles of a set first
