@@ -14,6 +14,8 @@
 //                  (32 for wide rows) are staged once for the four waves, double-buffered.
 //                  The loads of the next tile run beside the products of this one only with an LDS object per buffer (16 heads,
 //                  256 columns, 1024 rows of each of 2 sequences of 3000 and 6001 keys: 302 -> 233 us against two halves of one array).
+//                  That spares the plain reads only: the compiler waits for all vector memory, the next tile with it, in front of the
+//                  first transposed read of a tile.
 //   single kernel  sequences with one token: a workgroup takes up to 32 heads; its four waves take the key tiles of 32 in
 //                  turn, each staging its own (no barrier in the loop), and join their states through LDS.
 //

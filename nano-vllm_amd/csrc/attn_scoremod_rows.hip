@@ -12,11 +12,14 @@
 // the same in 64 bits (2-norms relative to the output rows, bf16), on either.  Exponentials relative to the soft cap, without any
 // maximum: 0.0028 and 119 us; the same with probabilities as the sum of two bf16 numbers: 0.0022 and 148 us.
 //
-// What bounds it: the vector units.  64 soft-capped scores cost a SIMD two exponentials and a reciprocal at quarter rate, about 70
-// cycles with what is around them, beside 32 cycles of matrix products.  Measured (4 prompts of 1777 .. 2048 tokens, 16 / 8 heads of 128,
-// soft cap and sink, the call with its preparation of 21 us): 116 us (127 with an XCD's pairs one after the other, see there; 129 with the
-// denominator as a product of rounded weights with ones, 3 us more with a polynomial in place of the cap's exponential and reciprocal); with the launch on 16 x 16 tiles, values transposed through registers, which other sizes still take, 496 us (44 of them
-// preparation).
+// What bounds it: waiting.  A key tile takes 2.1 us by itself and 3.2 beside the CU's other workgroup, where 64 soft-capped scores cost a SIMD about 70
+// cycles (two exponentials and a reciprocal at quarter rate with what is around them) beside 32 of matrix products, and fewer vector
+// instructions do not help: 3 us more with a polynomial in place of the cap's exponential and reciprocal.  The compiler cannot tell a transposed
+// read from the LDS-DMA in flight and puts a wait for all vector memory in front of the first one of every tile, so for the next
+// tile, whose loads start at the head of the same step; and the products of the first key block each wait for the two reads just before them.
+// 4 prompts of 1777 .. 2048 tokens, 16 / 8 heads of 128, soft cap and sink, the call with its preparation of 21 us: 117 us (127 with an XCD's pairs
+// one after the other, see there; 129 with the denominator as a product of rounded weights with ones); with the launch on 16 x 16
+// tiles, values transposed through registers, which other sizes still take, 496 us (44 of them preparation).
 #include <algorithm>
 #include <type_traits>
 

@@ -13,11 +13,15 @@
 // nv_moe_down           out[pair, :] = weight[pair] * (D_e y[position, :]), fp32, at the pair's own row: the caller sums
 //                       the `top` rows of a token in a fixed order (no atomics, bitwise reproducible).
 //
-// Both products are one grouped matrix product on the matrix cores: a workgroup of four waves takes one row tile
-// (16 to 128 rows of ONE expert) and 64 or 128 output columns, stages 64-deep (fp32: 32-deep) slices of the rows and of the
-// expert's weight rows through LDS, the next slices already on their way into registers, and issues v_mfma_f32_16x16x32_bf16 (bfloat16) or v_mfma_f32_16x16x4_f32 (true fp32) on them; a
-// wave owns 16 or 32 columns and all row sub-tiles.  Weights are
-// [E, rows_out, rows_in] with the contraction index contiguous, as stored.  The launch is sized for the most tiles any
+// Both products are grouped matrix products on the matrix cores, a row tile (16 to 128 rows of ONE expert) and some columns a workgroup of
+// four waves, in one of three kernels:
+//   moe_big_kernel      tiles of 128 rows, bf16: 256 weight rows, both operands by LDS-DMA, v_mfma_f32_32x32x16_bf16
+//   moe_rows_kernel     tiles of 16, 32 and 64 rows, bf16, few tiles that read the same weights: 64 weight rows straight from memory into
+//                       the operands' registers, the waves share the contraction
+//   moe_grouped_kernel  everything else (float32, sizes and addresses that are not in 16-byte pieces, many small tiles of the same
+//                       weights): 64 or 128 weight rows, 64-deep (fp32: 32-deep) slices of both operands through LDS, the next slices
+//                       on their way into registers, v_mfma_f32_16x16x32_bf16 or v_mfma_f32_16x16x4_f32 (true fp32)
+// Weights are [E, rows_out, rows_in] with the contraction index contiguous, as stored.  The launch is sized for the most tiles any
 // routing can produce; workgroups beyond the table's count return at once.
 #include <algorithm>
 #include <type_traits>
@@ -489,7 +493,8 @@ __device__ __forceinline__ float moe_glu(float g, float u, float limit, float al
 // ones; neither is written.
 // Launches that leave a CU one workgroup, and rows or weights 4 GiB apart, take slices 32 deep by address, three buffers and two slices in flight.
 // What bounds it: the way of the slices from L2 (11 TB/s through the CUs' vector caches).  Slices 32 deep take half a cache line of every row
-// and the same line again for the next slice: 340 and 240 us for both products of the call below.  Without any loads behind the first slice it is 217 and 136 us, with all of them in the vector caches 226 and 145, in L2 263 and 160.
+// and the same line again for the next slice: 340 and 240 us for both products of the call below.  Without any loads behind the first slice it
+// is 217 and 136 us, with all of them in the vector caches 226 and 145, in L2 263 and 160 (these, and the next lines', with the cheaper gated unit).
 // Buffer loads, because the compiler waits for all LDS reads behind a global load into LDS (and has no 64-bit addresses to add up): 336 -> 281
 // us; the products at a higher priority than the other workgroup's reads: 299 -> 281.  256 x 256 by one workgroup a CU, two buffers: four
 // waves of 128 x 128 319 and 211 us, eight of 64 x 128 349 and 220; a load of the lines two slices ahead into L2: no gain.

@@ -19,7 +19,8 @@ _retired: list[torch.Tensor] = []   # outgrown workspaces stay alive: captured g
 
 # The helpers below run several times a call, and a call of one token is bound by them: the raw stream without a Stream object around
 # it, messages only where they are raised.  Host time a call, before and after: paged attention of one sequence 28 and 20 us,
-# attention with modified scores 37 and 30, routed experts 32 and 27; 18, 28 and 19 since the entry points are CPython callables.
+# attention with modified scores 37 and 30, routed experts 32 and 27; 18, 28 and 19 since the entry points are CPython callables and
+# the experts' routing and sort one of them.
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)      # (not in builds of torch without a GPU)
 
 
