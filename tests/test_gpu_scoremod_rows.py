@@ -177,10 +177,12 @@ def test_every_row_whatever_the_order(H, G, n_qs):
 
 @pytest.mark.parametrize("H,G,n_qs,n_ks", [
     (8, 8, [2500] * 4, None),                         # all resident, 4 rounds of 20: workgroups 32 .. 63 of an XCD's group go back
-    (16, 8, [900] * 9, None),                         # more than are resident, 9 rounds: the last group has one pair, the others turn
-    (16, 4, [300] * 6, [310, 330, 350, 340, 320, 300]),   # chunks of about the same length, a group of three pairs
-    (16, 4, [300] * 6, [2000, 330, 1200, 340, 700, 300]),  # and of very different ones: one after the other
-    (16, 4, [300, 1, 300, 40, 1], [1000, 3000, 980, 990, 64]),     # single rows between them
+    (16, 8, [900] * 9, None),                         # more than are resident, 9 rounds: sets of five and four pairs that turn
+    (16, 4, [400] * 6, [410, 430, 450, 440, 420, 400]),   # chunks of about the same length, a set of three pairs
+    (16, 4, [400] * 6, [2000, 430, 1200, 440, 700, 400]),  # and of very different ones: one after the other
+    (16, 4, [300] * 6, [310, 330, 350, 340, 320, 300]),   # too few workgroups to look at their lengths
+    (16, 4, [430, 1, 430, 40, 1], [1000, 3000, 980, 990, 64]),     # single rows between them
+    (16, 8, [200] * 13, [201 + i for i in range(13)]),    # sets of five, four and four
     (16, 8, [700, 90, 350, 300, 410], None)])         # prompts of very different lengths
 def test_orders_of_pairs(H, G, n_qs, n_ks):
     """Every order that the launch chooses from: every row is written once, by the workgroup that has its keys."""
