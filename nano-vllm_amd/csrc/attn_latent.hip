@@ -11,11 +11,14 @@
 // running maximum is per lane pair and raised only when a score exceeds it by 2^8, so the accumulators are seldom rescaled.
 //
 //   rows kernel    sequences with several tokens in the step: a workgroup of four waves takes 128 rows; key tiles of 64
-//                  (32 for wide rows) are staged once for the four waves, double-buffered.
-//                  The loads of the next tile run beside the products of this one only with an LDS object per buffer (16 heads,
-//                  256 columns, 1024 rows of each of 2 sequences of 3000 and 6001 keys: 302 -> 233 us against two halves of one array).
-//                  That spares the plain reads only: the compiler waits for all vector memory, the next tile with it, in front of the
-//                  first transposed read of a tile.
+//                  (32 for wide rows) are staged once for the four waves by loads that the compiler does not know (it would wait for all of
+//                  them in front of a tile's first transposed read).  Where a wave has a SIMD to itself it multiplies the next
+//                  tile's scores beside the weights of this one, with operands four and eight products ahead (two and four elsewhere, where the
+//                  other wave has its turn), the accumulators held in their half of the registers, so that no tile moves them.
+//                  What bounds it then is power: a tile takes 3140 cycles instead of 4400 (2048 of them products), but at 1.4 to 1.66 GHz, with
+//                  the same work, where it was 1.7 to 2.  16 heads, 256 columns, 1024 rows of each of 2 sequences of 3000 and 6001 keys: the call
+//                  164 -> 153 us; a prompt of 2000 tokens 74 -> 65, 37 rows on 3000 keys 37 -> 32.  One wave a SIMD for rows of 160 columns too:
+//                  54 us instead of 58 for a prompt of 2000, but 66 for 59 where 700 rows come on top of up to 2300 keys.
 //   single kernel  sequences with one token: a workgroup takes up to 32 heads; its four waves take the key tiles of 32 in
 //                  turn, each staging its own (no barrier in the loop), and join their states through LDS.
 //
@@ -86,13 +89,20 @@ __device__ __forceinline__ void lat_piece(int piece, int lane, int& row, int& ch
 }
 
 // The state of one wave: 32 rows of queries against the keys it is shown.
-template <int D32, int DV32, int KB>
+template <int D32, int DV32, int KB, bool HOLD>
 struct LatentWave {
     bf16x8 qf[2 * D32];
     f32x16 oacc[DV32];
     float m_run, l_run;
+    uint32_t key_at[2], value_at[2];           // where the lane's operands of a tile at LDS address 0 begin
 
-    __device__ __forceinline__ void init(const __bf16* qrow, int h) {
+    __device__ __forceinline__ void init(const __bf16* qrow, int lane, int dv0) {
+        const int r = lane & 31, h = lane >> 5, i16 = lane & 15, g16 = (lane >> 4) & 1;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            key_at[i] = lat_off<D32>(r, 2 * i + h);
+            value_at[i] = lat_off<D32>(8 * i + 4 * h + (i16 >> 2), 2 * g16 + ((i16 & 3) >> 1)) + 8 * (i16 & 1) + 512 * dv0;
+        }
 #pragma unroll
         for (int s = 0; s < 2 * D32; ++s) qf[s] = *(const bf16x8*)(qrow + 16 * s + 8 * h);
 #pragma unroll
@@ -103,111 +113,237 @@ struct LatentWave {
         l_run = 0.f;
     }
 
-    // A tile of 32 KB keys at `lds`, the first of them key kt; the lane's row sees keys <= qpos (masked: some row of the wave
-    // does not see all of the tile).  The wave accumulates the value columns from 32 dv0 on.
-    // FAR: operands of the first product two steps ahead, the key blocks in turn (rows kernel: 233 -> 221 us at the call above; the
-    // single kernel, whose waves cover each other, lost 1 % with it).
-    template <bool FAR>
-    __device__ __forceinline__ void step(const unsigned char* lds, int lane, int kt, int qpos, bool masked, float scale_log2,
-                                         int dv0) {
-        const int r = lane & 31, h = lane >> 5, i16 = lane & 15, g16 = (lane >> 4) & 1;
-        f32x16 sacc[KB];
+    static constexpr int KSTEPS = 2 * D32, VSTEPS = 2 * KB * DV32;                      // products a key block and tile
+    static constexpr int AHEAD = HOLD ? 4 : 2, KA = KSTEPS < AHEAD ? KSTEPS : AHEAD, VA = VSTEPS < 2 * AHEAD ? VSTEPS : 2 * AHEAD;
+    typedef bf16x8 Keys[KA][KB];
+    typedef bf16x8 Values[VA];
+    // The lane's way through a tile; operands lie at constant distances from it.
+    struct Tile {
+        const lds_byte *key[2], *value[2];
+    };
+    __device__ __forceinline__ Tile tile(uint32_t at) const {
+        return {{(const lds_byte*)(key_at[0] + at), (const lds_byte*)(key_at[1] + at)}, {(const lds_byte*)(value_at[0] + at), (const lds_byte*)(value_at[1] + at)}};
+    }
+    // Operand c of the first product: 32 keys of each block, columns 16 c ...
+    __device__ __forceinline__ void keys(const Tile& t, int c, Keys& a) {
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)
+            a[c % KA][kb] = *(const __attribute__((address_space(3))) bf16x8*)(t.key[c & 1] + 2048 * D32 * kb + 512 * (c >> 1));
+    }
+    __device__ __forceinline__ void first_keys(const Tile& t, Keys& a) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) sacc[kb][i] = 0.f;
-        if constexpr (!FAR) {
+        for (int c = 0; c < KA; ++c) keys(t, c, a);
+    }
+    // Scores of a tile's 32 KB keys (register i of block kb is key 32 kb + (i & 3) + 8 (i >> 2) + 4 h of the tile).  The first operands are in
+    // `a`, the others come as many products ahead; beside() is what the wave does beside the products of a step.
+    template <class F>
+    __device__ __forceinline__ void scores(const Tile& t, f32x16 (&s)[KB], Keys& a, F beside) {
+        constexpr f32x16 zero = {};
 #pragma unroll
-            for (int kb = 0; kb < KB; ++kb)
+        for (int c = 0; c < KSTEPS; ++c) {
+            __builtin_amdgcn_sched_barrier(0);                       // (left alone, a product waits for the read just before it)
 #pragma unroll
-                for (int s = 0; s < 2 * D32; ++s) {
-                    const bf16x8 a = *(const bf16x8*)(lds + lat_off<D32>(kb * 32 + r, 2 * s + h));
-                    sacc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[s], sacc[kb], 0, 0, 0);
-                }
-        } else {
-            constexpr int AHEAD = 2;                                 // operand steps on their way before a product needs them
-            bf16x8 a[2 * D32][KB];
-            auto fetch = [&](int s) {
-#pragma unroll
-                for (int kb = 0; kb < KB; ++kb) a[s][kb] = *(const bf16x8*)(lds + lat_off<D32>(kb * 32 + r, 2 * s + h));
-            };
-#pragma unroll
-            for (int s = 0; s < AHEAD; ++s) fetch(s);
-#pragma unroll
-            for (int s = 0; s < 2 * D32; ++s) {
-                __builtin_amdgcn_sched_barrier(0);                   // (left alone, a product waits for the read just before it)
-                if (s + AHEAD < 2 * D32) fetch(s + AHEAD);
-#pragma unroll
-                for (int kb = 0; kb < KB; ++kb) sacc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s][kb], qf[s], sacc[kb], 0, 0, 0);
-            }
+            for (int kb = 0; kb < KB; ++kb) s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[c % KA][kb], qf[c], c ? s[kb] : zero, 0, 0, 0);
+            if (c + KA < KSTEPS) keys(t, c + KA, a);
+            beside(c);
         }
-        // register i of block kb is key kt + 32 kb + (i & 3) + 8 (i >> 2) + 4 h
-        if (masked) {
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // Weights of the scores, as operands of the second product; their sum goes to `sum`.  Score i in three steps that lie apart beside products.
+    typedef float Scores[16 * KB];             // (numbers, not vectors: they would be carried in the accumulators' half of the registers)
+    __device__ __forceinline__ void relate(Scores& s, int i, float scale_log2) { s[i] = __builtin_fmaf(s[i], scale_log2, -m_run); }
+    __device__ __forceinline__ void power(Scores& s, int i) { s[i] = __builtin_amdgcn_exp2f(s[i]); }
+    __device__ __forceinline__ void take(Scores& s, int i, bf16x8 (&p)[2 * KB], float (&sum)[2]) {
+        sum[i & 1] += s[i];
+        if ((i & 7) == 7) {
 #pragma unroll
-            for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int key = kt + kb * 32 + (i & 3) + 8 * (i >> 2) + 4 * h;
-                    sacc[kb][i] = key <= qpos ? sacc[kb][i] : -INFINITY;
-                }
+            for (int j = 0; j < 8; ++j) p[i >> 3][j] = (__bf16)s[i - 7 + j];
+            asm volatile("" : "+v"(p[i >> 3]));                      // (here and not where it is needed)
         }
-        float tmax = sacc[0][0];
+    }
+    // Operand n of the second product: 16 keys (n / DV32) x 32 columns (n % DV32, from 32 dv0 on), transposed on its way.  Keys of element
+    // j: 16 (n / DV32) + 8 (j >> 2) + 4 h + (j & 3).
+    __device__ __forceinline__ bf16x8 value(const Tile& t, int n) {
+        const int off = 1024 * D32 * (n / DV32) + 512 * (n % DV32);
+        const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(t.value[0] + off));
+        const s16x4 v2 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(t.value[1] + off));
+        return __builtin_bit_cast(bf16x8, __builtin_shufflevector(v1, v2, 0, 1, 2, 3, 4, 5, 6, 7));
+    }
+    // Adds the tile's values with these weights; the first VA operands are in `a`, the others come as many products ahead.  beside() as in scores().
+    template <class F>
+    __device__ __forceinline__ void values(const Tile& t, const bf16x8 (&p)[2 * KB], Values& a, F beside) {
 #pragma unroll
-        for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, sacc[kb][i]);
-        tmax = lat_max_xor32(tmax) * scale_log2;                 // (scale > 0)
-        if (!__all(tmax <= m_run + kLatRaise)) {                 // rare after the first tiles
-            const float m_new = fmaxf(m_run, tmax);
-            const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-            m_run = m_new;
-            l_run *= alpha;
-#pragma unroll
-            for (int d = 0; d < DV32; ++d)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) oacc[d][i] *= alpha;
+        for (int n = 0; n < VSTEPS; ++n) {
+            __builtin_amdgcn_sched_barrier(0);
+            oacc[n % DV32] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[n % VA], p[n / DV32], oacc[n % DV32], 0, 0, 0);
+            if (n + VA < VSTEPS) a[n % VA] = value(t, n + VA);
+            beside(n);
         }
-        float psum = 0.f;
+        __builtin_amdgcn_sched_barrier(0);
+        hold();
+    }
+    __device__ __forceinline__ void values(const Tile& t, const bf16x8 (&p)[2 * KB]) {
+        Values a;
+#pragma unroll
+        for (int n = 0; n < VA; ++n) a[n] = value(t, n);
+        values(t, p, a, [](int) {});
+    }
+    // The lane's row sees keys <= qpos of a tile that starts at key kt.
+    __device__ __forceinline__ void mask(Scores& s, int lane, int kt, int qpos) {
+        asm volatile("");                                            // (a branch around it, not 32 selections in every tile)
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[kb][i], scale_log2, -m_run));
-                sacc[kb][i] = e;
-                psum += e;
+                const int key = kt + kb * 32 + (i & 3) + 8 * (i >> 2) + 4 * (lane >> 5);
+                s[16 * kb + i] = key <= qpos ? s[16 * kb + i] : -INFINITY;
             }
-        l_run += psum;
+    }
+    // Raises the running maximum where a row's largest score (`tmax`, in log2 units) asks for it.
+    __device__ __forceinline__ bool high(float tmax) { return !__all(tmax <= m_run + kLatRaise); }       // rare after the first tiles
+    __device__ __forceinline__ void raise(float tmax) {
+        const float m_new = fmaxf(m_run, tmax);
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        m_run = m_new;
+        l_run *= alpha;
 #pragma unroll
-        for (int s = 0; s < 2 * KB; ++s) {
-            const int kb = s >> 1, s2 = s & 1;
-            bf16x8 pb;
+        for (int d = 0; d < DV32; ++d) {                             // (a block at a time: all of them would drive others out of their registers)
+            if constexpr (HOLD) asm volatile("" : "+a"(oacc[d]));
 #pragma unroll
-            for (int j = 0; j < 8; ++j) pb[j] = (__bf16)sacc[kb][8 * s2 + j];
-            // keys of element j: 32 kb + 16 s2 + 8 (j >> 2) + 4 h + (j & 3)
-            const int row1 = kb * 32 + 16 * s2 + 4 * h + (i16 >> 2);
-#pragma unroll
-            for (int d = 0; d < DV32; ++d) {
-                const int ch = d * 4 + 2 * g16 + ((i16 & 3) >> 1), sub = 8 * (i16 & 1);
-                const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(lds + 512 * dv0 + lat_off<D32>(row1, ch) + sub));
-                const s16x4 v2 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(lds + 512 * dv0 + lat_off<D32>(row1 + 8, ch) + sub));
-                s16x8 va;
-                va[0] = v1[0]; va[1] = v1[1]; va[2] = v1[2]; va[3] = v1[3];
-                va[4] = v2[0]; va[5] = v2[1]; va[6] = v2[2]; va[7] = v2[3];
-                oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, va), pb, oacc[d], 0, 0, 0);
-            }
+            for (int i = 0; i < 16; ++i) oacc[d][i] *= alpha;
+            if constexpr (HOLD) asm volatile("" : "+a"(oacc[d]));
+            else asm volatile("" : "+v"(oacc[d]));
+            __builtin_amdgcn_sched_barrier(0);
         }
+    }
+    // The queries have come (the compiler would wait for them, and with them for the tiles on their way, in front of every product).
+    __device__ __forceinline__ void settle() {
+#pragma unroll
+        for (int s = 0; s < 2 * D32; ++s) {
+            if constexpr (HOLD) asm volatile("" : "+a"(qf[s]));
+            else asm volatile("" : "+v"(qf[s]));
+        }
+    }
+    // The accumulators stay in the accumulators' half of the registers where the raise joins the way past it.
+    __device__ __forceinline__ void hold() {
+#pragma unroll
+        for (int d = 0; d < DV32; ++d) {
+            if constexpr (HOLD) asm volatile("" : "+a"(oacc[d]));
+            else asm volatile("" : "+v"(oacc[d]));
+        }
+    }
+    __device__ __forceinline__ float largest(const Scores& s) {
+        float top = s[0];
+#pragma unroll
+        for (int i = 0; i < 16 * KB; ++i) top = fmaxf(top, s[i]);
+        return top;
+    }
+    // A tile by itself, the first of its keys key kt (masked: some row of the wave does not see all of the tile).
+    __device__ __forceinline__ void step(uint32_t at, int lane, int kt, int qpos, bool masked, float scale_log2) {
+        Scores s;
+        first(at, s, lane, kt, qpos, masked, scale_log2);
+        last(at, s, scale_log2);
+    }
+    __device__ __forceinline__ void first(uint32_t at, Scores& s, int lane, int kt, int qpos, bool masked, float scale_log2) {
+        const Tile t = tile(at);
+        Keys a;
+        f32x16 n[KB];
+        first_keys(t, a);
+        scores(t, n, a, [](int) {});
+#pragma unroll
+        for (int i = 0; i < 16 * KB; ++i) s[i] = n[i >> 4][i & 15];
+        if (masked) mask(s, lane, kt, qpos);
+        const float tmax = lat_max_xor32(largest(s)) * scale_log2;   // (scale > 0)
+        if (high(tmax)) raise(tmax);
+        keep(s);
+    }
+    // The scores stay in the other half from one tile to the next.
+    __device__ __forceinline__ void keep(Scores& s) {
+#pragma unroll
+        for (int i = 0; i < 16 * KB; ++i) asm volatile("" : "+v"(s[i]));
+    }
+    // The weights and values of the tile at `now`, whose scores are s, and beside them the scores of the one at `next` (its first key kt), which
+    // take their place: the weights beside the products of the scores, the largest of those beside the products of the values.  The first
+    // operands of `next` are in `a`, those of the tile behind it are when it returns; half_way() is called between the two, begin() and
+    // load(i), where there are loads, beside the products of the values.
+    template <int LOADS, class S, class B, class F>
+    __device__ __forceinline__ void turn(uint32_t now_at, uint32_t next_at, uint32_t behind_at, Scores& s, Keys& a, int lane, int kt, int qpos,
+                                         bool masked, float scale_log2, S half_way, B begin, F load) {
+        const Tile now = tile(now_at), next = tile(next_at), behind = tile(behind_at);
+        f32x16 n[KB];
+        bf16x8 p[2 * KB];
+        Values v;
+        float sum[2] = {0.f, 0.f};
+        constexpr int ALL = 16 * KB, W = KSTEPS > 4 ? KSTEPS - 2 : KSTEPS, PER = (ALL + W - 1) / W;
+        auto weigh = [&](int c) {
+#pragma unroll
+            for (int i = 0; i < ALL; ++i) {
+                if (i / PER == c) relate(s, i, scale_log2);
+                if (i / PER == c - 1) power(s, i);
+                if (i / PER == c - 2) take(s, i, p, sum);
+            }
+        };
+        scores(next, n, a, [&](int c) {
+            weigh(c);
+#pragma unroll
+            for (int i = 0; i < VA; ++i)                             // (its first operands, where no more keys come)
+                if (c == (KSTEPS > KA ? KSTEPS - KA + i * KA / VA : KSTEPS - 1)) v[i] = value(now, i);
+        });
+#pragma unroll
+        for (int c = KSTEPS; c <= (ALL - 1) / PER + 2; ++c) weigh(c);
+        l_run += sum[0] + sum[1];
+        asm volatile("" : "+v"(l_run));                              // (here, not behind the products of the values)
+        half_way();
+        // The scores are in the accumulators' half of the registers; they move a block at a time, well behind the last product of theirs.
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) asm volatile("" : "+a"(n[kb]));
+        constexpr bool LONG = VSTEPS >= 8 * KB;                      // (products enough to do it beside)
+        constexpr int MOVE = LONG ? VSTEPS / 8 : 0, MAXES = LONG ? VSTEPS / 2 / KB : 1, EACH = 16 / MAXES + (16 % MAXES != 0);
+        constexpr int END = MOVE + (LONG ? MAXES : 0) * KB;
+        float top[2] = {-INFINITY, -INFINITY};
+        values(now, p, v, [&](int c) {
+            if (LOADS > 0 && c == 0) begin();
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i)
+                if (c == (VSTEPS > 4 ? 1 : 0) + i * VSTEPS / (2 * LOADS)) load(i);        // (in the first half)
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb) {
+                const int at = c - MOVE - kb * MAXES;
+                if (LONG ? at == 0 : c == 0) asm volatile("" : "+v"(n[kb]));
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if (LONG ? i / EACH == at : c == 0) top[i & 1] = fmaxf(top[i & 1], n[kb][i]);
+            }
+            if (LONG && c == END) top[0] = lat_max_xor32(fmaxf(top[0], top[1])) * scale_log2;
+            if (c == VSTEPS - 1) first_keys(behind, a);
+        });
+        if constexpr (!LONG || END >= VSTEPS) top[0] = lat_max_xor32(fmaxf(top[0], top[1])) * scale_log2;
+#pragma unroll
+        for (int i = 0; i < ALL; ++i) s[i] = n[i >> 4][i & 15];
+        if (masked) {
+            mask(s, lane, kt, qpos);
+            top[0] = lat_max_xor32(largest(s)) * scale_log2;
+        }
+        if (high(top[0])) raise(top[0]);
+        keep(s);
+    }
+    __device__ __forceinline__ void last(uint32_t at, Scores& s, float scale_log2) {
+        bf16x8 p[2 * KB];
+        float sum[2] = {0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 16 * KB; ++i) {
+            relate(s, i, scale_log2);
+            power(s, i);
+            take(s, i, p, sum);
+        }
+        l_run += sum[0] + sum[1];
+        values(tile(at), p);
     }
 };
 
-__device__ __forceinline__ void lat_dma(const unsigned char* src, unsigned char* dst) {
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                     (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
-}
-
 // first byte of the tile that starts at key `kt` (tiles do not straddle blocks; table entries are clamped into the cache)
 __device__ __forceinline__ const unsigned char* lat_tile_base(const LatentParams& p, int entry, int off, int row_bytes) {
-    const int64_t last = p.num_blocks - 1;
-    const int64_t phys = entry < 0 ? 0 : (entry > last ? last : entry);
+    const int64_t phys = min(max(entry, 0), (int)p.num_blocks - 1);         // (fewer than 2^31)
     return (const unsigned char*)p.cache + (phys * p.block_size + off) * (int64_t)row_bytes;
 }
 
@@ -252,11 +388,12 @@ __device__ __forceinline__ int lat_share(const LatentParams& p, int lane) {
 template <int D32, int DV32, int KB, int OCC, bool EVEN>
 __global__ __launch_bounds__(256, OCC) void attn_latent_rows_kernel(const LatentParams p) {
     constexpr int D = 32 * D32, KT = 32 * KB, kTile = KT * D * 2, kPieces = D32 * KB / 2;
+    constexpr bool TURN = OCC == 1 || D32 <= 3;
     static_assert(D32 * KB % 2 == 0, "a wave stages whole pieces");
     // A tile each; two waves' output staging areas at the end.  Two objects, not one array: the compiler tells a tile's reads from
     // the other tile's LDS-DMA by the object, and with one array it waits for the DMA just issued before the first read.
     constexpr int BUF = kTile > 2 * kLatRows * kLatStageRow ? kTile : 2 * kLatRows * kLatStageRow;
-    __shared__ __attribute__((aligned(16))) unsigned char buf0[BUF], buf1[BUF];
+    __shared__ __attribute__((aligned(16))) unsigned char buf[TURN ? 4 : 2][BUF];
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int split = blockIdx.y, dv0 = blockIdx.z * DV32, Dv = p.Dv;
@@ -283,48 +420,133 @@ __global__ __launch_bounds__(256, OCC) void attn_latent_rows_kernel(const Latent
     if (split >= ranges) return;
     const int wave_first_pos = start + min(rw0, rows - 1) / p.H, wave_last_pos = start + min(rw0 + kLatRows - 1, rows - 1) / p.H;
 
-    LatentWave<D32, DV32, KB> w;
-    w.init(p.q + ((int64_t)q_begin * p.H + my_row) * D, h);
+    LatentWave<D32, DV32, KB, TURN> w;
+    w.init(p.q + ((int64_t)q_begin * p.H + my_row) * D, lane, dv0);
 
     const int* table = p.block_tables + (int64_t)b * p.max_blocks;
-    int dma_row[kPieces];
     uint32_t dma_off[kPieces];
 #pragma unroll
     for (int i = 0; i < kPieces; ++i) {
-        int ch;
-        lat_piece<D32>(wave * kPieces + i, lane, dma_row[i], ch);
-        dma_off[i] = (uint32_t)(dma_row[i] * (D * 2) + ch * 16);
+        int row, ch;
+        lat_piece<D32>(wave * kPieces + i, lane, row, ch);
+        dma_off[i] = (uint32_t)(row * (D * 2) + ch * 16);
     }
-    auto stage = [&](unsigned char* buf, int entry, int t) {
-        const unsigned char* base = lat_tile_base(p, __builtin_amdgcn_readfirstlane(entry), (t % p.tiles_per_block) * KT, D * 2);
-        const int last = n_k - 1 - t * KT;                   // rows behind the sequence's end re-read its last row
-        unsigned char* dst = buf + wave * kPieces * 1024;
+    // The tile that is staged next: its number, its place in its block, and the block's entry of the table, fetched a tile ahead (the first
+    // ones together: the wait for an entry is one for the tiles in front of it too).  Without branches, so that it goes beside products.
+    const int first_block = t_begin / p.tiles_per_block, last_block = max(t_end - 1, 0) / p.tiles_per_block;
+    constexpr int EARLY = TURN ? 3 : 2;
+    int st = t_begin, st_in = t_begin - first_block * p.tiles_per_block, st_block = first_block, entry[EARLY];
 #pragma unroll
-        for (int i = 0; i < kPieces; ++i)
-            lat_dma(base + (dma_off[i] - (uint32_t)(max(dma_row[i] - last, 0) * (D * 2))), dst + i * 1024);
+    for (int i = 0, in = st_in, at = first_block; i < EARLY; ++i) {
+        entry[i] = table[min(at, last_block)];
+        const int wrap = ++in == p.tiles_per_block;
+        in = wrap ? 0 : in;
+        at += wrap;
+    }
+#pragma unroll
+    for (int i = 0; i < EARLY; ++i) entry[i] = __builtin_amdgcn_readfirstlane(entry[i]);
+    const unsigned char* st_base = nullptr;
+    const uint32_t buf_at = lds_address(buf);
+    uint32_t st_to = 0;
+    auto stage_from = [&](int to) {
+        st_base = lat_tile_base(p, __builtin_amdgcn_readfirstlane(entry[0]), st_in * KT, D * 2);
+        st_to = buf_at + to * BUF + wave * kPieces * 1024;
+        ++st;
+        const int wrap = ++st_in == p.tiles_per_block;
+        st_in = wrap ? 0 : st_in;
+        st_block += wrap;
     };
-    int entry_next = 0;
-    if (t_begin < t_end) stage(buf0, table[t_begin / p.tiles_per_block], t_begin);
-    if (t_begin + 1 < t_end) entry_next = table[(t_begin + 1) / p.tiles_per_block];
-    auto tile_step = [&](const unsigned char* now, unsigned char* next, int t) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();                                     // tile t has landed for all, the other buffer is free
-        if (t + 1 < t_end) stage(next, entry_next, t + 1);
-        if (t + 2 < t_end) entry_next = table[(t + 2) / p.tiles_per_block];
-        const int kt = t * KT;
-        if (wave_live && kt <= wave_last_pos)                // (uniform per wave)
-            w.template step<true>(now, lane, kt, qpos, kt + KT - 1 > wave_first_pos, p.scale_log2, dv0);
+    auto next_entry = [&] { entry[0] = table[min(st_block, last_block)]; };       // (in front of the tile's loads: there when the wait for them is over)
+    auto stage_piece = [&](int i) { lds_load16(st_base, dma_off[i], st_to + i * 1024); };
+    auto stage = [&](int to, auto next) {
+        const int last = n_k - 1 - st * KT;                  // rows behind the sequence's end re-read its last row (no tile comes behind that one)
+        if (last < KT - 1) {
+#pragma unroll
+            for (int i = 0; i < kPieces; ++i) {
+                int row, ch;
+                lat_piece<D32>(wave * kPieces + i, lane, row, ch);
+                dma_off[i] -= (uint32_t)(max(row - last, 0) * (D * 2));
+            }
+        }
+        stage_from(to);
+        next();
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) stage_piece(i);
     };
-    for (int t = t_begin; t < t_end; t += 2) {
-        tile_step(buf0, buf1, t);
-        if (t + 1 < t_end) tile_step(buf1, buf0, t + 1);
+    auto shift = [&] {
+#pragma unroll
+        for (int i = 1; i < EARLY; ++i) entry[i - 1] = entry[i];
+    };
+    const int w_end = wave_live ? min(t_end, wave_last_pos / KT + 1) : t_begin;      // behind the wave's last tile
+    const int full = wave_first_pos + 1 - KT;                // a tile that starts there at the latest is seen by all rows of the wave
+    int t = t_begin, now = 0;
+    if constexpr (TURN) {
+        // Tile t's values and tile t + 1's scores in a step.  Half way through it tile t + 2 has landed for all and tile t - 1 is done with, so
+        // the loads of tile t + 3 go out.
+        auto sync = [&] {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        };
+        if (t < t_end) stage(0, shift);
+        if (t + 1 < t_end) stage(1, shift);
+        if (t + 2 < t_end) {
+            stage(2, next_entry);
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPieces) : "memory");
+        } else {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+        w.settle();
+        __syncthreads();
+        typename LatentWave<D32, DV32, KB, TURN>::Scores sc;
+        typename LatentWave<D32, DV32, KB, TURN>::Keys keys;
+        if (t < w_end) {
+            w.first(buf_at, sc, lane, t * KT, qpos, t * KT > full, p.scale_log2);
+            w.first_keys(w.tile(buf_at + BUF), keys);
+        }
+        auto turn = [&](auto more) {
+            w.template turn<decltype(more)::value ? kPieces : 0>(
+                buf_at + now * BUF, buf_at + ((now + 1) & 3) * BUF, buf_at + ((now + 2) & 3) * BUF, sc, keys, lane, (t + 1) * KT, qpos, (t + 1) * KT > full,
+                p.scale_log2,
+                [&] {
+                    sync();
+                    if constexpr (!decltype(more)::value)
+                        if (t + 3 < t_end) stage((now + 3) & 3, next_entry);
+                },
+                [&] {
+                    stage_from((now + 3) & 3);
+                    next_entry();
+                },
+                stage_piece);
+        };
+        const int whole = min(t_end, n_k / KT);              // (a tile that the sequence ends in is staged by itself)
+        for (; t + 1 < w_end && t + 3 < whole; ++t, now = (now + 1) & 3) turn(std::true_type{});
+        for (; t + 1 < w_end; ++t, now = (now + 1) & 3) turn(std::false_type{});
+        if (t < w_end) w.last(buf_at + now * BUF, sc, p.scale_log2);
+        for (; t < t_end; ++t, now = (now + 1) & 3) {        // (loads for the waves that have more tiles)
+            sync();
+            if (t + 3 < t_end) stage((now + 3) & 3, next_entry);
+        }
+    } else {
+        if (t < t_end) stage(0, shift);
+        w.settle();
+        auto head = [&] {                                    // tile t has landed for all, the other buffer is free
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (t + 1 < t_end) stage(now ^ 1, next_entry);
+        };
+        for (; t < w_end; ++t, now ^= 1) {
+            head();
+            w.step(buf_at + now * BUF, lane, t * KT, qpos, t * KT > full, p.scale_log2);
+        }
+        for (; t < t_end; ++t, now ^= 1) head();
     }
     const float l_tot = lat_sum_xor32(w.l_run);
     __syncthreads();                                         // every wave is done reading tiles
     if (!wave_live) return;
     // Lane (r, h) holds columns 32 d + 8 (i >> 2) + 4 h + (i & 3) of row r: through the wave's staging area to 128-byte row
     // segments.
-    unsigned char* stg = (wave < 2 ? buf0 : buf1) + (wave & 1) * (kLatRows * kLatStageRow);
+    unsigned char* stg = buf[wave >> 1] + (wave & 1) * (kLatRows * kLatStageRow);
     const int rows_here = rows - rw0;
     const int64_t grow = (int64_t)q_begin * p.H + rw0;
     if (ranges > 1) {
@@ -402,17 +624,17 @@ __global__ __launch_bounds__(256, OCC) void attn_latent_single_kernel(const Late
         for (int i = 0; i < kPieces; ++i) {
             int row, ch;
             lat_piece<D32>(i, lane, row, ch);
-            lat_dma(base + (uint32_t)(min(row, last) * (D * 2) + ch * 16), mine + buf * kTile + i * 1024);
+            lds_load16(base, (uint32_t)(min(row, last) * (D * 2) + ch * 16), lds_address(mine + buf * kTile + i * 1024));
         }
     };
-    LatentWave<D32, DV32, 1> w;
+    LatentWave<D32, DV32, 1, false> w;
     int t = t_begin + wave, buf = 0;
     if (t < t_end) stage(0, t);
-    w.init(p.q + ((int64_t)t0 * p.H + head0 + min(r, heads - 1)) * D, h);
+    w.init(p.q + ((int64_t)t0 * p.H + head0 + min(r, heads - 1)) * D, lane, dv0);
     for (; t < t_end; t += 4) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // this wave's own tile has landed
         if (NBUF == 2 && t + 4 < t_end) stage(buf ^ 1, t + 4);
-        w.template step<false>(mine + buf * kTile, lane, t * KT, n_k - 1, t * KT + KT > n_k, p.scale_log2, dv0);
+        w.step(lds_address(mine + buf * kTile), lane, t * KT, n_k - 1, t * KT + KT > n_k, p.scale_log2);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // its reads are done before the buffer is filled again
         if (NBUF == 1 && t + 4 < t_end) stage(0, t + 4);
         if (NBUF == 2) buf ^= 1;

@@ -81,6 +81,17 @@ __device__ __forceinline__ uint4 load_stream16(const uint4* p) {
     return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
+// ---- memory to LDS ---------------------------------------------------------------
+// 16 bytes a lane from `base` + `off` straight into LDS: lane l fills bytes 16 l .. of the KiB at LDS address `to` (base and to uniform).  The
+// compiler does not know this load: it puts no wait in front of LDS reads that it cannot tell from the load's target, and none at all.  The
+// caller waits for it (vmcnt) and puts a barrier where other waves read.  Waits that the compiler counts for its own loads come out longer, never shorter.
+// (m0 is not named as overwritten, since it is a reserved register: a kernel takes either this or the builtins that set m0.)
+__device__ __forceinline__ void lds_load16(const void* base, uint32_t off, uint32_t to) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(to)), "v"(off), "s"(base) : "memory");
+}
+typedef __attribute__((address_space(3))) unsigned char lds_byte;
+__device__ __forceinline__ uint32_t lds_address(const void* p) { return (uint32_t)(uintptr_t)(const lds_byte*)p; }
+
 // ---- cross-lane helpers (wave64) --------------------------------------------------
 template <int CTRL>
 __device__ __forceinline__ float dpp_f32(float x) {
