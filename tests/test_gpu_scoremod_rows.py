@@ -193,3 +193,17 @@ def test_orders_of_pairs(H, G, n_qs, n_ks):
     nv.set_context(None)
     # (as in test_portions)
     torch.testing.assert_close(o.float(), o_r.float(), rtol=2e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("H,G,D,Dv", [(4, 2, 128, 128), (8, 2, 64, 64), (4, 2, 64, 128)])
+@pytest.mark.parametrize("softcap,spread", [(30.0, 0.5), (30.0, 1.0), (8.0, 1.0), (2.0, 1.0), (0.5, 1.0), (30.0, 6.0), (1e-3, 1.0), (1e4, 1.0)])
+def test_caps_far_above_and_below_the_scores(H, G, D, Dv, softcap, spread):
+    """Scores from a hundredth of the cap to far beyond it: tiles within 0.4 caps take another form of tanh than the others, and some tiles of
+    a row may be either.  Tiles whose rows see all of them, and edges."""
+    n_qs, n_ks = [150, 64, 33], [700, 64, 290]
+    a, r, ctx, pos, q, k, v, kc, vc = _step(H, G, D, Dv, 64, n_qs, n_ks, spread=spread, softcap=softcap, use_sink=True)
+    nv.set_context(ctx)
+    o, o_r = a(q, k, v, pos, kc.clone(), vc.clone()), r(q, k, v, pos, kc.clone(), vc.clone())
+    nv.set_context(None)
+    # probabilities and outputs are rounded to bf16 (2^-9 each), values are of order `spread`
+    torch.testing.assert_close(o.float(), o_r.float(), rtol=2e-2, atol=1e-2 * spread)
