@@ -485,3 +485,41 @@ def test_fast_decays(form, rows, rate):
     nv.set_context(None)
     torch.testing.assert_close(got, want, rtol=5e-5, atol=5e-5)          # (the bounds of test_portions)
     torch.testing.assert_close(got_state, want_state, rtol=2e-5, atol=2e-6 * want_state.abs().max().item())
+
+
+@pytest.mark.parametrize("form,H,D,Dv,seqs", [("gated", 16, 128, 128, 96), ("general", 16, 128, 128, 93), ("write", 16, 64, 64, 400),
+                                              ("gated", 8, 96, 80, 400), ("write", 4, 32, 32, 6000)])
+def test_single_tokens_of_more_states_than_the_cache_keeps(form, H, D, Dv, seqs):
+    """Launches of single tokens whose states pass by the caches against the same sequences in launches of half as many, whose states do not:
+    the same bits, fresh states among carried ones, and no other state is touched."""
+    assert seqs * H * D * Dv * 4 >= 92 << 20 > seqs // 2 * H * D * Dv * 4
+    g = torch.Generator(device=DEV).manual_seed(D + seqs)
+    mk = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    a, _ = _layers(form, H, D, Dv, mk)
+    G = H // 2 if form == "gated" else H
+    q, k, v = (x.to(torch.bfloat16) for x in (mk(seqs, G, D), mk(seqs, H if form == "write" else G, D), mk(seqs, H, Dv)))
+    gate, w, rate, b = (x.to(torch.bfloat16) for x in (mk(seqs, H * Dv), mk(seqs, H * D), mk(seqs, H * D), mk(seqs, H)))
+    state = mk(seqs + 3, H, D, Dv)
+    slots = torch.randperm(seqs + 3, generator=g, device=DEV)[:seqs].to(torch.int32)
+
+    def run(lo, hi, state):
+        n = hi - lo
+        cu = torch.arange(n + 1, dtype=torch.int32, device=DEV)
+        before = torch.tensor([0 if i % 7 == 3 else 5 for i in range(lo, hi)])
+        cu_k = torch.tensor([0] + (1 + before).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+        nv.set_context(nv.CacheContext(cu_seqlens_q=cu, cu_seqlens_k=cu_k, state_slots=slots[lo:hi].contiguous(), max_seqlen_q=1, num_leading_decode=n,
+                                       portion_kinds=ops.portion_kinds([])))
+        at = slice(lo, hi)
+        if form == "gated":
+            out = a(q[at], k[at], v[at], w[at], b[at], gate[at], state)
+        elif form == "general":
+            out = a(q[at], k[at], v[at], w[at], rate[at], gate[at], state)
+        else:
+            out = a(q[at], k[at], v[at], {"state": state})
+        nv.set_context(None)
+        return out
+
+    one, two = state.clone(), state.clone()
+    out = run(0, seqs, one)
+    parts = torch.cat([run(0, seqs // 2, two), run(seqs // 2, seqs, two)])
+    assert torch.equal(out, parts) and torch.equal(one, two) and not torch.equal(one, state)
