@@ -140,4 +140,9 @@ NV_HD bool moe_streams(int tile_rows, int64_t pairs, int E, int ff) {
     return pairs < line * (int64_t)E;
 }
 
+// Outputs of the second product (fp32, a row a pair) past the caches: they drive the weights and rows that other column blocks read out of the L2, and
+// large ones are gone before the caller adds a token's rows up.  The call with that sum, through / past, us, top 4 of 32 experts, 2048, 1024: 8192 tokens
+// (268 MB) 538 / 527, 4096 316 / 313, 2048 (67 MB) 214 / 208;  top 2 of 16, 1024, 1024: 8000 (66 MB) 165.7 / 168.3.
+NV_HD bool moe_streams_out(int64_t pairs, int width) { return pairs * width * 4 >= 64LL << 20; }
+
 }  // namespace nv

@@ -498,7 +498,7 @@ __device__ __forceinline__ float moe_glu(float g, float u, float limit, float al
 // Buffer loads, because the compiler waits for all LDS reads behind a global load into LDS (and has no 64-bit addresses to add up): 336 -> 281
 // us; the products at a higher priority than the other workgroup's reads: 299 -> 281.  256 x 256 by one workgroup a CU, two buffers: four
 // waves of 128 x 128 319 and 211 us, eight of 64 x 128 349 and 220; a load of the lines two slices ahead into L2: no gain.
-// 8192 tokens, top 4 of 32 experts, width 2048, ff 1024: gate and up 340 -> 297 us, down 240 -> 187; the call 604 -> 497.
+// 8192 tokens, top 4 of 32 experts, width 2048, ff 1024: gate and up 340 -> 297 us, down 240 -> 187; the call 604 -> 497, with the outputs past the caches 485.
 constexpr int kMoeBigRows = 128;
 
 // D: depth of a slice, 64 or 32.  A piece of 1 KiB is 512 / D rows of 2 D bytes, lane l fills bytes 16 l .. of it.
@@ -506,7 +506,8 @@ template <int D>
 __device__ __forceinline__ int big_off(int row, int ch) {
     return row * 2 * D + ((ch ^ (D == 64 ? (row >> 1) & 7 : (row >> 2) & 3)) * 16);
 }
-template <int MODE, int D>
+// STREAM: outputs pass by the caches (moe_streams_out).
+template <int MODE, int D, bool STREAM = false>
 __global__ __launch_bounds__(256, 2) void moe_big_kernel(
     const __bf16* __restrict__ a, int64_t a_stride, const __bf16* __restrict__ w, const int* __restrict__ sorted_pairs,
     const int* __restrict__ meta, const float* __restrict__ pair_w, __bf16* __restrict__ y, float* __restrict__ out, int top, int N,
@@ -730,8 +731,10 @@ __global__ __launch_bounds__(256, 2) void moe_big_kernel(
                     if (r < rows && n < N) {
                         const int pair = src_row[r];
                         const float f = weight[r];
-                        v.x *= f; v.y *= f; v.z *= f; v.w *= f;
-                        *(float4*)(out + (int64_t)pair * N + n) = v;
+                        const f32x4 o = {v.x * f, v.y * f, v.z * f, v.w * f};
+                        f32x4* to = (f32x4*)(out + (int64_t)pair * N + n);
+                        if constexpr (STREAM) __builtin_nontemporal_store(o, to);
+                        else *to = o;
                     }
                 }
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -1000,12 +1003,16 @@ static void launch_grouped(const void* a, int64_t a_stride, const void* w, const
             constexpr int cols = MODE == 1 ? 128 : 256;
             const int n_cols = (N + cols - 1) / cols;
             const dim3 grid((unsigned)(((int64_t)max_tiles * n_cols + 7) / 8 * 8));
+#define NV_MOE_BIG(D, STREAM)                                                                                                            \
+    hipLaunchKernelGGL((moe_big_kernel<MODE, D, STREAM>), grid, dim3(256), 0, s, (const T*)a, a_stride, (const T*)w, sorted_pairs, meta, pair_w, \
+                       (T*)y, out, top, N, K, limit, alpha, up_shift)
             if (moe_few_blocks(pairs, E, n_cols) || !moe_offsets_ok(MODE == 0 ? kMoeBigRows : a_rows, a_stride, (MODE == 1 ? 2 : 1) * (int64_t)N, K))
-                hipLaunchKernelGGL((moe_big_kernel<MODE, 32>), grid, dim3(256), 0, s, (const T*)a, a_stride, (const T*)w, sorted_pairs, meta, pair_w,
-                                   (T*)y, out, top, N, K, limit, alpha, up_shift);
+                NV_MOE_BIG(32, false);
+            else if (MODE == 0 && moe_streams_out(pairs, N))
+                NV_MOE_BIG(64, MODE == 0);
             else
-                hipLaunchKernelGGL((moe_big_kernel<MODE, 64>), grid, dim3(256), 0, s, (const T*)a, a_stride, (const T*)w, sorted_pairs, meta, pair_w,
-                                   (T*)y, out, top, N, K, limit, alpha, up_shift);
+                NV_MOE_BIG(64, false);
+#undef NV_MOE_BIG
             return;
         }
     }

@@ -59,3 +59,15 @@ def test_rows_far_apart():
     gate_up, down, logits = mk(E, 2 * ff, W, scale=W ** -0.5), mk(E, W, ff, scale=ff ** -0.5), torch.randn(T, E, generator=g, device=DEV)
     a = moe.MoEExperts(top, 1.5)
     torch.testing.assert_close(a(h, logits, gate_up, down), a(near, logits, gate_up, down), **_tol())
+
+
+def test_outputs_past_the_caches():
+    """Outputs of 64 MiB and more pass by the caches: the rows of two calls of half the tokens, whose outputs do not, to the bit."""
+    T, E, top, W, ff = 2100, 16, 4, 2048, 64
+    assert T * top * W * 4 >= 64 << 20 > T // 2 * top * W * 4
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    h, logits = rn(T, W).to(torch.bfloat16), rn(T, E)
+    gate_up, down = (W ** -0.5 * rn(E, 2 * ff, W)).to(torch.bfloat16), (ff ** -0.5 * rn(E, W, ff)).to(torch.bfloat16)
+    call = lambda at: ops.moe_experts(h[at].contiguous(), logits[at].contiguous(), gate_up, down, top, 7.0, 1.702)
+    assert torch.equal(call(slice(0, T)), torch.cat([call(slice(0, T // 2)), call(slice(T // 2, T))]))
