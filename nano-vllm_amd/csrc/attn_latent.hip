@@ -17,7 +17,7 @@
 //                  other wave has its turn), the accumulators held in their half of the registers, so that no tile moves them.
 //                  What bounds it then is power: a tile takes 3140 cycles instead of 4400 (2048 of them products), but at 1.4 to 1.66 GHz, with
 //                  the same work, where it was 1.7 to 2.  16 heads, 256 columns, 1024 rows of each of 2 sequences of 3000 and 6001 keys: the call
-//                  164 -> 153 us; a prompt of 2000 tokens 74 -> 65, 37 rows on 3000 keys 37 -> 32.  One wave a SIMD for rows of 160 columns too:
+//                  164 -> 144 to 153 us by the card; a prompt of 2000 tokens 74 -> 65, 37 rows on 3000 keys 37 -> 32.  One wave a SIMD for rows of 160 columns too:
 //                  54 us instead of 58 for a prompt of 2000, but 66 for 59 where 700 rows come on top of up to 2300 keys.
 //   single kernel  sequences with one token: a workgroup takes up to 32 heads; its four waves take the key tiles of 32 in
 //                  turn, each staging its own (no barrier in the loop), and join their states through LDS.
