@@ -19,8 +19,9 @@
 // the next scores would cost one or two of them: 8 prompts of 1024, 16 / 4 heads of 64, 51 us, so 49, with two waves 56), and tiles come by loads that the
 // compiler does not know (it would wait for the next tile in front of the first transposed read).  Nothing of a wave's is spilled: scratch memory costs a
 // launch about a microsecond.
-// 4 prompts of 1777 .. 2048 tokens, 16 / 8 heads of 128, soft cap and sink, the call with its preparation of 21 us: 115 us (117 with the exponential form of tanh and a tile's work one after the other, then 127 with an XCD's pairs
-// one after the other, see there; 129 with the denominator as a product of rounded weights with ones); with the launch on 16 x 16
+// 4 prompts of 1777 .. 2048 tokens, 16 / 8 heads of 128, soft cap and sink, the call with its preparation of 21 us: 115 us; 117 with tanh from an
+// exponential and a tile's work one after the other, and that way 127 with an XCD's pairs one after the other (see there) and 129
+// with the denominator as a product of rounded weights with ones; with the launch on 16 x 16
 // tiles, values transposed through registers, which other sizes still take, 496 us (44 of them preparation).
 #include <algorithm>
 #include <type_traits>
