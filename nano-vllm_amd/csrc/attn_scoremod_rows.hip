@@ -12,17 +12,18 @@
 // the same in 64 bits (2-norms relative to the output rows, bf16), on either.  Exponentials relative to the soft cap, without any
 // maximum: 0.0028 and 119 us; the same with probabilities as the sum of two bf16 numbers: 0.0022 and 148 us.
 //
-// What bounds it: the instructions of the scores, at a clock of 1.6 GHz (power).  64 soft-capped scores are seven and a half vector instructions and
-// one at quarter rate for a row beside 32 cycles of matrix products; an SIMD takes 2350 cycles for a wave's tile with nine and
-// three, whatever else is in the way.  So tanh is a polynomial where a tile's products allow it (about 250 cycles fewer), the weights of a tile are made
-// beside the scores of the next one (rows of 128 columns, two waves a SIMD; with rows of 64 columns four waves take turns, and the registers of
-// the next scores would cost one or two of them: 8 prompts of 1024, 16 / 4 heads of 64, 51 us, so 49, with two waves 56), and tiles come by loads that the
-// compiler does not know (it would wait for the next tile in front of the first transposed read).  Nothing of a wave's is spilled: scratch memory costs a
-// launch about a microsecond.
-// 4 prompts of 1777 .. 2048 tokens, 16 / 8 heads of 128, soft cap and sink, the call with its preparation of 21 us: 115 us; 117 with tanh from an
-// exponential and a tile's work one after the other, and that way 127 with an XCD's pairs one after the other (see there) and 129
-// with the denominator as a product of rounded weights with ones; with the launch on 16 x 16
+// What bounds it: the instructions of the scores.  64 soft-capped scores are nine vector instructions and three at quarter rate (two exponentials, a
+// reciprocal) for a row beside 32 cycles of matrix products.  So the weights of a tile are made beside the scores of the next one and the next scores capped
+// beside the values of this one (rows of 128 columns, two waves a SIMD; with rows of 64 columns more waves take turns, and the registers of
+// the next scores would cost one or two of them: 8 prompts of 1024, 16 / 4 heads of 64, 51 us, so with two waves 56), and tiles come by loads that the
+// compiler does not know (it would wait for the next tile in front of the first transposed read).
+// 4 prompts of 1777 .. 2048 tokens, 16 / 8 heads of 128, soft cap and sink, the call with its preparation of 21 us: 112 us on a card where a tile's work one
+// after the other takes 114; 3 prompts of 700 .. 1900 71 and 75, 2 portions of 1000 on 3000 .. 4000 117 and 121.  On another card 117 for that order, 127 with an
+// XCD's pairs one after the other (see there) and 129 with the denominator as a product of rounded weights with ones; with the launch on 16 x 16
 // tiles, values transposed through registers, which other sizes still take, 496 us (44 of them preparation).
+// Not taken: an odd polynomial of tanh where a tile's products are within 0.4 caps (the same call 112; 8 prompts of 300 .. 800, 16 / 4 heads of 64, 39 us instead
+// of 42).  Whether a tile takes it depends on the portion a row comes in, and with it the row's bits; its coefficients
+// overflow with caps below about 1e-8, its squares with products above 1.8e19.
 #include <algorithm>
 #include <type_traits>
 
@@ -237,18 +238,12 @@ __global__ __launch_bounds__(256, D32 + V32 == 4 ? (MOD == kSrGeneral ? 3 : 4) :
         __builtin_amdgcn_sched_barrier(0);
     };
     // A score from its product to log2 units: cap tanh(x / cap) = cap - 2 cap / (exp(2 x / cap) + 1), its scale or, elsewhere, a bias on top.
-    // Where no product of the tile (and wave) is beyond 0.4 caps, an odd polynomial of tanh beside the weights instead, off by 1e-7 of
-    // the value at most: two of three quarter-rate instructions fewer.  The products then stay what they are until their weights are made.
-    constexpr bool CAP = MOD == kSrCap, BESIDE = MOD != kSrGeneral;           // (a bias comes from memory: all of them together)
-    const float per_cap = p.cap_in * (0.5f / kSrLog2e), per_cap2 = per_cap * per_cap;
-    const float t0 = cap2 * per_cap * 0.99999990f, t1 = cap2 * per_cap * per_cap2 * -0.33331362f;
-    const float t2 = cap2 * per_cap * per_cap2 * per_cap2 * 0.13270977f, t3 = cap2 * per_cap * per_cap2 * per_cap2 * per_cap2 * -0.0475536f;
+    constexpr bool BESIDE = MOD != kSrGeneral;        // (a bias comes from memory: all of them together)
     auto capped = [&](float x) { return cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x * p.cap_in) + 1.0f); };
-    bool products = false;                            // s are products
-    auto modify = [&](int i, float& top, float& low) __attribute__((always_inline)) {
-        s[i] = CAP ? n[i >> 4][i & 15] : n[i >> 4][i & 15] * p.scale_log2;
+    auto modify = [&](int i, float& top) __attribute__((always_inline)) {
+        const float x = n[i >> 4][i & 15];
+        s[i] = MOD == kSrCap ? capped(x) : x * p.scale_log2;
         top = fmaxf(top, s[i]);
-        if (CAP) low = fminf(low, s[i]);
     };
     auto all_general = [&](int kt) __attribute__((always_inline)) {
 #pragma unroll
@@ -260,19 +255,9 @@ __global__ __launch_bounds__(256, D32 + V32 == 4 ? (MOD == kSrGeneral ? 3 : 4) :
         }
     };
     // Hides what a row does not see of the tile at key kt, where some row of the wave does not see all of it, and raises the running maximum.
-    // top, low: this lane's extremes (of products, where there is a cap).
-    auto settle = [&](int kt, float top, float low) __attribute__((always_inline)) {
+    // top: the largest of this lane's scores.
+    auto settle = [&](int kt, float top) __attribute__((always_inline)) {
         const bool edge = kt + kSrTile - 1 > rw0 + shift;
-        products = CAP && !edge && p.cap_in > 0.f && __all(fmaxf(top, -low) * per_cap <= 0.4f);
-        if (CAP && !products) {
-            asm volatile("");
-            top = -INFINITY;
-#pragma unroll
-            for (int i = 0; i < 32; ++i) {
-                s[i] = capped(s[i]);
-                top = fmaxf(top, s[i]);
-            }
-        }
         if (edge) {
             asm volatile("");                         // (a branch around it, not 32 selections in every tile)
             top = -INFINITY;
@@ -281,10 +266,6 @@ __global__ __launch_bounds__(256, D32 + V32 == 4 ? (MOD == kSrGeneral ? 3 : 4) :
                 s[i] = kt + (i >> 4) * 32 + (i & 3) + 8 * ((i & 15) >> 2) + 4 * hh <= qpos ? s[i] : -INFINITY;
                 top = fmaxf(top, s[i]);
             }
-        }
-        if (products) {
-            const float u = top * top;
-            top *= __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(t3, u, t2), u, t1), u, t0);
         }
         const float tmax = sr_max_xor32(top);
         if (!__all(tmax <= m_run)) {                  // rare after the first tiles
@@ -299,18 +280,12 @@ __global__ __launch_bounds__(256, D32 + V32 == 4 ? (MOD == kSrGeneral ? 3 : 4) :
             }
         }
     };
-    float l_part[2];
-    auto weigh = [&](auto poly, int i, int step, float (&h)[32], bf16x8 (&pb)[4]) __attribute__((always_inline)) {
-        if constexpr (decltype(poly)::value) {
-            const float u = s[i] * s[i];
-            if (step == 0) h[i] = __builtin_fmaf(__builtin_fmaf(t3, u, t2), u, t1);
-            if (step == 1) s[i] = __builtin_fmaf(s[i], __builtin_fmaf(h[i], u, t0), -m_run);
-        } else if (step == 1) {
-            s[i] -= m_run;
-        }
-        if (step == 2) s[i] = __builtin_amdgcn_exp2f(s[i]);
-        if (step == 3) {
-            l_part[i & 1] += s[i];
+    float l_part[4];
+    auto weigh = [&](int i, int step, bf16x8 (&pb)[4]) __attribute__((always_inline)) {
+        if (step == 0) s[i] -= m_run;
+        if (step == 1) s[i] = __builtin_amdgcn_exp2f(s[i]);
+        if (step == 2) {
+            l_part[i & 3] += s[i];
             if ((i & 7) == 7) {
 #pragma unroll
                 for (int j = 0; j < 8; ++j) pb[i >> 3][j] = (__bf16)s[i - 7 + j];
@@ -321,49 +296,44 @@ __global__ __launch_bounds__(256, D32 + V32 == 4 ? (MOD == kSrGeneral ? 3 : 4) :
     // The weights of tile t, and beside them the scores of tile t + 1 (MORE).
     auto weights = [&](int t, auto more, bf16x8 (&pb)[4]) __attribute__((always_inline)) {
         constexpr bool MORE = decltype(more)::value;
-        l_part[0] = l_part[1] = 0.f;
-        auto in_steps = [&](auto poly) __attribute__((always_inline)) {
-            constexpr int W = KSTEPS > 4 ? KSTEPS - 2 : KSTEPS, PER = LEAN ? 2 : (32 + W - 1) / W;
-            float h[32];
-            auto weighs = [&](int c) {
+        constexpr int W = KSTEPS > 4 ? KSTEPS - 2 : KSTEPS, PER = LEAN ? 2 : (32 + W - 1) / W;
+        l_part[0] = l_part[1] = l_part[2] = l_part[3] = 0.f;
+        auto weighs = [&](int c) {
 #pragma unroll
-                for (int i = 0; i < 32; ++i)
+            for (int i = 0; i < 32; ++i)
 #pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        if (i / PER == c - k) weigh(poly, i, k, h, pb);
-            };
-            if constexpr (MORE) scores(t + 1, weighs);
-#pragma unroll
-            for (int c = MORE ? KSTEPS : 0; c <= 31 / PER + 3; ++c) weighs(c);
+                for (int k = 0; k < 3; ++k)
+                    if (i / PER == c - k) weigh(i, k, pb);
         };
-        if (CAP && products) in_steps(std::integral_constant<bool, CAP>{});
-        else in_steps(std::false_type{});
-        l_run += l_part[0] + l_part[1];
+        if constexpr (MORE) scores(t + 1, weighs);
+#pragma unroll
+        for (int c = MORE ? KSTEPS : 0; c <= 31 / PER + 2; ++c) weighs(c);
+        l_run += (l_part[0] + l_part[1]) + (l_part[2] + l_part[3]);
         asm volatile("" : "+v"(l_run));
     };
     auto first_scores = [&](int t) __attribute__((always_inline)) {
-        float top = -INFINITY, low = INFINITY;
+        float top = -INFINITY;
         scores(t, [](int) {});
         if constexpr (!BESIDE) all_general(t * kSrTile);
 #pragma unroll
         for (int i = 0; i < 32; ++i) {
-            if constexpr (BESIDE) modify(i, top, low);
+            if constexpr (BESIDE) modify(i, top);
             else top = fmaxf(top, s[i]);
         }
-        settle(t * kSrTile, top, low);
+        settle(t * kSrTile, top);
     };
     // A step: the weights of tile t beside the scores of tile t + 1 (MORE), then the values of tile t.
     auto step = [&](int t, auto more) __attribute__((always_inline)) {
         constexpr bool MORE = decltype(more)::value;
         bf16x8 pb[4];
         weights(t, more, pb);
-        float top[2] = {-INFINITY, -INFINITY}, low[2] = {INFINITY, INFINITY};
+        float top[2] = {-INFINITY, -INFINITY};
         constexpr int EACH = (32 + VSTEPS - 2) / (VSTEPS - 1);
         values(t, pb, [&](int c) {
             if constexpr (MORE && BESIDE) {
 #pragma unroll
                 for (int i = 0; i < 32; ++i)
-                    if (i / EACH == c - 1) modify(i, top[i & 1], low[i & 1]);
+                    if (i / EACH == c - 1) modify(i, top[i & 1]);
             }
         });
         if constexpr (MORE) {
@@ -372,7 +342,7 @@ __global__ __launch_bounds__(256, D32 + V32 == 4 ? (MOD == kSrGeneral ? 3 : 4) :
 #pragma unroll
                 for (int i = 0; i < 32; ++i) top[i & 1] = fmaxf(top[i & 1], s[i]);
             }
-            settle((t + 1) * kSrTile, fmaxf(top[0], top[1]), fminf(low[0], low[1]));
+            settle((t + 1) * kSrTile, fmaxf(top[0], top[1]));
         }
     };
 

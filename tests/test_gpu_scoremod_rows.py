@@ -198,8 +198,7 @@ def test_orders_of_pairs(H, G, n_qs, n_ks):
 @pytest.mark.parametrize("H,G,D,Dv", [(4, 2, 128, 128), (8, 2, 64, 64), (4, 2, 64, 128)])
 @pytest.mark.parametrize("softcap,spread", [(30.0, 0.5), (30.0, 1.0), (8.0, 1.0), (2.0, 1.0), (0.5, 1.0), (30.0, 6.0), (1e-3, 1.0), (1e4, 1.0)])
 def test_caps_far_above_and_below_the_scores(H, G, D, Dv, softcap, spread):
-    """Scores from a hundredth of the cap to far beyond it: tiles within 0.4 caps take another form of tanh than the others, and some tiles of
-    a row may be either.  Tiles whose rows see all of them, and edges."""
+    """Scores from a hundredth of the cap to far beyond it.  Tiles whose rows see all of them, and edges."""
     n_qs, n_ks = [150, 64, 33], [700, 64, 290]
     a, r, ctx, pos, q, k, v, kc, vc = _step(H, G, D, Dv, 64, n_qs, n_ks, spread=spread, softcap=softcap, use_sink=True)
     nv.set_context(ctx)
@@ -207,3 +206,33 @@ def test_caps_far_above_and_below_the_scores(H, G, D, Dv, softcap, spread):
     nv.set_context(None)
     # probabilities and outputs are rounded to bf16 (2^-9 each), values are of order `spread`
     torch.testing.assert_close(o.float(), o_r.float(), rtol=2e-2, atol=1e-2 * spread)
+
+
+@pytest.mark.parametrize("D,Dv", [(128, 128), (64, 64), (64, 128), (128, 64)])
+@pytest.mark.parametrize("softcap,spread", [(30.0, 1.0), (8.0, 0.5), (300.0, 3.0), (0.0, 1.0)])
+def test_a_row_in_portions_that_begin_elsewhere(D, Dv, softcap, spread):
+    """A row's bits do not depend on the other rows of its portion: a tile that all rows of its wave see in one portion is at the diagonal of a row of its
+    wave in another, and one in which no row's maximum rises in one may raise another row's."""
+    H, G, bs, n_k = 4, 2, 64, 704
+    a, r, ctx, pos, q, k, v, kc, vc = _step(H, G, D, Dv, bs, [n_k], [n_k], spread=spread, softcap=softcap, use_sink=True)
+    cu = lambda n: torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    got = {n: ops.attn_scoremod_paged(q[n_k - n:], kc, vc, cu(n), cu(n_k), ctx.block_tables, D ** -0.5, softcap, a.sink, None, n, n_k, 0).view(n, -1)
+           for n in (144, 140, 128, 97)}
+    for n, o in got.items():
+        assert torch.equal(o, got[144][144 - n:]), n
+
+
+@pytest.mark.parametrize("D,Dv", [(128, 128), (64, 64)])
+@pytest.mark.parametrize("softcap,rows,keys", [(1e-9, 0.0, 1.0), (1e-12, 0.0, 1.0), (1e24, 1e12, 1e10), (1e30, 1e10, 1e10)])
+def test_caps_beyond_all_measure(D, Dv, softcap, rows, keys):
+    """Scores of zero under a cap near zero weigh all keys alike; products far beyond 2^64 under a cap still larger leave finite outputs."""
+    H, G, bs, n_q, n_k = 4, 2, 64, 70, 330
+    a, r, ctx, pos, q, k, v, kc, vc = _step(H, G, D, Dv, bs, [n_q], [n_k], softcap=softcap)
+    got = ops.attn_scoremod_paged(q * rows, kc * keys, vc, ctx.cu_seqlens_q, ctx.cu_seqlens_k, ctx.block_tables, D ** -0.5, softcap, None, None, n_q, n_k, 0)
+    assert torch.isfinite(got.float()).all()
+    if rows == 0.0:
+        vals = vc[ctx.block_tables[0].long()].flatten(0, 1)[:n_k].float().repeat_interleave(H // G, dim=1)
+        seen = torch.arange(n_k - n_q, n_k, device=DEV) + 1
+        want = vals.cumsum(0)[seen - 1] / seen[:, None, None]
+        # (the mean of hundreds of values of order one, about 0.06, rounded to bf16)
+        torch.testing.assert_close(got.view(n_q, H, Dv).float(), want, rtol=2 ** -8, atol=1e-4)
