@@ -116,6 +116,12 @@ NV_HD PairPlace scoremod_order(const PairGroup& g, int index, int slots_per_pair
     return {g.pair + one * g.step, (rank << xs_shift) + (index & ((1 << xs_shift) - 1))};
 }
 
+// Score-modified attention, prompt portions: the loop for launches of several tiles, from four on and wherever a bias is added.  Shorter ones have few steps to
+// gain in and more in front of the first.  Short loop / long, us, the call with its preparation, 16 heads, soft cap: rows of 128, one prompt of 64 tokens
+// 10.55 / 10.76, 13 of 20 .. 64 13.0 / 13.3, 8 of 100 .. 190 18.1 / 18.2, 3 of 200 .. 256 19.1 / 18.9, 2 of 385 .. 762 32.9 / 31.9;  rows of 64, one of 54 8.75 / 8.88,
+// 2 of 121 .. 395 16.81 / 16.85, 3 of 900 .. 2000 71.1 / 69.7.  With a bias, the launch alone: one prompt of 54 tokens, rows of 128, 7.2 / 6.7, 3 of 700 .. 1900 86 / 63.
+NV_HD bool scoremod_long(int max_k, bool biased) { return biased || max_k > 192; }
+
 // Tiles of 128 rows, no more blocks than CUs: slices 32 deep, since nothing else runs on a CU while its one workgroup waits for a slice.  Tiles of an
 // expert: one, from 100 pairs on as many as its pairs fill and a half.  First / second product of 16 or 32 experts, us, 64 and 32 deep:
 //   128 blocks   width 2048, ff 1024: 41.5 and 36.7 / 23.9 and 21.8;  width 1024, ff 512: 25.7 and 23.0 / 15.7 and 15.3

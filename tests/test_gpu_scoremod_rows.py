@@ -236,3 +236,20 @@ def test_caps_beyond_all_measure(D, Dv, softcap, rows, keys):
         want = vals.cumsum(0)[seen - 1] / seen[:, None, None]
         # (the mean of hundreds of values of order one, about 0.06, rounded to bf16)
         torch.testing.assert_close(got.view(n_q, H, Dv).float(), want, rtol=2 ** -8, atol=1e-4)
+
+
+@pytest.mark.parametrize("D,Dv", [(128, 128), (64, 64), (64, 128), (128, 64)])
+@pytest.mark.parametrize("form", ["plain", "cap", "bias", "cap_bias"])
+def test_short_and_long_launches(D, Dv, form):
+    """Launches of up to three key tiles take another loop than longer ones (without a bias): the same rows with a longer sequence behind them have the
+    same bits; prompts and portions that end around the tiles' edges."""
+    H, G, bs = 4, 2, 64
+    n_qs, n_ks = [1, 2, 33, 64, 100, 128, 70, 192, 200], [1, 2, 33, 64, 129, 128, 190, 192, 700]
+    cap = 25.0 if "cap" in form else 0.0
+    a, r, ctx, pos, q, k, v, kc, vc = _step(H, G, D, Dv, bs, n_qs, n_ks, softcap=cap, use_sink=True, spread=2.0)
+    bias = torch.randn(H, 90, device=DEV) if "bias" in form else None
+    call = lambda n, T: ops.attn_scoremod_paged(q[:T], kc, vc, ctx.cu_seqlens_q[:n + 1], ctx.cu_seqlens_k[:n + 1], ctx.block_tables[:n].contiguous(), D ** -0.5, cap,
+                                                a.sink, bias, max(n_qs[:n]), max(n_ks[:n]), -1)
+    T = sum(n_qs[:-1])
+    assert max(n_ks[:-1]) <= 192 < n_ks[-1]
+    assert torch.equal(call(len(n_qs) - 1, T), call(len(n_qs), sum(n_qs))[:T])
