@@ -85,9 +85,13 @@ __device__ __forceinline__ uint4 load_stream16(const uint4* p) {
 // 16 bytes a lane from `base` + `off` straight into LDS: lane l fills bytes 16 l .. of the KiB at LDS address `to` (base and to uniform).  The
 // compiler does not know this load: it puts no wait in front of LDS reads that it cannot tell from the load's target, and none at all.  The
 // caller waits for it (vmcnt) and puts a barrier where other waves read.  Waits that the compiler counts for its own loads come out longer, never shorter.
+// Nor does it keep what it does not know away from registers just written: a vector memory instruction may read a scalar register that a vector instruction
+// wrote (readfirstlane, readlane, so a restored spill too) only five wait states later, so `base` goes through a scalar copy here, which waits
+// for such writes by itself and is read at once; it is also the wait state between m0 and the load.
 // (m0 is not named as overwritten, since it is a reserved register: a kernel takes either this or the builtins that set m0.)
 __device__ __forceinline__ void lds_load16(const void* base, uint32_t off, uint32_t to) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(to)), "v"(off), "s"(base) : "memory");
+    uint64_t at;
+    asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0" : "=&s"(at) : "s"(__builtin_amdgcn_readfirstlane(to)), "v"(off), "s"(base) : "memory");
 }
 typedef __attribute__((address_space(3))) unsigned char lds_byte;
 __device__ __forceinline__ uint32_t lds_address(const void* p) { return (uint32_t)(uintptr_t)(const lds_byte*)p; }
