@@ -12,13 +12,17 @@
 //
 //   rows kernel    sequences with several tokens in the step: a workgroup of four waves takes 128 rows; key tiles of 64
 //                  (32 for wide rows) are staged once for the four waves by loads that the compiler does not know (it would wait for all of
-//                  them in front of a tile's first transposed read).  Where a wave has a SIMD to itself it multiplies the next
-//                  tile's scores beside the weights of this one, with operands four and eight products ahead (two and four elsewhere, where the
-//                  other wave has its turn), the accumulators held in their half of the registers, so that no tile moves them.
-//                  What bounds it then is power: a tile takes 3140 cycles instead of 4400 (2048 of them products), but at 1.4 to 1.66 GHz, with
-//                  the same work, where it was 1.7 to 2.  16 heads, 256 columns, 1024 rows of each of 2 sequences of 3000 and 6001 keys: the call
-//                  164 -> 144 to 153 us by the card; a prompt of 2000 tokens 74 -> 65, 37 rows on 3000 keys 37 -> 32.  One wave a SIMD for rows of 160 columns too:
-//                  54 us instead of 58 for a prompt of 2000, but 66 for 59 where 700 rows come on top of up to 2300 keys.
+//                  them in front of a tile's first transposed read).  Where a wave has a SIMD to itself (rows beyond 160 columns, but for 192 with
+//                  values of 128) it multiplies the next tile's scores beside the weights of this one, with operands four and eight products ahead, the
+//                  accumulators held in their half of the registers, so that no tile moves them: a tile takes 3140 cycles instead of 4400 (2048 of them
+//                  products).  16 heads, 256 columns, 1024 rows of each of 2 sequences of 3000 and 6001 keys: the call 160 -> 139 us; a prompt
+//                  of 2000 tokens 71 -> 62, 37 rows on 3000 keys 34 -> 29.  One wave a SIMD for rows of 160 columns too: 54 us instead of 58 for a
+//                  prompt of 2000, but 66 for 59 where 700 rows come on top of up to 2300 keys.
+//                  Elsewhere two to four waves take turns, a tile's work one after the other, operands of the first product two ahead.  With the next
+//                  scores beside, rows of 32, 64 and 96 columns lost a wave a SIMD or two: 4 prompts of 1900 .. 2048, rows of 64, 44.3 us before, 47.9
+//                  so, 43.4 as it is; rows of 96 57.8, 60.6 and 54.2.  The second product is in order with operands four ahead for those, and left to
+//                  the compiler for wider ones, whose waves are often alone at a launch's end: 3 prompts of 700 .. 1900, rows of 160, 48.3 before, 48.7
+//                  in order, 47.1 as it is; the 4 prompts 85.2, 79.7 and 79.8; rows of 64, 3 prompts, 30.3, 29.3 and 30.4.
 //   single kernel  sequences with one token: a workgroup takes up to 32 heads; its four waves take the key tiles of 32 in
 //                  turn, each staging its own (no barrier in the loop), and join their states through LDS.
 //
@@ -113,6 +117,8 @@ struct LatentWave {
         l_run = 0.f;
     }
 
+    // Rows kernel with several waves a SIMD, rows of 128 columns and more: the weights and the second product in the compiler's order (see the header).
+    static constexpr bool FREE = !HOLD && KB == 2 && D32 >= 4;
     static constexpr int KSTEPS = 2 * D32, VSTEPS = 2 * KB * DV32;                      // products a key block and tile
     static constexpr int AHEAD = HOLD ? 4 : 2, KA = KSTEPS < AHEAD ? KSTEPS : AHEAD, VA = VSTEPS < 2 * AHEAD ? VSTEPS : 2 * AHEAD;
     typedef bf16x8 Keys[KA][KB];
@@ -158,7 +164,7 @@ struct LatentWave {
         if ((i & 7) == 7) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) p[i >> 3][j] = (__bf16)s[i - 7 + j];
-            asm volatile("" : "+v"(p[i >> 3]));                      // (here and not where it is needed)
+            if constexpr (!FREE) asm volatile("" : "+v"(p[i >> 3]));  // (here and not where it is needed)
         }
     }
     // Operand n of the second product: 16 keys (n / DV32) x 32 columns (n % DV32, from 32 dv0 on), transposed on its way.  Keys of element
@@ -183,6 +189,11 @@ struct LatentWave {
         hold();
     }
     __device__ __forceinline__ void values(const Tile& t, const bf16x8 (&p)[2 * KB]) {
+        if constexpr (FREE) {
+#pragma unroll
+            for (int n = 0; n < VSTEPS; ++n) oacc[n % DV32] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(value(t, n), p[n / DV32], oacc[n % DV32], 0, 0, 0);
+            return;
+        }
         Values a;
 #pragma unroll
         for (int n = 0; n < VA; ++n) a[n] = value(t, n);
@@ -260,7 +271,8 @@ struct LatentWave {
     // The scores stay in the other half from one tile to the next.
     __device__ __forceinline__ void keep(Scores& s) {
 #pragma unroll
-        for (int i = 0; i < 16 * KB; ++i) asm volatile("" : "+v"(s[i]));
+        for (int i = 0; i < 16 * KB; ++i)
+            if constexpr (!FREE) asm volatile("" : "+v"(s[i]));
     }
     // The weights and values of the tile at `now`, whose scores are s, and beside them the scores of the one at `next` (its first key kt), which
     // take their place: the weights beside the products of the scores, the largest of those beside the products of the values.  The first
@@ -388,10 +400,10 @@ __device__ __forceinline__ int lat_share(const LatentParams& p, int lane) {
 template <int D32, int DV32, int KB, int OCC, bool EVEN>
 __global__ __launch_bounds__(256, OCC) void attn_latent_rows_kernel(const LatentParams p) {
     constexpr int D = 32 * D32, KT = 32 * KB, kTile = KT * D * 2, kPieces = D32 * KB / 2;
-    constexpr bool TURN = OCC == 1 || D32 <= 3;
+    constexpr bool TURN = OCC == 1;                          // the next tile's scores beside this one's weights
     static_assert(D32 * KB % 2 == 0, "a wave stages whole pieces");
-    // A tile each; two waves' output staging areas at the end.  Two objects, not one array: the compiler tells a tile's reads from
-    // the other tile's LDS-DMA by the object, and with one array it waits for the DMA just issued before the first read.
+    // A tile each; two waves' output staging areas at the end.  Only the wait for the loads and the barrier, half way through a turn or at the head
+    // of a step, keep a tile's reads apart from the loads into its buffer.
     constexpr int BUF = kTile > 2 * kLatRows * kLatStageRow ? kTile : 2 * kLatRows * kLatStageRow;
     __shared__ __attribute__((aligned(16))) unsigned char buf[TURN ? 4 : 2][BUF];
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;

@@ -10,7 +10,7 @@ from test_gpu_nekodra_layers import DEV, reference_rows, rn
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("D,Dv", [(256, 256), (160, 160), (96, 96), (320, 320), (576, 512)])
+@pytest.mark.parametrize("D,Dv", [(256, 256), (160, 160), (96, 96), (64, 64), (32, 32), (128, 128), (192, 128), (320, 320), (576, 512)])
 @pytest.mark.parametrize("n_k", [2, 31, 64, 65, 128, 129, 191, 192, 257, 320, 385])
 @pytest.mark.parametrize("rows", [2, 70])
 def test_few_tiles(D, Dv, n_k, rows):
