@@ -702,7 +702,7 @@ __global__ __launch_bounds__(256, OCC) void attn_latent_single_kernel(const Late
                 }
             } else {
                 const float inv = lat_finish(m, l, p.sink, head0 + hr);
-                *(uint2*)(p.out + grow * Dw + c) = make_uint2(pack_bf16(s.x * inv, s.y * inv), pack_bf16(s.z * inv, s.w * inv));
+                *(uint2*)(p.out + grow * Dv + dv0 * 32 + c) = make_uint2(pack_bf16(s.x * inv, s.y * inv), pack_bf16(s.z * inv, s.w * inv));
             }
         }
     }
