@@ -24,7 +24,10 @@
 //                  the compiler for wider ones, whose waves are often alone at a launch's end: 3 prompts of 700 .. 1900, rows of 160, 48.3 before, 48.7
 //                  in order, 47.1 as it is; the 4 prompts 85.2, 79.7 and 79.8; rows of 64, 3 prompts, 30.3, 29.3 and 30.4.
 //   single kernel  sequences with one token: a workgroup takes up to 32 heads; its four waves take the key tiles of 32 in
-//                  turn, each staging its own (no barrier in the loop), and join their states through LDS.
+//                  turn, each staging its own (no barrier in the loop), and join their states through LDS.  Rows up to 192 columns in order with operands
+//                  ahead, by loads that the compiler does not know; wider ones, one wave a SIMD, in the compiler's order by loads that it knows (the
+//                  addresses of 32 and more pieces a tile do not stay in scalar registers).  In order / in the compiler's, us: 256 sequences of
+//                  513 .. 768 keys, rows of 160 25.3 / 26.1, 256 36.1 / 34.1;  32 of 500 .. 4000, 128 heads, rows of 576, 144 / 134.
 //
 // When a launch would leave most of the chip idle the keys are cut into ranges; the ranges' unnormalised states go through
 // a workspace and a second launch.
@@ -254,6 +257,64 @@ struct LatentWave {
         Scores s;
         first(at, s, lane, kt, qpos, masked, scale_log2);
         last(at, s, scale_log2);
+    }
+    // The same in the compiler's order, from a tile at `lds` that came by loads which the compiler knows.
+    __device__ __forceinline__ void plain_step(const unsigned char* lds, int lane, int kt, int qpos, bool masked, float scale_log2, int dv0) {
+        const int r = lane & 31, h = lane >> 5, i16 = lane & 15, g16 = (lane >> 4) & 1;
+        f32x16 s[KB];
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[kb][i] = 0.f;
+#pragma unroll
+            for (int c = 0; c < KSTEPS; ++c)
+                s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(lds + lat_off<D32>(kb * 32 + r, 2 * c + h)), qf[c], s[kb], 0, 0, 0);
+        }
+        if (masked) {
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s[kb][i] = kt + kb * 32 + (i & 3) + 8 * (i >> 2) + 4 * h <= qpos ? s[kb][i] : -INFINITY;
+        }
+        float tmax = s[0][0];
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, s[kb][i]);
+        tmax = lat_max_xor32(tmax) * scale_log2;                 // (scale > 0)
+        if (high(tmax)) {
+            const float m_new = fmaxf(m_run, tmax), alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+            m_run = m_new;
+            l_run *= alpha;
+#pragma unroll
+            for (int d = 0; d < DV32; ++d)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) oacc[d][i] *= alpha;
+        }
+        float psum = 0.f;
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                s[kb][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kb][i], scale_log2, -m_run));
+                psum += s[kb][i];
+            }
+        l_run += psum;
+#pragma unroll
+        for (int k = 0; k < 2 * KB; ++k) {
+            bf16x8 pb;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) pb[j] = (__bf16)s[k >> 1][8 * (k & 1) + j];
+            const int row = 16 * k + 4 * h + (i16 >> 2);
+#pragma unroll
+            for (int d = 0; d < DV32; ++d) {
+                const unsigned char* at = lds + 512 * dv0 + 8 * (i16 & 1);
+                const int ch = d * 4 + 2 * g16 + ((i16 & 3) >> 1);
+                const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + lat_off<D32>(row, ch)));
+                const s16x4 v2 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + lat_off<D32>(row + 8, ch)));
+                oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, __builtin_shufflevector(v1, v2, 0, 1, 2, 3, 4, 5, 6, 7)), pb, oacc[d], 0, 0, 0);
+            }
+        }
     }
     __device__ __forceinline__ void first(uint32_t at, Scores& s, int lane, int kt, int qpos, bool masked, float scale_log2) {
         const Tile t = tile(at);
@@ -613,6 +674,7 @@ __global__ __launch_bounds__(256, OCC) void attn_latent_rows_kernel(const Latent
 template <int D32, int DV32, int NBUF, int OCC>
 __global__ __launch_bounds__(256, OCC) void attn_latent_single_kernel(const LatentParams p) {
     constexpr int D = 32 * D32, Dw = 32 * DV32, KT = 32, kTile = KT * D * 2, kPieces = 2 * D32;
+    constexpr bool PLAIN = OCC == 1;                         // (see the header)
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];      // [4 waves][NBUF tiles], then [4][32] (m, l)
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -636,7 +698,12 @@ __global__ __launch_bounds__(256, OCC) void attn_latent_single_kernel(const Late
         for (int i = 0; i < kPieces; ++i) {
             int row, ch;
             lat_piece<D32>(i, lane, row, ch);
-            lds_load16(base, (uint32_t)(min(row, last) * (D * 2) + ch * 16), lds_address(mine + buf * kTile + i * 1024));
+            const uint32_t off = (uint32_t)(min(row, last) * (D * 2) + ch * 16);
+            unsigned char* to = mine + buf * kTile + i * 1024;
+            if constexpr (PLAIN)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(base + off), (__attribute__((address_space(3))) void*)to, 16, 0, 0);
+            else
+                lds_load16(base, off, lds_address(to));
         }
     };
     LatentWave<D32, DV32, 1, false> w;
@@ -646,7 +713,8 @@ __global__ __launch_bounds__(256, OCC) void attn_latent_single_kernel(const Late
     for (; t < t_end; t += 4) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // this wave's own tile has landed
         if (NBUF == 2 && t + 4 < t_end) stage(buf ^ 1, t + 4);
-        w.step(lds_address(mine + buf * kTile), lane, t * KT, n_k - 1, t * KT + KT > n_k, p.scale_log2);
+        if constexpr (PLAIN) w.plain_step(mine + buf * kTile, lane, t * KT, n_k - 1, t * KT + KT > n_k, p.scale_log2, dv0);
+        else w.step(lds_address(mine + buf * kTile), lane, t * KT, n_k - 1, t * KT + KT > n_k, p.scale_log2);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // its reads are done before the buffer is filled again
         if (NBUF == 1 && t + 4 < t_end) stage(0, t + 4);
         if (NBUF == 2) buf ^= 1;
