@@ -131,7 +131,7 @@ struct LatentWave {
         const lds_byte *key[2], *value[2];
     };
     __device__ __forceinline__ Tile tile(uint32_t at) const {
-        return {{(const lds_byte*)(key_at[0] + at), (const lds_byte*)(key_at[1] + at)}, {(const lds_byte*)(value_at[0] + at), (const lds_byte*)(value_at[1] + at)}};
+        return {{lds_pointer(key_at[0] + at), lds_pointer(key_at[1] + at)}, {lds_pointer(value_at[0] + at), lds_pointer(value_at[1] + at)}};
     }
     // Operand c of the first product: 32 keys of each block, columns 16 c ...
     __device__ __forceinline__ void keys(const Tile& t, int c, Keys& a) {
@@ -375,10 +375,12 @@ struct LatentWave {
         constexpr int END = MOVE + (LONG ? MAXES : 0) * KB;
         float top[2] = {-INFINITY, -INFINITY};
         values(now, p, v, [&](int c) {
-            if (LOADS > 0 && c == 0) begin();
+            if constexpr (LOADS > 0) {
+                if (c == 0) begin();
 #pragma unroll
-            for (int i = 0; i < LOADS; ++i)
-                if (c == (VSTEPS > 4 ? 1 : 0) + i * VSTEPS / (2 * LOADS)) load(i);        // (in the first half)
+                for (int i = 0; i < LOADS; ++i)
+                    if (c == (VSTEPS > 4 ? 1 : 0) + i * VSTEPS / (2 * LOADS)) load(i);    // (in the first half)
+            }
 #pragma unroll
             for (int kb = 0; kb < KB; ++kb) {
                 const int at = c - MOVE - kb * MAXES;

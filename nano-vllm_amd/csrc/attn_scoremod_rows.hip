@@ -207,7 +207,7 @@ __global__ __launch_bounds__(256, !LONG ? 2 : D32 + V32 == 4 ? (MOD == kSrGenera
         float s[32];                                      // a tile's scores, then weights: 16 kb + i is key kt + 32 kb + (i & 3) + 8 (i >> 2) + 4 hh; row rw0 + r
         f32x16 n[2];                                      // the next tile's as they are multiplied
         auto scores = [&](int t, auto beside) __attribute__((always_inline)) {
-            const Tile tile = {{(const lds_byte*)(key_at[0] + (t & 1) * KB), (const lds_byte*)(key_at[1] + (t & 1) * KB)}};
+            const Tile tile = {{lds_pointer(key_at[0] + (t & 1) * KB), lds_pointer(key_at[1] + (t & 1) * KB)}};
             constexpr f32x16 zero = {};
             if constexpr (!AHEAD) {
 #pragma unroll
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(256, !LONG ? 2 : D32 + V32 == 4 ? (MOD == kSrGenera
             __builtin_amdgcn_sched_barrier(0);
         };
         auto values = [&](int t, const bf16x8 (&pb)[4], auto beside) __attribute__((always_inline)) {
-            const Tile tile = {{(const lds_byte*)(value_at[0] + (t & 1) * VB), (const lds_byte*)(value_at[1] + (t & 1) * VB)}};
+            const Tile tile = {{lds_pointer(value_at[0] + (t & 1) * VB), lds_pointer(value_at[1] + (t & 1) * VB)}};
             if constexpr (!AHEAD) {
 #pragma unroll
                 for (int c = 0; c < VSTEPS; ++c) oacc[c % V32] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(value(tile, c), pb[c / V32], oacc[c % V32], 0, 0, 0);

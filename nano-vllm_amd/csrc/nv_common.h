@@ -95,6 +95,7 @@ __device__ __forceinline__ void lds_load16(const void* base, uint32_t off, uint3
 }
 typedef __attribute__((address_space(3))) unsigned char lds_byte;
 __device__ __forceinline__ uint32_t lds_address(const void* p) { return (uint32_t)(uintptr_t)(const lds_byte*)p; }
+__device__ __forceinline__ const lds_byte* lds_pointer(uint32_t address) { return (const lds_byte*)(uintptr_t)address; }
 
 // ---- cross-lane helpers (wave64) --------------------------------------------------
 template <int CTRL>
