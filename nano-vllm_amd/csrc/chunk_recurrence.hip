@@ -45,7 +45,7 @@
 // waits for, is multiplied while the parts of K S are exchanged.  Whole calls, chunks of 8 against 16, 16 heads 128 x 128, bf16 rows:
 // gated, 4 prompts of 1501 .. 2048 tokens 285 -> 248 us; general, 3 prompts of 700 .. 2000: 286 -> 266; write, 8 portions of 509 over
 // carried states: 114 -> 96, one prompt of 2048: 197 -> 119.  Token by token: gated 3123, general 3645, write 431; gated, 256 single
-// tokens: 393 -> 113, and 99 past the caches (5.5 TB/s of states).
+// tokens, the states of three layers in turn: 393 -> 113, and 99 past the caches (5.4 TB/s of states).
 // In a profile of the 248-us call (286 us there) the first launch is 82 us, the second 177, 128 chunks in a row at 1.38 us: 0.83 us of MFMAs
 // (15.3 ns each, back to back), the rest LDS latency and the chain; the read-outs' norm is 26.  Tried and slower: all large products as six bf16 products of three parts each, split by the
 // movers (198 us for the second launch: the LDS traffic of the parts; 144 without them), the same for the updates alone (176), four
@@ -65,6 +65,7 @@
 #include <algorithm>
 
 #include "chunk_recurrence_parts.h"
+#include "launch_order.h"
 #include "../../include/nanovllm_hip_mixers.h"
 
 namespace nv {
@@ -790,8 +791,7 @@ __global__ __launch_bounds__(256) void recurrence_finish_kernel(const ChunkRecur
 // registers, four neighbouring columns of ROWS rows a thread (all loads in flight at once); what the token finds in the old state
 // and what it reads out come from one pass: with p = S^T k (decayed as the form wants it) the read-out of the new state
 // is that of the decayed old one plus the write's part, which is a number per token (k . q and the like) times the columns written.
-// STREAM: the states pass by the caches, for launches whose states are more than the last cache keeps from one step to the next (see
-// cr_states_stream).
+// STREAM: the states pass by the caches (see recurrence_streams).
 template <typename T, int FORM, int ROWS, bool STREAM>
 __global__ __launch_bounds__(256) void single_recurrence_kernel(const ChunkRecurrenceArgs a, const int pieces) {
     constexpr int NX = FORM == kCrGated ? 3 : FORM == kCrGeneral ? 4 : 2;
@@ -1001,12 +1001,6 @@ static int chunks_of(const ChunkRecurrenceArgs& a, int first_seq, int tokens, bo
     return check_launch("chunked recurrence");
 }
 
-// States of a launch of single tokens that do not stay in the last cache (256 MB, shared with what the rest of a step touches) until they are read again
-// pass by the caches instead of driving out each other.  Same states step after step, us, through the caches / past them, 16 heads: gated 128 x 128,
-// 64 sequences (67 MB) 24.2 / 30.3, 80 (84 MB) 31.2 / 36.2, 96 (101 MB) 47.2 / 42.6, 128 62.6 / 51.1, 256 112.6 / 99.4 (5.5 TB/s);
-// 64 x 64, 256 sequences (67 MB) 36.1 / 44.9, 384 (101 MB) 73.7 / 66.2; general, 128 x 128, 128 sequences 66.8 / 51.1, write 58.4 / 49.2.
-static bool cr_states_stream(int64_t seqs, int H, int D, int Dv) { return seqs * H * D * Dv * 4 >= (92LL << 20); }
-
 template <typename T, int FORM, bool STREAM>
 static void singles_rows(const ChunkRecurrenceArgs& a, int pieces, int rows, hipStream_t s) {
     const dim3 grid((unsigned)a.num_seqs, (unsigned)a.H), block(256);
@@ -1015,12 +1009,13 @@ static void singles_rows(const ChunkRecurrenceArgs& a, int pieces, int rows, hip
     else if (rows <= 16) hipLaunchKernelGGL((single_recurrence_kernel<T, FORM, 16, STREAM>), grid, block, 0, s, a, pieces);
     else hipLaunchKernelGGL((single_recurrence_kernel<T, FORM, 32, STREAM>), grid, block, 0, s, a, pieces);
 }
+// singles: sequences known to be of one token
 template <typename T, int FORM>
-static int singles_of(const ChunkRecurrenceArgs& a, hipStream_t s) {
+static int singles_of(const ChunkRecurrenceArgs& a, int singles, hipStream_t s) {
     int pieces = 1;
     while (pieces * 4 < a.Dv) pieces *= 2;            // at most 64
     const int rows = (a.D + 256 / pieces - 1) / (256 / pieces);
-    if (cr_states_stream(a.num_seqs, a.H, a.D, a.Dv)) singles_rows<T, FORM, true>(a, pieces, rows, s);
+    if (recurrence_streams(singles, a.H, a.D, a.Dv)) singles_rows<T, FORM, true>(a, pieces, rows, s);
     else singles_rows<T, FORM, false>(a, pieces, rows, s);
     return check_launch("single-token recurrence");
 }
@@ -1036,8 +1031,8 @@ static int launch_chunk_recurrence(int form, const ChunkRecurrenceArgs& a, int f
                                    hipStream_t s) {
     NV_CR_DISPATCH(chunks_of, a, first_seq, tokens, singles_behind, dtype, s);
 }
-static int launch_single_recurrence(int form, const ChunkRecurrenceArgs& a, int dtype, hipStream_t s) {
-    NV_CR_DISPATCH(singles_of, a, s);
+static int launch_single_recurrence(int form, const ChunkRecurrenceArgs& a, int singles, int dtype, hipStream_t s) {
+    NV_CR_DISPATCH(singles_of, a, singles, s);
 }
 #undef NV_CR_DISPATCH
 
@@ -1061,7 +1056,7 @@ bool run_recurrence_portions(int form, ChunkRecurrenceArgs a, int lead, int port
     if (lead > 0 || singles_behind) {
         ChunkRecurrenceArgs one = a;
         if (!singles_behind) one.num_seqs = lead;
-        *rc = launch_single_recurrence(form, one, dtype, s);
+        *rc = launch_single_recurrence(form, one, recurrence_singles(a.num_seqs, lead, rest), dtype, s);
         if (*rc != NV_OK) return true;
     }
     a.chunks = (float*)workspace;

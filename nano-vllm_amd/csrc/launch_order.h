@@ -146,6 +146,23 @@ NV_HD bool moe_streams(int tile_rows, int64_t pairs, int E, int ff) {
     return pairs < line * (int64_t)E;
 }
 
+// Recurrences, single tokens: sequences known to be of one token in a launch over those in front (`lead`) and, among longer portions (`rest`), behind
+// them.  Only their states are read and written by it.
+NV_HD int recurrence_singles(int num_seqs, int lead, bool rest) { return rest ? lead : num_seqs; }
+// Whether their states pass by the caches (loads and stores).  What pays depends on whether the last cache (256 MB) keeps a layer's states until its next step,
+// so on what the step touches in between, which a launch does not know.  Through / past, us, 16 heads 128 x 128, gated, states of as many layers in turn:
+//                         1              3              6 and 12             1, written just before   a state's first pass
+//   32 seqs (34 MB)   13.9 / 13.2    16.6 / 14.7    16.4 / 15.2, 20.1 / 15.5
+//   64 (67 MB)        25.0 / 27.6    24.7 / 29.5    39.2 / 30.0, 39.3 / 30.0
+//   80 (84 MB)        31.1 / 33.1    31.3 / 35.5    44.0 / 35.4, 43.9 / 36.3
+//   92 (96 MB)        33.8 / 38.5    40.6 / 40.5    49.4 / 40.7, 49.5 / 40.8
+//   128 (134 MB)      44.1 / 49.4    60.5 / 50.5    60.9 / 50.8, 60.6 / 50.9       46.0 / 46.7               83 / 88
+//   256 (268 MB)      100 / 98       113 / 99       112 / 99, 112 / 99             95.6 / 92.6              129 / 145
+//   64 x 64, 256 (67 MB)  37.2 / 45.0, 36.9 / 45.2, 51.1 / 45.2, 51.1 / 45.2;  384 (101 MB)  51.7 / 66.4, 71.8 / 66.7, 73.2 / 66.7, 73.2 / 66.8
+// The line is where three layers' states stop fitting.  A model of more layers would gain from less on and loses nothing at it; one whose
+// states all stay loses up to 28 % between 96 and 200 MB.  General and write as gated.  Only loads or only stores past the caches: 106 and 114 for 256.
+NV_HD bool recurrence_streams(int singles, int H, int D, int Dv) { return (int64_t)singles * H * D * Dv * 4 >= 92LL << 20; }
+
 // Outputs of the second product (fp32, a row a pair) past the caches: they drive the weights and rows that other column blocks read out of the L2, and
 // large ones are gone before the caller adds a token's rows up.  The call with that sum, through / past, us, top 4 of 32 experts, 2048, 1024: 8192 tokens
 // (268 MB) 538 / 527, 4096 316 / 313, 2048 (67 MB) 214 / 208;  top 2 of 16, 1024, 1024: 8000 (66 MB) 165.7 / 168.3.

@@ -46,6 +46,9 @@ extern "C" int scored_pairs(int64_t grid_base, int num_seqs, int64_t total_q, in
     return scoremod_pairs(grid_base, num_seqs, total_q, max_q, max_k);
 }
 extern "C" int streams(int tile_rows, int64_t pairs, int E, int ff) { return moe_streams(tile_rows, pairs, E, ff); }
+extern "C" int states_past(int num_seqs, int lead, int rest, int H, int D, int Dv) {
+    return recurrence_streams(recurrence_singles(num_seqs, lead, rest != 0), H, D, Dv);
+}
 extern "C" int few_blocks(int64_t pairs, int E, int n_cols) { return moe_few_blocks(pairs, E, n_cols); }
 """
 
@@ -187,3 +190,11 @@ def test_prompt_pairs_together(order):
     for H, G, lens, max_k, want in ((16, 8, [2048] * 4, 2048, 2), (16, 8, [1024] * 8, 1024, 4), (16, 8, [1365, 1180, 1000] * 2, 1365, 3), (32, 8, [600, 2048], 2048, 1),
                                     (32, 8, [1100, 850, 600] * 2, 1100, 1), (16, 8, [1000] * 4, 3000, 1), (32, 8, [2048] * 4, 2048, 1)):
         assert order.pairs_together(wgs(lens, H, G), sum(lens), len(lens), max(lens), max_k) == want, (H, lens)
+
+
+def test_states_past_the_caches(order):
+    """From 92 MiB of single-token states on: portions behind them do not count (nor does 32-bit arithmetic)."""
+    assert [order.states_past(n, n, 0, 16, 128, 128) for n in (1, 91, 92, 4096)] == [0, 0, 1, 1]
+    assert [order.states_past(n, 0, 0, 16, 128, 128) for n in (91, 92)] == [0, 1]            # (not known to lead, but all of one token)
+    assert [order.states_past(200, lead, 1, 16, 128, 128) for lead in (0, 91, 92)] == [0, 0, 1]
+    assert order.states_past(65535, 65535, 0, 64, 256, 256)
