@@ -163,9 +163,20 @@ NV_HD int recurrence_singles(int num_seqs, int lead, bool rest) { return rest ? 
 // states all stay loses up to 28 % between 96 and 200 MB.  General and write as gated.  Only loads or only stores past the caches: 106 and 114 for 256.
 NV_HD bool recurrence_streams(int singles, int H, int D, int Dv) { return (int64_t)singles * H * D * Dv * 4 >= 92LL << 20; }
 
-// Outputs of the second product (fp32, a row a pair) past the caches: they drive the weights and rows that other column blocks read out of the L2, and
-// large ones are gone before the caller adds a token's rows up.  The call with that sum, through / past, us, top 4 of 32 experts, 2048, 1024: 8192 tokens
-// (268 MB) 538 / 527, 4096 316 / 313, 2048 (67 MB) 214 / 208;  top 2 of 16, 1024, 1024: 8000 (66 MB) 165.7 / 168.3.
-NV_HD bool moe_streams_out(int64_t pairs, int width) { return pairs * width * 4 >= 64LL << 20; }
+// Outputs of the second product (fp32, a row a pair) past the caches, where they and the experts' weights (three matrices of ff x width each) together do not
+// stay in the last cache (256 MB, beside rows and activations): they drive out what other blocks read, and themselves before the caller adds a token's
+// rows up.  The call with that sum, through / past, us, weights of one layer, of six layers in turn (MiB of outputs + weights; experts, top, width, ff):
+//   64 + 384 (32, 4, 2048, 1024)   215 / 208, 221 / 215        64 + 192 (16, 2, 2048, 1024)   190 / 190, 195 / 197
+//   256 + 384                      560 / 550, 541 / 527        128 + 192                      303 / 295, 310 / 300
+//   64 + 192 (32, 2, 2048, 512)    139 / 139, 142 / 144        128 + 192                      219 / 214, 226 / 221
+//   128 + 96 (16, 4, 2048, 512)    190 / 188, 193 / 197        256 + 96                       342 / 318, 339 / 321
+// and below the line:
+//   64 + 96 (16, 4, 2048, 512)     107 / 109, 120 / 121        93 + 96                        124 / 127, 133 / 135
+//   64 + 96 (16, 2, 1024, 1024)    168 / 170, 180 / 182        128 + 48 (16, 4, 1024, 512)    180 / 181, 181 / 186
+// Without the sum they pay from less on (64 + 192 of 32 experts, 115 / 95); outputs of less than 64 MiB made no difference to the call with it.
+NV_HD bool moe_streams_out(int64_t pairs, int width, int E, int ff) {
+    const int64_t out = pairs * width * 4, weights = (int64_t)E * ff * width * 6;
+    return out >= 64LL << 20 && out + weights >= 224LL << 20;
+}
 
 }  // namespace nv

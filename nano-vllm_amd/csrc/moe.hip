@@ -1008,7 +1008,7 @@ static void launch_grouped(const void* a, int64_t a_stride, const void* w, const
                        (T*)y, out, top, N, K, limit, alpha, up_shift)
             if (moe_few_blocks(pairs, E, n_cols) || !moe_offsets_ok(MODE == 0 ? kMoeBigRows : a_rows, a_stride, (MODE == 1 ? 2 : 1) * (int64_t)N, K))
                 NV_MOE_BIG(32, false);
-            else if (MODE == 0 && moe_streams_out(pairs, N))
+            else if (MODE == 0 && moe_streams_out(pairs, N, E, K))
                 NV_MOE_BIG(64, MODE == 0);
             else
                 NV_MOE_BIG(64, false);

@@ -62,9 +62,9 @@ def test_rows_far_apart():
 
 
 def test_outputs_past_the_caches():
-    """Outputs of 64 MiB and more pass by the caches: the rows of two calls of half the tokens, whose outputs do not, to the bit."""
-    T, E, top, W, ff = 2100, 16, 4, 2048, 64
-    assert T * top * W * 4 >= 64 << 20 > T // 2 * top * W * 4
+    """Outputs of 64 MiB and more pass by the caches beside 160 MiB of weights: the rows of two calls of half the tokens, whose outputs do not, to the bit."""
+    T, E, top, W, ff = 2100, 32, 4, 2048, 448
+    assert T * top * W * 4 >= 64 << 20 > T // 2 * top * W * 4 and T * top * W * 4 + 6 * E * ff * W >= 224 << 20
     g = torch.Generator(device="cuda").manual_seed(5)
     rn = lambda *s: torch.randn(*s, generator=g, device="cuda")
     h, logits = rn(T, W).to(torch.bfloat16), rn(T, E)

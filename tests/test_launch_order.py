@@ -46,6 +46,7 @@ extern "C" int scored_pairs(int64_t grid_base, int num_seqs, int64_t total_q, in
     return scoremod_pairs(grid_base, num_seqs, total_q, max_q, max_k);
 }
 extern "C" int streams(int tile_rows, int64_t pairs, int E, int ff) { return moe_streams(tile_rows, pairs, E, ff); }
+extern "C" int outputs_past(int64_t pairs, int width, int E, int ff) { return moe_streams_out(pairs, width, E, ff); }
 extern "C" int states_past(int num_seqs, int lead, int rest, int H, int D, int Dv) {
     return recurrence_streams(recurrence_singles(num_seqs, lead, rest != 0), H, D, Dv);
 }
@@ -198,3 +199,12 @@ def test_states_past_the_caches(order):
     assert [order.states_past(n, 0, 0, 16, 128, 128) for n in (91, 92)] == [0, 1]            # (not known to lead, but all of one token)
     assert [order.states_past(200, lead, 1, 16, 128, 128) for lead in (0, 91, 92)] == [0, 0, 1]
     assert order.states_past(65535, 65535, 0, 64, 256, 256)
+
+
+def test_expert_outputs_past_the_caches(order):
+    """From 64 MiB of outputs on, where they and the experts' weights come to 224 MiB; in 64 bits."""
+    past = lambda tokens, E, top, width, ff: order.outputs_past(C.c_int64(tokens * top), width, E, ff)
+    assert past(8192, 32, 4, 2048, 1024) and past(2048, 32, 4, 2048, 1024) and past(4096, 32, 2, 2048, 512) and not past(2047, 32, 4, 2048, 1024)
+    assert not past(8000, 16, 2, 1024, 1024) and not past(8192, 16, 2, 1024, 1024) and past(16384, 16, 2, 1024, 1024)
+    assert not past(3000, 16, 4, 2048, 512) and past(4096, 16, 4, 2048, 512) and not past(8192, 16, 4, 1024, 512)
+    assert past(1 << 20, 256, 8, 8192, 8192) and not past(1, 256, 8, 8192, 8192)
