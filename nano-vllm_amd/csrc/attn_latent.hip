@@ -436,9 +436,9 @@ __device__ __forceinline__ float lat_finish(float m, float l, const float* sink,
 // ------------------------------------------------------------------------------------------------ several tokens
 // Key tiles of a range: what the step has for every slot, not less than the launch has room for.  All row tiles get a whole range
 // first, longest first, and what is left of the long ones goes to the slots whose row tile was short: 16 heads, 256 columns, 1024 rows
-// of each of 2 sequences of 3000 and 6001 keys take 63 tiles the longest way, where ranges of half the longest sequence take 94: with the order
-// of the workgroups 220 -> 164 us a call; 500 rows of each of 4 sequences of 1000 .. 3000 keys 138 -> 106, 16 prompts of 200 .. 512 tokens
-// 67 -> 53 (device times, 256 columns; rows of one range write no state).
+// of each of 2 sequences of 3000 and 6001 keys take 63 tiles the longest way, where ranges of half the longest sequence take 94:
+// 152 -> 137 us a call; 500 rows of each of 4 sequences of 1000 .. 3000 keys 87 -> 82; with the order of the workgroups alone 16 prompts of 200 .. 512 tokens
+// 56 -> 43 (device times, 256 columns; rows of one range write no state).
 template <int KT>
 __device__ __forceinline__ int lat_share(const LatentParams& p, int lane) {
     int64_t total = 0;

@@ -69,7 +69,8 @@ __global__ __launch_bounds__(256, !LONG ? 2 : D32 + V32 == 4 ? (MOD == kSrGenera
     // the pairs turn by one every time.  Where all workgroups are there from the start, 32 (one for each CU) go there and the next 32
     // back instead, so that a CU that has a heavy one gets a light one with it (one heavy after the other is better where
     // CUs that have ended take the next).  Pairs of very different lengths are no order of weight that way and go one after the other:
-    // 16 / 4 heads of 64, 16 chunks of 300 rows on 600 .. 4000 keys 121 us, together 145, 6 prompts of 300 .. 1300 50 and 57, 6 of 466 .. 862 50 and 37.
+    // 16 / 4 heads of 64, the launch alone, 16 chunks of 300 rows on 600 .. 4000 keys 106 us, together 133, 6 prompts of 300 .. 1300 36 and 44, 6 of 466 .. 862
+    // 36 and 23.
     const int split = blockIdx.x / p.grid_base, bid = blockIdx.x - split * p.grid_base;
     const PairGroup group = scoremod_group(bid, p.sets, p.slots_per_pair, p.xs_shift);
     bool even = p.even > 0;

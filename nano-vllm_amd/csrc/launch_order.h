@@ -16,14 +16,17 @@ NV_HD int latent_share(int64_t total_tiles, int slots, int fewest) {
     return (int)(share < fewest ? fewest : share > most ? most : share);
 }
 // Chunks behind at least three quarters of the longest sequence: all row tiles are about as long, so equal ranges of each, as the host plans them, are
-// even already, and a share for every slot leaves whole row tiles over for a second round.  Share / equal ranges, 16 heads: 7 chunks of 290 rows
-// on 2966 .. 3257 keys, rows of 256, 199 / 181 us (174 where every row tile has all ranges), 9 of 161 on 3708 .. 3828, rows of 160, 100.2 / 99.6 (94.0).
-// With less in front: 8 of 256 on 3053 .. 4036, rows of 256, 147 / 166.
+// even already, and a share for every slot may leave whole row tiles over for a second round.  Share / equal ranges, us, 16 heads: rows of 256, 7 chunks of 290
+// rows on 2966 .. 3257 keys 156 / 152, 6 of 183 on 5003 .. 5427 141 / 124, 5 of 194 on 6422 .. 7383 126 / 131;  rows of 320, 8 of 136 on 2808 .. 3466
+// 177 / 159;  rows of 160, 9 of 161 on 3708 .. 3828 89 / 91.  With less in front: rows of 256, 8 of 256 on 3053 .. 4036 125 / 144.  The line dates
+// from a slower loop over the tiles: of 40 such launches now, those of few row tiles were mostly faster with a share (3 chunks of 25 rows on 6717 .. 7748,
+// rows of 320, 54 / 82), larger ones about even; 1.08 times as fast over all.
 NV_HD bool latent_alike(int least_in_front, int longest) { return (int64_t)least_in_front * 4 >= (int64_t)longest * 3; }
 // Launches of more than one round without key ranges: whether the order of workgroups is turned.  Their sequences come in turn, so each of 2, 4, 8 ..
 // keeps to some of the XCDs and shader engines, and those of the longest are what the launch waits for; any other number, and sequences
-// of about the same length, spread by themselves.  Rows of 320, us, as they come / turned: 4 prompts of 446 .. 931 101 / 78, 4 chunks of 456 rows on 865
-// 105 / 77, 13 prompts of 103 .. 164 28 / 35, 9 of 616 .. 805 144 / 158;  256: 8 of 318 .. 670 61 / 49, 8 of 1000 .. 1024 106 / 109, 7 of 309 .. 542 35 / 40.
+// of about the same length, spread by themselves.  16 heads, us, as they come / turned: rows of 320, 4 prompts of 446 .. 931 70.6 / 53.9,
+// 13 of 103 .. 164 20.7 / 26.1, 9 of 616 .. 805 110 / 116;  256: 2 of 1000 .. 2048 62.6 / 54.9, 8 of 318 .. 670 46.1 / 33.4, 16 of 200 .. 500 55.6 / 42.8,
+// 8 of 1000 .. 1024 83.1 / 86.2, 7 of 309 .. 542 25.9 / 28.1;  160: 4 of 1000 .. 2048 69.5 / 60.8;  96: 8 of 600 .. 1024 30.1 / 28.7.
 NV_HD bool latent_turns(int num_seqs, int64_t total_q, int max_q, int max_k) {
     return num_seqs > 1 && (num_seqs & (num_seqs - 1)) == 0 && (max_q != max_k || total_q * 9 < (int64_t)num_seqs * max_q * 8);
 }
@@ -78,9 +81,10 @@ NV_HD RoundPlace prefill_order(int slot, int slots_per_pair, const PairSets& set
 
 // Score-modified attention, prompt portions: workgroup (of a key range) -> its pair of sequence and kv head and its place in the pair, heaviest query
 // tile first.  Workgroups go to the eight XCDs in turn; an XCD has `rounds` pairs (8 >> xs_shift of them a round over all XCDs) in sets of three to
-// five: what four at a time leave over begins with its heaviest tile when the others end.  One after the other / fours and the rest last /
-// so: 3 prompts of 1893 .. 2197, 16 heads of 128 each, 127 / 138 / 117 us, 12 of 444 .. 676, 16 / 4 of 64, 43.6 / 47.0 / 41.8; 70
-// launches of a number of pairs that fours do not divide 1 / 0.991 / 0.975 on average, 1.05 at most (1.08 with the rest last).
+// five: what four at a time leave over begins with its heaviest tile when the others end.  One after the other /
+// so, the launch alone: 3 prompts of 1893 .. 2197, 16 heads of 128 each, 97 / 86 us, 12 of 444 .. 676, 16 / 4 of 64, 29.8 / 28.3.  With an earlier loop
+// over the tiles, 70 launches of a number of pairs that fours do not divide, one after the other / fours and the rest last / so: 1 / 0.991 / 0.975 on
+// average, 1.05 at most (1.08 with the rest last).
 // grid: 8 * rounds * slots_per_pair; places past a pair's workgroups and pairs past the last one are for the caller to leave out.
 NV_HD PairSets scoremod_sets(int rounds) { return pair_sets(rounds, rounds < 6 ? 1 : (rounds + 2) / 4); }
 struct PairGroup {
@@ -101,7 +105,7 @@ NV_HD bool scoremod_even(int64_t keys, int64_t longest, int n, int whole_prompts
 }
 // What a launch knows of that: 1 and 0, or -1 where a group of chunks is to look at its own lengths.  Chunks of no more workgroups of a key range than CUs
 // do not look, which takes half a microsecond of 13 to 21, and go one after the other: with several key ranges the order is not without
-// effect there, 5 of 230 rows on 2194 .. 3955 keys, 16 / 8 heads of 128, 83 us so and 96 together, 2 of 431 on 3229 .. 4093 73 and 84; 80 such
+// effect there, 5 of 230 rows on 2194 .. 3955 keys, 16 / 8 heads of 128, 73 us so and 91 together, 2 of 431 on 3229 .. 4093 64 and 75; with an earlier loop 80 such
 // steps, from 0.90 to 1.14 of the time and 1.005 on average together, 0.997 looking first (7 of them 2 to 4 % slower for it).
 NV_HD int scoremod_pairs(int64_t grid_base, int num_seqs, int64_t total_q, int max_q, int max_k) {
     if (max_q == max_k) return scoremod_even(total_q, max_q, num_seqs, 1);
