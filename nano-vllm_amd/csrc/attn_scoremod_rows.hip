@@ -13,10 +13,10 @@
 // maximum: 0.0028 and 119 us; the same with probabilities as the sum of two bf16 numbers: 0.0022 and 148 us.
 //
 // What bounds it: the instructions of the scores.  64 soft-capped scores are nine vector instructions and three at quarter rate (two exponentials, a
-// reciprocal) for a row beside 32 cycles of matrix products.  So, in launches of several tiles, tiles come by loads that the compiler does not know (it would
-// wait for the next tile in front of the first transposed read), and with rows of 128 columns, two waves a SIMD, the weights of a tile are made beside the
-// scores of the next one, which are capped beside the values of this one.  With rows of 64 columns more waves take turns, and the registers of the next scores
-// would cost one or two of them: 8 prompts of 1024, 16 / 4 heads of 64, 51 us, so with two waves 56.
+// reciprocal) for a row beside 32 cycles of matrix products, which are 34 % of the busy cycles of the call below.  So, in launches
+// of several tiles, tiles come by loads that the compiler does not know (it would wait for the next tile in front of the first transposed read), and with
+// rows of 128 columns, two waves a SIMD, the weights of a tile are made beside the scores of the next one, which are capped beside the values of this one.
+// With rows of 64 columns more waves take turns, and the registers of the next scores would cost one or two of them: 8 prompts of 1024, 16 / 4 heads of 64, 51 us, so with two waves 56.
 // 4 prompts of 1777 .. 2048 tokens, 16 / 8 heads of 128, soft cap and sink, the call with its preparation of 21 us: 112 us on a card where a tile's work one
 // after the other takes 114; 3 prompts of 700 .. 1900 71 and 75, 2 portions of 1000 on 3000 .. 4000 117 and 121.  On another card 117 for that order, 127 with an
 // XCD's pairs one after the other (see there) and 129 with the denominator as a product of rounded weights with ones; with the launch on 16 x 16
