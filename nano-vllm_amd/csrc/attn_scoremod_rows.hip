@@ -465,16 +465,17 @@ __global__ __launch_bounds__(256, !LONG ? 2 : D32 + V32 == 4 ? (MOD == kSrGenera
                                                  (__attribute__((address_space(3))) void*)(lds + AT + KB + (wave + 4 * i) * 1024), 16, 0, 0);
             }
         };
+        auto entry_of = [&](int t) { return bt[min(t / tpb, p.max_blocks - 1)]; };
         int entry = 0;                                    // block-table entry of the tile staged next, fetched a tile ahead
-        if (t_begin < nt) stage(std::integral_constant<int, 0>{}, t_begin, bt[t_begin / tpb]);
-        if (t_begin + 1 < nt) entry = bt[(t_begin + 1) / tpb];
+        if (t_begin < nt) stage(std::integral_constant<int, 0>{}, t_begin, entry_of(t_begin));
+        if (t_begin + 1 < nt) entry = entry_of(t_begin + 1);
 
         auto tile_step = [&](auto buf_tag, int t) {
             constexpr int B = decltype(buf_tag)::value;
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this tile has landed, and everybody is done with the other buffer
             __syncthreads();
             const int use = entry;
-            if (t + 2 < nt) entry = bt[(t + 2) / tpb];
+            if (t + 2 < nt) entry = entry_of(t + 2);
             if (t + 1 < nt) stage(std::integral_constant<int, 1 - B>{}, t + 1, use);
             const unsigned char* ldsK = lds + B * BUF;
             const unsigned char* ldsV = ldsK + KB;
